@@ -50,7 +50,9 @@ EXTRA_FLAGS = {
     # the resident-tile 1x1 kernel's leading scalar arguments: preloaded as well
     "ehip_gemm1x1.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=16"],
     # the Winograd kernel whose requantized values take the accumulators' place in the vector registers
-    "ehip_wino_lanes.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    "ehip_wino_lanes.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1", "-mllvm", "-amdgpu-kernarg-preload-count=16"],
+    "ehip_wino.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=16"],
+    "ehip_fewch.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=16"],
     "ehip_gemm1x1w.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=16", "-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     # and those of the 1x1 kernels with few input channels
     "ehip_gemm.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=16"],

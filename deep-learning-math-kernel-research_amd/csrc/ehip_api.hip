@@ -28,6 +28,8 @@ void set_error(const std::string &msg) { g_last_error = msg; }
     }                                                                                              \
   } while (0)
 
+constexpr int kMaxPlans = 3;
+
 struct ehip_conv {
   ehip_conv_desc_t d;
   int family = 0;
@@ -56,22 +58,17 @@ struct ehip_conv {
   int T = 1, Tr = 1, wtb = 1;
   // Winograd
   int ht = 0, wt = 0, nt = 0, t = 0, wino_tile = 6;
-  int chunk_n = 0;   // images per pass of the three-stage pipeline (intermediates sized for it)
   bool fused = true; // GEMM and output transform in one kernel (no f32 GEMM result in memory)
   uint8_t *tin = nullptr;
   bool tin_blocked = false;   // Winograd, fused schedule: tin as [t / 32][36][ic2][32][16]
   float *tout = nullptr;
   size_t tin_bytes = 0, tout_bytes = 0;
 
-  // launch plans of the steady state (filled by the first execute, see LaunchPlan); the Winograd ones are
-  // used only when the layer runs in one pass (no chunking)
-  int stage_mask = 7;   // Winograd: which stages execute() launches (ehip_conv_execute_stages)
-  LaunchPlan<GemmArgs> plan_gemm;
-  LaunchPlan<Conv3x3Args> plan_3x3;
-  LaunchPlan<FewChArgs> plan_fewch;
-  LaunchPlan<DepthwiseArgs> plan_dw;
-  LaunchPlan<WinoArgs> plan_wino_in, plan_wino_out;
-  LaunchPlan<WinoFusedArgs> plan_wino_fused;
+  // what an execute launches, in order, and the stage bit (ehip_conv_execute_stages) each launch belongs to
+  LaunchPlan plan[kMaxPlans];
+  int plan_stage[kMaxPlans] = {7, 7, 7};
+  int nplans = 0;
+  void *args_dev = nullptr;   // [kMaxPlans][kArgBlock]
 };
 
 namespace {
@@ -88,7 +85,7 @@ void free_all(ehip_conv *c)
 {
   // (scale, shift and comp are one allocation: see setup_workspace)
   void *ptrs[] = {c->wpacked, c->scale, c->absmax, c->wsum, c->tin, c->tout,
-                  c->cls_h, c->cls_w, c->rects, c->shift_tab};
+                  c->cls_h, c->cls_w, c->rects, c->shift_tab, c->args_dev};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
 }
@@ -395,9 +392,8 @@ int setup_workspace(ehip_conv *c)
     c->nt = c->ht * c->wt;
     // One pass over the whole batch.  (Running the stages over a few images at a time, with the intermediates
     // sized for one pass, was measured on MI355X and only costs: the 256 MB memory-side cache does not keep the
-    // intermediates away from HBM.  The pass loop of execute stays: chunk_n images per pass.)
-    c->chunk_n = d.n;
-    c->t = c->nt * c->chunk_n;   // tiles per pass
+    // intermediates away from HBM.)
+    c->t = c->nt * d.n;
     if ((long long)c->t >= (1ll << 31) / 64) return fail(EHIP_UNIMPLEMENTED, "winograd: too many tiles");
     c->variant = gemm_pick_variant(c->t, c->oc2, c->ic2, c->nbatch, 1);
     c->units_pad = up(c->ic2, gemm_variant_chunk(c->variant));
@@ -445,6 +441,8 @@ int setup_workspace(ehip_conv *c)
   c->comp = reinterpret_cast<int *>(c->scale + 2 * c->per_oc);
   if ((rc = dev_alloc(&c->absmax, c->per_oc, true)) != EHIP_OK) return rc;
   if ((rc = dev_alloc(&c->wsum, c->per_oc, true)) != EHIP_OK) return rc;
+  if ((rc = dev_alloc(reinterpret_cast<uint8_t **>(&c->args_dev), kMaxPlans * kArgBlock, false)) != EHIP_OK) return rc;
+  for (int i = 0; i < kMaxPlans; ++i) c->plan[i].args_dev = static_cast<uint8_t *>(c->args_dev) + i * kArgBlock;
   if (c->nclass > 1 && (rc = dev_alloc(&c->shift_tab, (size_t)c->nclass * c->ocpp, true)) != EHIP_OK) return rc;
   return EHIP_OK;
 }
@@ -534,6 +532,160 @@ EHIP_API int ehip_conv_destroy(ehip_conv_t *c)
 
 EHIP_API const char *ehip_conv_kernel_name(ehip_conv_t *c) { return c ? c->kernel_name.c_str() : ""; }
 
+// Development aid: a build with -DEHIP_TRACE takes the address of a device buffer for the kernels' clock
+// stamps from the environment; the product build passes null and never looks.
+static long long *trace_buffer()
+{
+#ifdef EHIP_TRACE
+  const char *env = getenv("EHIP_TRACE_PTR");
+  return reinterpret_cast<long long *>(env ? strtoull(env, nullptr, 0) : 0ull);
+#else
+  return nullptr;
+#endif
+}
+
+// What an execute will launch: everything but the tensors (LaunchPlan), with the argument structures written to the
+// handle's device memory on stream s, like the packed weights.
+static int plan_execute(ehip_conv *c, hipStream_t s)
+{
+  const ehip_conv_desc_t &d = c->d;
+  LaunchPlan *p = &c->plan[0];
+  switch (c->family) {
+  case FAM_GEMM_1X1: {
+    GemmArgs a;
+    memset(&a, 0, sizeof(a));
+    a.w = c->wpacked;
+    a.ep = make_epilogue(c, d.output_type, d.with_ip_sum && d.algorithm == EHIP_CONV_DIRECT_1X1, d.with_relu);
+    a.p_total = d.n * d.oh * d.ow;
+    a.ohw = d.oh * d.ow; a.ow = d.ow;
+    a.ohw_magic = div_magic(a.ohw); a.ow_magic = div_magic(a.ow);
+    a.ihw = d.ih * d.iw; a.iw = d.iw;
+    a.stride_h = d.stride_h; a.stride_w = d.stride_w;
+    a.ic2 = c->ic2; a.units_pad = c->units_pad; a.oc2 = c->oc2; a.ocpp = c->ocpp;
+    a.in_nhwc = d.input_fmt == EHIP_NHWC; a.out_nhwc = d.output_fmt == EHIP_NHWC;
+    a.kh = d.kh; a.kw = d.kw; a.pad_t = d.pad_t; a.pad_l = d.pad_l; a.ih = d.ih;
+    if (c->nclass > 1) {
+      a.ep.shift_tab = c->shift_tab; a.ep.tab_stride = c->ocpp;
+      a.cls_h = c->cls_h; a.cls_w = c->cls_w; a.ncls_w = c->ncls_w;
+    }
+    a.trace = trace_buffer();
+    HIP_TRY(plan_gemm(*p, a, 1, c->variant, s));
+    if (p->name) c->kernel_name = p->name;   // the choice depends on the epilogue
+    break;
+  }
+  case FAM_CONV_FEWCH: {
+    FewChArgs a;
+    memset(&a, 0, sizeof(a));
+    a.w = c->wpacked;
+    a.ep = make_epilogue(c, d.output_type, false, d.with_relu);
+    a.n = d.n; a.ih = d.ih; a.iw = d.iw; a.oh = d.oh; a.ow = d.ow; a.ic = d.ic; a.kh = d.kh; a.kw = d.kw;
+    a.stride_h = d.stride_h; a.stride_w = d.stride_w; a.pad_t = d.pad_t; a.pad_l = d.pad_l;
+    a.oc2 = c->oc2; a.ocpp = c->ocpp; a.icl = c->icl;
+    a.in_nhwc = d.input_fmt == EHIP_NHWC; a.out_nhwc = d.output_fmt == EHIP_NHWC;
+    if (c->nclass > 1) {
+      a.ep.shift_tab = c->shift_tab; a.ep.tab_stride = c->ocpp;
+      a.cls_h = c->cls_h; a.cls_w = c->cls_w; a.ncls_w = c->ncls_w; a.nclass = c->nclass;
+    }
+    HIP_TRY(plan_conv_fewch(*p, a, s));
+    c->kernel_name = p->name;
+    break;
+  }
+  case FAM_CONV_3X3: {
+    Conv3x3Args a;
+    memset(&a, 0, sizeof(a));
+    a.w = c->wpacked;
+    a.ep = make_epilogue(c, d.output_type, false, d.with_relu);
+    a.ih = d.ih; a.iw = d.iw; a.oh = d.oh; a.ow = d.ow;
+    a.pad_t = d.pad_t; a.pad_l = d.pad_l;
+    a.ic2 = c->ic2; a.units_pad = c->units_pad; a.oc2 = c->oc2; a.ocpp = c->ocpp;
+    a.chunk_units = c->chunk_units;
+    a.vw = d.stride_h == 2 ? d.ow + 1 : d.ow + 2;
+    a.vw_magic = div_magic(a.vw);
+    a.trace = trace_buffer();
+    HIP_TRY(plan_conv3x3v(*p, a, d.n, c->variant, s));
+    break;
+  }
+  case FAM_DEPTHWISE: {
+    DepthwiseArgs a;
+    memset(&a, 0, sizeof(a));
+    a.w = c->wpacked;
+    a.scale = c->scale; a.shift = c->shift; a.wsum = c->wsum;
+    a.wdiag = reinterpret_cast<const uint4 *>(c->wpacked + (size_t)c->oc2 * 192);
+    a.n = d.n; a.g2 = c->oc2; a.ih = d.ih; a.iw = d.iw; a.oh = d.oh; a.ow = d.ow;
+    a.stride = d.stride_h;
+    a.pad_t = d.pad_t; a.pad_l = d.pad_l;
+    a.T = c->T; a.Tr = c->Tr; a.wt = c->wtb;
+    a.out_type = d.output_type; a.with_relu = d.with_relu;
+    a.lo = d.relu_lower; a.hi = d.relu_upper;
+    HIP_TRY(plan_depthwise(*p, a, s));
+    break;
+  }
+  case FAM_WINOGRAD: {
+    WinoArgs w = make_wino_args(d, c->ic2, c->oc2);
+    w.tin = c->tin;
+    w.tin_blocked = c->tin_blocked;
+    w.tout = c->tout;
+    // mrepS = input_S * (1 / tinput_S), z = ceil(tinput_z)
+    // (src/elx_conv_wino_trans_input.cpp:617-618, src/elx_int8_conv_wino.cpp:270-276)
+    const float tin_repS = 1.0f / d.tinput_scale;
+    w.mrepS = d.input_scale * tin_repS;
+    w.mz = ceilf(d.tinput_z);
+    HIP_TRY(plan_wino_trans_input(c->plan[0], w, s));
+    c->plan_stage[0] = 1;
+    c->plan_stage[1] = 2;
+    if (c->fused) {
+      WinoFusedArgs f;
+      memset(&f, 0, sizeof(f));
+      f.tin = c->tin; f.tin_blocked = c->tin_blocked; f.w = c->wpacked;
+      f.scale = c->scale; f.shift = c->shift; f.comp = c->comp;
+      f.n = w.n; f.ic2 = c->ic2; f.units_pad = c->units_pad; f.oc2 = c->oc2; f.ocpp = c->ocpp;
+      f.oh = d.oh; f.ow = d.ow; f.ht = w.ht; f.wt = w.wt; f.nt = w.nt; f.t = w.t;
+      f.with_bias = d.with_bias; f.with_relu = d.with_relu; f.with_sum = d.with_ip_sum; f.tile = d.tile_size;
+      f.out_type = w.out_type; f.out_repS = w.out_repS; f.out_z = w.out_z;
+      f.out_nhwc = w.out_nhwc;
+      f.tpart = c->tout_bytes > 16 ? reinterpret_cast<float4 *>(c->tout) : nullptr;
+      f.trace = trace_buffer();
+      HIP_TRY(plan_wino_gemm_output(c->plan[1], f, s));
+      if (c->plan[1].name) c->kernel_name = std::string("k_wino_trans_input_u8 + ") + c->plan[1].name;
+      c->nplans = 2;
+      return EHIP_OK;
+    }
+    GemmArgs a;
+    memset(&a, 0, sizeof(a));
+    a.in = c->tin;
+    a.w = c->wpacked;
+    a.out = c->tout;
+    a.ep = make_epilogue(c, EHIP_F32, false, false);
+    a.p_total = w.t;
+    a.ohw = w.t; a.ow = w.t; a.ihw = w.t; a.iw = w.t;
+    a.ohw_magic = div_magic(a.ohw); a.ow_magic = div_magic(a.ow);
+    a.stride_h = 1; a.stride_w = 1;
+    a.ic2 = c->ic2; a.units_pad = c->units_pad; a.oc2 = c->oc2; a.ocpp = c->ocpp;
+    a.in_batch_stride = (long long)c->ic2 * w.t * 16;
+    a.out_batch_stride = (long long)c->oc2 * w.t * 16;
+    HIP_TRY(plan_gemm(c->plan[1], a, c->nbatch, c->variant, s));
+    HIP_TRY(plan_wino_trans_output(c->plan[2], w, s));
+    c->plan_stage[2] = 4;
+    c->nplans = 3;
+    return EHIP_OK;
+  }
+  default:
+    return fail(EHIP_GENERAL_ERROR, "internal: no executor");
+  }
+  c->nplans = 1;
+  return EHIP_OK;
+}
+
+static int run_plans(const ehip_conv *c, void *out, const void *in, const void *bias, int stages, hipStream_t s)
+{
+  if (c->family == FAM_CONV_FEWCH && c->d.input_fmt == EHIP_NHWC && (reinterpret_cast<uintptr_t>(in) & 3))
+    return fail(EHIP_GENERAL_ERROR, "nhwc input of a few-channel layer must be 4-byte aligned");
+  if (c->family == FAM_WINOGRAD && c->d.with_bias && !bias) return fail(EHIP_GENERAL_ERROR, "Parameter error. Invalid input data!");
+  for (int i = 0; i < c->nplans; ++i)
+    if (c->plan_stage[i] & stages) HIP_TRY(plan_launch(c->plan[i], in, out, bias, s));
+  return EHIP_OK;
+}
+
 EHIP_API int ehip_conv_prepare(ehip_conv_t *c, const void *weights_dev, const void *bias_dev, void *hip_stream)
 {
   if (!c || !weights_dev) return fail(EHIP_GENERAL_ERROR, "Parameter error. Invalid input data!");
@@ -579,20 +731,9 @@ EHIP_API int ehip_conv_prepare(ehip_conv_t *c, const void *weights_dev, const vo
   default:
     return fail(EHIP_GENERAL_ERROR, "internal: no executor");
   }
-  c->prepared = true;
-  return EHIP_OK;
-}
-
-// Development aid: a build with -DEHIP_TRACE takes the address of a device buffer for the kernels' clock
-// stamps from the environment; the product build passes null and never looks.
-static long long *trace_buffer()
-{
-#ifdef EHIP_TRACE
-  const char *env = getenv("EHIP_TRACE_PTR");
-  return reinterpret_cast<long long *>(env ? strtoull(env, nullptr, 0) : 0ull);
-#else
-  return nullptr;
-#endif
+  const int rc = plan_execute(c, s);
+  c->prepared = rc == EHIP_OK;
+  return rc;
 }
 
 EHIP_API int ehip_conv_execute(ehip_conv_t *c, void *output_dev, const void *input_dev, const void *weights_dev,
@@ -603,149 +744,7 @@ EHIP_API int ehip_conv_execute(ehip_conv_t *c, void *output_dev, const void *inp
     int rc = ehip_conv_prepare(c, weights_dev, bias_dev, hip_stream);
     if (rc != EHIP_OK) return rc;
   }
-  hipStream_t s = static_cast<hipStream_t>(hip_stream);
-  const ehip_conv_desc_t &d = c->d;
-  switch (c->family) {
-  case FAM_GEMM_1X1: {
-    GemmArgs a;
-    memset(&a, 0, sizeof(a));
-    a.in = static_cast<const uint8_t *>(input_dev);
-    a.w = c->wpacked;
-    a.out = output_dev;
-    a.ep = make_epilogue(c, d.output_type, d.with_ip_sum && d.algorithm == EHIP_CONV_DIRECT_1X1, d.with_relu);
-    a.p_total = d.n * d.oh * d.ow;
-    a.ohw = d.oh * d.ow; a.ow = d.ow;
-    a.ohw_magic = div_magic(a.ohw); a.ow_magic = div_magic(a.ow);
-    a.ihw = d.ih * d.iw; a.iw = d.iw;
-    a.stride_h = d.stride_h; a.stride_w = d.stride_w;
-    a.ic2 = c->ic2; a.units_pad = c->units_pad; a.oc2 = c->oc2; a.ocpp = c->ocpp;
-    a.in_nhwc = d.input_fmt == EHIP_NHWC; a.out_nhwc = d.output_fmt == EHIP_NHWC;
-    a.kh = d.kh; a.kw = d.kw; a.pad_t = d.pad_t; a.pad_l = d.pad_l; a.ih = d.ih;
-    if (c->nclass > 1) {
-      a.ep.shift_tab = c->shift_tab; a.ep.tab_stride = c->ocpp;
-      a.cls_h = c->cls_h; a.cls_w = c->cls_w; a.ncls_w = c->ncls_w;
-    }
-    a.trace = trace_buffer();
-    HIP_TRY(launch_gemm(a, 1, c->variant, s, &c->plan_gemm));
-    if (c->plan_gemm.name) c->kernel_name = c->plan_gemm.name;   // the launcher's choice depends on the epilogue
-    break;
-  }
-  case FAM_CONV_FEWCH: {
-    FewChArgs a;
-    memset(&a, 0, sizeof(a));
-    a.in = static_cast<const uint8_t *>(input_dev);
-    a.w = c->wpacked;
-    a.out = output_dev;
-    a.ep = make_epilogue(c, d.output_type, false, d.with_relu);
-    a.n = d.n; a.ih = d.ih; a.iw = d.iw; a.oh = d.oh; a.ow = d.ow; a.ic = d.ic; a.kh = d.kh; a.kw = d.kw;
-    a.stride_h = d.stride_h; a.stride_w = d.stride_w; a.pad_t = d.pad_t; a.pad_l = d.pad_l;
-    a.oc2 = c->oc2; a.ocpp = c->ocpp; a.icl = c->icl;
-    a.in_nhwc = d.input_fmt == EHIP_NHWC; a.out_nhwc = d.output_fmt == EHIP_NHWC;
-    if (c->nclass > 1) {
-      a.ep.shift_tab = c->shift_tab; a.ep.tab_stride = c->ocpp;
-      a.cls_h = c->cls_h; a.cls_w = c->cls_w; a.ncls_w = c->ncls_w; a.nclass = c->nclass;
-    }
-    if (a.in_nhwc && (reinterpret_cast<uintptr_t>(input_dev) & 3))
-      return fail(EHIP_GENERAL_ERROR, "nhwc input of a few-channel layer must be 4-byte aligned");
-    HIP_TRY(launch_conv_fewch(a, s, &c->plan_fewch));
-    if (c->plan_fewch.name) c->kernel_name = c->plan_fewch.name;
-    break;
-  }
-  case FAM_CONV_3X3: {
-    Conv3x3Args a;
-    memset(&a, 0, sizeof(a));
-    a.in = static_cast<const uint8_t *>(input_dev);
-    a.w = c->wpacked;
-    a.out = output_dev;
-    a.ep = make_epilogue(c, d.output_type, false, d.with_relu);
-    a.ih = d.ih; a.iw = d.iw; a.oh = d.oh; a.ow = d.ow;
-    a.pad_t = d.pad_t; a.pad_l = d.pad_l;
-    a.ic2 = c->ic2; a.units_pad = c->units_pad; a.oc2 = c->oc2; a.ocpp = c->ocpp;
-    a.chunk_units = c->chunk_units;
-    a.vw = d.stride_h == 2 ? d.ow + 1 : d.ow + 2;
-    a.vw_magic = div_magic(a.vw);
-    a.trace = trace_buffer();
-    HIP_TRY(launch_conv3x3v(a, d.n, c->variant, s, &c->plan_3x3));
-    break;
-  }
-  case FAM_DEPTHWISE: {
-    DepthwiseArgs a;
-    memset(&a, 0, sizeof(a));
-    a.in = static_cast<const uint8_t *>(input_dev);
-    a.w = c->wpacked;
-    a.out = output_dev;
-    a.scale = c->scale; a.shift = c->shift; a.wsum = c->wsum;
-    a.wdiag = reinterpret_cast<const uint4 *>(c->wpacked + (size_t)c->oc2 * 192);
-    a.n = d.n; a.g2 = c->oc2; a.ih = d.ih; a.iw = d.iw; a.oh = d.oh; a.ow = d.ow;
-    a.stride = d.stride_h;
-    a.pad_t = d.pad_t; a.pad_l = d.pad_l;
-    a.T = c->T; a.Tr = c->Tr; a.wt = c->wtb;
-    a.out_type = d.output_type; a.with_relu = d.with_relu;
-    a.lo = d.relu_lower; a.hi = d.relu_upper;
-    HIP_TRY(launch_depthwise(a, s, &c->plan_dw));
-    break;
-  }
-  case FAM_WINOGRAD: {
-    if (d.with_bias && !bias_dev) return fail(EHIP_GENERAL_ERROR, "Parameter error. Invalid input data!");
-    const bool one_pass = c->chunk_n >= d.n;   // the launch plans hold ONE pass's arguments
-    for (int n0 = 0; n0 < d.n; n0 += c->chunk_n) {
-      ehip_conv_desc_t dc = d;
-      dc.n = d.n - n0 < c->chunk_n ? d.n - n0 : c->chunk_n;
-      WinoArgs w = make_wino_args(dc, c->ic2, c->oc2);
-      const size_t in_esz = d.input_type == EHIP_U8 ? 1 : 4, out_esz = d.output_type == EHIP_F32 ? 4 : 1;
-      w.in = static_cast<const uint8_t *>(input_dev) + (size_t)n0 * c->ic2 * d.ih * d.iw * 16 * in_esz;
-      w.tin = c->tin;
-      w.tin_blocked = c->tin_blocked;
-      w.tout = c->tout;
-      w.out = static_cast<uint8_t *>(output_dev) + (size_t)n0 * c->oc2 * d.oh * d.ow * 16 * out_esz;
-      w.bias = static_cast<const float *>(bias_dev);
-      // mrepS = input_S * (1 / tinput_S), z = ceil(tinput_z)
-      // (src/elx_conv_wino_trans_input.cpp:617-618, src/elx_int8_conv_wino.cpp:270-276)
-      const float tin_repS = 1.0f / d.tinput_scale;
-      w.mrepS = d.input_scale * tin_repS;
-      w.mz = ceilf(d.tinput_z);
-      if (c->stage_mask & 1) HIP_TRY(launch_wino_trans_input(w, s, one_pass ? &c->plan_wino_in : nullptr));
-      if (c->fused) {
-        if (!(c->stage_mask & 2)) continue;
-        WinoFusedArgs f;
-        memset(&f, 0, sizeof(f));
-        f.tin = c->tin; f.tin_blocked = c->tin_blocked; f.w = c->wpacked; f.out = w.out; f.bias = w.bias;
-        f.scale = c->scale; f.shift = c->shift; f.comp = c->comp;
-        f.n = w.n; f.ic2 = c->ic2; f.units_pad = c->units_pad; f.oc2 = c->oc2; f.ocpp = c->ocpp;
-        f.oh = d.oh; f.ow = d.ow; f.ht = w.ht; f.wt = w.wt; f.nt = w.nt; f.t = w.t;
-        f.with_bias = d.with_bias; f.with_relu = d.with_relu; f.with_sum = d.with_ip_sum; f.tile = d.tile_size;
-        f.out_type = w.out_type; f.out_repS = w.out_repS; f.out_z = w.out_z;
-        f.out_nhwc = w.out_nhwc;
-        f.tpart = c->tout_bytes > 16 ? reinterpret_cast<float4 *>(c->tout) : nullptr;
-        f.trace = trace_buffer();
-        HIP_TRY(launch_wino_gemm_output(f, s, one_pass ? &c->plan_wino_fused : nullptr));
-        // (which form of the fused stage runs is the launcher's choice: known from the first execute on)
-        if (c->plan_wino_fused.name && c->kernel_name.find(c->plan_wino_fused.name) == std::string::npos)
-          c->kernel_name = std::string("k_wino_trans_input_u8 + ") + c->plan_wino_fused.name;
-        continue;
-      }
-      GemmArgs a;
-      memset(&a, 0, sizeof(a));
-      a.in = c->tin;
-      a.w = c->wpacked;
-      a.out = c->tout;
-      a.ep = make_epilogue(c, EHIP_F32, false, false);
-      a.p_total = w.t;
-      a.ohw = w.t; a.ow = w.t; a.ihw = w.t; a.iw = w.t;
-      a.ohw_magic = div_magic(a.ohw); a.ow_magic = div_magic(a.ow);
-      a.stride_h = 1; a.stride_w = 1;
-      a.ic2 = c->ic2; a.units_pad = c->units_pad; a.oc2 = c->oc2; a.ocpp = c->ocpp;
-      a.in_batch_stride = (long long)c->ic2 * w.t * 16;
-      a.out_batch_stride = (long long)c->oc2 * w.t * 16;
-      if (c->stage_mask & 2) HIP_TRY(launch_gemm(a, c->nbatch, c->variant, s, one_pass ? &c->plan_gemm : nullptr));
-      if (c->stage_mask & 4) HIP_TRY(launch_wino_trans_output(w, s, one_pass ? &c->plan_wino_out : nullptr));
-    }
-    break;
-  }
-  default:
-    return fail(EHIP_GENERAL_ERROR, "internal: no executor");
-  }
-  return EHIP_OK;
+  return run_plans(c, output_dev, input_dev, bias_dev, 7, static_cast<hipStream_t>(hip_stream));
 }
 
 EHIP_API int ehip_conv_execute_stages(ehip_conv_t *c, void *output_dev, const void *input_dev, const void *bias_dev,
@@ -754,10 +753,10 @@ EHIP_API int ehip_conv_execute_stages(ehip_conv_t *c, void *output_dev, const vo
   if (!c || !c->prepared) return fail(EHIP_GENERAL_ERROR, "execute_stages needs a prepared handle");
   if (c->family != FAM_WINOGRAD) return fail(EHIP_GENERAL_ERROR, "execute_stages: not a Winograd layer");
   if (stages < 1 || stages > 7) return fail(EHIP_GENERAL_ERROR, "execute_stages: stages is a mask of 1 | 2 | 4");
-  c->stage_mask = stages;
+  if (!output_dev || !input_dev) return fail(EHIP_GENERAL_ERROR, "Parameter error. Invalid input data!");
   int rc = EHIP_OK;
-  for (int i = 0; i < count && rc == EHIP_OK; ++i) rc = ehip_conv_execute(c, output_dev, input_dev, nullptr, bias_dev, hip_stream);
-  c->stage_mask = 7;
+  for (int i = 0; i < count && rc == EHIP_OK; ++i)
+    rc = run_plans(c, output_dev, input_dev, bias_dev, stages, static_cast<hipStream_t>(hip_stream));
   return rc;
 }
 
@@ -832,7 +831,6 @@ EHIP_API int ehip_conv_query(ehip_conv_t *c, int what, void *host_dst, size_t *b
   }
   case EHIP_Q_TINPUT_U8:
     if (c->family != FAM_WINOGRAD) return fail(EHIP_GENERAL_ERROR, "not a Winograd handle");
-    if (c->chunk_n < d.n) return fail(EHIP_UNIMPLEMENTED, "the intermediates of a multi-pass layer hold its last pass only");
     if (c->tin_blocked) {   // back to the canonical [pos][ic2][t][16]
       const size_t canon = (size_t)c->nbatch * c->ic2 * c->t * 16;
       if (!want(canon)) return EHIP_OK;
@@ -851,7 +849,6 @@ EHIP_API int ehip_conv_query(ehip_conv_t *c, int what, void *host_dst, size_t *b
     return EHIP_OK;
   case EHIP_Q_TOUTPUT_F32:
     if (c->family != FAM_WINOGRAD) return fail(EHIP_GENERAL_ERROR, "not a Winograd handle");
-    if (c->chunk_n < d.n) return fail(EHIP_UNIMPLEMENTED, "the intermediates of a multi-pass layer hold its last pass only");
     if (c->fused) return fail(EHIP_UNIMPLEMENTED, "the fused schedule keeps the GEMM result on chip (set EHIP_WINO_FUSED=0)");
     if (!want(c->tout_bytes)) return EHIP_OK;
     HIP_TRY(hipMemcpy(host_dst, c->tout, c->tout_bytes, hipMemcpyDeviceToHost));

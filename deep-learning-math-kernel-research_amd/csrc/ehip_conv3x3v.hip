@@ -506,28 +506,23 @@ __device__ __forceinline__ void conv3x3v_body(const Conv3x3Args &a)
 // staging addresses are made of -- is passed as leading scalar arguments, which the dispatcher preloads into
 // scalar registers with the wave (the file is compiled with -amdgpu-kernarg-preload-count=16): the wave
 // starts computing addresses at once instead of after a round trip to the kernel-argument memory (~0.5 us,
-// of a 6 us kernel).  The rest of the argument block is loaded as usual while the staging loads fly.
+// of a 6 us kernel).  The rest of the argument structure (`rest`, see LaunchPlan) is loaded while the staging loads
+// fly.  pads_cu = pad_t | pad_l << 8 | chunk_units << 16.
 #define EHIP_CONV3X3V_HEAD                                                                                            \
-  const uint8_t *in, int ih, int iw, int oh, int ow, int pad_t, int pad_l, int ic2, int chunk_units, int vw,         \
+  const uint8_t *in, const Conv3x3Args *rest, int ih, int iw, int oh, int ow, unsigned pads_cu, int ic2, int vw,        \
       unsigned vw_magic, int gx, int gy, int tiles, int tiles_per_xcd
 template <int WM, int WN, int TM, int TN, int CT, int NPASS, int PAIRS = 0, bool SP = false, bool SL = false, int S = 1>
-__global__ __launch_bounds__(kBlock, 2) void k_conv3x3v_u8s8(EHIP_CONV3X3V_HEAD, Conv3x3Args rest)
+__global__ __launch_bounds__(kBlock, 2) void k_conv3x3v_u8s8(EHIP_CONV3X3V_HEAD, void *out)
 {
-  Conv3x3Args a = rest;
-  a.in = in; a.ih = ih; a.iw = iw; a.oh = oh; a.ow = ow; a.pad_t = pad_t; a.pad_l = pad_l; a.ic2 = ic2;
-  a.chunk_units = chunk_units; a.vw = vw; a.vw_magic = vw_magic; a.gx = gx; a.gy = gy; a.tiles = tiles;
+  Conv3x3Args a = load_args(rest);
+  a.in = in; a.out = out; a.ih = ih; a.iw = iw; a.oh = oh; a.ow = ow; a.pad_t = (int)(pads_cu & 0xffu); a.pad_l = (int)((pads_cu >> 8) & 0xffu);
+  a.ic2 = ic2; a.chunk_units = (int)(pads_cu >> 16); a.vw = vw; a.vw_magic = vw_magic; a.gx = gx; a.gy = gy; a.tiles = tiles;
   a.tiles_per_xcd = tiles_per_xcd;
   conv3x3v_body<WM, WN, TM, TN, CT, NPASS, PAIRS, SP, SL, S>(a);
 }
 
 namespace {
-typedef void (*conv3x3v_kernel_t)(EHIP_CONV3X3V_HEAD, Conv3x3Args);
-inline hipError_t conv3x3v_enqueue(conv3x3v_kernel_t kernel, dim3 grid, unsigned lds, const Conv3x3Args &a, hipStream_t s)
-{
-  hipLaunchKernelGGL(kernel, grid, dim3(kBlock), lds, s, a.in, a.ih, a.iw, a.oh, a.ow, a.pad_t, a.pad_l, a.ic2, a.chunk_units,
-                     a.vw, a.vw_magic, a.gx, a.gy, a.tiles, a.tiles_per_xcd, a);
-  return hipGetLastError();
-}
+typedef void (*conv3x3v_kernel_t)(EHIP_CONV3X3V_HEAD, void *out);
 struct Variant {
   const char *name;
   int oc_t, p_t, cells;   // cells: staged cells per unit a tile may span
@@ -684,15 +679,8 @@ int conv3x3v_pick_variant(int n, int oh, int ow, int oc2, int stride)
   return best;
 }
 
-hipError_t launch_conv3x3v(const Conv3x3Args &a0, int n, int variant, hipStream_t s, LaunchPlan<Conv3x3Args> *plan)
+hipError_t plan_conv3x3v(LaunchPlan &plan, const Conv3x3Args &a0, int n, int variant, hipStream_t s)
 {
-  if (plan && plan->valid) {   // everything but the tensors is as on the first launch
-    Conv3x3Args local = plan->args;   // a copy: the kept plan is only read (executes from several threads or streams)
-    local.in = a0.in;
-    local.out = a0.out;
-    // (the plan keeps this kernel's pointer under the one-argument type of its slot)
-    return conv3x3v_enqueue(reinterpret_cast<conv3x3v_kernel_t>(plan->kernel), plan->grid, plan->lds, local, s);
-  }
   const Variant &k = kVariants[variant];
   Conv3x3Args a = a0;
   const size_t lds_bytes = (size_t)a.chunk_units * k.ustride * 16;
@@ -722,21 +710,10 @@ hipError_t launch_conv3x3v(const Conv3x3Args &a0, int n, int variant, hipStream_
       if (k.split[slot] && (a.lean & 1) && !(a.lean & 4) && want) kernel = k.split[slot];
     }
   }
-  if (lds_bytes > 48 * 1024) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
-    if (e != hipSuccess) return e;
-  }
-  const hipError_t e = conv3x3v_enqueue(kernel, grid, (unsigned)lds_bytes, a, s);
-  if (plan && e == hipSuccess) {   // kept only once the first launch has gone out
-    plan->kernel = reinterpret_cast<void (*)(Conv3x3Args)>(kernel);
-    plan->grid = grid;
-    plan->block = dim3(kBlock);
-    plan->lds = (unsigned)lds_bytes;
-    plan->args = a;
-    plan->valid = true;
-  }
-  return e;
+  if (a.pad_t > 255 || a.pad_l > 255 || a.chunk_units >= 65536) return hipErrorInvalidValue;   // pads_cu's fields
+  return plan_set(plan, kernel, grid, dim3(kBlock), lds_bytes, a, s, ArgIn{a.in}, ArgBlock{}, a.ih, a.iw, a.oh, a.ow,
+                  (unsigned)a.pad_t | (unsigned)a.pad_l << 8 | (unsigned)a.chunk_units << 16, a.ic2, a.vw, a.vw_magic, a.gx, a.gy,
+                  a.tiles, a.tiles_per_xcd, ArgOut{a.out});
 }
 
 }  // namespace ehip

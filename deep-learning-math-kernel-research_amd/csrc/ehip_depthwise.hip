@@ -82,21 +82,21 @@ __device__ __forceinline__ uint2 swap_halves(unsigned x, unsigned y)
 // the clamp is the instruction's own saturation.
 // Both kernels take what a wave's first loads need -- three pointers and the geometry the addresses are made of,
 // packed into 16 dwords -- as leading scalar arguments, which the dispatcher preloads into scalar registers with
-// the wave (the file is compiled with -amdgpu-kernarg-preload-count=16); the rest of the argument block is loaded
-// as usual meanwhile.  ihw = ih | iw << 16, ohw = oh | ow << 16, geom = pad_t | pad_l << 8 | stride << 16,
-// ppb_lp = planes_per_block | lanes_padded << 16.
+// the wave (the file is compiled with -amdgpu-kernarg-preload-count=16); the rest of the argument structure (`rest`,
+// see LaunchPlan) is loaded meanwhile.  ihw = ih | iw << 16, ohw = oh | ow << 16, geom = pad_t | pad_l << 4 |
+// stride << 8 | planes_per_block << 12 | lanes_padded << 16, walk = lanes_per_plane (dot4 kernel) or strips_per_wg.
 #define EHIP_DW_HEAD                                                                                                   \
-  const uint8_t *in_, const int8_t *w_, const int *wsum_, int n_, int g2_, unsigned ihw_, unsigned ohw_, unsigned geom_, \
-      int blocks_per_plane_, int lanes_per_plane_, unsigned ppb_lp_, unsigned wp_magic_, int strips_per_wg_
+  const uint8_t *in_, const int8_t *w_, const int *wsum_, const DepthwiseArgs *rest, int n_, int g2_, unsigned ihw_,    \
+      unsigned ohw_, unsigned geom_, int blocks_per_plane_, int walk_, unsigned wp_magic_, void *out_
 #define EHIP_DW_UNPACK                                                                                                 \
-  DepthwiseArgs a = rest;                                                                                              \
-  a.in = in_; a.w = w_; a.wsum = wsum_; a.n = n_; a.g2 = g2_; a.ih = (int)(ihw_ & 0xffffu); a.iw = (int)(ihw_ >> 16);  \
-  a.oh = (int)(ohw_ & 0xffffu); a.ow = (int)(ohw_ >> 16); a.pad_t = (int)(geom_ & 0xffu);                              \
-  a.pad_l = (int)((geom_ >> 8) & 0xffu); a.stride = (int)(geom_ >> 16); a.blocks_per_plane = blocks_per_plane_;        \
-  a.lanes_per_plane = lanes_per_plane_; a.planes_per_block = (int)(ppb_lp_ & 0xffffu);                                 \
-  a.lanes_padded = (int)(ppb_lp_ >> 16); a.wp_magic = wp_magic_; a.strips_per_wg = strips_per_wg_
+  DepthwiseArgs a = load_args(rest);                                                                                   \
+  a.out = out_; a.in = in_; a.w = w_; a.wsum = wsum_; a.n = n_; a.g2 = g2_; a.ih = (int)(ihw_ & 0xffffu); a.iw = (int)(ihw_ >> 16);  \
+  a.oh = (int)(ohw_ & 0xffffu); a.ow = (int)(ohw_ >> 16); a.pad_t = (int)(geom_ & 15u);                                \
+  a.pad_l = (int)((geom_ >> 4) & 15u); a.stride = (int)((geom_ >> 8) & 15u);                                           \
+  a.planes_per_block = (int)((geom_ >> 12) & 15u); a.lanes_padded = (int)(geom_ >> 16);                                \
+  a.blocks_per_plane = blocks_per_plane_; a.lanes_per_plane = a.strips_per_wg = walk_; a.wp_magic = wp_magic_
 template <int RB, int MODE, int S>
-__global__ __launch_bounds__(kBlock) void k_depthwise3x3_u8s8(EHIP_DW_HEAD, DepthwiseArgs rest)
+__global__ __launch_bounds__(kBlock) void k_depthwise3x3_u8s8(EHIP_DW_HEAD)
 {
   EHIP_DW_UNPACK;
   constexpr int NPX = S == 1 ? 4 : 5;          // input pixels per row a lane touches
@@ -114,7 +114,7 @@ __global__ __launch_bounds__(kBlock) void k_depthwise3x3_u8s8(EHIP_DW_HEAD, Dept
   if (plane_id >= a.n * a.g2) return;   // whole waves
   const int wp = (a.ow + 1) >> 1;
   const int local = a.planes_per_block > 1 ? (int)threadIdx.x - sub * a.lanes_padded
-                                           : (seq - pgrp * a.blocks_per_plane) * (int)blockDim.x + (int)threadIdx.x;
+                                           : (seq - pgrp * a.blocks_per_plane) * a.lanes_padded + (int)threadIdx.x;
   if (local >= a.lanes_per_plane) return;
   const int q = local & 3;
   const int hb = fastdiv(local >> 2, wp, a.wp_magic);
@@ -272,7 +272,7 @@ __global__ __launch_bounds__(kBlock) void k_depthwise3x3_u8s8(EHIP_DW_HEAD, Dept
 // other half of a double LDS buffer once the arithmetic is done (one barrier per strip).  A layer this short (57.8 MB,
 // 9 us for a plain copy) has no time for workgroups that load, compute and store one after the other.
 template <int MODE, int NC>
-__global__ __launch_bounds__(kBlock) void k_depthwise3x3_mfma(EHIP_DW_HEAD, DepthwiseArgs rest)
+__global__ __launch_bounds__(kBlock) void k_depthwise3x3_mfma(EHIP_DW_HEAD)
 {
   EHIP_DW_UNPACK;
   constexpr int R = 8, WL = 32 * NC + 2, CELLS = (R + 2) * WL, PER = (CELLS + kBlock - 1) / kBlock;
@@ -282,7 +282,7 @@ __global__ __launch_bounds__(kBlock) void k_depthwise3x3_mfma(EHIP_DW_HEAD, Dept
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // strips [first, last) of this workgroup: XCD x (workgroups x, x + 8, ...) walks the x-th eighth of all
   // strips, a workgroup a contiguous run of it -- neighbouring strips share two input rows in that XCD's L2
-  const int per_xcd = gridDim.x >> 3;
+  const int per_xcd = a.lanes_padded;   // (this kernel: an eighth of the grid)
   const int w_lin = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
   const int first = w_lin * a.strips_per_wg;
   const int total = a.n * a.g2 * a.blocks_per_plane;    // blocks_per_plane = strips per plane
@@ -453,33 +453,19 @@ hipError_t launch_depthwise_diag(const int8_t *wpacked, int g2n, void *diag, hip
 }
 
 namespace {
-typedef void (*dw_kernel_t)(EHIP_DW_HEAD, DepthwiseArgs);
-hipError_t dw_enqueue(const LaunchPlan<DepthwiseArgs> &plan, hipStream_t s)
-{
-  const DepthwiseArgs &a = plan.args;
-  hipLaunchKernelGGL(reinterpret_cast<dw_kernel_t>(plan.kernel), plan.grid, plan.block, plan.lds, s, a.in, a.w, a.wsum, a.n, a.g2,
-                     (unsigned)a.ih | (unsigned)a.iw << 16, (unsigned)a.oh | (unsigned)a.ow << 16,
-                     (unsigned)a.pad_t | (unsigned)a.pad_l << 8 | (unsigned)a.stride << 16, a.blocks_per_plane, a.lanes_per_plane,
-                     (unsigned)a.planes_per_block | (unsigned)a.lanes_padded << 16, a.wp_magic, a.strips_per_wg, a);
-  return hipGetLastError();
-}
-hipError_t dw_launch(LaunchPlan<DepthwiseArgs> *plan, dw_kernel_t kernel, dim3 grid, dim3 block, const DepthwiseArgs &a, hipStream_t s)
+typedef void (*dw_kernel_t)(EHIP_DW_HEAD);
+hipError_t dw_set(LaunchPlan &plan, dw_kernel_t kernel, dim3 grid, dim3 block, const DepthwiseArgs &a, int walk, hipStream_t s)
 {
   // what the packed leading arguments can hold
-  if (a.ih >= 65536 || a.iw >= 65536 || a.oh >= 65536 || a.ow >= 65536 || a.pad_t < 0 || a.pad_t > 255 || a.pad_l < 0 ||
-      a.pad_l > 255 || a.planes_per_block >= 65536 || a.lanes_padded >= 65536) {
+  if (a.ih >= 65536 || a.iw >= 65536 || a.oh >= 65536 || a.ow >= 65536 || a.pad_t < 0 || a.pad_t > 15 || a.pad_l < 0 ||
+      a.pad_l > 15 || a.planes_per_block > 15 || a.lanes_padded >= 65536) {
     set_error("depthwise: plane or padding too large");
     return hipErrorInvalidValue;
   }
-  LaunchPlan<DepthwiseArgs> local;
-  LaunchPlan<DepthwiseArgs> *p = plan ? plan : &local;
-  p->kernel = reinterpret_cast<void (*)(DepthwiseArgs)>(kernel);
-  p->grid = grid;
-  p->block = block;
-  p->lds = 0;
-  p->args = a;
-  p->enqueue = dw_enqueue;
-  return plan_first_launch(p, s);
+  const unsigned geom = (unsigned)a.pad_t | (unsigned)a.pad_l << 4 | (unsigned)a.stride << 8 | (unsigned)a.planes_per_block << 12 |
+      (unsigned)a.lanes_padded << 16;
+  return plan_set(plan, kernel, grid, block, 0, a, s, ArgIn{a.in}, a.w, a.wsum, ArgBlock{}, a.n, a.g2, (unsigned)a.ih | (unsigned)a.iw << 16,
+                  (unsigned)a.oh | (unsigned)a.ow << 16, geom, a.blocks_per_plane, walk, a.wp_magic, ArgOut{a.out});
 }
 template <int RB, int S>
 dw_kernel_t kernel_rbs(int mode)
@@ -514,11 +500,8 @@ bool depthwise_mfma_applies(int stride, int oh, int ow, int pad_t, int pad_l, in
   return 32.0 * nc * 8.0 * strips <= 1.35 * ow * oh;
 }
 
-hipError_t launch_depthwise(const DepthwiseArgs &a0, hipStream_t s, LaunchPlan<DepthwiseArgs> *plan)
+hipError_t plan_depthwise(LaunchPlan &plan, const DepthwiseArgs &a0, hipStream_t s)
 {
-  if (plan && plan->valid) {   // everything but the tensors is as on the first launch
-    return plan_relaunch(*plan, [&](DepthwiseArgs &x) { x.in = a0.in; x.out = a0.out; }, s);
-  }
   DepthwiseArgs a = a0;
   if (a.stride != 1 && a.stride != 2) {
     set_error("depthwise: stride must be 1 or 2");
@@ -545,11 +528,13 @@ hipError_t launch_depthwise(const DepthwiseArgs &a0, hipStream_t s, LaunchPlan<D
     if (per_wg < 1) per_wg = 1;
     a.strips_per_wg = per_wg;
     const long long wgs = 8 * ((((total + per_wg - 1) / per_wg) + 7) / 8);
+    a.planes_per_block = 1;
+    a.lanes_padded = (int)(wgs / 8);   // (per_wg: at most 1024 workgroups and a few)
     dw_kernel_t kernel = nullptr;
 #define EHIP_DWM(NC) (full ? k_depthwise3x3_mfma<2, NC> : k_depthwise3x3_mfma<1, NC>)
     kernel = nc == 1 ? EHIP_DWM(1) : (nc == 2 ? EHIP_DWM(2) : (nc == 3 ? EHIP_DWM(3) : EHIP_DWM(4)));
 #undef EHIP_DWM
-    return dw_launch(plan, kernel, dim3((unsigned)wgs), dim3(kBlock), a, s);
+    return dw_set(plan, kernel, dim3((unsigned)wgs), dim3(kBlock), a, a.strips_per_wg, s);
   }
   // four rows per lane on tall planes (seven where that divides the height: 28, 56, 112 -- fewer halo
   // rows re-read, 2-5 % on the MobileNet layers), fewer where that would leave lanes idle
@@ -585,7 +570,7 @@ hipError_t launch_depthwise(const DepthwiseArgs &a0, hipStream_t s, LaunchPlan<D
   dim3 grid((unsigned)(8 * ((groups + 7) / 8) * a.blocks_per_plane), 1, 1);
   const dw_kernel_t kernel = rb == 7 ? kernel_rb<7>(a.stride, mode)
       : (rb == 4 ? kernel_rb<4>(a.stride, mode) : (rb == 2 ? kernel_rb<2>(a.stride, mode) : kernel_rb<1>(a.stride, mode)));
-  return dw_launch(plan, kernel, grid, dim3(block), a, s);
+  return dw_set(plan, kernel, grid, dim3(block), a, a.lanes_per_plane, s);
 }
 
 }  // namespace ehip

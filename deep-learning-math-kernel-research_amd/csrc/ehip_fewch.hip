@@ -207,8 +207,10 @@ __device__ __forceinline__ FewChTables fewch_stage(const FewChArgs &a, unsigned 
 }
 
 template <int KS>
-__global__ __launch_bounds__(kBlock, 3) void k_conv_fewch_u8s8(FewChArgs a)
+__global__ __launch_bounds__(kBlock, 3) void k_conv_fewch_u8s8(const FewChArgs *rest, const uint8_t *in, void *out)
 {
+  FewChArgs a = load_args(rest);
+  a.in = in; a.out = out;
   // [nrows_in][lrow / 4] staged rows; with border classes kept on chip (a.tab_lds): the shift rows of
   // the workgroup's channels [class][wo * 32], then the class of each of the strip's output rows
   // (times ncls_w) and of each output column
@@ -349,8 +351,10 @@ __global__ __launch_bounds__(kBlock, 3) void k_conv_fewch_u8s8(FewChArgs a)
 // comes from LDS): nothing but that epilogue, so the tile loop is straight-line code with 32-bit output offsets,
 // and the cells of a wave's next tile are read while the present one is scaled and stored.
 template <int KS, bool CLAMP, bool TAB>
-__global__ __launch_bounds__(kBlock, 3) void k_conv_fewch_lean(FewChArgs a)
+__global__ __launch_bounds__(kBlock, 3) void k_conv_fewch_lean(const FewChArgs *rest, const uint8_t *in, void *out)
 {
+  FewChArgs a = load_args(rest);
+  a.in = in; a.out = out;
   extern __shared__ unsigned rows_lds[];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -480,14 +484,10 @@ int conv_fewch_row_pitch(int icl, int kw, int iw, int ow, int stride_w, int pad_
   return icl == 4 ? up(need + 4, 16) : up(need + 4, 4) + 4;
 }
 
-// Fills the derived fields (cells, strip height, LDS row pitch, wave split) and launches.
-// Expects in a: tensors, epilogue, n, ih, iw, oh, ow, ic, kh, kw, strides, pads, oc2, ocpp, formats, classes.
-hipError_t launch_conv_fewch(FewChArgs &a, hipStream_t s, LaunchPlan<FewChArgs> *plan)
+// Fills the derived fields (cells, strip height, LDS row pitch, wave split) and the plan.
+// Expects in a: weights, epilogue, n, ih, iw, oh, ow, ic, kh, kw, strides, pads, oc2, ocpp, formats, classes.
+hipError_t plan_conv_fewch(LaunchPlan &plan, FewChArgs &a, hipStream_t s)
 {
-  if (plan && plan->valid) {   // everything but the tensors is as on the first launch
-    if (a.in_nhwc && (reinterpret_cast<uintptr_t>(a.in) & 3)) return hipErrorInvalidValue;   // aligned dword loads
-    return plan_relaunch(*plan, [&](FewChArgs &x) { x.in = a.in; x.out = a.out; }, s);
-  }
   {
     // lean_mode() but for the per-pixel shift rows, which this kernel's lean path reads itself
     Epilogue e = a.ep;
@@ -500,7 +500,6 @@ hipError_t launch_conv_fewch(FewChArgs &a, hipStream_t s, LaunchPlan<FewChArgs> 
   a.nu = (a.kw + a.ppc - 1) / a.ppc;
   a.cells = a.kh * a.nu;
   if (!conv_fewch_applies(a.ic, a.kh, a.kw)) return hipErrorInvalidValue;
-  if (a.in_nhwc && (reinterpret_cast<uintptr_t>(a.in) & 3)) return hipErrorInvalidValue;   // aligned dword loads
   a.lrow = conv_fewch_row_pitch(a.icl, a.kw, a.iw, a.ow, a.stride_w, a.pad_l);
   const int octiles = up(a.oc2 * 16, 32) / 32;   // <= ocpp / 32
   a.wo = octiles % 4 == 0 ? 4 : octiles % 2 == 0 ? 2 : 1;
@@ -569,7 +568,7 @@ hipError_t launch_conv_fewch(FewChArgs &a, hipStream_t s, LaunchPlan<FewChArgs> 
   if ((long long)a.nrows_in * (a.lrow / 4) * (a.lrow / 4) >= (1ll << 32) || (long long)a.nrows_in * a.iw * a.iw >= (1ll << 32))
     return hipErrorInvalidValue;
   const int ks = (a.cells + 1) / 2;
-  void (*kern)(FewChArgs) = ks <= 2 ? k_conv_fewch_u8s8<2> : ks == 3 ? k_conv_fewch_u8s8<3> : ks == 4 ? k_conv_fewch_u8s8<4>
+  void (*kern)(const FewChArgs *, const uint8_t *, void *) = ks <= 2 ? k_conv_fewch_u8s8<2> : ks == 3 ? k_conv_fewch_u8s8<3> : ks == 4 ? k_conv_fewch_u8s8<4>
       : ks == 5 ? k_conv_fewch_u8s8<5> : k_conv_fewch_u8s8<7>;
   const char *name = "k_conv_fewch_u8s8";
   // the kernel of the lean epilogue alone: shift rows per channel or on chip, an image's output below 2 GB
@@ -583,9 +582,8 @@ hipError_t launch_conv_fewch(FewChArgs &a, hipStream_t s, LaunchPlan<FewChArgs> 
 #undef FL
     name = "k_conv_fewch_lean";
   }
-  const hipError_t e = plan_launch(plan, kern, dim3(a.n * a.strips, gy), dim3(kBlock), lds, a, s);
-  if (plan) plan->name = name;
-  return e;
+  plan.name = name;
+  return plan_set(plan, kern, dim3(a.n * a.strips, gy), dim3(kBlock), lds, a, s, ArgBlock{}, ArgIn{a.in}, ArgOut{a.out});
 }
 
 }  // namespace ehip

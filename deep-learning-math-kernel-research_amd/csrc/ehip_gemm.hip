@@ -42,8 +42,10 @@
 namespace ehip {
 
 template <int WM, int WN, int TM, int TN, int KC, int D, bool NHWC, int CONV>
-__global__ __launch_bounds__(kBlock, 2) void k_gemm_u8s8(GemmArgs a)
+__global__ __launch_bounds__(kBlock, 2) void k_gemm_u8s8(const GemmArgs *rest, const uint8_t *in, void *out)
 {
+  GemmArgs a = load_args(rest);
+  a.in = in; a.out = out;
   static_assert(!(NHWC && CONV == 1), "nhwc kh x kw input works the tap out per cell");
   constexpr int OC_T = WM * TM * 32;
   constexpr int P_T = WN * TN * 32;
@@ -360,19 +362,19 @@ __global__ __launch_bounds__(kBlock, 2) void k_gemm_u8s8(GemmArgs a)
 // so the activations reach the CU once.  grid: (workgroups over pixel tiles, 4-wave channel blocks).
 // What a wave's first loads need -- the two pointers and the geometry their addresses are made of -- is passed as
 // leading scalar arguments, which the dispatcher preloads into scalar registers with the wave (the file is compiled
-// with -amdgpu-kernarg-preload-count=16); the rest of the argument block is loaded as usual meanwhile.
-// geom = stride_h | stride_w << 8 | dense << 16 | in_nhwc << 17 | out_nhwc << 18 | sk_wo << 20.
+// with -amdgpu-kernarg-preload-count=16); the rest of the argument structure (`rest`, see LaunchPlan) is loaded meanwhile.
+// geom = stride_h | stride_w << 8 | dense << 16 | in_nhwc << 17 | out_nhwc << 18 | sk_wo << 20 | ic2 << 24.
 #define EHIP_SMALLK_HEAD                                                                                             \
-  const uint8_t *in, const int8_t *w, int p_total, int ohw, unsigned ohw_magic, int ihw, int ic2, int ocpp, int oc2, \
-      unsigned geom, int iw, int ow, unsigned ow_magic
+  const uint8_t *in, const int8_t *w, const GemmArgs *rest, int p_total, int ohw, unsigned ohw_magic, int ihw, int ocpp, \
+      int oc2, unsigned geom, int iw, int ow, unsigned ow_magic
 template <int TNW, int KS>
-__global__ __launch_bounds__(kBlock, 2) void k_gemm_smallk_u8s8(EHIP_SMALLK_HEAD, GemmArgs rest)
+__global__ __launch_bounds__(kBlock, 2) void k_gemm_smallk_u8s8(EHIP_SMALLK_HEAD, void *out)
 {
-  GemmArgs a = rest;
-  a.in = in; a.w = w; a.p_total = p_total; a.ohw = ohw; a.ohw_magic = ohw_magic; a.ihw = ihw; a.ic2 = ic2; a.ocpp = ocpp;
+  GemmArgs a = load_args(rest);
+  a.in = in; a.out = out; a.w = w; a.p_total = p_total; a.ohw = ohw; a.ohw_magic = ohw_magic; a.ihw = ihw; a.ic2 = (int)(geom >> 24); a.ocpp = ocpp;
   a.oc2 = oc2; a.iw = iw; a.ow = ow; a.ow_magic = ow_magic;
   a.stride_h = (int)(geom & 0xffu); a.stride_w = (int)((geom >> 8) & 0xffu);
-  a.in_nhwc = (int)((geom >> 17) & 1u); a.out_nhwc = (int)((geom >> 18) & 1u); a.sk_wo = (int)(geom >> 20);
+  a.in_nhwc = (int)((geom >> 17) & 1u); a.out_nhwc = (int)((geom >> 18) & 1u); a.sk_wo = (int)((geom >> 20) & 7u);
   __shared__ v4i xpatch[4 * 256];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -419,7 +421,7 @@ __global__ __launch_bounds__(kBlock, 2) void k_gemm_smallk_u8s8(EHIP_SMALLK_HEAD
 
   // a wave-tile is TNW x 32 consecutive pixels
   const int ntiles = (a.p_total + 32 * TNW - 1) / (32 * TNW);
-  const int tstep = wpn * gridDim.x;
+  const int tstep = wpn * a.nx;   // (nx: the grid's first dimension; gridDim itself would be a hidden argument)
   int tile = wpn * blockIdx.x + wp;
   v4i breg[TNW][KS];
   auto load_b = [&](int t) {
@@ -502,13 +504,13 @@ __global__ __launch_bounds__(kBlock, 2) void k_gemm_smallk_u8s8(EHIP_SMALLK_HEAD
 // wave's channels sit in a wave-private piece of LDS -- in registers they would take 48 per tile -- and every
 // lane of a half-wave reads the same 16 bytes of them (a broadcast).
 template <int KS, int OCW>
-__global__ __launch_bounds__(kBlock, 2) void k_gemm_smallk_lean(EHIP_SMALLK_HEAD, GemmArgs rest)
+__global__ __launch_bounds__(kBlock, 2) void k_gemm_smallk_lean(EHIP_SMALLK_HEAD, void *out)
 {
-  GemmArgs a = rest;
-  a.in = in; a.w = w; a.p_total = p_total; a.ohw = ohw; a.ohw_magic = ohw_magic; a.ihw = ihw; a.ic2 = ic2; a.ocpp = ocpp;
+  GemmArgs a = load_args(rest);
+  a.in = in; a.out = out; a.w = w; a.p_total = p_total; a.ohw = ohw; a.ohw_magic = ohw_magic; a.ihw = ihw; a.ic2 = (int)(geom >> 24); a.ocpp = ocpp;
   a.oc2 = oc2; a.iw = iw; a.ow = ow; a.ow_magic = ow_magic;
   a.stride_h = (int)(geom & 0xffu); a.stride_w = (int)((geom >> 8) & 0xffu);
-  a.in_nhwc = (int)((geom >> 17) & 1u); a.out_nhwc = (int)((geom >> 18) & 1u); a.sk_wo = (int)(geom >> 20);
+  a.in_nhwc = (int)((geom >> 17) & 1u); a.out_nhwc = (int)((geom >> 18) & 1u); a.sk_wo = (int)((geom >> 20) & 7u);
   __shared__ float4 cst_lds[4 * OCW * 24];   // [wave][tile][scale | shift | compensation][8 cells of 4 channels]
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -553,7 +555,7 @@ __global__ __launch_bounds__(kBlock, 2) void k_gemm_smallk_lean(EHIP_SMALLK_HEAD
   const long long ustride = a.in_nhwc ? 16 : unit_stride;
 
   const int ntiles = (a.p_total + 31) / 32;
-  const int tstep = wpn * gridDim.x;
+  const int tstep = wpn * a.nx;   // (nx: the grid's first dimension; gridDim itself would be a hidden argument)
   int tile = wpn * blockIdx.x + wp;
   v4i breg[KS];
   auto load_b = [&](int t) {
@@ -619,16 +621,17 @@ __global__ __launch_bounds__(kBlock, 2) void k_gemm_smallk_lean(EHIP_SMALLK_HEAD
 }
 
 namespace {
+typedef void (*gemm_kernel_t)(const GemmArgs *, const uint8_t *, void *);
 struct Variant {
   const char *name;
   int oc_t, p_t, kc;
   // [blocked | nhwc | blocked kh x kw, ic2 % KC == 0 | blocked kh x kw, any ic2 | nhwc kh x kw][prefetch depth 1, 2, 4]
   // (null: not built)
-  void (*kernel[5][3])(GemmArgs);
+  gemm_kernel_t kernel[5][3];
 };
 // depth 4 only where four fills of staging fit in 96 registers
 template <int WM, int WN, int TM, int TN, int KC, bool NHWC>
-constexpr void (*deep_or_null())(GemmArgs)
+constexpr gemm_kernel_t deep_or_null()
 {
   if constexpr (4 * ((WM * TM + WN * TN) * 32 * KC / kBlock) * 4 <= 96) return k_gemm_u8s8<WM, WN, TM, TN, KC, 4, NHWC, 0>;
   else return nullptr;
@@ -689,35 +692,23 @@ int gemm_pick_variant(int p_total, int oc2, int ic2, int nbatch, int stride)
 }
 
 namespace {
-typedef void (*smallk_kernel_t)(EHIP_SMALLK_HEAD, GemmArgs);
+typedef void (*smallk_kernel_t)(EHIP_SMALLK_HEAD, void *out);
 template <int KS>
 smallk_kernel_t smallk_kernel(int tnw)
 {
   (void)tnw;   // (two pixel tiles per iteration cost more in occupancy than they gain in overlap: one)
   return k_gemm_smallk_u8s8<1, KS>;
 }
-hipError_t smallk_enqueue(const LaunchPlan<GemmArgs> &plan, hipStream_t s)
+hipError_t smallk_set(LaunchPlan &plan, smallk_kernel_t kernel, dim3 grid, const GemmArgs &a0, hipStream_t s)
 {
-  const GemmArgs &a = plan.args;
+  GemmArgs a = a0;
+  a.nx = (int)grid.x;
+  if (a.stride_h > 255 || a.stride_w > 255 || a.ic2 > 255) return hipErrorInvalidValue;   // geom's fields
   const bool dense = a.stride_h == 1 && a.stride_w == 1 && a.iw == a.ow;
   const unsigned geom = (unsigned)a.stride_h | (unsigned)a.stride_w << 8 | (dense ? 1u << 16 : 0u) | (a.in_nhwc ? 1u << 17 : 0u) |
-      (a.out_nhwc ? 1u << 18 : 0u) | (unsigned)a.sk_wo << 20;
-  hipLaunchKernelGGL(reinterpret_cast<smallk_kernel_t>(plan.kernel), plan.grid, plan.block, plan.lds, s, a.in, a.w, a.p_total,
-                     a.ohw, a.ohw_magic, a.ihw, a.ic2, a.ocpp, a.oc2, geom, a.iw, a.ow, a.ow_magic, a);
-  return hipGetLastError();
-}
-hipError_t smallk_launch(LaunchPlan<GemmArgs> *plan, smallk_kernel_t kernel, dim3 grid, const GemmArgs &a, hipStream_t s)
-{
-  if (a.stride_h > 255 || a.stride_w > 255) return hipErrorInvalidValue;   // geom's fields
-  LaunchPlan<GemmArgs> local;
-  LaunchPlan<GemmArgs> *p = plan ? plan : &local;
-  p->kernel = reinterpret_cast<void (*)(GemmArgs)>(kernel);
-  p->grid = grid;
-  p->block = dim3(kBlock);
-  p->lds = 0;
-  p->args = a;
-  p->enqueue = smallk_enqueue;
-  return plan_first_launch(p, s);
+      (a.out_nhwc ? 1u << 18 : 0u) | (unsigned)a.sk_wo << 20 | (unsigned)a.ic2 << 24;
+  return plan_set(plan, kernel, grid, dim3(kBlock), 0, a, s, ArgIn{a.in}, a.w, ArgBlock{}, a.p_total, a.ohw, a.ohw_magic, a.ihw,
+                  a.ocpp, a.oc2, geom, a.iw, a.ow, a.ow_magic, ArgOut{a.out});
 }
 }  // namespace
 
@@ -730,7 +721,7 @@ bool gemm_smallk_applies(int ic2, int taps, int nbatch)
   return nbatch == 1 && taps <= 1 && ic2 <= 8;
 }
 
-hipError_t launch_gemm_smallk(const GemmArgs &a0, hipStream_t s, LaunchPlan<GemmArgs> *plan = nullptr)
+hipError_t plan_gemm_smallk(LaunchPlan &plan, const GemmArgs &a0, hipStream_t s)
 {
   GemmArgs a = a0;
   a.lean = lean_mode(a.ep, false);   // blocked and nhwc output alike
@@ -770,27 +761,24 @@ hipError_t launch_gemm_smallk(const GemmArgs &a0, hipStream_t s, LaunchPlan<Gemm
     if (ks == 1) lk = ocw == 4 ? k_gemm_smallk_lean<1, 4> : k_gemm_smallk_lean<1, 2>;
     else if (ks == 2) lk = ocw == 4 ? k_gemm_smallk_lean<2, 4> : k_gemm_smallk_lean<2, 2>;
     else lk = k_gemm_smallk_lean<4, 2>;
-    if (plan) {
+    {
       static const char *const names[3][2] = {{"k_gemm_smallk_lean<1,2>", "k_gemm_smallk_lean<1,4>"},
                                               {"k_gemm_smallk_lean<2,2>", "k_gemm_smallk_lean<2,4>"},
                                               {"k_gemm_smallk_lean<4,2>", "k_gemm_smallk_lean<4,2>"}};
-      plan->name = names[ks == 1 ? 0 : (ks == 2 ? 1 : 2)][ocw == 4 ? 1 : 0];
+      plan.name = names[ks == 1 ? 0 : (ks == 2 ? 1 : 2)][ocw == 4 ? 1 : 0];
     }
-    return smallk_launch(plan, lk, dim3(nx2, ny2), a, s);
+    return smallk_set(plan, lk, dim3(nx2, ny2), a, s);
   }
-  return smallk_launch(plan, kernel, dim3(nx, ny), a, s);
+  return smallk_set(plan, kernel, dim3(nx, ny), a, s);
 }
 
-hipError_t launch_gemm(const GemmArgs &a0, int nbatch, int variant, hipStream_t s, LaunchPlan<GemmArgs> *plan)
+hipError_t plan_gemm(LaunchPlan &plan, const GemmArgs &a0, int nbatch, int variant, hipStream_t s)
 {
-  if (plan && plan->valid) {   // everything but the tensors is as on the first launch
-    return plan_relaunch(*plan, [&](GemmArgs &x) { x.in = a0.in; x.out = a0.out; }, s);
-  }
-  if (gemm1x1_wres_applies(a0, nbatch)) return launch_gemm1x1_wres(a0, s, plan);
-  if (gemm_smallk_applies(a0.ic2, a0.kh * a0.kw, nbatch)) return launch_gemm_smallk(a0, s, plan);
+  if (gemm1x1_wres_applies(a0, nbatch)) return plan_gemm1x1_wres(plan, a0, s);
+  if (gemm_smallk_applies(a0.ic2, a0.kh * a0.kw, nbatch)) return plan_gemm_smallk(plan, a0, s);
   {
     const int rv = gemm1x1_res_pick(a0, nbatch);
-    if (rv >= 0) return launch_gemm1x1_res(a0, rv, s, plan);
+    if (rv >= 0) return plan_gemm1x1_res(plan, a0, rv, s);
   }
   const Variant &k = kVariants[variant];
   GemmArgs a = a0;
@@ -810,7 +798,7 @@ hipError_t launch_gemm(const GemmArgs &a0, int nbatch, int variant, hipStream_t 
   if (taps > 1 && (taps > 64 || nbatch != 1)) return hipErrorInvalidValue;
   const int fmt = taps > 1 ? (a.in_nhwc ? 4 : (a.ic2 % k.kc == 0 ? 2 : 3)) : (a.in_nhwc ? 1 : 0);
   while (dl > 0 && (nchunks % (1 << dl) != 0 || !k.kernel[fmt][dl])) --dl;
-  return plan_launch(plan, k.kernel[fmt][dl], grid, dim3(kBlock), 0, a, s);
+  return plan_set(plan, k.kernel[fmt][dl], grid, dim3(kBlock), 0, a, s, ArgBlock{}, ArgIn{a.in}, ArgOut{a.out});
 }
 
 }  // namespace ehip

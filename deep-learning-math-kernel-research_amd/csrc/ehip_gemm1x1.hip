@@ -93,17 +93,19 @@ __device__ __forceinline__ void wait_loads_but(int n)
 // What a wave's first instructions need -- the three pointers its first loads go through and the geometry
 // their addresses are made of -- is passed as leading scalar arguments, which the dispatcher preloads into scalar
 // registers with the wave (the file is compiled with -amdgpu-kernarg-preload-count=16); the rest of the argument
-// block is loaded as usual while those loads fly.  geom = stride_h | stride_w << 8 | dense << 16 | oc2 << 20.
+// structure (`rest`, see LaunchPlan) is loaded while those loads fly.  geom = stride_h | stride_w << 8 | dense << 16 |
+// oc2 << 20 (the padded channel count follows from it), units = ic2 | units_pad << 16.
 #define EHIP_RES_HEAD                                                                                                  \
-  const uint8_t *in, const int8_t *w, const int *comp, int nx, int ny, int p_total, int ohw, unsigned ohw_magic, int ihw, \
-      int ic2, int units_pad, int ocpp, unsigned geom
+  const uint8_t *in, const int8_t *w, const int *comp, const GemmArgs *rest, int nx, int ny, int p_total, int ohw,      \
+      unsigned ohw_magic, int ihw, unsigned units, unsigned geom
 template <int TM, int TN, int NKS, bool NHWC = false>
-__global__ __launch_bounds__(kBlock, 1) void k_gemm1x1_res(EHIP_RES_HEAD, GemmArgs rest)
+__global__ __launch_bounds__(kBlock, 1) void k_gemm1x1_res(EHIP_RES_HEAD, void *out)
 {
-  GemmArgs a = rest;
-  a.in = in; a.w = w; a.ep.comp = comp; a.nx = nx; a.ny = ny; a.p_total = p_total; a.ohw = ohw; a.ohw_magic = ohw_magic;
-  a.ihw = ihw; a.ic2 = ic2; a.units_pad = units_pad; a.ocpp = ocpp;
+  GemmArgs a = load_args(rest);
+  a.in = in; a.out = out; a.w = w; a.ep.comp = comp; a.nx = nx; a.ny = ny; a.p_total = p_total; a.ohw = ohw; a.ohw_magic = ohw_magic;
+  a.ihw = ihw; a.ic2 = (int)(units & 0xffffu); a.units_pad = (int)(units >> 16);
   a.stride_h = (int)(geom & 0xffu); a.stride_w = (int)((geom >> 8) & 0xffu); a.oc2 = (int)(geom >> 20);
+  a.ocpp = (a.oc2 * 16 + kOcTile - 1) / kOcTile * kOcTile;
   constexpr int OC_T = 4 * TM * 32;
   constexpr int P_T = TN * 32;
   // Weight ring: k-steps requested ahead.  A kernel launch starts with cold L2s, and in a layer of ONE
@@ -364,7 +366,7 @@ __global__ __launch_bounds__(kBlock, 1) void k_gemm1x1_res(EHIP_RES_HEAD, GemmAr
 }
 
 namespace {
-typedef void (*res_kernel_t)(EHIP_RES_HEAD, GemmArgs);
+typedef void (*res_kernel_t)(EHIP_RES_HEAD, void *out);
 struct ResVariant {
   const char *name;
   int oc_t, p_t;
@@ -373,15 +375,6 @@ struct ResVariant {
   res_kernel_t generic_nhwc;  // nhwc input (64-pixel tiles only), or null
   res_kernel_t unrolled_nhwc[3];
 };
-hipError_t res_enqueue(const LaunchPlan<GemmArgs> &plan, hipStream_t s)
-{
-  const GemmArgs &a = plan.args;
-  const bool dense = a.stride_h == 1 && a.stride_w == 1 && a.iw == a.ow;
-  const unsigned geom = (unsigned)a.stride_h | (unsigned)a.stride_w << 8 | (dense ? 1u << 16 : 0u) | (unsigned)a.oc2 << 20;
-  hipLaunchKernelGGL(reinterpret_cast<res_kernel_t>(plan.kernel), plan.grid, plan.block, plan.lds, s, a.in, a.w, a.ep.comp,
-                     a.nx, a.ny, a.p_total, a.ohw, a.ohw_magic, a.ihw, a.ic2, a.units_pad, a.ocpp, geom, a);
-  return hipGetLastError();
-}
 #define RV(TM, TN)                                                                                           \
   { "k_gemm1x1_res<" #TM "," #TN ">", 4 * TM * 32, TN * 32, k_gemm1x1_res<TM, TN, 0>,                        \
     {k_gemm1x1_res<TM, TN, 8>, k_gemm1x1_res<TM, TN, 16>, k_gemm1x1_res<TM, TN, 32>}, nullptr, {nullptr, nullptr, nullptr} }
@@ -464,7 +457,7 @@ int gemm1x1_res_pick(const GemmArgs &a, int nbatch)
 
 const char *gemm1x1_res_name(int v) { return kRes[v].name; }
 
-hipError_t launch_gemm1x1_res(const GemmArgs &a0, int v, hipStream_t s, LaunchPlan<GemmArgs> *plan)
+hipError_t plan_gemm1x1_res(LaunchPlan &plan, const GemmArgs &a0, int v, hipStream_t s)
 {
   const ResVariant &k = kRes[v];
   GemmArgs a = a0;
@@ -483,21 +476,14 @@ hipError_t launch_gemm1x1_res(const GemmArgs &a0, int v, hipStream_t s, LaunchPl
   if (!kernel) return hipErrorInvalidValue;
   a.u1_magic = div_magic(a.units_pad + 1);
   const size_t lds_bytes = res_lds_bytes(a, k.p_t);
-  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     (int)lds_bytes);
-  if (e != hipSuccess) return e;
   dim3 grid(8 * a.ny * ((a.nx + 7) / 8));
-  if (a.stride_h > 255 || a.stride_w > 255 || a.oc2 >= 4096) return hipErrorInvalidValue;   // geom's fields
-  LaunchPlan<GemmArgs> local;
-  LaunchPlan<GemmArgs> *p = plan ? plan : &local;
-  p->kernel = reinterpret_cast<void (*)(GemmArgs)>(kernel);
-  p->grid = grid;
-  p->block = dim3(kBlock);
-  p->lds = (unsigned)lds_bytes;
-  p->args = a;
-  p->enqueue = res_enqueue;
-  p->name = k.name;   // (nhwc output: the handle could not tell at creation whether the lean epilogue applies)
-  return plan_first_launch(p, s);
+  if (a.stride_h > 255 || a.stride_w > 255 || a.oc2 >= 4096 || a.units_pad >= 65536 || a.ocpp != up(a.oc2 * 16, kOcTile))
+    return hipErrorInvalidValue;   // the packed arguments' fields
+  const bool dense = a.stride_h == 1 && a.stride_w == 1 && a.iw == a.ow;
+  const unsigned geom = (unsigned)a.stride_h | (unsigned)a.stride_w << 8 | (dense ? 1u << 16 : 0u) | (unsigned)a.oc2 << 20;
+  plan.name = k.name;   // (nhwc output: the handle could not tell at creation whether the lean epilogue applies)
+  return plan_set(plan, kernel, grid, dim3(kBlock), lds_bytes, a, s, ArgIn{a.in}, a.w, a.ep.comp, ArgBlock{}, a.nx, a.ny, a.p_total,
+                  a.ohw, a.ohw_magic, a.ihw, (unsigned)a.ic2 | (unsigned)a.units_pad << 16, geom, ArgOut{a.out});
 }
 
 }  // namespace ehip

@@ -75,18 +75,21 @@ struct PixInfo {
 
 // geom = stride_h | stride_w << 8 | dense << 16 | nb << 20 (channel blocks of 4 x TM x 32)
 // (the leading arguments are what the first tile's loads, the per-channel constants and the weight loads need: they
-// arrive in scalar registers with the wave, while the rest of the argument block is still being fetched;
-// owiw = ow | iw << 16; consts = [3][ocpp]: scale, shift, compensation, one allocation)
+// arrive in scalar registers with the wave, while the rest of the argument structure (`rest`, see LaunchPlan) is still
+// being fetched; owiw = ow | iw << 16; nreg_oc = runs | ocpp / 256 << 16; consts = [3][ocpp]: scale, shift, compensation,
+// one allocation)
 #define EHIP_WRES_HEAD                                                                                                  \
-  const uint8_t *in, const int8_t *w, const float *consts, int p_total, int ohw, unsigned ohw_magic, int ihw, int ocpp, \
-      unsigned geom, int nreg, unsigned owiw, unsigned ow_magic
+  const uint8_t *in, const int8_t *w, const float *consts, const GemmArgs *rest, int p_total, int ohw, unsigned ohw_magic, \
+      int ihw, unsigned geom, unsigned nreg_oc, unsigned owiw, unsigned ow_magic
 // NW waves per workgroup: four, two workgroups per CU; or eight in one workgroup per CU, which then share ONE copy
 // of every pixel tile (1024 input channels, where a wave can only hold the weights of 32 channels: eight waves own
 // the 256 channels that four own with fewer input channels)
 template <int NKS, int TM, int SUM, int NW>   // SUM: 0 none, 1 the old output is u8, 2 it is s8
-__global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void k_gemm1x1_wres(EHIP_WRES_HEAD, GemmArgs rest)
+__global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void k_gemm1x1_wres(EHIP_WRES_HEAD, void *out)
 {
-  GemmArgs a = rest;
+  GemmArgs a = load_args(rest);
+  const int ocpp = (int)(nreg_oc >> 16) * kOcTile, nreg = (int)(nreg_oc & 0xffffu);
+  a.out = out;
   a.in = in; a.w = w; a.p_total = p_total; a.ohw = ohw; a.ohw_magic = ohw_magic;
   a.ihw = ihw; a.ic2 = 2 * NKS; a.ocpp = ocpp; a.ow = (int)(owiw & 0xffffu); a.iw = (int)(owiw >> 16); a.ow_magic = ow_magic;
   constexpr int stage_bytes = NKS * 1024 + (SUM ? NW * TM * 1024 : 0);
@@ -367,18 +370,8 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void k_gemm1x1_wres(EHIP_
 }
 
 namespace {
-typedef void (*wres_kernel_t)(EHIP_WRES_HEAD, GemmArgs);
+typedef void (*wres_kernel_t)(EHIP_WRES_HEAD, void *out);
 constexpr size_t kWresLds = 80 * 1024;   // two workgroups per CU
-
-hipError_t wres_enqueue(const LaunchPlan<GemmArgs> &plan, hipStream_t s)
-{
-  const GemmArgs &a = plan.args;
-  const bool dense = a.stride_h == 1 && a.stride_w == 1 && a.iw == a.ow;
-  const unsigned geom = (unsigned)a.stride_h | (unsigned)a.stride_w << 8 | (dense ? 1u << 16 : 0u) | (unsigned)a.ny << 20;
-  hipLaunchKernelGGL(reinterpret_cast<wres_kernel_t>(plan.kernel), plan.grid, plan.block, plan.lds, s, a.in, a.w, a.ep.scale, a.p_total,
-                     a.ohw, a.ohw_magic, a.ihw, a.ocpp, geom, a.nx, (unsigned)a.ow | (unsigned)a.iw << 16, a.ow_magic, a);
-  return hipGetLastError();
-}
 
 // TM: 32-channel tiles per wave.  Two with up to 512 input channels (the weights of 64 channels are 128 registers),
 // one with 1024.
@@ -478,7 +471,7 @@ bool gemm1x1_wres_applies(const GemmArgs &a, int nbatch)
   return wres_geom(a, g);
 }
 
-hipError_t launch_gemm1x1_wres(const GemmArgs &a0, hipStream_t s, LaunchPlan<GemmArgs> *plan)
+hipError_t plan_gemm1x1_wres(LaunchPlan &plan, const GemmArgs &a0, hipStream_t s)
 {
   GemmArgs a = a0;
   a.lean = lean_mode(a.ep, false);
@@ -491,19 +484,13 @@ hipError_t launch_gemm1x1_wres(const GemmArgs &a0, hipStream_t s, LaunchPlan<Gem
   a.wr_region = g.tiles;
   a.wr_stage = g.stage;
   a.wr_nbuf = g.nbuf;
-  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     (int)g.lds_bytes);
-  if (e != hipSuccess) return e;
-  LaunchPlan<GemmArgs> local;
-  LaunchPlan<GemmArgs> *p = plan ? plan : &local;
-  p->kernel = reinterpret_cast<void (*)(GemmArgs)>(kernel);
-  p->grid = dim3(8 * g.nb * ((g.nreg + 7) / 8));
-  p->block = dim3(g.nw * 64);
-  p->lds = (unsigned)g.lds_bytes;
-  p->args = a;
-  p->enqueue = wres_enqueue;
-  p->name = "k_gemm1x1_wres";
-  return plan_first_launch(p, s);
+  if (a.nx >= 65536 || a.ocpp % kOcTile || a.ocpp / kOcTile >= 65536) return hipErrorInvalidValue;   // nreg_oc's fields
+  const bool dense = a.stride_h == 1 && a.stride_w == 1 && a.iw == a.ow;
+  const unsigned geom = (unsigned)a.stride_h | (unsigned)a.stride_w << 8 | (dense ? 1u << 16 : 0u) | (unsigned)a.ny << 20;
+  plan.name = "k_gemm1x1_wres";
+  return plan_set(plan, kernel, dim3(8 * g.nb * ((g.nreg + 7) / 8)), dim3(g.nw * 64), g.lds_bytes, a, s, ArgIn{a.in}, a.w, a.ep.scale,
+                  ArgBlock{}, a.p_total, a.ohw, a.ohw_magic, a.ihw, geom, (unsigned)a.nx | (unsigned)(a.ocpp / kOcTile) << 16,
+                  (unsigned)a.ow | (unsigned)a.iw << 16, a.ow_magic, ArgOut{a.out});
 }
 
 }  // namespace ehip

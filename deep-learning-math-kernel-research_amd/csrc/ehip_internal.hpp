@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <stdlib.h>
+#include <string.h>
 #include <string>
 
 #include "euler_hip.h"
@@ -137,70 +138,94 @@ struct WinoFusedArgs {
   int tile;             // tile size A: 6 (or 0), 5, 4
   int out_nhwc;         // output as [n][h][w][c] (c % 16 == 0)
   int nx, ny;           // set by the launcher: blocks of 32 tiles, of 64 channels
+  int slots;            // set by the lanes launcher: workgroups per XCD and channel block
   float4 *tpart;        // first-stage results parked between the two passes of the 512-channel lanes kernel (wino_lanes_tpart_bytes)
   long long *trace;     // development aid, normally null (see EHIP_TRACE)
 };
 
 // ---- launch plans -------------------------------------------------------------------------------
-// What a launcher works out from the layer -- kernel, grid, LDS size, derived arguments, the EHIP_* knobs
-// read from the environment, the one-off hipFuncSetAttribute -- is kept in the handle after the first
-// launch: later executes of the handle patch the tensor pointers into the kept argument block and launch.
-template <typename Args>
+// Everything about a launch but the tensors is worked out once, when the handle is prepared (planned): kernel, grid,
+// LDS size, the derived arguments, the EHIP_* knobs read from the environment.  The argument structure goes to device
+// memory owned by the handle (written on the stream that packs the weights, so it is there when they are), and a launch
+// passes its ADDRESS beside the tensors and the few scalars a wave's first loads need: at most kMaxKernarg bytes.
+// What that buys: HIP writes kernel arguments into device memory across PCIe, and a launch with 300 bytes of them
+// costs the host 3.4 us where 16-96 bytes cost 2.6 (128: 3.25, 256: 3.45; empty kernel, back to back) -- as long as a
+// small layer's kernel takes on the GPU.
+constexpr size_t kMaxKernarg = 104;   // (the step is between 104 and 128)
+constexpr size_t kArgBlock = 512;     // device memory of one argument structure
 struct LaunchPlan {
-  bool valid = false;
-  void (*kernel)(Args) = nullptr;
+  void *args_dev = nullptr;     // kArgBlock bytes of device memory, set when the handle is created
+  hipFunction_t fn = nullptr;   // of the device the handle was prepared on
   dim3 grid, block;
   unsigned lds = 0;
-  Args args;
-  const char *name = nullptr;   // set by a launcher whose choice of kernel the handle cannot know beforehand
-  // set by a launcher whose kernel takes leading scalar arguments besides the block (`kernel` is then that
-  // kernel's pointer under the one-argument type): how to launch the plan
-  hipError_t (*enqueue)(const LaunchPlan &, hipStream_t) = nullptr;
+  const char *name = nullptr;   // set by a planner whose choice of kernel the handle cannot know beforehand
+  unsigned karg_bytes = 0;
+  unsigned in_at = kMaxKernarg, out_at = kMaxKernarg, bias_at = kMaxKernarg;   // (kMaxKernarg: none; see plan_launch)
+  alignas(8) unsigned char karg[kMaxKernarg] = {};
 };
-template <typename Args>
-inline hipError_t plan_launch(LaunchPlan<Args> *plan, void (*kernel)(Args), dim3 grid, dim3 block, size_t lds, const Args &a,
-                              hipStream_t s)
-{
-  hipLaunchKernelGGL(kernel, grid, block, lds, s, a);
-  const hipError_t e = hipGetLastError();
-  if (plan && e == hipSuccess) {   // kept only once the first launch has gone out
-    plan->kernel = kernel;
-    plan->grid = grid;
-    plan->block = block;
-    plan->lds = (unsigned)lds;
-    plan->args = a;
-    plan->valid = true;
+// kernel arguments that a launch fills in (a `fixed` pointer that is not null is filled in for good)
+struct ArgIn { const void *fixed; };
+struct ArgOut { void *fixed; };
+struct ArgBias {};
+struct ArgBlock {};   // the address of the argument structure
+
+hipError_t launch_store_args(const void *args, size_t bytes, void *dst_dev, hipStream_t s);   // (ehip_prepare.hip)
+
+struct KernargWriter {
+  LaunchPlan &p;
+  bool fits = true;
+  void raw(const void *v, size_t bytes, unsigned *at = nullptr)
+  {
+    const size_t off = (p.karg_bytes + bytes - 1) / bytes * bytes;   // natural alignment: pointers and 32-bit values
+    if (off + bytes > kMaxKernarg) { fits = false; return; }
+    if (v) memcpy(p.karg + off, v, bytes);
+    if (at) *at = (unsigned)off;
+    p.karg_bytes = (unsigned)(off + bytes);
   }
+  template <typename P> void put(const P &v) { static_assert(sizeof(P) == 4 || sizeof(P) == 8, "scalar"); raw(&v, sizeof(P)); }
+  template <typename P> void put(const ArgIn &v) { raw(&v.fixed, 8, v.fixed ? nullptr : &p.in_at); }
+  template <typename P> void put(const ArgOut &v) { raw(&v.fixed, 8, v.fixed ? nullptr : &p.out_at); }
+  template <typename P> void put(const ArgBias &) { raw(nullptr, 8, &p.bias_at); }
+  template <typename P> void put(const ArgBlock &) { raw(&p.args_dev, 8); }
+};
+// `a` in the order of the kernel's parameters, each converted to its parameter's type
+template <typename Args, typename... P, typename... A>
+inline hipError_t plan_set(LaunchPlan &p, void (*kernel)(P...), dim3 grid, dim3 block, size_t lds, const Args &args, hipStream_t s, A... a)
+{
+  static_assert(sizeof...(P) == sizeof...(A), "one value per kernel parameter");
+  static_assert(sizeof(Args) <= kArgBlock && sizeof(Args) % 4 == 0, "argument structure");
+  p.grid = grid;
+  p.block = block;
+  p.lds = (unsigned)lds;
+  p.karg_bytes = 0;
+  p.in_at = p.out_at = p.bias_at = kMaxKernarg;
+  KernargWriter w{p};
+  (w.put<P>(a), ...);
+  if (!w.fits) return hipErrorInvalidValue;
+  hipError_t e = hipSuccess;
+  if (lds > 48 * 1024)
+    e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  if (e == hipSuccess) e = hipGetFuncBySymbol(&p.fn, reinterpret_cast<const void *>(kernel));
+  if (e == hipSuccess) e = launch_store_args(&args, sizeof(Args), p.args_dev, s);
   return e;
 }
-// A launcher that fills a plan by hand launches through this: the plan becomes valid when the launch has gone out.
-template <typename Args>
-inline hipError_t plan_first_launch(LaunchPlan<Args> *p, hipStream_t s)
+// The kept plan is only read: the tensors of this call go into a copy of the kernel arguments, so executes of one
+// handle from several threads or streams never see each other's pointers.
+inline hipError_t plan_launch(const LaunchPlan &p, const void *in, void *out, const void *bias, hipStream_t s)
 {
-  hipError_t e;
-  if (p->enqueue) {
-    e = p->enqueue(*p, s);
-  } else {
-    hipLaunchKernelGGL(p->kernel, p->grid, p->block, p->lds, s, p->args);
-    e = hipGetLastError();
-  }
-  p->valid = e == hipSuccess;
-  return e;
-}
-// Later launches of a valid plan: the kept plan is only read.  The tensors of this call are patched into a COPY of
-// the argument block, so executes of one handle from several threads or streams never see each other's pointers.
-template <typename Args, typename Patch>
-inline hipError_t plan_relaunch(const LaunchPlan<Args> &plan, Patch patch, hipStream_t s)
-{
-  LaunchPlan<Args> local = plan;
-  patch(local.args);
-  if (local.enqueue) return local.enqueue(local, s);
-  hipLaunchKernelGGL(local.kernel, local.grid, local.block, local.lds, s, local.args);
-  return hipGetLastError();
+  alignas(8) unsigned char k[kMaxKernarg + 8];   // (the last eight bytes take a pointer the kernel has no parameter for)
+  memcpy(k, p.karg, kMaxKernarg);
+  memcpy(k + p.in_at, &in, 8);
+  memcpy(k + p.out_at, &out, 8);
+  memcpy(k + p.bias_at, &bias, 8);
+  size_t bytes = p.karg_bytes;
+  void *extra[] = {HIP_LAUNCH_PARAM_BUFFER_POINTER, k, HIP_LAUNCH_PARAM_BUFFER_SIZE, &bytes, HIP_LAUNCH_PARAM_END};
+  return hipModuleLaunchKernel(p.fn, p.grid.x, p.grid.y, p.grid.z, p.block.x, p.block.y, p.block.z, p.lds, s, nullptr, extra);
 }
 
-// ---- launchers (implemented next to their kernels) ------------------------------------------
-hipError_t launch_gemm(const GemmArgs &a, int nbatch, int variant, hipStream_t s, LaunchPlan<GemmArgs> *plan = nullptr);
+// ---- planners and launchers (implemented next to their kernels) -----------------------------
+// A planner chooses the kernel and fills the plan; a.in / a.out null = given at each launch.
+hipError_t plan_gemm(LaunchPlan &plan, const GemmArgs &a, int nbatch, int variant, hipStream_t s);
 bool gemm_smallk_applies(int ic2, int taps, int nbatch);
 int gemm_pick_variant(int p_total, int oc2, int ic2, int nbatch, int stride);
 int gemm_variant_chunk(int variant);
@@ -210,29 +235,29 @@ const char *gemm_variant_name(int variant);
 // 1x1 layers with many input channels, blocked activations: pixel tile resident in LDS, weights streamed
 int gemm1x1_res_pick(const GemmArgs &a, int nbatch);   // variant, or -1 when the layer is not one for it
 const char *gemm1x1_res_name(int variant);
-hipError_t launch_gemm1x1_res(const GemmArgs &a, int variant, hipStream_t s, LaunchPlan<GemmArgs> *plan = nullptr);
+hipError_t plan_gemm1x1_res(LaunchPlan &plan, const GemmArgs &a, int variant, hipStream_t s);
 // 1x1 layers of 256 / 512 / 1024 input channels with the lean epilogue: weights resident in registers, pixels streamed
 bool gemm1x1_wres_applies(const GemmArgs &a, int nbatch);
-hipError_t launch_gemm1x1_wres(const GemmArgs &a, hipStream_t s, LaunchPlan<GemmArgs> *plan = nullptr);
+hipError_t plan_gemm1x1_wres(LaunchPlan &plan, const GemmArgs &a, hipStream_t s);
 
-hipError_t launch_conv3x3v(const Conv3x3Args &a, int n, int variant, hipStream_t s, LaunchPlan<Conv3x3Args> *plan = nullptr);
+hipError_t plan_conv3x3v(LaunchPlan &plan, const Conv3x3Args &a, int n, int variant, hipStream_t s);
 int conv3x3v_pick_variant(int n, int oh, int ow, int oc2, int stride);   // stride 1 or 2 (both directions); -1: rows too wide for every variant
 int conv3x3v_chunk_units(int variant, int ic2);
 int conv3x3v_num_variants();
 const char *conv3x3v_variant_name(int variant);
 
-hipError_t launch_depthwise(const DepthwiseArgs &a, hipStream_t s, LaunchPlan<DepthwiseArgs> *plan = nullptr);
+hipError_t plan_depthwise(LaunchPlan &plan, const DepthwiseArgs &a, hipStream_t s);
 hipError_t launch_depthwise_diag(const int8_t *wpacked, int g2n, void *diag, hipStream_t s);
 bool depthwise_mfma_applies(int stride, int oh, int ow, int pad_t, int pad_l, int out_type, int with_relu, float lo, float hi,
                             long long planes, int ih, int iw);
-hipError_t launch_wino_trans_input(const WinoArgs &a, hipStream_t s, LaunchPlan<WinoArgs> *plan = nullptr);
-hipError_t launch_wino_trans_output(const WinoArgs &a, hipStream_t s, LaunchPlan<WinoArgs> *plan = nullptr);
-hipError_t launch_wino_gemm_output(const WinoFusedArgs &a, hipStream_t s, LaunchPlan<WinoFusedArgs> *plan = nullptr);
+hipError_t plan_wino_trans_input(LaunchPlan &plan, const WinoArgs &a, hipStream_t s);
+hipError_t plan_wino_trans_output(LaunchPlan &plan, const WinoArgs &a, hipStream_t s);
+hipError_t plan_wino_gemm_output(LaunchPlan &plan, const WinoFusedArgs &a, hipStream_t s);
 // at most 256 input channels, u8 / s8 output: the form without an exchange between GEMMs and transform (ehip_wino_lanes.hip)
 bool wino_lanes_applies(const WinoFusedArgs &a);
 // device memory the lanes kernel needs besides the tensors (0 for most layers): a.tpart
 size_t wino_lanes_tpart_bytes(int tile, int ic2, int oc2, int t);
-hipError_t launch_wino_gemm_output_lanes(const WinoFusedArgs &a, hipStream_t s, LaunchPlan<WinoFusedArgs> *plan = nullptr);
+hipError_t plan_wino_gemm_output_lanes(LaunchPlan &plan, const WinoFusedArgs &a, hipStream_t s);
 // min / max of the transformed input: partials = 2 * a.ic2 dwords of device scratch, result = two floats
 // of device memory (min, max); three launches on `s`, nothing else
 hipError_t launch_wino_range(const WinoArgs &a, int ic_real, unsigned *partials, float *minmax_out_dev, hipStream_t s);
@@ -275,7 +300,7 @@ struct FewChArgs {
 int conv_fewch_icl(int ic, int kw);
 bool conv_fewch_applies(int ic, int kh, int kw);
 int conv_fewch_row_pitch(int icl, int kw, int iw, int ow, int stride_w, int pad_l);   // icl: conv_fewch_icl()
-hipError_t launch_conv_fewch(FewChArgs &a, hipStream_t s, LaunchPlan<FewChArgs> *plan = nullptr);
+hipError_t plan_conv_fewch(LaunchPlan &plan, FewChArgs &a, hipStream_t s);
 hipError_t launch_prepare_direct_px(const float *w, const float *bias, int oc, int ic, int icl, int kh, int kw, int ppc, int nu,
                                     int ocpp, const ehip_conv_desc_t &d, float *absmax, int8_t *wpacked, float *scale,
                                     float *shift, int *wsum, int *comp, hipStream_t s);
@@ -306,6 +331,52 @@ void set_error(const std::string &msg);
 // ---- device helpers -----------------------------------------------------------------------------
 #if defined(__HIPCC__)
 namespace ehip {
+
+// The argument structure of a launch, from the handle's device memory (LaunchPlan).  Read through the constant address
+// space: scalar loads, issued at the kernel's start like those of arguments passed by value.  Pointers are taken member
+// by member: the compiler knows that a pointer loaded from that address space is to global memory, but not one that
+// went through the copy of the whole structure (accesses through it would be flat ones).
+#if defined(__HIP_DEVICE_COMPILE__)
+#define EHIP_CONSTANT __attribute__((address_space(4)))
+#else
+#define EHIP_CONSTANT
+#endif
+__device__ __forceinline__ void load_pointers(Epilogue &e, const EHIP_CONSTANT Epilogue *c)
+{
+  e.scale = c->scale; e.shift = c->shift; e.comp = c->comp; e.shift_tab = c->shift_tab;
+}
+__device__ __forceinline__ void load_pointers(GemmArgs &a, const EHIP_CONSTANT GemmArgs *c)
+{
+  a.w = c->w; a.cls_h = c->cls_h; a.cls_w = c->cls_w; a.trace = c->trace;
+  load_pointers(a.ep, &c->ep);
+}
+__device__ __forceinline__ void load_pointers(Conv3x3Args &a, const EHIP_CONSTANT Conv3x3Args *c)
+{
+  a.w = c->w; a.trace = c->trace;
+  load_pointers(a.ep, &c->ep);
+}
+__device__ __forceinline__ void load_pointers(DepthwiseArgs &a, const EHIP_CONSTANT DepthwiseArgs *c)
+{
+  a.scale = c->scale; a.shift = c->shift; a.wdiag = c->wdiag;
+}
+__device__ __forceinline__ void load_pointers(FewChArgs &a, const EHIP_CONSTANT FewChArgs *c)
+{
+  a.w = c->w; a.cls_h = c->cls_h; a.cls_w = c->cls_w;
+  load_pointers(a.ep, &c->ep);
+}
+__device__ __forceinline__ void load_pointers(WinoArgs &a, const EHIP_CONSTANT WinoArgs *c) { a.tin = c->tin; a.tout = c->tout; }
+__device__ __forceinline__ void load_pointers(WinoFusedArgs &a, const EHIP_CONSTANT WinoFusedArgs *c)
+{
+  a.tin = c->tin; a.w = c->w; a.scale = c->scale; a.shift = c->shift; a.comp = c->comp; a.tpart = c->tpart; a.trace = c->trace;
+}
+template <typename Args>
+__device__ __forceinline__ Args load_args(const Args *p)
+{
+  const EHIP_CONSTANT Args *c = (const EHIP_CONSTANT Args *)p;
+  Args a = *(const Args *)c;
+  load_pointers(a, c);
+  return a;
+}
 
 // round-to-nearest-even float -> s32 with the x86 "integer indefinite" for NaN / out of range
 __device__ __forceinline__ int cvt_s32_rne(float f)

@@ -239,8 +239,10 @@ __device__ __forceinline__ void gather_tile_wide(const WinoArgs &, const TileCoo
 // branch-free form of the transform instead of both forms under complementary masks.
 // Cell = float4 (f32 user input) or unsigned (u8 user input: four codes per lane and pixel).
 template <typename Cell, int A = 6>
-__global__ __launch_bounds__(kBlock) void k_wino_trans_input_u8(WinoArgs a)
+__global__ __launch_bounds__(kBlock) void k_wino_trans_input_u8(const WinoArgs *rest, const void *in)
 {
+  WinoArgs a = load_args(rest);
+  a.in = in;
   constexpr int AA = A * A;
   constexpr bool kCodes = sizeof(Cell) == sizeof(unsigned);
   const int q = threadIdx.x & 3;
@@ -521,8 +523,10 @@ __device__ __forceinline__ void output_tile(const float4 *m, const float4 &bias,
 
 // grid: (ceil(t / 64), oc2); block: 64 tiles x 4 channel quads
 template <int OUT, int A = 6>
-__global__ __launch_bounds__(kBlock) void k_wino_trans_output(WinoArgs a)
+__global__ __launch_bounds__(kBlock) void k_wino_trans_output(const WinoArgs *rest, void *out, const float *bias_)
 {
+  WinoArgs a = load_args(rest);
+  a.out = out; a.bias = bias_;
   constexpr int AA = A * A;
   const int q = threadIdx.x & 3;
   const int t = blockIdx.x * 64 + (threadIdx.x >> 2);
@@ -579,8 +583,10 @@ __global__ __launch_bounds__(kBlock) void k_wino_trans_output(WinoArgs a)
 // The ring then runs ahead over the wave's positions as one flat sequence of steps -- with a ring of one position
 // every position costs a trip to memory (64 -> 64: 36 MFMAs per wave in 16 K clocks).
 template <int KS, int A = 6, bool SUM = false, int NT = 1, int NH = 2, int NKSF = 0>
-__global__ __launch_bounds__(kBlock, 1) void k_wino_gemm_output(WinoFusedArgs a)
+__global__ __launch_bounds__(kBlock, 1) void k_wino_gemm_output(const WinoFusedArgs *rest, void *out, const float *bias_)
 {
+  WinoFusedArgs a = load_args(rest);
+  a.out = out; a.bias = bias_;
   constexpr int AA = A * A, PW = (AA + 3) / 4, CN = PW * 24, NJ = (CN + 63) / 64;
   extern __shared__ float4 xl[];   // [AA][32 tiles][8 cells of 4 channels], cell ^ ((tile / 2) & 7)
   const int tid = threadIdx.x;
@@ -650,7 +656,7 @@ __global__ __launch_bounds__(kBlock, 1) void k_wino_gemm_output(WinoFusedArgs a)
       const int row = idx >> 3, cell = idx & 7;
       const int i = row / 3, arr = row - 3 * i;
       const int p = p0 + i < AA ? p0 + i : AA - 1;   // (a wave with fewer positions: rows nobody reads)
-      const float *src = arr == 0 ? a.scale : (arr == 1 ? a.shift : reinterpret_cast<const float *>(a.comp));
+      const float *src = a.scale + (size_t)arr * AA * a.ocpp;   // (scale, shift, compensation: one allocation, [3][AA][ocpp])
       cst[j] = *reinterpret_cast<const float4 *>(src + (long long)p * a.ocpp + oc0 + 32 * h + 4 * cell);
     }
   };
@@ -795,11 +801,8 @@ __global__ __launch_bounds__(kBlock, 1) void k_wino_gemm_output(WinoFusedArgs a)
   }
 }
 
-hipError_t launch_wino_trans_input(const WinoArgs &a0, hipStream_t s, LaunchPlan<WinoArgs> *plan)
+hipError_t plan_wino_trans_input(LaunchPlan &plan, const WinoArgs &a0, hipStream_t s)
 {
-  if (plan && plan->valid) {   // everything but the tensors is as on the first launch
-    return plan_relaunch(*plan, [&](WinoArgs &x) { x.in = a0.in; }, s);
-  }
   WinoArgs a = a0;
   {
     const unsigned long long bytes = (unsigned long long)a.n * a.ic2 * a.ih * a.iw * 16 * (a.in_u8 ? 1 : 4);
@@ -811,20 +814,17 @@ hipError_t launch_wino_trans_input(const WinoArgs &a0, hipStream_t s, LaunchPlan
   a.nblocks = (a.t + 63) / 64;
   a.items_per_xcd = (int)(((long long)a.nblocks * a.ic2 + 7) / 8);
   dim3 grid(8 * a.items_per_xcd, 1);
-  void (*kern)(WinoArgs) = nullptr;
+  void (*kern)(const WinoArgs *, const void *) = nullptr;
   if (a.tile == 4) kern = a.in_u8 ? k_wino_trans_input_u8<unsigned, 4> : k_wino_trans_input_u8<float4, 4>;
   else if (a.tile == 5) kern = a.in_u8 ? k_wino_trans_input_u8<unsigned, 5> : k_wino_trans_input_u8<float4, 5>;
   else kern = a.in_u8 ? k_wino_trans_input_u8<unsigned, 6> : k_wino_trans_input_u8<float4, 6>;
-  return plan_launch(plan, kern, grid, dim3(kBlock), 0, a, s);
+  return plan_set(plan, kern, grid, dim3(kBlock), 0, a, s, ArgBlock{}, ArgIn{a.in});
 }
 
-hipError_t launch_wino_trans_output(const WinoArgs &a, hipStream_t s, LaunchPlan<WinoArgs> *plan)
+hipError_t plan_wino_trans_output(LaunchPlan &plan, const WinoArgs &a, hipStream_t s)
 {
-  if (plan && plan->valid) {   // everything but the tensors is as on the first launch
-    return plan_relaunch(*plan, [&](WinoArgs &x) { x.out = a.out; x.bias = a.bias; }, s);
-  }
   dim3 grid((a.t + 63) / 64, a.oc2);
-  void (*kern)(WinoArgs) = nullptr;
+  void (*kern)(const WinoArgs *, void *, const float *) = nullptr;
 #define EHIP_WO(A)                                                                                         \
   kern = a.out_type == EHIP_U8 ? k_wino_trans_output<EHIP_U8, A>                                           \
       : (a.out_type == EHIP_S8 ? k_wino_trans_output<EHIP_S8, A> : k_wino_trans_output<EHIP_F32, A>)
@@ -832,18 +832,15 @@ hipError_t launch_wino_trans_output(const WinoArgs &a, hipStream_t s, LaunchPlan
   else if (a.tile == 5) EHIP_WO(5);
   else EHIP_WO(6);
 #undef EHIP_WO
-  return plan_launch(plan, kern, grid, dim3(kBlock), 0, a, s);
+  return plan_set(plan, kern, grid, dim3(kBlock), 0, a, s, ArgBlock{}, ArgOut{a.out}, ArgBias{});
 }
 
 // k-steps per ring block: the largest of 8, 4, 2 that divides the k-steps of a position
-hipError_t launch_wino_gemm_output(const WinoFusedArgs &a0, hipStream_t s, LaunchPlan<WinoFusedArgs> *plan)
+hipError_t plan_wino_gemm_output(LaunchPlan &plan, const WinoFusedArgs &a0, hipStream_t s)
 {
-  if (plan && plan->valid) {   // everything but the tensors is as on the first launch
-    return plan_relaunch(*plan, [&](WinoFusedArgs &x) { x.out = a0.out; x.bias = a0.bias; }, s);
-  }
   WinoFusedArgs a = a0;
   const int A = a.tile ? a.tile : 6, AA = A * A;
-  if (wino_lanes_applies(a)) return launch_wino_gemm_output_lanes(a, s, plan);
+  if (wino_lanes_applies(a)) return plan_wino_gemm_output_lanes(plan, a, s);
   const int ntb = A == 4 ? 2 : 1;   // blocks of 32 tiles per workgroup
   a.nx = (a.t + 32 * ntb - 1) / (32 * ntb);
   // 64 channels per workgroup; 32 where that would leave a quarter of the CUs or more without a workgroup
@@ -860,7 +857,7 @@ hipError_t launch_wino_gemm_output(const WinoFusedArgs &a0, hipStream_t s, Launc
   if (const char *env = getenv("EHIP_WINO_KS")) ks_max = atoi(env);
   bool flat = true;   // 64 / 128 input channels: the ring runs ahead over positions
   if (const char *env = getenv("EHIP_WINO_FLAT")) flat = env[0] != '0';
-  void (*kernel)(WinoFusedArgs) = nullptr;
+  void (*kernel)(const WinoFusedArgs *, void *, const float *) = nullptr;
 #define EHIP_WF1(AV, SV, NHV)                                                                          \
   kernel = (nks == 2 && flat) ? k_wino_gemm_output<8, AV, SV, AV == 4 ? 2 : 1, NHV, 2>                  \
       : (nks == 4 && flat) ? k_wino_gemm_output<8, AV, SV, AV == 4 ? 2 : 1, NHV, 4>                     \
@@ -884,9 +881,7 @@ hipError_t launch_wino_gemm_output(const WinoFusedArgs &a0, hipStream_t s, Launc
 #undef EHIP_WF
 #undef EHIP_WF1
   if (nks % 2 != 0) return hipErrorInvalidValue;
-  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  if (e != hipSuccess) return e;
-  return plan_launch(plan, kernel, grid, dim3(kBlock), lds, a, s);
+  return plan_set(plan, kernel, grid, dim3(kBlock), lds, a, s, ArgBlock{}, ArgOut{a.out}, ArgBias{});
 }
 
 // partials: 2 * a.ic2 dwords of device memory; minmax_out_dev: two floats of device memory

@@ -197,8 +197,10 @@ __device__ __forceinline__ void out_1d(const float *f, float *o)
 // Workgroup = 32 channels x 32 tiles (one block of the blocked tinput); wave = (half of the channels, half of the
 // tiles); NKS = k-steps of 64 channels per position (1, 2 or 4).
 template <int A, bool SUM, int NKS>
-__global__ __launch_bounds__(kBlock, 2) void k_wino_gemm_output_lanes(WinoFusedArgs a)
+__global__ __launch_bounds__(kBlock, 2) void k_wino_gemm_output_lanes(const WinoFusedArgs *rest, void *out, const float *bias_)
 {
+  WinoFusedArgs a = load_args(rest);
+  a.out = out; a.bias = bias_;
   constexpr int AA = A * A, D = 8, STEPS = AA * NKS;
   extern __shared__ float4 cl[];   // [AA][3][8 quads of the workgroup's 32 channels]: scale, shift, compensation
   const int tid = threadIdx.x;
@@ -251,7 +253,7 @@ __global__ __launch_bounds__(kBlock, 2) void k_wino_gemm_output_lanes(WinoFusedA
       int idx = tid + j * kBlock;
       idx = idx < AA * 24 ? idx : AA * 24 - 1;
       const int p = idx / 24, rem = idx - 24 * p, arr = rem >> 3, cell = rem & 7;
-      const float *src = arr == 0 ? a.scale : (arr == 1 ? a.shift : reinterpret_cast<const float *>(a.comp));
+      const float *src = a.scale + (size_t)arr * AA * a.ocpp;   // (scale, shift, compensation: one allocation, [3][AA][ocpp])
       cst[j] = *reinterpret_cast<const float4 *>(src + (long long)p * a.ocpp + oc0 + 4 * cell);
     }
 #pragma unroll
@@ -340,8 +342,10 @@ __global__ __launch_bounds__(kBlock, 2) void k_wino_gemm_output_lanes(WinoFusedA
 // a.nx = blocks of 16 NW tiles, a.ny = groups of 16 packed rows; grid = 8 XCDs x a.ny x slots, a slot walks over the
 // blocks slot * 8 + xcd, + 8 * slots, ...
 template <int A, bool SUM, int NKS, int NW = 4>
-__global__ __launch_bounds__(64 * NW, 2) void k_wino_gemm_output_lanes_wres(WinoFusedArgs a)
+__global__ __launch_bounds__(64 * NW, 2) void k_wino_gemm_output_lanes_wres(const WinoFusedArgs *rest, void *out, const float *bias_)
 {
+  WinoFusedArgs a = load_args(rest);
+  a.out = out; a.bias = bias_;
   constexpr int TB = 64 * NW;   // threads; a block of tiles of the workgroup = 16 NW tiles = NW / 2 blocks of 32
   constexpr int AA = A * A, STEPS = AA * NKS;
   constexpr int D = A == 6 ? (SUM ? 6 : 12) : (A == 5 ? 5 : 8);   // divides STEPS: a ring slot holds the same steps in every block
@@ -356,7 +360,7 @@ __global__ __launch_bounds__(64 * NW, 2) void k_wino_gemm_output_lanes_wres(Wino
   const int xcd = blockIdx.x & 7, seq = blockIdx.x >> 3;
   const int by = seq % a.ny;
   const int slot = seq / a.ny;
-  const int item_step = 8 * (int)(gridDim.x / (8u * a.ny));
+  const int item_step = 8 * a.slots;
   int item = slot * 8 + xcd;
   if (item >= a.nx) return;          // whole workgroup
   // the workgroup's 16 channels are one block of the output: of the group of 32 packed rows (row 8 gq + 4 h + j holds
@@ -415,7 +419,7 @@ __global__ __launch_bounds__(64 * NW, 2) void k_wino_gemm_output_lanes_wres(Wino
       int idx = tid + j * TB;
       idx = idx < AA * 12 ? idx : AA * 12 - 1;
       const int p = idx / 12, rem = idx - 12 * p, arr = rem >> 2, gq = rem & 3;
-      const float *src = arr == 0 ? a.scale : (arr == 1 ? a.shift : reinterpret_cast<const float *>(a.comp));
+      const float *src = a.scale + (size_t)arr * AA * a.ocpp;   // (scale, shift, compensation: one allocation, [3][AA][ocpp])
       cst[j] = *reinterpret_cast<const float4 *>(src + (long long)p * a.ocpp + oc0 + 16 * h + 4 * gq);
     }
 #pragma unroll
@@ -654,8 +658,10 @@ __device__ __forceinline__ void finish_columns(const WinoFusedArgs &a, float (&T
 // 16 bytes per lane and value in lane order.
 // a.tpart: [a.ny][a.nx][NW][(A - 2) x C0][64 lanes] float4, C0 = columns of the first pass (wino_lanes_tpart_bytes).
 template <int A, bool SUM, int NKS, int NW>
-__global__ __launch_bounds__(64 * NW, 2) void k_wino_gemm_output_lanes_wres2(WinoFusedArgs a)
+__global__ __launch_bounds__(64 * NW, 2) void k_wino_gemm_output_lanes_wres2(const WinoFusedArgs *rest, void *out, const float *bias_)
 {
+  WinoFusedArgs a = load_args(rest);
+  a.out = out; a.bias = bias_;
   static_assert(A == 6 || A == 5, "tile sizes with a column-wise transform");
   constexpr int TB = 64 * NW;
   constexpr int AA = A * A, M = A - 2;
@@ -673,7 +679,7 @@ __global__ __launch_bounds__(64 * NW, 2) void k_wino_gemm_output_lanes_wres2(Win
   const int xcd = blockIdx.x & 7, seq = blockIdx.x >> 3;
   const int by = seq % a.ny;
   const int slot = seq / a.ny;
-  const int item_step = 8 * (int)(gridDim.x / (8u * a.ny));
+  const int item_step = 8 * a.slots;
   const int item0 = slot * 8 + xcd;
   if (item0 >= a.nx) return;          // whole workgroup
   const int oc0 = (by >> 1) * 32, h = by & 1;   // (the workgroup's 16 channels: see the kernel above)
@@ -739,7 +745,7 @@ __global__ __launch_bounds__(64 * NW, 2) void k_wino_gemm_output_lanes_wres2(Win
           int idx = tid + j * TB;
           idx = idx < AA * 12 ? idx : AA * 12 - 1;
           const int p = idx / 12, rem = idx - 12 * p, arr = rem >> 2, gq = rem & 3;
-          const float *src = arr == 0 ? a.scale : (arr == 1 ? a.shift : reinterpret_cast<const float *>(a.comp));
+          const float *src = a.scale + (size_t)arr * AA * a.ocpp;   // (scale, shift, compensation: one allocation, [3][AA][ocpp])
           cst[j] = *reinterpret_cast<const float4 *>(src + (long long)p * a.ocpp + oc0 + 16 * h + 4 * gq);
         }
       }
@@ -850,8 +856,9 @@ __global__ __launch_bounds__(64 * NW, 2) void k_wino_gemm_output_lanes_wres2(Win
 }
 
 namespace {
+typedef void (*lanes_kernel_t)(const WinoFusedArgs *, void *, const float *);
 template <int A, bool SUM>
-auto pick_wres_nks(int nks64, int nw) -> void (*)(WinoFusedArgs)
+auto pick_wres_nks(int nks64, int nw) -> lanes_kernel_t
 {
   switch (nks64) {
     case 1: return k_wino_gemm_output_lanes_wres<A, SUM, 1>;
@@ -865,7 +872,7 @@ auto pick_wres_nks(int nks64, int nw) -> void (*)(WinoFusedArgs)
     default: return nullptr;
   }
 }
-auto pick_wres(int A, bool sum, int nks64, int nw) -> void (*)(WinoFusedArgs)
+auto pick_wres(int A, bool sum, int nks64, int nw) -> lanes_kernel_t
 {
   if (A == 4) return sum ? pick_wres_nks<4, true>(nks64, nw) : pick_wres_nks<4, false>(nks64, nw);
   if (A == 5) return sum ? pick_wres_nks<5, true>(nks64, nw) : pick_wres_nks<5, false>(nks64, nw);
@@ -916,12 +923,12 @@ bool wino_lanes_applies(const WinoFusedArgs &a)
       !(env && env[0] == '0');
 }
 
-hipError_t launch_wino_gemm_output_lanes(const WinoFusedArgs &a0, hipStream_t s, LaunchPlan<WinoFusedArgs> *plan)
+hipError_t plan_wino_gemm_output_lanes(LaunchPlan &plan, const WinoFusedArgs &a0, hipStream_t s)
 {
   WinoFusedArgs a = a0;
   const int A = a.tile ? a.tile : 6, AA = A * A;
   const int nks64 = (a.ic2 + 3) / 4;
-  void (*kernel)(WinoFusedArgs) = nullptr;
+  lanes_kernel_t kernel = nullptr;
   const char *env = getenv("EHIP_WINO_LANES_WRES");
   if (!(env && env[0] == '0') || nks64 == 3 || nks64 > 4) {   // (the streamed form below has 1, 2 and 4 k-steps only)
     // weights resident: the weights of 16 channels in LDS, workgroups walking over blocks of tiles.  Up to 128 input
@@ -941,13 +948,11 @@ hipError_t launch_wino_gemm_output_lanes(const WinoFusedArgs &a0, hipStream_t s,
     slots = slots < 1 ? 1 : slots;
     const int need = (a.nx + 7) / 8;
     slots = slots < need ? slots : need;
+    a.slots = slots;
     kernel = pick_wres(A, a.with_sum != 0, nks64, nw);
     if (!kernel) return hipErrorInvalidValue;
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e != hipSuccess) return e;
-    const hipError_t rc = plan_launch(plan, kernel, dim3(8 * a.ny * slots), dim3(64 * nw), lds, a, s);
-    if (plan && rc == hipSuccess) plan->name = "k_wino_gemm_output_lanes_wres";
-    return rc;
+    plan.name = "k_wino_gemm_output_lanes_wres";
+    return plan_set(plan, kernel, dim3(8 * a.ny * slots), dim3(64 * nw), lds, a, s, ArgBlock{}, ArgOut{a.out}, ArgBias{});
   }
   a.nx = (a.t + 31) / 32;
   a.ny = (a.oc2 * 16 + 31) / 32;
@@ -961,9 +966,8 @@ hipError_t launch_wino_gemm_output_lanes(const WinoFusedArgs &a0, hipStream_t s,
   else EHIP_WL(6);
 #undef EHIP_WL
   const size_t lds = (size_t)AA * 24 * sizeof(float4);
-  const hipError_t rc = plan_launch(plan, kernel, dim3(8 * a.ny * ((a.nx + 7) / 8)), dim3(kBlock), lds, a, s);
-  if (plan && rc == hipSuccess) plan->name = "k_wino_gemm_output_lanes";
-  return rc;
+  plan.name = "k_wino_gemm_output_lanes";
+  return plan_set(plan, kernel, dim3(8 * a.ny * ((a.nx + 7) / 8)), dim3(kBlock), lds, a, s, ArgBlock{}, ArgOut{a.out}, ArgBias{});
 }
 
 }  // namespace ehip
