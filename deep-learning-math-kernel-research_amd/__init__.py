@@ -2,7 +2,9 @@
 
 The compute lives in ``libeuler_hip.so`` (hand-written HIP kernels behind ``include/euler_hip.h``);
 this module only loads it with ctypes and mirrors the descriptor of ``eld_conv_t`` so that tests and
-benchmarks read like the reference's harness: fill a descriptor, ``setup()``, then ``execute()``.
+benchmarks read like the reference's harness: fill a descriptor, ``setup()``, then ``execute()``.  The
+calls of a running model's loop (execute, input quantization, activation reorders) go through a small
+extension module instead of ctypes (``csrc/ehip_call.cpp``).
 Device memory and streams come from the caller (torch tensors or raw device pointers).
 
 There is no CPU fallback: if the library is missing or fails to load, importing this package
@@ -95,9 +97,20 @@ EXPORTED_SYMBOLS = (
 )
 
 
+try:
+    from . import _ehip_call
+except ImportError as e:
+    raise ImportError("_ehip_call.so is not built; run `python -c 'import __graft_entry__ as g; g.build()'`") from e
+
+
 def _check(rc):
     if rc != EHIP_OK:
         raise EulerHipError(rc, lib.ehip_last_error().decode(errors="replace"))
+
+
+_ehip_call.bind(*(ctypes.cast(f, ctypes.c_void_p).value for f in (
+    lib.ehip_conv_execute, lib.ehip_quantize_input_u8, lib.ehip_reorder_nchw_to_blocked,
+    lib.ehip_reorder_blocked_to_nchw)), _check)
 
 
 def _ptr(x):
@@ -142,15 +155,16 @@ def make_desc(n, ic, oc, ih, iw, kh=1, kw=1, pad=0, stride=1, g=1, algorithm=CON
     return d
 
 
-class Conv:
+class Conv(_ehip_call.ConvBase):
     """One convolution layer on the GPU: setup (ehip_conv_create), first-run weight preparation
-    (ehip_conv_prepare) and execute (ehip_conv_execute), all through the C-ABI."""
+    (ehip_conv_prepare) and execute (ehip_conv_execute), all through the C-ABI.  The base class holds
+    the handle and has ``execute(output, input, weights=None, bias=None, stream=0)``."""
 
     def __init__(self, desc):
         self.desc = desc
         h = ctypes.c_void_p()
         _check(lib.ehip_conv_create(ctypes.byref(desc), ctypes.byref(h)))
-        self._h = h
+        self._h = h.value
 
     def close(self):
         if getattr(self, "_h", None) and lib is not None:
@@ -165,10 +179,6 @@ class Conv:
 
     def prepare(self, weights, bias=None, stream=0):
         _check(lib.ehip_conv_prepare(self._h, _ptr(weights), _ptr(bias), ctypes.c_void_p(stream)))
-
-    def execute(self, output, input, weights=None, bias=None, stream=0):
-        _check(lib.ehip_conv_execute(self._h, _ptr(output), _ptr(input), _ptr(weights), _ptr(bias),
-                                     ctypes.c_void_p(stream)))
 
     def execute_repeat(self, output, input, count, bias=None, stream=0):
         _check(lib.ehip_conv_execute_repeat(self._h, _ptr(output), _ptr(input), _ptr(bias), count,
@@ -191,8 +201,8 @@ class Conv:
         return buf
 
 
-def quantize_input_u8(dst, src, count, scale, z, stream=0):
-    _check(lib.ehip_quantize_input_u8(_ptr(dst), _ptr(src), count, scale, z, ctypes.c_void_p(stream)))
+# quantize_input_u8(dst, src, count, scale, z, stream=0)
+quantize_input_u8 = _ehip_call.quantize_input_u8
 
 
 def wino_tinput_range(desc, input):
@@ -223,12 +233,9 @@ def calibrate_output_quant(desc, out_min, out_max, sum_absmax=0.0, representatio
     return s.value, z.value, ss.value
 
 
-def reorder_nchw_to_blocked(dst, src, elem_size, n, c, h, w, stream=0):
-    _check(lib.ehip_reorder_nchw_to_blocked(_ptr(dst), _ptr(src), elem_size, n, c, h, w, ctypes.c_void_p(stream)))
-
-
-def reorder_blocked_to_nchw(dst, src, elem_size, n, c, h, w, stream=0):
-    _check(lib.ehip_reorder_blocked_to_nchw(_ptr(dst), _ptr(src), elem_size, n, c, h, w, ctypes.c_void_p(stream)))
+# reorder_*(dst, src, elem_size, n, c, h, w, stream=0)
+reorder_nchw_to_blocked = _ehip_call.reorder_nchw_to_blocked
+reorder_blocked_to_nchw = _ehip_call.reorder_blocked_to_nchw
 
 
 def reorder_oihw_to_blocked(dst, src, o, i, h, w, stream=0):

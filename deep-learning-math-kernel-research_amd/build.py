@@ -7,6 +7,7 @@ The library is written next to this file so that it travels with the source tree
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -91,6 +92,12 @@ def build(verbose=True, jobs=8, incremental=False):
     if verbose:
         print(" ".join(cmd), flush=True)
     subprocess.check_call(cmd)
+    # the Python binding's extension module (host code only; the library's addresses are handed to it at run time)
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden", "-Wall",
+           "-I" + sysconfig.get_paths()["include"], os.path.join(CSRC, "ehip_call.cpp"), "-o", os.path.join(HERE, "_ehip_call.so")]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    procs.append(("ehip_call.cpp", subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT)))
     # the MFMA rate probe of the benchmark: a library of its own, not part of the product's C-ABI
     cmd = [hipcc] + FLAGS + ["-shared", os.path.join(CSRC, "ehip_probe.hip"), "-o", os.path.join(objdir, "libehip_probe.so")]
     if verbose:
