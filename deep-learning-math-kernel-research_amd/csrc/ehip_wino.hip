@@ -281,7 +281,7 @@ __global__ __launch_bounds__(kBlock) void k_wino_trans_input_u8(const WinoArgs *
       float f[AA], v[AA];
 #pragma unroll
       for (int e = 0; e < AA; ++e) f[e] = comp_of(d[e], k);
-      if (mixed) wino::tile_input_lanes<A>(f, v, c.border);
+      if (kCodes || mixed) wino::tile_input_lanes<A, kCodes>(f, v, c.border);
       else wino::tile_input<A>(f, v, false);
       if (watch) {
         float y[AA];
@@ -319,7 +319,7 @@ __global__ __launch_bounds__(kBlock) void k_wino_trans_input_u8(const WinoArgs *
     }
     return kCodes ? (seen_min < -0.5f || odd_consts) : (seen_u > 0xbf000000u || seen_s > 0x7f800000);
   };
-  const bool mixed = __ballot(c.border) != 0;   // wave-uniform
+  const bool mixed = !kCodes && __ballot(c.border) != 0;   // wave-uniform
   bool again;
   if (mixed) again = channels(true, true);
   else again = channels(false, true);
@@ -359,7 +359,7 @@ __global__ __launch_bounds__(kBlock) void k_wino_tinput_range(WinoArgs a, int ic
       float f[AA], v[AA];
 #pragma unroll
       for (int e = 0; e < AA; ++e) f[e] = comp_of(d[e], k);
-      wino::tile_input_lanes<A>(f, v, c.border);
+      wino::tile_input_lanes<A, sizeof(Cell) == sizeof(unsigned)>(f, v, c.border);
 #pragma unroll
       for (int e = 0; e < AA; ++e) {
         mn = v[e] < mn ? v[e] : mn;
@@ -694,7 +694,7 @@ __global__ __launch_bounds__(kBlock, 1) void k_wino_gemm_output(const WinoFusedA
     for (int s = 0; s < PW * NKSF; ++s) {
 #pragma unroll
       for (int j = 0; j < NT; ++j) {
-        const v4i b = rb[s % KS][j] ^ (int)0x80808080;
+        const v4i b = rb[s % KS][j] ;
 #pragma unroll
         for (int h = 0; h < NH; ++h)
           acc[s / NKSF][h][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ra[s % KS][h], b, acc[s / NKSF][h][j], 0, 0, 0);
@@ -711,7 +711,7 @@ __global__ __launch_bounds__(kBlock, 1) void k_wino_gemm_output(const WinoFusedA
       for (int k = 0; k < KS; ++k) {
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
-          const v4i b = rb[k][j] ^ (int)0x80808080;
+          const v4i b = rb[k][j] ;
 #pragma unroll
           for (int h = 0; h < NH; ++h)
             acc[i][h][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ra[k][h], b, acc[i][h][j], 0, 0, 0);

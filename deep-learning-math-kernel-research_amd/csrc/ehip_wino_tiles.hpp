@@ -213,46 +213,40 @@ __device__ __forceinline__ void tile_input<4>(const float *d, float *v, bool)
 #undef V
 }
 
-// tile_input with the border flag per lane (see fma_or_mul_add): what a wave with both kinds of tile runs
-template <int A>
-__device__ __forceinline__ void tile_input_lanes(const float *d, float *v, bool border);
-template <>
-__device__ __forceinline__ void tile_input_lanes<6>(const float *d, float *v, bool border)
+// tile_input with the border flag per lane (see fma_or_mul_add): what a wave with both kinds of tile runs.
+// CODES: the tile holds u8 codes.  The column pass is then exact whichever way it is rounded -- its results are multiples
+// of 1/256 below 2^10 (A = 6: products with 225/256, 169/64, 25/64, ...; A = 5: of 1/2) -- so the two kinds of tile
+// differ in one product of the last row pass (A = 6) or not at all: 145 vector instructions fewer per tile and channel.
+template <int A, bool CODES>
+__device__ __forceinline__ void tile_input_lanes(const float *d, float *v, bool border)
 {
-  float m[36];
+  if constexpr (A == 4) tile_input<4>(d, v, border);
+  else {
+    float m[A * A];
 #pragma unroll
-  for (int j = 0; j < 6; ++j) {
-    float f[6], o[6];
+    for (int j = 0; j < A; ++j) {
+      float f[A], o[A];
 #pragma unroll
-    for (int i = 0; i < 6; ++i) f[i] = d[6 * i + j];
-    in6_1d_lanes(f, o, border, false);
+      for (int i = 0; i < A; ++i) f[i] = d[A * i + j];
+      if constexpr (A == 6) {
+        if (CODES) in6_1d(f, o, false, false);
+        else in6_1d_lanes(f, o, border, false);
+      } else {
+        if (CODES) in5_1d(f, o, true);
+        else in5_1d_lanes(f, o, border);
+      }
 #pragma unroll
-    for (int i = 0; i < 6; ++i) m[6 * i + j] = o[i];
+      for (int i = 0; i < A; ++i) m[A * i + j] = o[i];
+    }
+    if constexpr (A == 6) {
+#pragma unroll
+      for (int i = 0; i < 5; ++i) in6_1d(&m[6 * i], &v[6 * i], false, false);
+      in6_1d_lanes(&m[30], &v[30], false, border);
+    } else {
+#pragma unroll
+      for (int i = 0; i < A; ++i) in5_1d(&m[A * i], &v[A * i], true);
+    }
   }
-#pragma unroll
-  for (int i = 0; i < 5; ++i) in6_1d(&m[6 * i], &v[6 * i], false, false);
-  in6_1d_lanes(&m[30], &v[30], false, border);
-}
-template <>
-__device__ __forceinline__ void tile_input_lanes<5>(const float *d, float *v, bool border)
-{
-  float m[25];
-#pragma unroll
-  for (int j = 0; j < 5; ++j) {
-    float f[5], o[5];
-#pragma unroll
-    for (int i = 0; i < 5; ++i) f[i] = d[5 * i + j];
-    in5_1d_lanes(f, o, border);
-#pragma unroll
-    for (int i = 0; i < 5; ++i) m[5 * i + j] = o[i];
-  }
-#pragma unroll
-  for (int i = 0; i < 5; ++i) in5_1d(&m[5 * i], &v[5 * i], true);
-}
-template <>
-__device__ __forceinline__ void tile_input_lanes<4>(const float *d, float *v, bool border)
-{
-  tile_input<4>(d, v, border);
 }
 
 // g: [3][3] (kh, kw)
