@@ -23,6 +23,7 @@ SOURCES = [
     "ehip_depthwise.hip",
     "ehip_wino.hip",
     "ehip_wino_lanes.hip",
+    "ehip_wino_ring.hip", "ehip_wino_ring6.hip", "ehip_wino_ring5.hip", "ehip_wino_ring4.hip",
     "ehip_prepare.hip",
     "ehip_harness.hip",
     "ehip_api.hip",
@@ -52,6 +53,9 @@ EXTRA_FLAGS = {
     "ehip_gemm1x1.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=16"],
     # the Winograd kernel whose requantized values take the accumulators' place in the vector registers
     "ehip_wino_lanes.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1", "-mllvm", "-amdgpu-kernarg-preload-count=16"],
+    # (and the straight-line column of positions of the ring kernels)
+    **{"ehip_wino_ring%d.hip" % a: ["-mllvm", "-amdgpu-mfma-vgpr-form=1", "-mllvm", "-pragma-unroll-threshold=1000000", "-mllvm",
+                                    "-amdgpu-kernarg-preload-count=16"] for a in (6, 5, 4)},
     "ehip_wino.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=16"],
     "ehip_fewch.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=16"],
     "ehip_gemm1x1w.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=16", "-mllvm", "-amdgpu-mfma-vgpr-form=1"],

@@ -397,6 +397,7 @@ int setup_workspace(ehip_conv *c)
     if ((long long)c->t >= (1ll << 31) / 64) return fail(EHIP_UNIMPLEMENTED, "winograd: too many tiles");
     c->variant = gemm_pick_variant(c->t, c->oc2, c->ic2, c->nbatch, 1);
     c->units_pad = up(c->ic2, gemm_variant_chunk(c->variant));
+    if (c->ic2 > 16) c->units_pad = up(c->units_pad, 8);   // (whole stages of the ring kernels)
     {
       const char *env = getenv("EHIP_WINO_FUSED");
       // every tile size, with or without the in-place sum, runs the fused GEMM + output transform, as the
@@ -409,13 +410,9 @@ int setup_workspace(ehip_conv *c)
     // (blocked: whole blocks of 32 tiles)  allocated with one pad unit behind it
     c->tin_bytes = (size_t)c->nbatch * c->ic2 * (c->tin_blocked ? up(c->t, 32) : c->t) * 16;
     c->tout_bytes = c->fused ? 16 : (size_t)c->nbatch * c->oc2 * c->t * 16 * sizeof(float);
-    if (c->fused) {   // (the fused stage's own parking space, where its kernel asks for one)
-      const size_t park = wino_lanes_tpart_bytes(d.tile_size, c->ic2, c->oc2, c->t);
-      if (park > c->tout_bytes) c->tout_bytes = park;
-    }
-    // (the pad: an odd unit count makes the last k-step read one unit past its position -- in the blocked layout
-    // 512 bytes past the last one, multiplied by zero weights)
-    if ((rc = dev_alloc(&c->tin, c->tin_bytes + ((size_t)c->t * 16 > 1024 ? (size_t)c->t * 16 : 1024), true)) != EHIP_OK) return rc;
+    // (the pad: the last k-steps of a unit count that does not fill them read up to seven units past their position -- in
+    // the blocked layout 3584 bytes past the last one, multiplied by zero weights)
+    if ((rc = dev_alloc(&c->tin, c->tin_bytes + ((size_t)c->t * 16 > 4096 ? (size_t)c->t * 16 : 4096), true)) != EHIP_OK) return rc;
     if ((rc = dev_alloc(reinterpret_cast<uint8_t **>(&c->tout), c->tout_bytes, false)) != EHIP_OK) return rc;
     break;
   }
@@ -643,7 +640,6 @@ static int plan_execute(ehip_conv *c, hipStream_t s)
       f.with_bias = d.with_bias; f.with_relu = d.with_relu; f.with_sum = d.with_ip_sum; f.tile = d.tile_size;
       f.out_type = w.out_type; f.out_repS = w.out_repS; f.out_z = w.out_z;
       f.out_nhwc = w.out_nhwc;
-      f.tpart = c->tout_bytes > 16 ? reinterpret_cast<float4 *>(c->tout) : nullptr;
       f.trace = trace_buffer();
       HIP_TRY(plan_wino_gemm_output(c->plan[1], f, s));
       if (c->plan[1].name) c->kernel_name = std::string("k_wino_trans_input_u8 + ") + c->plan[1].name;
@@ -831,7 +827,7 @@ EHIP_API int ehip_conv_query(ehip_conv_t *c, int what, void *host_dst, size_t *b
   }
   case EHIP_Q_TINPUT_U8:
     if (c->family != FAM_WINOGRAD) return fail(EHIP_GENERAL_ERROR, "not a Winograd handle");
-    if (c->tin_blocked) {   // back to the canonical [pos][ic2][t][16]
+    if (c->tin_blocked) {   // back to the canonical [pos][ic2][t][16], and from signed bytes to the codes
       const size_t canon = (size_t)c->nbatch * c->ic2 * c->t * 16;
       if (!want(canon)) return EHIP_OK;
       std::vector<uint8_t> raw(c->tin_bytes);
@@ -840,8 +836,9 @@ EHIP_API int ehip_conv_query(ehip_conv_t *c, int what, void *host_dst, size_t *b
       for (int p = 0; p < c->nbatch; ++p)
         for (int u = 0; u < c->ic2; ++u)
           for (int t = 0; t < c->t; ++t)
-            memcpy(dst + (((size_t)p * c->ic2 + u) * c->t + t) * 16,
-                   raw.data() + ((((size_t)(t >> 5) * c->nbatch + p) * c->ic2 + u) * 32 + (t & 31)) * 16, 16);
+            for (int k = 0; k < 16; ++k)
+              dst[(((size_t)p * c->ic2 + u) * c->t + t) * 16 + k] =
+                  raw[((((size_t)(t >> 5) * c->nbatch + p) * c->ic2 + u) * 32 + (t & 31)) * 16 + k] ^ 0x80;
       return EHIP_OK;
     }
     if (!want(c->tin_bytes)) return EHIP_OK;

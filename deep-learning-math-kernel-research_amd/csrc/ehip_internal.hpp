@@ -105,7 +105,7 @@ struct DepthwiseArgs {
 
 struct WinoArgs {
   const void *in;       // [n][ic2][ih][iw][16] f32, or u8 codes (in_u8)
-  uint8_t *tin;         // [36][ic2][t][16], or (tin_blocked) [t / 32][36][ic2][32][16]
+  uint8_t *tin;         // [36][ic2][t][16], or (tin_blocked) [t / 32][36][ic2][32][16] of code - 128
   int tin_blocked;      // the fused schedule's layout: everything a block of 32 tiles needs is one contiguous run
   const float *tout;    // [36][oc2][t][16]
   void *out;            // [n][oc2][oh][ow][16] f32 / u8 / s8 (out_type)
@@ -123,7 +123,7 @@ struct WinoArgs {
 };
 
 struct WinoFusedArgs {
-  const uint8_t *tin;   // [36][ic2][t][16] u8, or (tin_blocked) [t / 32][36][ic2][32][16]
+  const uint8_t *tin;   // (tin_blocked) [t / 32][36][ic2][32][16]: code - 128 (the general kernel also reads [36][ic2][t][16])
   int tin_blocked;
   const int8_t *w;      // [36][units_pad][OCpp][16] s8
   void *out;            // [n][oc2][oh][ow][16] f32 / u8 / s8 (out_type)
@@ -139,7 +139,7 @@ struct WinoFusedArgs {
   int out_nhwc;         // output as [n][h][w][c] (c % 16 == 0)
   int nx, ny;           // set by the launcher: blocks of 32 tiles, of 64 channels
   int slots;            // set by the lanes launcher: workgroups per XCD and channel block
-  float4 *tpart;        // first-stage results parked between the two passes of the 512-channel lanes kernel (wino_lanes_tpart_bytes)
+  int nkc;              // set by the ring launcher: stages per position
   long long *trace;     // development aid, normally null (see EHIP_TRACE)
 };
 
@@ -253,11 +253,20 @@ bool depthwise_mfma_applies(int stride, int oh, int ow, int pad_t, int pad_l, in
 hipError_t plan_wino_trans_input(LaunchPlan &plan, const WinoArgs &a, hipStream_t s);
 hipError_t plan_wino_trans_output(LaunchPlan &plan, const WinoArgs &a, hipStream_t s);
 hipError_t plan_wino_gemm_output(LaunchPlan &plan, const WinoFusedArgs &a, hipStream_t s);
-// at most 256 input channels, u8 / s8 output: the form without an exchange between GEMMs and transform (ehip_wino_lanes.hip)
+// at most 256 input channels: the form without an exchange between GEMMs and transform (ehip_wino_lanes.hip)
 bool wino_lanes_applies(const WinoFusedArgs &a);
-// device memory the lanes kernel needs besides the tensors (0 for most layers): a.tpart
-size_t wino_lanes_tpart_bytes(int tile, int ic2, int oc2, int t);
 hipError_t plan_wino_gemm_output_lanes(LaunchPlan &plan, const WinoFusedArgs &a, hipStream_t s);
+// both operands through an LDS ring (ehip_wino_ring.hip): the form for the layer, or -1
+int wino_ring_pick(const WinoFusedArgs &a);
+struct RingForm {
+  void (*kernel)(const WinoFusedArgs *, void *, const float *);
+  int oct, tt;                     // channels and tiles of a workgroup
+  int waves, stage_kb, stages, kc; // waves, KB and number of the ring's stages, k-steps of 64 channels per stage
+};
+RingForm wino_ring_form6(int form, int nks);   // tile sizes 6, 5, 4; nks = k-steps of a position
+RingForm wino_ring_form5(int form, int nks);
+RingForm wino_ring_form4(int form, int nks);
+hipError_t plan_wino_gemm_output_ring(LaunchPlan &plan, const WinoFusedArgs &a, int form, hipStream_t s);
 // min / max of the transformed input: partials = 2 * a.ic2 dwords of device scratch, result = two floats
 // of device memory (min, max); three launches on `s`, nothing else
 hipError_t launch_wino_range(const WinoArgs &a, int ic_real, unsigned *partials, float *minmax_out_dev, hipStream_t s);
@@ -367,7 +376,7 @@ __device__ __forceinline__ void load_pointers(FewChArgs &a, const EHIP_CONSTANT 
 __device__ __forceinline__ void load_pointers(WinoArgs &a, const EHIP_CONSTANT WinoArgs *c) { a.tin = c->tin; a.tout = c->tout; }
 __device__ __forceinline__ void load_pointers(WinoFusedArgs &a, const EHIP_CONSTANT WinoFusedArgs *c)
 {
-  a.tin = c->tin; a.w = c->w; a.scale = c->scale; a.shift = c->shift; a.comp = c->comp; a.tpart = c->tpart; a.trace = c->trace;
+  a.tin = c->tin; a.w = c->w; a.scale = c->scale; a.shift = c->shift; a.comp = c->comp; a.trace = c->trace;
 }
 template <typename Args>
 __device__ __forceinline__ Args load_args(const Args *p)

@@ -334,9 +334,12 @@ __global__ __launch_bounds__(kBlock) void k_wino_trans_input_u8(const WinoArgs *
   const uint8_t *base = a.tin_blocked ? a.tin + ((size_t)t32 * AA * a.ic2 + c2) * 512 : a.tin + (size_t)c2 * a.t * 16;
   const unsigned voff = a.tin_blocked ? (unsigned)((t & 31) * 4 + q) * 4u : (unsigned)(t * 4 + q) * 4u;
   const size_t pos_stride = a.tin_blocked ? (size_t)a.ic2 * 512 : (size_t)a.ic2 * a.t * 16;   // bytes
+  // (blocked layout: the fused stage's, whose matrix instructions take signed bytes -- the codes leave as u8 - 128, once
+  // here instead of in every channel block's workgroups)
+  const unsigned flip = a.tin_blocked ? 0x80808080u : 0u;
 #pragma unroll
   for (int e = 0; e < AA; ++e)
-    *reinterpret_cast<unsigned *>(const_cast<uint8_t *>(base) + e * pos_stride + voff) = packed[e];
+    *reinterpret_cast<unsigned *>(const_cast<uint8_t *>(base) + e * pos_stride + voff) = packed[e] ^ flip;
 }
 
 // partials[2 * c2] = ordered-min, [2 * c2 + 1] = ordered-max (see f2ord) of 16-channel unit c2; real
@@ -840,6 +843,8 @@ hipError_t plan_wino_gemm_output(LaunchPlan &plan, const WinoFusedArgs &a0, hipS
 {
   WinoFusedArgs a = a0;
   const int A = a.tile ? a.tile : 6, AA = A * A;
+  const int ring = wino_ring_pick(a);
+  if (ring >= 0) return plan_wino_gemm_output_ring(plan, a, ring, s);
   if (wino_lanes_applies(a)) return plan_wino_gemm_output_lanes(plan, a, s);
   const int ntb = A == 4 ? 2 : 1;   // blocks of 32 tiles per workgroup
   a.nx = (a.t + 32 * ntb - 1) / (32 * ntb);

@@ -607,3 +607,35 @@ def test_wino_replayed_from_a_hip_graph(tile):
         g.replay()
         torch.cuda.synchronize()
         assert np.array_equal(host(out), exp)
+
+
+# ---- both operands through the LDS ring (more than 256 input channels; 193-256 with form 2) --------------
+@pytest.mark.parametrize("tile", [6, 5, 4])
+@pytest.mark.parametrize("out_type,with_sum,with_relu", [(ol.S8, 1, True), (ol.U8, 0, False), (ol.F32, 0, True)])
+@pytest.mark.parametrize("form,n,ic,oc,hw", [("0", 3, 272, 72, 19), ("0", 2, 512, 144, 26), ("1", 3, 448, 48, 19), ("1", 1, 330, 80, 9),
+                                             ("0", 1, 560, 72, 13), ("1", 2, 560, 32, 18), ("2", 3, 256, 72, 19), ("2", 1, 200, 32, 40)])
+def test_wino_fused_ring(form, tile, out_type, with_sum, with_relu, n, ic, oc, hw, monkeypatch):
+    """Operand bytes that do not fill a stage, channel counts that leave a workgroup's last blocks empty, tile counts around the
+    32 and 64 of a workgroup (one and several blocks per workgroup), and every count of stages per position"""
+    import torch
+    monkeypatch.setenv("EHIP_WINO_RING", form)
+    E, p, d, xq, wb, bias = make_wino_u8(n, ic, oc, hw, seed=17 + tile + ic + out_type, out_type=out_type, tile=tile,
+                                         with_relu=with_relu, out_z=1.6 if out_type == ol.U8 else 0.0)
+    p.with_sum = with_sum
+    d.with_ip_sum = with_sum
+    p.tin_scale, p.tin_z = 22.0 / 255.0, 104.0
+    d.tinput_scale, d.tinput_z = p.tin_scale, p.tin_z
+    rng = np.random.default_rng(5 + tile + hw)
+    shape = (n, ol.up16(oc) // 16, hw, hw, 16)
+    old = rng.integers(-30 if out_type == ol.S8 else 0, 60, shape).astype(ol.NP_OF[out_type])
+    twq, tscale, tshift = ol.wino_prepare(p, wb)
+    tout, _ = ol.wino_gemm(p, ol.wino_trans_input(p, xq.astype(f32)), twq, tscale, tshift)
+    exp = ol.wino_trans_output(p, tout, bias, out_init=old if with_sum else None)
+    conv = E.Conv(d)
+    d_out, d_b = dev(old), dev(bias)
+    conv.prepare(dev(wb), d_b)
+    conv.execute(d_out, dev(xq), None, d_b)
+    torch.cuda.synchronize()
+    assert conv.kernel_name.endswith("k_wino_gemm_output_lanes_wres")
+    got = host(d_out)
+    assert np.array_equal(bits(got), bits(exp)), "output differs at %d of %d" % (int((got != exp).sum()), got.size)
