@@ -615,6 +615,7 @@ static int plan_execute(ehip_conv *c, hipStream_t s)
     a.out_type = d.output_type; a.with_relu = d.with_relu;
     a.lo = d.relu_lower; a.hi = d.relu_upper;
     HIP_TRY(plan_depthwise(*p, a, s));
+    if (p->name) c->kernel_name = p->name;   // small layers
     break;
   }
   case FAM_WINOGRAD: {

@@ -482,6 +482,16 @@ dw_kernel_t kernel_rb(int stride, int mode)
 // The matrix-core kernel: stride 1, u8 output with a ReLU inside the code range, pads 0 / 1, and a plane
 // of up to four 32-column chunks whose chunks and 8-row strips are mostly real pixels (EHIP_DW_MFMA=0 / 1
 // overrides the last condition).
+// Lanes of a dot4 launch with one output row per lane.  Small layers are bound by the latency of a lane's chain of loads and
+// rows and by CUs without work, not by the halo rows read again: they take one row per lane, and none runs on the matrix
+// cores, whose workgroups start from eight staged rows.  Measured (us; one row / two / the choice of the large layers):
+// stride 1: 14 x 14 x 512 N = 1 3.0 / 3.2 / 4.7, N = 16 (200 K lanes) 4.2 / 4.0 / 5.0, N = 32 6.0 / 5.2 / 5.2; 112 x 112 x 32
+// N = 1 (50 K) 3.4 / 3.2 / 5.0, N = 4 4.1 / 3.9 / 5.1, N = 8 (400 K) 5.7 / 5.0 / 5.3; 56 x 56 x 128 N = 1 3.0 / 3.3 / 4.0,
+// N = 8 5.7 / 5.1 / 4.9; 7 x 7 x 1024 N = 8 (57 K) 3.1 / 3.4 / 3.4, N = 32 4.4 / 4.0 / 4.0.  Stride 2: 56 -> 28, 128 channels, N = 1
+// 3.0 / 3.4 / 5.6, N = 32 (400 K) 6.0 / 6.1 / 6.8, N = 64 9.3 / 10.1 / 10.1.
+constexpr long long kOneRow = 110000, kTwoRows = 260000, kOneRowStride2 = 450000;
+static long long one_row_lanes(long long planes, int oh, int ow) { return planes * oh * ((ow + 1) / 2) * 4; }
+
 bool depthwise_mfma_applies(int stride, int oh, int ow, int pad_t, int pad_l, int out_type, int with_relu, float lo, float hi,
                             long long planes, int ih, int iw)
 {
@@ -507,8 +517,10 @@ hipError_t plan_depthwise(LaunchPlan &plan, const DepthwiseArgs &a0, hipStream_t
     set_error("depthwise: stride must be 1 or 2");
     return hipErrorInvalidValue;
   }
-  if (depthwise_mfma_applies(a.stride, a.oh, a.ow, a.pad_t, a.pad_l, a.out_type, a.with_relu, a.lo, a.hi, (long long)a.n * a.g2, a.ih,
-                             a.iw)) {
+  const long long lanes1 = one_row_lanes((long long)a.n * a.g2, a.oh, a.ow);
+  const bool small = lanes1 <= kTwoRows && !getenv("EHIP_DW_MFMA");
+  if (!small && depthwise_mfma_applies(a.stride, a.oh, a.ow, a.pad_t, a.pad_l, a.out_type, a.with_relu, a.lo, a.hi,
+                                       (long long)a.n * a.g2, a.ih, a.iw)) {
     const int nc = (a.ow + 31) / 32;
     const bool full = a.lo == 0.0f && a.hi == 255.0f;
     a.T_magic = div_magic(a.T);
@@ -544,6 +556,12 @@ hipError_t plan_depthwise(LaunchPlan &plan, const DepthwiseArgs &a0, hipStream_t
   // seven: 15 input rows of five pixels per lane are too many loads in flight)
   if (a.stride == 1 && a.oh == 14) rb = 7;
   if (a.stride == 2 && a.oh >= 56) rb = 2;
+  plan.name = "k_depthwise3x3_u8s8";   // (also for layers the handle took for the matrix cores')
+  if (a.stride == 2) {
+    if (lanes1 <= kOneRowStride2 || rb == 7) rb = 1;
+  } else if (lanes1 <= kTwoRows) {
+    rb = lanes1 <= kOneRow ? 1 : 2;
+  }
   const int ohb = (a.oh + rb - 1) / rb;
   const int wp = (a.ow + 1) / 2;
   a.lanes_per_plane = ohb * wp * 4;

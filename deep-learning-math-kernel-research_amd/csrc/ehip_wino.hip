@@ -697,7 +697,7 @@ __global__ __launch_bounds__(kBlock, 1) void k_wino_gemm_output(const WinoFusedA
     for (int s = 0; s < PW * NKSF; ++s) {
 #pragma unroll
       for (int j = 0; j < NT; ++j) {
-        const v4i b = rb[s % KS][j] ;
+        const v4i b = rb[s % KS][j];
 #pragma unroll
         for (int h = 0; h < NH; ++h)
           acc[s / NKSF][h][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ra[s % KS][h], b, acc[s / NKSF][h][j], 0, 0, 0);
@@ -714,7 +714,7 @@ __global__ __launch_bounds__(kBlock, 1) void k_wino_gemm_output(const WinoFusedA
       for (int k = 0; k < KS; ++k) {
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
-          const v4i b = rb[k][j] ;
+          const v4i b = rb[k][j];
 #pragma unroll
           for (int h = 0; h < NH; ++h)
             acc[i][h][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ra[k][h], b, acc[i][h][j], 0, 0, 0);

@@ -742,3 +742,12 @@ def test_prepared_handle_on_other_buffers(kind):
     res = run_and_compare(layer)
     again = layer.rerun_gpu(res["conv"])
     assert again.shape == res["out"].shape and (again == res["out"]).all(), kind
+
+
+# ---- depthwise: rows per lane by the size of the layer ----------------------------------------------------
+@pytest.mark.parametrize("n,g,hw,stride", [(1, 32, 14, 1), (1, 16, 57, 1), (4, 64, 28, 1), (6, 32, 56, 1), (1, 48, 28, 2), (2, 32, 57, 2),
+                                           (64, 32, 7, 1)])
+def test_depthwise_rows_per_lane(n, g, hw, stride):
+    for out_type in (ol.U8, ol.S8):
+        run_and_compare(Layer(n, g, g, hw, k=3, pad=1, stride=stride, out_type=out_type, depthwise=True, T=min(28, (hw - 1) // stride + 1),
+                              w_sigma=0.1, seed=830 + g + hw))
