@@ -18,6 +18,7 @@ SOURCES = [
     "ehip_gemm.hip",
     "ehip_gemm1x1.hip",
     "ehip_gemm1x1w.hip",
+    "ehip_gemm1x1s.hip",
     "ehip_conv3x3v.hip",
     "ehip_fewch.hip",
     "ehip_depthwise.hip",
@@ -58,6 +59,7 @@ EXTRA_FLAGS = {
                                     "-amdgpu-kernarg-preload-count=16"] for a in (6, 5, 4)},
     "ehip_wino.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=16"],
     "ehip_fewch.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=16"],
+    "ehip_gemm1x1s.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=16"],
     "ehip_gemm1x1w.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=16", "-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     # and those of the 1x1 kernels with few input channels
     "ehip_gemm.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=16"],

@@ -774,6 +774,7 @@ hipError_t plan_gemm_smallk(LaunchPlan &plan, const GemmArgs &a0, hipStream_t s)
 
 hipError_t plan_gemm(LaunchPlan &plan, const GemmArgs &a0, int nbatch, int variant, hipStream_t s)
 {
+  if (gemm1x1_split_applies(a0, nbatch)) return plan_gemm1x1_split(plan, a0, s);
   if (gemm1x1_wres_applies(a0, nbatch)) return plan_gemm1x1_wres(plan, a0, s);
   if (gemm_smallk_applies(a0.ic2, a0.kh * a0.kw, nbatch)) return plan_gemm_smallk(plan, a0, s);
   {

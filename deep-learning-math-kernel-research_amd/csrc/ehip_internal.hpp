@@ -240,6 +240,10 @@ hipError_t plan_gemm1x1_res(LaunchPlan &plan, const GemmArgs &a, int variant, hi
 bool gemm1x1_wres_applies(const GemmArgs &a, int nbatch);
 hipError_t plan_gemm1x1_wres(LaunchPlan &plan, const GemmArgs &a, hipStream_t s);
 
+// 1x1 layers with few output values: K split over the waves of a workgroup
+bool gemm1x1_split_applies(const GemmArgs &a, int nbatch);
+hipError_t plan_gemm1x1_split(LaunchPlan &plan, const GemmArgs &a, hipStream_t s);
+
 hipError_t plan_conv3x3v(LaunchPlan &plan, const Conv3x3Args &a, int n, int variant, hipStream_t s);
 int conv3x3v_pick_variant(int n, int oh, int ow, int oc2, int stride);   // stride 1 or 2 (both directions); -1: rows too wide for every variant
 int conv3x3v_chunk_units(int variant, int ic2);

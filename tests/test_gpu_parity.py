@@ -751,3 +751,20 @@ def test_depthwise_rows_per_lane(n, g, hw, stride):
     for out_type in (ol.U8, ol.S8):
         run_and_compare(Layer(n, g, g, hw, k=3, pad=1, stride=stride, out_type=out_type, depthwise=True, T=min(28, (hw - 1) // stride + 1),
                               w_sigma=0.1, seed=830 + g + hw))
+
+
+# ---- 1x1 with the K loop split over a workgroup's waves --------------------------------------------------
+@pytest.mark.parametrize("n,ic,oc,hw,stride", [(1, 16, 48, 9, 1), (2, 40, 32, 7, 2), (1, 96, 80, 11, 1), (1, 128, 33, 6, 1), (3, 144, 80, 9, 1),
+                                               (1, 256, 16, 14, 2), (1, 272, 64, 5, 1), (1, 384, 48, 7, 1), (2, 528, 272, 7, 1),
+                                               (1, 1024, 64, 7, 1), (1, 1040, 48, 3, 1), (1, 2048, 32, 5, 1)])
+def test_conv1x1_k_split(n, ic, oc, hw, stride, monkeypatch):
+    """every count of k-steps per wave (waves without any included), odd unit counts, ragged channels and pixels, both layouts"""
+    monkeypatch.setenv("EHIP_GEMM1X1_SPLIT", "1")
+    for out_type, kw in ((ol.U8, {}), (ol.S8, {"with_sum": True}), (ol.U8, {"with_sum": True, "relu_hi": 200.0}), (ol.S8, {"with_relu": False}),
+                         (ol.F32, {}), (ol.S32, {})):
+        res = run_and_compare(Layer(n, ic, oc, hw, stride=stride, out_type=out_type, seed=810 + ic + oc + out_type, **kw))
+        assert "split" in res["conv"].kernel_name
+    if ic % 16 == 0 and oc % 16 == 0:
+        for out_type, sides in ((ol.U8, {"in_nhwc": True, "out_nhwc": True}), (ol.F32, {"in_nhwc": True})):
+            res = run_and_compare(Layer(n, ic, oc, hw, stride=stride, out_type=out_type, seed=820 + ic, **sides))
+            assert "split" in res["conv"].kernel_name
