@@ -13,11 +13,13 @@
 
 namespace ehip {
 
-// the leading scalar arguments: see EHIP_SMALLK_HEAD in ehip_gemm.hip.
-// geom = stride_h | stride_w << 8 | dense << 16 | in_nhwc << 17 | out_nhwc << 18 | ic2 << 24
+// What every load of a wave needs -- operands AND per-channel constants: behind the argument structure (`rest`) the latter
+// would be two more trips to memory one after the other -- as leading scalar arguments, preloaded with the wave.
+// ny_rows = channel blocks | packed rows / 256 << 16; geom = stride_h | stride_w << 8 | dense << 16 | in_nhwc << 17 |
+// out_nhwc << 18 | ic2 << 24; iow = iw | ow << 16; consts: [scale | shift | compensation][packed rows]
 #define EHIP_SPLIT_HEAD                                                                                              \
-  const uint8_t *in, const int8_t *w, const GemmArgs *rest, int p_total, int ohw, unsigned ohw_magic, int ihw, int ocpp, \
-      int ny, unsigned geom, int iw, int ow, unsigned ow_magic, void *out
+  const uint8_t *in, const int8_t *w, const float *consts, const GemmArgs *rest, int p_total, int ohw, unsigned ohw_magic,  \
+      int ihw, unsigned ny_rows, unsigned geom, unsigned iow, unsigned ow_magic, void *out
 
 template <int NW, int KPW>
 __global__ __launch_bounds__(64 * NW) void k_gemm1x1_res_split(EHIP_SPLIT_HEAD)
@@ -28,6 +30,7 @@ __global__ __launch_bounds__(64 * NW) void k_gemm1x1_res_split(EHIP_SPLIT_HEAD)
   const int l32 = lane & 31, lh = lane >> 5;
   // (channel blocks next to each other: block b runs on XCD b % 8, so with a multiple of eight of them an XCD's L2 holds the
   // weights of its own ones only)
+  const int ny = (int)(ny_rows & 0xffffu), ocpp = (int)(ny_rows >> 16) * kOcTile, iw = (int)(iow & 0xffffu), ow = (int)(iow >> 16);
   const int px = blockIdx.x / ny, oc0 = (blockIdx.x - px * ny) * 32;
   const int ic2 = (int)(geom >> 24), sh = (int)(geom & 0xffu), sw = (int)((geom >> 8) & 0xffu);
   const bool in_nhwc = (geom >> 17) & 1u, out_nhwc = (geom >> 18) & 1u, dense = (geom >> 16) & 1u;
@@ -55,16 +58,21 @@ __global__ __launch_bounds__(64 * NW) void k_gemm1x1_res_split(EHIP_SPLIT_HEAD)
     u = u < ic2 ? u : ic2 - 1;   // (an odd count's last unit multiplies zero weights)
     vb[i] = *reinterpret_cast<const v4i *>(src + u * ustride);
   }
-  GemmArgs a = load_args(rest);
-  const int oc_real = a.oc2 * 16;
   const int oc = oc0 + 16 * lh;
   OcConsts k;
+  if (wave == 0) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      k.sc[q] = *reinterpret_cast<const float4 *>(consts + oc + 4 * q);
+      k.sh[q] = *reinterpret_cast<const float4 *>(consts + ocpp + oc + 4 * q);
+      k.comp[q] = *reinterpret_cast<const v4i *>(consts + 2 * (size_t)ocpp + oc + 4 * q);
+    }
+  }
+  GemmArgs a = load_args(rest);
+  const int oc_real = a.oc2 * 16;
   v4i old;
   const size_t cell = out_nhwc ? (size_t)gp * oc_real + oc : (((size_t)n * a.oc2 + (oc >> 4)) * ohw + r) * 16;
-  if (wave == 0) {
-    load_consts(k, a.ep, oc);
-    if (a.ep.with_sum) old = *reinterpret_cast<const v4i *>(static_cast<const uint8_t *>(out) + (oc < oc_real ? cell : 0));
-  }
+  if (wave == 0 && a.ep.with_sum) old = *reinterpret_cast<const v4i *>(static_cast<const uint8_t *>(out) + (oc < oc_real ? cell : 0));
   v16i acc[1][1];
 #pragma unroll
   for (int v = 0; v < 16; ++v) acc[0][0][v] = 0;
@@ -125,15 +133,16 @@ split_kernel_t split_kernel(int nks, int &nw)
   if (nks <= 8) return k_gemm1x1_res_split<4, 2>;
   if (nks <= 12) return k_gemm1x1_res_split<4, 3>;
   if (nks <= 16) return k_gemm1x1_res_split<4, 4>;
-  if (nks <= 32) return k_gemm1x1_res_split<8, 4>;
-  return nks <= 64 ? k_gemm1x1_res_split<8, 8> : nullptr;
+  return nks <= 32 ? k_gemm1x1_res_split<8, 4> : k_gemm1x1_res_split<8, 8>;
 }
 }  // namespace
 
 bool gemm1x1_split_applies(const GemmArgs &a, int nbatch)
 {
   if (nbatch != 1 || a.kh * a.kw > 1 || a.ep.shift_tab || a.ic2 > 128) return false;
-  if (a.stride_h > 255 || a.stride_w > 255) return false;
+  if (a.stride_h > 255 || a.stride_w > 255 || a.iw >= 65536 || a.ow >= 65536 || a.oc2 >= 65536) return false;
+  // (scale, shift and compensation in one allocation)
+  if (a.ep.shift != a.ep.scale + a.ocpp || reinterpret_cast<const float *>(a.ep.comp) != a.ep.scale + 2 * (size_t)a.ocpp) return false;
   if (a.out_nhwc && !lean_mode(a.ep, false)) return false;
   for (const char *other : {"EHIP_GEMM1X1_RES", "EHIP_GEMM1X1_WRES", "EHIP_GEMM_VARIANT", "EHIP_GEMM_SMALLK"})   // (another kernel asked for)
     if (const char *env = getenv(other)) if (env[0]) return false;
@@ -157,15 +166,15 @@ hipError_t plan_gemm1x1_split(LaunchPlan &plan, const GemmArgs &a0, hipStream_t 
   a.lean = lean_mode(a.ep, false);
   int nw = 0;
   const split_kernel_t kernel = split_kernel((a.ic2 + 1) / 2, nw);
-  if (!kernel) return hipErrorInvalidValue;
   a.nx = (a.p_total + 31) / 32;
   a.ny = (a.oc2 * 16 + 31) / 32;
   const bool dense = a.stride_h == 1 && a.stride_w == 1 && a.iw == a.ow;
   const unsigned geom = (unsigned)a.stride_h | (unsigned)a.stride_w << 8 | (dense ? 1u << 16 : 0u) | (a.in_nhwc ? 1u << 17 : 0u) |
       (a.out_nhwc ? 1u << 18 : 0u) | (unsigned)a.ic2 << 24;
   plan.name = a.ic2 > 8 ? "k_gemm1x1_res_split" : (a.lean ? "k_gemm_smallk_lean_split" : "k_gemm_smallk_split");
-  return plan_set(plan, kernel, dim3((unsigned)(a.nx * a.ny)), dim3(64 * nw), 0, a, s, ArgIn{a.in}, a.w, ArgBlock{}, a.p_total, a.ohw,
-                  a.ohw_magic, a.ihw, a.ocpp, a.ny, geom, a.iw, a.ow, a.ow_magic, ArgOut{a.out});
+  return plan_set(plan, kernel, dim3((unsigned)(a.nx * a.ny)), dim3(64 * nw), 0, a, s, ArgIn{a.in}, a.w, a.ep.scale, ArgBlock{}, a.p_total,
+                  a.ohw, a.ohw_magic, a.ihw, (unsigned)a.ny | (unsigned)(a.ocpp / kOcTile) << 16, geom,
+                  (unsigned)a.iw | (unsigned)a.ow << 16, a.ow_magic, ArgOut{a.out});
 }
 
 }  // namespace ehip
