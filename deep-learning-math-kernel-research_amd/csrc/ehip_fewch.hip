@@ -414,7 +414,16 @@ __global__ __launch_bounds__(kBlock, 3) void k_conv_fewch_lean(const FewChArgs *
     ro = fastdiv(p, a.ow, a.ow_magic);
     ox = p - ro * a.ow;
     const int at0 = ro * row_step + ox * px_step;
-    if (a.icl == 4) {
+    if (a.icl == 4 && (a.stride_w & 1) == 0) {
+      // every cell starts on eight bytes: one read of twice eight bytes per cell, and neighbouring lanes' pieces follow each
+      // other (as four dwords, eight bytes apart from lane to lane, half of the banks idle)
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const uint2 *src = reinterpret_cast<const uint2 *>(reinterpret_cast<const char *>(rows_lds) + at0 + cell_at[ks]);
+        const uint2 lo = src[0], hi = src[1];
+        b[ks] = v4i{(int)lo.x, (int)lo.y, (int)hi.x, (int)hi.y};
+      }
+    } else if (a.icl == 4) {
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
         const unsigned *src = rows_lds + ((at0 + cell_at[ks]) >> 2);
