@@ -87,6 +87,17 @@ bool pointer_or_null(PyObject *x, void **p)
   return !x || as_pointer(x, p);
 }
 
+// a stream: its address as an int, None or not given for the default stream.  Not a tensor: one in the stream's place (one
+// positional argument too many) would hand the runtime its data as a stream.
+bool stream_or_null(PyObject *x, void **p)
+{
+  if (x && x != Py_None && !PyLong_Check(x)) {
+    PyErr_Format(PyExc_TypeError, "stream: an int or None, not %.100s", Py_TYPE(x)->tp_name);
+    return false;
+  }
+  return pointer_or_null(x, p);
+}
+
 bool as_int(PyObject *x, int *v)
 {
   const long l = PyLong_AsLong(x);
@@ -111,8 +122,9 @@ PyObject *conv_execute(PyObject *self, PyObject *const *args, Py_ssize_t nargs, 
   PyObject *v[5];
   void *p[5];
   if (!arguments("execute", names, 2, args, nargs, kwnames, v)) return nullptr;
-  for (int i = 0; i < 5; ++i)
+  for (int i = 0; i < 4; ++i)
     if (!pointer_or_null(v[i], &p[i])) return nullptr;
+  if (!stream_or_null(v[4], &p[4])) return nullptr;
   void *h = reinterpret_cast<ConvBase *>(self)->handle;
   int rc;
   Py_BEGIN_ALLOW_THREADS
@@ -137,7 +149,8 @@ int conv_set_h(PyObject *self, PyObject *v, void *)
 
 PyMethodDef conv_methods[] = {
     {"execute", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(conv_execute)), METH_FASTCALL | METH_KEYWORDS,
-     "execute(output, input, weights=None, bias=None, stream=0): ehip_conv_execute; tensors, device addresses or None"},
+     "execute(output, input, weights=None, bias=None, stream=0): ehip_conv_execute; tensors, device addresses or None, and "
+     "the stream's address"},
     {nullptr, nullptr, 0, nullptr}};
 PyGetSetDef conv_getset[] = {{"_h", conv_get_h, conv_set_h, "address of the C handle, or None", nullptr},
                              {nullptr, nullptr, nullptr, nullptr, nullptr}};
@@ -150,7 +163,7 @@ PyObject *quantize_input_u8(PyObject *, PyObject *const *args, Py_ssize_t nargs,
   PyObject *v[6];
   void *dst, *src, *stream;
   if (!arguments("quantize_input_u8", names, 5, args, nargs, kwnames, v)) return nullptr;
-  if (!as_pointer(v[0], &dst) || !as_pointer(v[1], &src) || !pointer_or_null(v[5], &stream)) return nullptr;
+  if (!as_pointer(v[0], &dst) || !as_pointer(v[1], &src) || !stream_or_null(v[5], &stream)) return nullptr;
   const size_t count = PyLong_AsSize_t(v[2]);
   if (PyErr_Occurred()) return nullptr;
   const double scale = PyFloat_AsDouble(v[3]);
@@ -171,7 +184,7 @@ PyObject *reorder(const char *fn, reorder_t f, PyObject *const *args, Py_ssize_t
   void *dst, *src, *stream;
   int d[5];
   if (!arguments(fn, names, 7, args, nargs, kwnames, v)) return nullptr;
-  if (!as_pointer(v[0], &dst) || !as_pointer(v[1], &src) || !pointer_or_null(v[7], &stream)) return nullptr;
+  if (!as_pointer(v[0], &dst) || !as_pointer(v[1], &src) || !stream_or_null(v[7], &stream)) return nullptr;
   for (int i = 0; i < 5; ++i)
     if (!as_int(v[2 + i], &d[i])) return nullptr;
   int rc;

@@ -46,3 +46,22 @@ def test_pointers_are_tensors_ints_or_none():
             f(16, 16, 1, 1 << 40, 1, 1, 1)
         with pytest.raises(TypeError):
             f(16, 16, 1, 1, 1, 1)
+
+
+class DeviceTensor:
+    def data_ptr(self):
+        return 256
+
+
+@pytest.mark.parametrize("stream", [DeviceTensor(), 1.0, "0", np.int64(0)])
+def test_a_stream_is_an_int_or_none(stream):
+    """a tensor in the stream's place (one positional argument too many) must not become the address of a stream"""
+    with pytest.raises(TypeError):
+        closed_conv().execute(1, 2, None, None, stream)
+    with pytest.raises(TypeError):
+        closed_conv().execute(1, 2, stream=stream)
+    with pytest.raises(TypeError):
+        E.quantize_input_u8(16, 16, 4, 0.0, 0.0, stream)
+    for f in (E.reorder_nchw_to_blocked, E.reorder_blocked_to_nchw):
+        with pytest.raises(TypeError):
+            f(16, 16, 2, 1, 1, 1, 1, stream)
