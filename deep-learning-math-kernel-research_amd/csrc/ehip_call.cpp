@@ -164,7 +164,10 @@ PyObject *quantize_input_u8(PyObject *, PyObject *const *args, Py_ssize_t nargs,
   void *dst, *src, *stream;
   if (!arguments("quantize_input_u8", names, 5, args, nargs, kwnames, v)) return nullptr;
   if (!as_pointer(v[0], &dst) || !as_pointer(v[1], &src) || !stream_or_null(v[5], &stream)) return nullptr;
-  const size_t count = PyLong_AsSize_t(v[2]);
+  PyObject *n = PyNumber_Index(v[2]);   // (whatever converts to an int without loss, a numpy integer for instance)
+  if (!n) return nullptr;
+  const size_t count = PyLong_AsSize_t(n);
+  Py_DECREF(n);
   if (PyErr_Occurred()) return nullptr;
   const double scale = PyFloat_AsDouble(v[3]);
   if (PyErr_Occurred()) return nullptr;

@@ -65,3 +65,14 @@ def test_a_stream_is_an_int_or_none(stream):
     for f in (E.reorder_nchw_to_blocked, E.reorder_blocked_to_nchw):
         with pytest.raises(TypeError):
             f(16, 16, 2, 1, 1, 1, 1, stream)
+
+
+@pytest.mark.parametrize("integer", [int, np.int32, np.int64, np.uint8])
+def test_counts_and_sizes_take_numpy_integers(integer):
+    with pytest.raises(E.EulerHipError, match="scale is zero"):
+        E.quantize_input_u8(16, 16, integer(4), 0.0, 0.0)
+    for f in (E.reorder_nchw_to_blocked, E.reorder_blocked_to_nchw):
+        with pytest.raises(E.EulerHipError, match="bad argument"):
+            f(16, 16, integer(2), integer(1), integer(1), integer(1), integer(1))
+    with pytest.raises(TypeError):
+        E.quantize_input_u8(16, 16, 4.0, 0.0, 0.0)
