@@ -502,23 +502,6 @@ EHIP_API int ehip_init(int device)
   return EHIP_OK;
 }
 
-EHIP_API int ehip_conv_create(const ehip_conv_desc_t *desc, ehip_conv_t **out)
-{
-  if (!desc || !out) return fail(EHIP_GENERAL_ERROR, "null argument");
-  *out = nullptr;
-  ehip_conv *c = new ehip_conv();
-  c->d = *desc;
-  int rc = classify(c);
-  if (rc == EHIP_OK) rc = setup_workspace(c);
-  if (rc != EHIP_OK) {
-    free_all(c);
-    delete c;
-    return rc;
-  }
-  *out = c;
-  return EHIP_OK;
-}
-
 EHIP_API int ehip_conv_destroy(ehip_conv_t *c)
 {
   if (!c) return EHIP_OK;
@@ -542,8 +525,8 @@ static long long *trace_buffer()
 }
 
 // What an execute will launch: everything but the tensors (LaunchPlan), with the argument structures written to the
-// handle's device memory on stream s, like the packed weights.
-static int plan_execute(ehip_conv *c, hipStream_t s)
+// handle's device memory.
+static int plan_execute(ehip_conv *c)
 {
   const ehip_conv_desc_t &d = c->d;
   LaunchPlan *p = &c->plan[0];
@@ -566,8 +549,7 @@ static int plan_execute(ehip_conv *c, hipStream_t s)
       a.cls_h = c->cls_h; a.cls_w = c->cls_w; a.ncls_w = c->ncls_w;
     }
     a.trace = trace_buffer();
-    HIP_TRY(plan_gemm(*p, a, 1, c->variant, s));
-    if (p->name) c->kernel_name = p->name;   // the choice depends on the epilogue
+    HIP_TRY(plan_gemm(*p, a, 1, c->variant));
     break;
   }
   case FAM_CONV_FEWCH: {
@@ -583,8 +565,7 @@ static int plan_execute(ehip_conv *c, hipStream_t s)
       a.ep.shift_tab = c->shift_tab; a.ep.tab_stride = c->ocpp;
       a.cls_h = c->cls_h; a.cls_w = c->cls_w; a.ncls_w = c->ncls_w; a.nclass = c->nclass;
     }
-    HIP_TRY(plan_conv_fewch(*p, a, s));
-    c->kernel_name = p->name;
+    HIP_TRY(plan_conv_fewch(*p, a));
     break;
   }
   case FAM_CONV_3X3: {
@@ -599,7 +580,7 @@ static int plan_execute(ehip_conv *c, hipStream_t s)
     a.vw = d.stride_h == 2 ? d.ow + 1 : d.ow + 2;
     a.vw_magic = div_magic(a.vw);
     a.trace = trace_buffer();
-    HIP_TRY(plan_conv3x3v(*p, a, d.n, c->variant, s));
+    HIP_TRY(plan_conv3x3v(*p, a, d.n, c->variant));
     break;
   }
   case FAM_DEPTHWISE: {
@@ -614,8 +595,7 @@ static int plan_execute(ehip_conv *c, hipStream_t s)
     a.T = c->T; a.Tr = c->Tr; a.wt = c->wtb;
     a.out_type = d.output_type; a.with_relu = d.with_relu;
     a.lo = d.relu_lower; a.hi = d.relu_upper;
-    HIP_TRY(plan_depthwise(*p, a, s));
-    if (p->name) c->kernel_name = p->name;   // small layers
+    HIP_TRY(plan_depthwise(*p, a));
     break;
   }
   case FAM_WINOGRAD: {
@@ -628,7 +608,7 @@ static int plan_execute(ehip_conv *c, hipStream_t s)
     const float tin_repS = 1.0f / d.tinput_scale;
     w.mrepS = d.input_scale * tin_repS;
     w.mz = ceilf(d.tinput_z);
-    HIP_TRY(plan_wino_trans_input(c->plan[0], w, s));
+    HIP_TRY(plan_wino_trans_input(c->plan[0], w));
     c->plan_stage[0] = 1;
     c->plan_stage[1] = 2;
     if (c->fused) {
@@ -642,8 +622,7 @@ static int plan_execute(ehip_conv *c, hipStream_t s)
       f.out_type = w.out_type; f.out_repS = w.out_repS; f.out_z = w.out_z;
       f.out_nhwc = w.out_nhwc;
       f.trace = trace_buffer();
-      HIP_TRY(plan_wino_gemm_output(c->plan[1], f, s));
-      if (c->plan[1].name) c->kernel_name = std::string("k_wino_trans_input_u8 + ") + c->plan[1].name;
+      HIP_TRY(plan_wino_gemm_output(c->plan[1], f));
       c->nplans = 2;
       return EHIP_OK;
     }
@@ -660,8 +639,8 @@ static int plan_execute(ehip_conv *c, hipStream_t s)
     a.ic2 = c->ic2; a.units_pad = c->units_pad; a.oc2 = c->oc2; a.ocpp = c->ocpp;
     a.in_batch_stride = (long long)c->ic2 * w.t * 16;
     a.out_batch_stride = (long long)c->oc2 * w.t * 16;
-    HIP_TRY(plan_gemm(c->plan[1], a, c->nbatch, c->variant, s));
-    HIP_TRY(plan_wino_trans_output(c->plan[2], w, s));
+    HIP_TRY(plan_gemm(c->plan[1], a, c->nbatch, c->variant));
+    HIP_TRY(plan_wino_trans_output(c->plan[2], w));
     c->plan_stage[2] = 4;
     c->nplans = 3;
     return EHIP_OK;
@@ -670,6 +649,31 @@ static int plan_execute(ehip_conv *c, hipStream_t s)
     return fail(EHIP_GENERAL_ERROR, "internal: no executor");
   }
   c->nplans = 1;
+  return EHIP_OK;
+}
+
+static int finish_on_null_stream()
+{
+  HIP_TRY(hipStreamSynchronize(nullptr));
+  return EHIP_OK;
+}
+
+EHIP_API int ehip_conv_create(const ehip_conv_desc_t *desc, ehip_conv_t **out)
+{
+  if (!desc || !out) return fail(EHIP_GENERAL_ERROR, "null argument");
+  *out = nullptr;
+  ehip_conv *c = new ehip_conv();
+  c->d = *desc;
+  int rc = classify(c);
+  if (rc == EHIP_OK) rc = setup_workspace(c);
+  if (rc == EHIP_OK) rc = plan_execute(c);
+  if (rc == EHIP_OK) rc = finish_on_null_stream();   // cleared workspaces and argument structures
+  if (rc != EHIP_OK) {
+    free_all(c);
+    delete c;
+    return rc;
+  }
+  *out = c;
   return EHIP_OK;
 }
 
@@ -728,9 +732,14 @@ EHIP_API int ehip_conv_prepare(ehip_conv_t *c, const void *weights_dev, const vo
   default:
     return fail(EHIP_GENERAL_ERROR, "internal: no executor");
   }
-  const int rc = plan_execute(c, s);
-  c->prepared = rc == EHIP_OK;
-  return rc;
+  // from here on the name is that of the kernel the planner chose
+  if (c->family == FAM_WINOGRAD) {
+    if (c->fused && c->plan[1].name) c->kernel_name = std::string("k_wino_trans_input_u8 + ") + c->plan[1].name;
+  } else if (c->plan[0].name) {
+    c->kernel_name = c->plan[0].name;
+  }
+  c->prepared = true;
+  return EHIP_OK;
 }
 
 EHIP_API int ehip_conv_execute(ehip_conv_t *c, void *output_dev, const void *input_dev, const void *weights_dev,

@@ -679,7 +679,7 @@ int conv3x3v_pick_variant(int n, int oh, int ow, int oc2, int stride)
   return best;
 }
 
-hipError_t plan_conv3x3v(LaunchPlan &plan, const Conv3x3Args &a0, int n, int variant, hipStream_t s)
+hipError_t plan_conv3x3v(LaunchPlan &plan, const Conv3x3Args &a0, int n, int variant)
 {
   const Variant &k = kVariants[variant];
   Conv3x3Args a = a0;
@@ -711,7 +711,7 @@ hipError_t plan_conv3x3v(LaunchPlan &plan, const Conv3x3Args &a0, int n, int var
     }
   }
   if (a.pad_t > 255 || a.pad_l > 255 || a.chunk_units >= 65536) return hipErrorInvalidValue;   // pads_cu's fields
-  return plan_set(plan, kernel, grid, dim3(kBlock), lds_bytes, a, s, ArgIn{a.in}, ArgBlock{}, a.ih, a.iw, a.oh, a.ow,
+  return plan_set(plan, kernel, grid, dim3(kBlock), lds_bytes, a, ArgIn{a.in}, ArgBlock{}, a.ih, a.iw, a.oh, a.ow,
                   (unsigned)a.pad_t | (unsigned)a.pad_l << 8 | (unsigned)a.chunk_units << 16, a.ic2, a.vw, a.vw_magic, a.gx, a.gy,
                   a.tiles, a.tiles_per_xcd, ArgOut{a.out});
 }

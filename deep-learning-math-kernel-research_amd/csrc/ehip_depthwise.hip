@@ -454,7 +454,7 @@ hipError_t launch_depthwise_diag(const int8_t *wpacked, int g2n, void *diag, hip
 
 namespace {
 typedef void (*dw_kernel_t)(EHIP_DW_HEAD);
-hipError_t dw_set(LaunchPlan &plan, dw_kernel_t kernel, dim3 grid, dim3 block, const DepthwiseArgs &a, int walk, hipStream_t s)
+hipError_t dw_set(LaunchPlan &plan, dw_kernel_t kernel, dim3 grid, dim3 block, const DepthwiseArgs &a, int walk)
 {
   // what the packed leading arguments can hold
   if (a.ih >= 65536 || a.iw >= 65536 || a.oh >= 65536 || a.ow >= 65536 || a.pad_t < 0 || a.pad_t > 15 || a.pad_l < 0 ||
@@ -464,7 +464,7 @@ hipError_t dw_set(LaunchPlan &plan, dw_kernel_t kernel, dim3 grid, dim3 block, c
   }
   const unsigned geom = (unsigned)a.pad_t | (unsigned)a.pad_l << 4 | (unsigned)a.stride << 8 | (unsigned)a.planes_per_block << 12 |
       (unsigned)a.lanes_padded << 16;
-  return plan_set(plan, kernel, grid, block, 0, a, s, ArgIn{a.in}, a.w, a.wsum, ArgBlock{}, a.n, a.g2, (unsigned)a.ih | (unsigned)a.iw << 16,
+  return plan_set(plan, kernel, grid, block, 0, a, ArgIn{a.in}, a.w, a.wsum, ArgBlock{}, a.n, a.g2, (unsigned)a.ih | (unsigned)a.iw << 16,
                   (unsigned)a.oh | (unsigned)a.ow << 16, geom, a.blocks_per_plane, walk, a.wp_magic, ArgOut{a.out});
 }
 template <int RB, int S>
@@ -510,7 +510,7 @@ bool depthwise_mfma_applies(int stride, int oh, int ow, int pad_t, int pad_l, in
   return 32.0 * nc * 8.0 * strips <= 1.35 * ow * oh;
 }
 
-hipError_t plan_depthwise(LaunchPlan &plan, const DepthwiseArgs &a0, hipStream_t s)
+hipError_t plan_depthwise(LaunchPlan &plan, const DepthwiseArgs &a0)
 {
   DepthwiseArgs a = a0;
   if (a.stride != 1 && a.stride != 2) {
@@ -546,7 +546,7 @@ hipError_t plan_depthwise(LaunchPlan &plan, const DepthwiseArgs &a0, hipStream_t
 #define EHIP_DWM(NC) (full ? k_depthwise3x3_mfma<2, NC> : k_depthwise3x3_mfma<1, NC>)
     kernel = nc == 1 ? EHIP_DWM(1) : (nc == 2 ? EHIP_DWM(2) : (nc == 3 ? EHIP_DWM(3) : EHIP_DWM(4)));
 #undef EHIP_DWM
-    return dw_set(plan, kernel, dim3((unsigned)wgs), dim3(kBlock), a, a.strips_per_wg, s);
+    return dw_set(plan, kernel, dim3((unsigned)wgs), dim3(kBlock), a, a.strips_per_wg);
   }
   // four rows per lane on tall planes (seven where that divides the height: 28, 56, 112 -- fewer halo
   // rows re-read, 2-5 % on the MobileNet layers), fewer where that would leave lanes idle
@@ -588,7 +588,7 @@ hipError_t plan_depthwise(LaunchPlan &plan, const DepthwiseArgs &a0, hipStream_t
   dim3 grid((unsigned)(8 * ((groups + 7) / 8) * a.blocks_per_plane), 1, 1);
   const dw_kernel_t kernel = rb == 7 ? kernel_rb<7>(a.stride, mode)
       : (rb == 4 ? kernel_rb<4>(a.stride, mode) : (rb == 2 ? kernel_rb<2>(a.stride, mode) : kernel_rb<1>(a.stride, mode)));
-  return dw_set(plan, kernel, grid, dim3(block), a, a.lanes_per_plane, s);
+  return dw_set(plan, kernel, grid, dim3(block), a, a.lanes_per_plane);
 }
 
 }  // namespace ehip

@@ -495,7 +495,7 @@ int conv_fewch_row_pitch(int icl, int kw, int iw, int ow, int stride_w, int pad_
 
 // Fills the derived fields (cells, strip height, LDS row pitch, wave split) and the plan.
 // Expects in a: weights, epilogue, n, ih, iw, oh, ow, ic, kh, kw, strides, pads, oc2, ocpp, formats, classes.
-hipError_t plan_conv_fewch(LaunchPlan &plan, FewChArgs &a, hipStream_t s)
+hipError_t plan_conv_fewch(LaunchPlan &plan, FewChArgs &a)
 {
   {
     // lean_mode() but for the per-pixel shift rows, which this kernel's lean path reads itself
@@ -592,7 +592,7 @@ hipError_t plan_conv_fewch(LaunchPlan &plan, FewChArgs &a, hipStream_t s)
     name = "k_conv_fewch_lean";
   }
   plan.name = name;
-  return plan_set(plan, kern, dim3(a.n * a.strips, gy), dim3(kBlock), lds, a, s, ArgBlock{}, ArgIn{a.in}, ArgOut{a.out});
+  return plan_set(plan, kern, dim3(a.n * a.strips, gy), dim3(kBlock), lds, a, ArgBlock{}, ArgIn{a.in}, ArgOut{a.out});
 }
 
 }  // namespace ehip

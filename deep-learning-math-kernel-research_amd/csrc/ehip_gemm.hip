@@ -699,7 +699,7 @@ smallk_kernel_t smallk_kernel(int tnw)
   (void)tnw;   // (two pixel tiles per iteration cost more in occupancy than they gain in overlap: one)
   return k_gemm_smallk_u8s8<1, KS>;
 }
-hipError_t smallk_set(LaunchPlan &plan, smallk_kernel_t kernel, dim3 grid, const GemmArgs &a0, hipStream_t s)
+hipError_t smallk_set(LaunchPlan &plan, smallk_kernel_t kernel, dim3 grid, const GemmArgs &a0)
 {
   GemmArgs a = a0;
   a.nx = (int)grid.x;
@@ -707,7 +707,7 @@ hipError_t smallk_set(LaunchPlan &plan, smallk_kernel_t kernel, dim3 grid, const
   const bool dense = a.stride_h == 1 && a.stride_w == 1 && a.iw == a.ow;
   const unsigned geom = (unsigned)a.stride_h | (unsigned)a.stride_w << 8 | (dense ? 1u << 16 : 0u) | (a.in_nhwc ? 1u << 17 : 0u) |
       (a.out_nhwc ? 1u << 18 : 0u) | (unsigned)a.sk_wo << 20 | (unsigned)a.ic2 << 24;
-  return plan_set(plan, kernel, grid, dim3(kBlock), 0, a, s, ArgIn{a.in}, a.w, ArgBlock{}, a.p_total, a.ohw, a.ohw_magic, a.ihw,
+  return plan_set(plan, kernel, grid, dim3(kBlock), 0, a, ArgIn{a.in}, a.w, ArgBlock{}, a.p_total, a.ohw, a.ohw_magic, a.ihw,
                   a.ocpp, a.oc2, geom, a.iw, a.ow, a.ow_magic, ArgOut{a.out});
 }
 }  // namespace
@@ -721,7 +721,7 @@ bool gemm_smallk_applies(int ic2, int taps, int nbatch)
   return nbatch == 1 && taps <= 1 && ic2 <= 8;
 }
 
-hipError_t plan_gemm_smallk(LaunchPlan &plan, const GemmArgs &a0, hipStream_t s)
+hipError_t plan_gemm_smallk(LaunchPlan &plan, const GemmArgs &a0)
 {
   GemmArgs a = a0;
   a.lean = lean_mode(a.ep, false);   // blocked and nhwc output alike
@@ -767,19 +767,19 @@ hipError_t plan_gemm_smallk(LaunchPlan &plan, const GemmArgs &a0, hipStream_t s)
                                               {"k_gemm_smallk_lean<4,2>", "k_gemm_smallk_lean<4,2>"}};
       plan.name = names[ks == 1 ? 0 : (ks == 2 ? 1 : 2)][ocw == 4 ? 1 : 0];
     }
-    return smallk_set(plan, lk, dim3(nx2, ny2), a, s);
+    return smallk_set(plan, lk, dim3(nx2, ny2), a);
   }
-  return smallk_set(plan, kernel, dim3(nx, ny), a, s);
+  return smallk_set(plan, kernel, dim3(nx, ny), a);
 }
 
-hipError_t plan_gemm(LaunchPlan &plan, const GemmArgs &a0, int nbatch, int variant, hipStream_t s)
+hipError_t plan_gemm(LaunchPlan &plan, const GemmArgs &a0, int nbatch, int variant)
 {
-  if (gemm1x1_split_applies(a0, nbatch)) return plan_gemm1x1_split(plan, a0, s);
-  if (gemm1x1_wres_applies(a0, nbatch)) return plan_gemm1x1_wres(plan, a0, s);
-  if (gemm_smallk_applies(a0.ic2, a0.kh * a0.kw, nbatch)) return plan_gemm_smallk(plan, a0, s);
+  if (gemm1x1_split_applies(a0, nbatch)) return plan_gemm1x1_split(plan, a0);
+  if (gemm1x1_wres_applies(a0, nbatch)) return plan_gemm1x1_wres(plan, a0);
+  if (gemm_smallk_applies(a0.ic2, a0.kh * a0.kw, nbatch)) return plan_gemm_smallk(plan, a0);
   {
     const int rv = gemm1x1_res_pick(a0, nbatch);
-    if (rv >= 0) return plan_gemm1x1_res(plan, a0, rv, s);
+    if (rv >= 0) return plan_gemm1x1_res(plan, a0, rv);
   }
   const Variant &k = kVariants[variant];
   GemmArgs a = a0;
@@ -799,7 +799,7 @@ hipError_t plan_gemm(LaunchPlan &plan, const GemmArgs &a0, int nbatch, int varia
   if (taps > 1 && (taps > 64 || nbatch != 1)) return hipErrorInvalidValue;
   const int fmt = taps > 1 ? (a.in_nhwc ? 4 : (a.ic2 % k.kc == 0 ? 2 : 3)) : (a.in_nhwc ? 1 : 0);
   while (dl > 0 && (nchunks % (1 << dl) != 0 || !k.kernel[fmt][dl])) --dl;
-  return plan_set(plan, k.kernel[fmt][dl], grid, dim3(kBlock), 0, a, s, ArgBlock{}, ArgIn{a.in}, ArgOut{a.out});
+  return plan_set(plan, k.kernel[fmt][dl], grid, dim3(kBlock), 0, a, ArgBlock{}, ArgIn{a.in}, ArgOut{a.out});
 }
 
 }  // namespace ehip

@@ -457,7 +457,7 @@ int gemm1x1_res_pick(const GemmArgs &a, int nbatch)
 
 const char *gemm1x1_res_name(int v) { return kRes[v].name; }
 
-hipError_t plan_gemm1x1_res(LaunchPlan &plan, const GemmArgs &a0, int v, hipStream_t s)
+hipError_t plan_gemm1x1_res(LaunchPlan &plan, const GemmArgs &a0, int v)
 {
   const ResVariant &k = kRes[v];
   GemmArgs a = a0;
@@ -482,7 +482,7 @@ hipError_t plan_gemm1x1_res(LaunchPlan &plan, const GemmArgs &a0, int v, hipStre
   const bool dense = a.stride_h == 1 && a.stride_w == 1 && a.iw == a.ow;
   const unsigned geom = (unsigned)a.stride_h | (unsigned)a.stride_w << 8 | (dense ? 1u << 16 : 0u) | (unsigned)a.oc2 << 20;
   plan.name = k.name;   // (nhwc output: the handle could not tell at creation whether the lean epilogue applies)
-  return plan_set(plan, kernel, grid, dim3(kBlock), lds_bytes, a, s, ArgIn{a.in}, a.w, a.ep.comp, ArgBlock{}, a.nx, a.ny, a.p_total,
+  return plan_set(plan, kernel, grid, dim3(kBlock), lds_bytes, a, ArgIn{a.in}, a.w, a.ep.comp, ArgBlock{}, a.nx, a.ny, a.p_total,
                   a.ohw, a.ohw_magic, a.ihw, (unsigned)a.ic2 | (unsigned)a.units_pad << 16, geom, ArgOut{a.out});
 }
 

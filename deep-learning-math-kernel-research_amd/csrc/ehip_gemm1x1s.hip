@@ -160,7 +160,7 @@ bool gemm1x1_split_applies(const GemmArgs &a, int nbatch)
   return tiles <= (nks <= 2 ? 1600 : (nks <= 16 ? 900 : 640));
 }
 
-hipError_t plan_gemm1x1_split(LaunchPlan &plan, const GemmArgs &a0, hipStream_t s)
+hipError_t plan_gemm1x1_split(LaunchPlan &plan, const GemmArgs &a0)
 {
   GemmArgs a = a0;
   a.lean = lean_mode(a.ep, false);
@@ -172,7 +172,7 @@ hipError_t plan_gemm1x1_split(LaunchPlan &plan, const GemmArgs &a0, hipStream_t 
   const unsigned geom = (unsigned)a.stride_h | (unsigned)a.stride_w << 8 | (dense ? 1u << 16 : 0u) | (a.in_nhwc ? 1u << 17 : 0u) |
       (a.out_nhwc ? 1u << 18 : 0u) | (unsigned)a.ic2 << 24;
   plan.name = a.ic2 > 8 ? "k_gemm1x1_res_split" : (a.lean ? "k_gemm_smallk_lean_split" : "k_gemm_smallk_split");
-  return plan_set(plan, kernel, dim3((unsigned)(a.nx * a.ny)), dim3(64 * nw), 0, a, s, ArgIn{a.in}, a.w, a.ep.scale, ArgBlock{}, a.p_total,
+  return plan_set(plan, kernel, dim3((unsigned)(a.nx * a.ny)), dim3(64 * nw), 0, a, ArgIn{a.in}, a.w, a.ep.scale, ArgBlock{}, a.p_total,
                   a.ohw, a.ohw_magic, a.ihw, (unsigned)a.ny | (unsigned)(a.ocpp / kOcTile) << 16, geom,
                   (unsigned)a.iw | (unsigned)a.ow << 16, a.ow_magic, ArgOut{a.out});
 }

@@ -471,7 +471,7 @@ bool gemm1x1_wres_applies(const GemmArgs &a, int nbatch)
   return wres_geom(a, g);
 }
 
-hipError_t plan_gemm1x1_wres(LaunchPlan &plan, const GemmArgs &a0, hipStream_t s)
+hipError_t plan_gemm1x1_wres(LaunchPlan &plan, const GemmArgs &a0)
 {
   GemmArgs a = a0;
   a.lean = lean_mode(a.ep, false);
@@ -488,7 +488,7 @@ hipError_t plan_gemm1x1_wres(LaunchPlan &plan, const GemmArgs &a0, hipStream_t s
   const bool dense = a.stride_h == 1 && a.stride_w == 1 && a.iw == a.ow;
   const unsigned geom = (unsigned)a.stride_h | (unsigned)a.stride_w << 8 | (dense ? 1u << 16 : 0u) | (unsigned)a.ny << 20;
   plan.name = "k_gemm1x1_wres";
-  return plan_set(plan, kernel, dim3(8 * g.nb * ((g.nreg + 7) / 8)), dim3(g.nw * 64), g.lds_bytes, a, s, ArgIn{a.in}, a.w, a.ep.scale,
+  return plan_set(plan, kernel, dim3(8 * g.nb * ((g.nreg + 7) / 8)), dim3(g.nw * 64), g.lds_bytes, a, ArgIn{a.in}, a.w, a.ep.scale,
                   ArgBlock{}, a.p_total, a.ohw, a.ohw_magic, a.ihw, geom, (unsigned)a.nx | (unsigned)(a.ocpp / kOcTile) << 16,
                   (unsigned)a.ow | (unsigned)a.iw << 16, a.ow_magic, ArgOut{a.out});
 }

@@ -144,10 +144,11 @@ struct WinoFusedArgs {
 };
 
 // ---- launch plans -------------------------------------------------------------------------------
-// Everything about a launch but the tensors is worked out once, when the handle is prepared (planned): kernel, grid,
+// Everything about a launch but the tensors is worked out once, when the handle is created (planned): kernel, grid,
 // LDS size, the derived arguments, the EHIP_* knobs read from the environment.  The argument structure goes to device
-// memory owned by the handle (written on the stream that packs the weights, so it is there when they are), and a launch
-// passes its ADDRESS beside the tensors and the few scalars a wave's first loads need: at most kMaxKernarg bytes.
+// memory owned by the handle, and a launch passes its ADDRESS beside the tensors and the few scalars a wave's first loads
+// need: at most kMaxKernarg bytes.  The structure holds pointers, so it is complete before the handle is handed out: a
+// launch finds it there on whatever stream it runs and whether or not that stream waits for the one that packs the weights.
 // What that buys: HIP writes kernel arguments into device memory across PCIe, and a launch with 300 bytes of them
 // costs the host 3.4 us where 16-96 bytes cost 2.6 (128: 3.25, 256: 3.45; empty kernel, back to back) -- as long as a
 // small layer's kernel takes on the GPU.
@@ -155,7 +156,7 @@ constexpr size_t kMaxKernarg = 104;   // (the step is between 104 and 128)
 constexpr size_t kArgBlock = 512;     // device memory of one argument structure
 struct LaunchPlan {
   void *args_dev = nullptr;     // kArgBlock bytes of device memory, set when the handle is created
-  hipFunction_t fn = nullptr;   // of the device the handle was prepared on
+  hipFunction_t fn = nullptr;   // of the device the handle was created on
   dim3 grid, block;
   unsigned lds = 0;
   const char *name = nullptr;   // set by a planner whose choice of kernel the handle cannot know beforehand
@@ -168,8 +169,6 @@ struct ArgIn { const void *fixed; };
 struct ArgOut { void *fixed; };
 struct ArgBias {};
 struct ArgBlock {};   // the address of the argument structure
-
-hipError_t launch_store_args(const void *args, size_t bytes, void *dst_dev, hipStream_t s);   // (ehip_prepare.hip)
 
 struct KernargWriter {
   LaunchPlan &p;
@@ -188,9 +187,10 @@ struct KernargWriter {
   template <typename P> void put(const ArgBias &) { raw(nullptr, 8, &p.bias_at); }
   template <typename P> void put(const ArgBlock &) { raw(&p.args_dev, 8); }
 };
-// `a` in the order of the kernel's parameters, each converted to its parameter's type
+// `a` in the order of the kernel's parameters, each converted to its parameter's type.  (The copy is complete once the null
+// stream has been waited for, as ehip_conv_create does.)
 template <typename Args, typename... P, typename... A>
-inline hipError_t plan_set(LaunchPlan &p, void (*kernel)(P...), dim3 grid, dim3 block, size_t lds, const Args &args, hipStream_t s, A... a)
+inline hipError_t plan_set(LaunchPlan &p, void (*kernel)(P...), dim3 grid, dim3 block, size_t lds, const Args &args, A... a)
 {
   static_assert(sizeof...(P) == sizeof...(A), "one value per kernel parameter");
   static_assert(sizeof(Args) <= kArgBlock && sizeof(Args) % 4 == 0, "argument structure");
@@ -206,7 +206,7 @@ inline hipError_t plan_set(LaunchPlan &p, void (*kernel)(P...), dim3 grid, dim3 
   if (lds > 48 * 1024)
     e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e == hipSuccess) e = hipGetFuncBySymbol(&p.fn, reinterpret_cast<const void *>(kernel));
-  if (e == hipSuccess) e = launch_store_args(&args, sizeof(Args), p.args_dev, s);
+  if (e == hipSuccess) e = hipMemcpy(p.args_dev, &args, sizeof(Args), hipMemcpyHostToDevice);
   return e;
 }
 // The kept plan is only read: the tensors of this call go into a copy of the kernel arguments, so executes of one
@@ -225,7 +225,7 @@ inline hipError_t plan_launch(const LaunchPlan &p, const void *in, void *out, co
 
 // ---- planners and launchers (implemented next to their kernels) -----------------------------
 // A planner chooses the kernel and fills the plan; a.in / a.out null = given at each launch.
-hipError_t plan_gemm(LaunchPlan &plan, const GemmArgs &a, int nbatch, int variant, hipStream_t s);
+hipError_t plan_gemm(LaunchPlan &plan, const GemmArgs &a, int nbatch, int variant);
 bool gemm_smallk_applies(int ic2, int taps, int nbatch);
 int gemm_pick_variant(int p_total, int oc2, int ic2, int nbatch, int stride);
 int gemm_variant_chunk(int variant);
@@ -235,31 +235,31 @@ const char *gemm_variant_name(int variant);
 // 1x1 layers with many input channels, blocked activations: pixel tile resident in LDS, weights streamed
 int gemm1x1_res_pick(const GemmArgs &a, int nbatch);   // variant, or -1 when the layer is not one for it
 const char *gemm1x1_res_name(int variant);
-hipError_t plan_gemm1x1_res(LaunchPlan &plan, const GemmArgs &a, int variant, hipStream_t s);
+hipError_t plan_gemm1x1_res(LaunchPlan &plan, const GemmArgs &a, int variant);
 // 1x1 layers of 256 / 512 / 1024 input channels with the lean epilogue: weights resident in registers, pixels streamed
 bool gemm1x1_wres_applies(const GemmArgs &a, int nbatch);
-hipError_t plan_gemm1x1_wres(LaunchPlan &plan, const GemmArgs &a, hipStream_t s);
+hipError_t plan_gemm1x1_wres(LaunchPlan &plan, const GemmArgs &a);
 
 // 1x1 layers with few output values: K split over the waves of a workgroup
 bool gemm1x1_split_applies(const GemmArgs &a, int nbatch);
-hipError_t plan_gemm1x1_split(LaunchPlan &plan, const GemmArgs &a, hipStream_t s);
+hipError_t plan_gemm1x1_split(LaunchPlan &plan, const GemmArgs &a);
 
-hipError_t plan_conv3x3v(LaunchPlan &plan, const Conv3x3Args &a, int n, int variant, hipStream_t s);
+hipError_t plan_conv3x3v(LaunchPlan &plan, const Conv3x3Args &a, int n, int variant);
 int conv3x3v_pick_variant(int n, int oh, int ow, int oc2, int stride);   // stride 1 or 2 (both directions); -1: rows too wide for every variant
 int conv3x3v_chunk_units(int variant, int ic2);
 int conv3x3v_num_variants();
 const char *conv3x3v_variant_name(int variant);
 
-hipError_t plan_depthwise(LaunchPlan &plan, const DepthwiseArgs &a, hipStream_t s);
+hipError_t plan_depthwise(LaunchPlan &plan, const DepthwiseArgs &a);
 hipError_t launch_depthwise_diag(const int8_t *wpacked, int g2n, void *diag, hipStream_t s);
 bool depthwise_mfma_applies(int stride, int oh, int ow, int pad_t, int pad_l, int out_type, int with_relu, float lo, float hi,
                             long long planes, int ih, int iw);
-hipError_t plan_wino_trans_input(LaunchPlan &plan, const WinoArgs &a, hipStream_t s);
-hipError_t plan_wino_trans_output(LaunchPlan &plan, const WinoArgs &a, hipStream_t s);
-hipError_t plan_wino_gemm_output(LaunchPlan &plan, const WinoFusedArgs &a, hipStream_t s);
+hipError_t plan_wino_trans_input(LaunchPlan &plan, const WinoArgs &a);
+hipError_t plan_wino_trans_output(LaunchPlan &plan, const WinoArgs &a);
+hipError_t plan_wino_gemm_output(LaunchPlan &plan, const WinoFusedArgs &a);
 // at most 256 input channels: the form without an exchange between GEMMs and transform (ehip_wino_lanes.hip)
 bool wino_lanes_applies(const WinoFusedArgs &a);
-hipError_t plan_wino_gemm_output_lanes(LaunchPlan &plan, const WinoFusedArgs &a, hipStream_t s);
+hipError_t plan_wino_gemm_output_lanes(LaunchPlan &plan, const WinoFusedArgs &a);
 // both operands through an LDS ring (ehip_wino_ring.hip): the form for the layer, or -1
 int wino_ring_pick(const WinoFusedArgs &a);
 struct RingForm {
@@ -270,7 +270,7 @@ struct RingForm {
 RingForm wino_ring_form6(int form, int nks);   // tile sizes 6, 5, 4; nks = k-steps of a position
 RingForm wino_ring_form5(int form, int nks);
 RingForm wino_ring_form4(int form, int nks);
-hipError_t plan_wino_gemm_output_ring(LaunchPlan &plan, const WinoFusedArgs &a, int form, hipStream_t s);
+hipError_t plan_wino_gemm_output_ring(LaunchPlan &plan, const WinoFusedArgs &a, int form);
 // min / max of the transformed input: partials = 2 * a.ic2 dwords of device scratch, result = two floats
 // of device memory (min, max); three launches on `s`, nothing else
 hipError_t launch_wino_range(const WinoArgs &a, int ic_real, unsigned *partials, float *minmax_out_dev, hipStream_t s);
@@ -313,7 +313,7 @@ struct FewChArgs {
 int conv_fewch_icl(int ic, int kw);
 bool conv_fewch_applies(int ic, int kh, int kw);
 int conv_fewch_row_pitch(int icl, int kw, int iw, int ow, int stride_w, int pad_l);   // icl: conv_fewch_icl()
-hipError_t plan_conv_fewch(LaunchPlan &plan, FewChArgs &a, hipStream_t s);
+hipError_t plan_conv_fewch(LaunchPlan &plan, FewChArgs &a);
 hipError_t launch_prepare_direct_px(const float *w, const float *bias, int oc, int ic, int icl, int kh, int kw, int ppc, int nu,
                                     int ocpp, const ehip_conv_desc_t &d, float *absmax, int8_t *wpacked, float *scale,
                                     float *shift, int *wsum, int *comp, hipStream_t s);

@@ -474,21 +474,6 @@ hipError_t launch_prepare_wino(const float *w, int oc, int ic, int tile, int uni
   return hipGetLastError();
 }
 
-// A launch's argument structure into the handle's device memory: by value in this kernel's arguments, so that it works
-// in a stream that is being captured, too.
-namespace {
-struct ArgBlob { unsigned d[kArgBlock / 4]; };
-__global__ __launch_bounds__(kArgBlock / 4) void k_store_args(ArgBlob a, unsigned *dst) { dst[threadIdx.x] = a.d[threadIdx.x]; }
-}  // namespace
-hipError_t launch_store_args(const void *args, size_t bytes, void *dst_dev, hipStream_t s)
-{
-  if (!dst_dev || bytes > kArgBlock) return hipErrorInvalidValue;
-  ArgBlob b = {};
-  memcpy(&b, args, bytes);
-  hipLaunchKernelGGL(k_store_args, dim3(1), dim3(kArgBlock / 4), 0, s, b, static_cast<unsigned *>(dst_dev));
-  return hipGetLastError();
-}
-
 hipError_t launch_quantize_input(uint8_t *dst, const float *src, size_t count, float scale, float z, hipStream_t s)
 {
   const size_t quads = count / 4;

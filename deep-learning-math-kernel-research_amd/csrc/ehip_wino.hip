@@ -804,7 +804,7 @@ __global__ __launch_bounds__(kBlock, 1) void k_wino_gemm_output(const WinoFusedA
   }
 }
 
-hipError_t plan_wino_trans_input(LaunchPlan &plan, const WinoArgs &a0, hipStream_t s)
+hipError_t plan_wino_trans_input(LaunchPlan &plan, const WinoArgs &a0)
 {
   WinoArgs a = a0;
   {
@@ -821,10 +821,10 @@ hipError_t plan_wino_trans_input(LaunchPlan &plan, const WinoArgs &a0, hipStream
   if (a.tile == 4) kern = a.in_u8 ? k_wino_trans_input_u8<unsigned, 4> : k_wino_trans_input_u8<float4, 4>;
   else if (a.tile == 5) kern = a.in_u8 ? k_wino_trans_input_u8<unsigned, 5> : k_wino_trans_input_u8<float4, 5>;
   else kern = a.in_u8 ? k_wino_trans_input_u8<unsigned, 6> : k_wino_trans_input_u8<float4, 6>;
-  return plan_set(plan, kern, grid, dim3(kBlock), 0, a, s, ArgBlock{}, ArgIn{a.in});
+  return plan_set(plan, kern, grid, dim3(kBlock), 0, a, ArgBlock{}, ArgIn{a.in});
 }
 
-hipError_t plan_wino_trans_output(LaunchPlan &plan, const WinoArgs &a, hipStream_t s)
+hipError_t plan_wino_trans_output(LaunchPlan &plan, const WinoArgs &a)
 {
   dim3 grid((a.t + 63) / 64, a.oc2);
   void (*kern)(const WinoArgs *, void *, const float *) = nullptr;
@@ -835,17 +835,17 @@ hipError_t plan_wino_trans_output(LaunchPlan &plan, const WinoArgs &a, hipStream
   else if (a.tile == 5) EHIP_WO(5);
   else EHIP_WO(6);
 #undef EHIP_WO
-  return plan_set(plan, kern, grid, dim3(kBlock), 0, a, s, ArgBlock{}, ArgOut{a.out}, ArgBias{});
+  return plan_set(plan, kern, grid, dim3(kBlock), 0, a, ArgBlock{}, ArgOut{a.out}, ArgBias{});
 }
 
 // k-steps per ring block: the largest of 8, 4, 2 that divides the k-steps of a position
-hipError_t plan_wino_gemm_output(LaunchPlan &plan, const WinoFusedArgs &a0, hipStream_t s)
+hipError_t plan_wino_gemm_output(LaunchPlan &plan, const WinoFusedArgs &a0)
 {
   WinoFusedArgs a = a0;
   const int A = a.tile ? a.tile : 6, AA = A * A;
   const int ring = wino_ring_pick(a);
-  if (ring >= 0) return plan_wino_gemm_output_ring(plan, a, ring, s);
-  if (wino_lanes_applies(a)) return plan_wino_gemm_output_lanes(plan, a, s);
+  if (ring >= 0) return plan_wino_gemm_output_ring(plan, a, ring);
+  if (wino_lanes_applies(a)) return plan_wino_gemm_output_lanes(plan, a);
   const int ntb = A == 4 ? 2 : 1;   // blocks of 32 tiles per workgroup
   a.nx = (a.t + 32 * ntb - 1) / (32 * ntb);
   // 64 channels per workgroup; 32 where that would leave a quarter of the CUs or more without a workgroup
@@ -886,7 +886,7 @@ hipError_t plan_wino_gemm_output(LaunchPlan &plan, const WinoFusedArgs &a0, hipS
 #undef EHIP_WF
 #undef EHIP_WF1
   if (nks % 2 != 0) return hipErrorInvalidValue;
-  return plan_set(plan, kernel, grid, dim3(kBlock), lds, a, s, ArgBlock{}, ArgOut{a.out}, ArgBias{});
+  return plan_set(plan, kernel, grid, dim3(kBlock), lds, a, ArgBlock{}, ArgOut{a.out}, ArgBias{});
 }
 
 // partials: 2 * a.ic2 dwords of device memory; minmax_out_dev: two floats of device memory

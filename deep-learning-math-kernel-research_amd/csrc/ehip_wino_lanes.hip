@@ -459,7 +459,7 @@ bool wino_lanes_applies(const WinoFusedArgs &a)
       !(env && env[0] == '0');
 }
 
-hipError_t plan_wino_gemm_output_lanes(LaunchPlan &plan, const WinoFusedArgs &a0, hipStream_t s)
+hipError_t plan_wino_gemm_output_lanes(LaunchPlan &plan, const WinoFusedArgs &a0)
 {
   WinoFusedArgs a = a0;
   const int A = a.tile ? a.tile : 6, AA = A * A;
@@ -487,7 +487,7 @@ hipError_t plan_wino_gemm_output_lanes(LaunchPlan &plan, const WinoFusedArgs &a0
     kernel = pick_wres(A, a.with_sum != 0, nks64, nw);
     if (!kernel) return hipErrorInvalidValue;
     plan.name = "k_wino_gemm_output_lanes_wres";
-    return plan_set(plan, kernel, dim3(8 * a.ny * slots), dim3(64 * nw), lds, a, s, ArgBlock{}, ArgOut{a.out}, ArgBias{});
+    return plan_set(plan, kernel, dim3(8 * a.ny * slots), dim3(64 * nw), lds, a, ArgBlock{}, ArgOut{a.out}, ArgBias{});
   }
   a.nx = (a.t + 31) / 32;
   a.ny = (a.oc2 * 16 + 31) / 32;
@@ -502,7 +502,7 @@ hipError_t plan_wino_gemm_output_lanes(LaunchPlan &plan, const WinoFusedArgs &a0
 #undef EHIP_WL
   const size_t lds = (size_t)AA * 24 * sizeof(float4);
   plan.name = "k_wino_gemm_output_lanes";
-  return plan_set(plan, kernel, dim3(8 * a.ny * ((a.nx + 7) / 8)), dim3(kBlock), lds, a, s, ArgBlock{}, ArgOut{a.out}, ArgBias{});
+  return plan_set(plan, kernel, dim3(8 * a.ny * ((a.nx + 7) / 8)), dim3(kBlock), lds, a, ArgBlock{}, ArgOut{a.out}, ArgBias{});
 }
 
 }  // namespace ehip

@@ -29,7 +29,7 @@ int wino_ring_pick(const WinoFusedArgs &a)
   return 36 * ((large + 255) / 256) < (small <= 256 ? 20 : 30) * ((small + 511) / 512) ? 0 : 1;
 }
 
-hipError_t plan_wino_gemm_output_ring(LaunchPlan &plan, const WinoFusedArgs &a0, int form, hipStream_t s)
+hipError_t plan_wino_gemm_output_ring(LaunchPlan &plan, const WinoFusedArgs &a0, int form)
 {
   WinoFusedArgs a = a0;
   const int A = a.tile ? a.tile : 6, AA = A * A;
@@ -47,7 +47,7 @@ hipError_t plan_wino_gemm_output_ring(LaunchPlan &plan, const WinoFusedArgs &a0,
   const int need = (a.nx + 7) / 8;
   a.slots = slots < need ? slots : need;
   plan.name = "k_wino_gemm_output_lanes_wres";   // (the family of the lanes kernels that read their weights from LDS)
-  return plan_set(plan, f.kernel, dim3(8 * a.ny * a.slots), dim3(64 * f.waves), lds, a, s, ArgBlock{}, ArgOut{a.out}, ArgBias{});
+  return plan_set(plan, f.kernel, dim3(8 * a.ny * a.slots), dim3(64 * f.waves), lds, a, ArgBlock{}, ArgOut{a.out}, ArgBias{});
 }
 
 }  // namespace ehip

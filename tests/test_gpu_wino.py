@@ -609,6 +609,34 @@ def test_wino_replayed_from_a_hip_graph(tile):
         assert np.array_equal(host(out), exp)
 
 
+@pytest.mark.parametrize("ic,fused", [(48, "1"), (272, "1"), (48, "0")])
+def test_wino_prepared_on_one_stream_and_run_on_another(ic, fused, monkeypatch):
+    """ehip_conv_prepare of a Winograd layer returns when its weights are ready, so a caller may execute on any other stream
+    at once: everything that the kernels read, their argument structures included, has to be in place by then.  Both streams
+    are new for every handle, and the preparing one is busy with work of its own."""
+    import torch
+    monkeypatch.setenv("EHIP_WINO_FUSED", fused)
+    E, p, d, xq, wb, bias = make_wino_u8(2, ic, 48, 13, seed=610 + ic, out_type=ol.S8)
+    p.tin_scale, p.tin_z = 22.0 / 255.0, 104.0
+    d.tinput_scale, d.tinput_z = p.tin_scale, p.tin_z
+    _, exp = _oracle_u8(p, xq, wb, bias)
+    d_x, d_w, d_b = dev(xq), dev(wb), dev(bias)
+    busy = torch.zeros(1 << 24, device="cuda")
+    for _ in range(3):
+        preparing, running = torch.cuda.Stream(), torch.cuda.Stream()
+        d_out = torch.full(exp.shape, 9, dtype=torch.int8, device="cuda")
+        torch.cuda.synchronize()
+        with torch.cuda.stream(preparing):
+            for _ in range(20):
+                busy.add_(1.0)
+        conv = E.Conv(d)
+        conv.prepare(d_w, d_b, stream=preparing.cuda_stream)
+        conv.execute(d_out, d_x, None, d_b, stream=running.cuda_stream)
+        running.synchronize()
+        assert np.array_equal(host(d_out), exp)
+        torch.cuda.synchronize()
+
+
 # ---- both operands through the LDS ring (more than 256 input channels; 193-256 with form 2) --------------
 @pytest.mark.parametrize("tile", [6, 5, 4])
 @pytest.mark.parametrize("out_type,with_sum,with_relu", [(ol.S8, 1, True), (ol.U8, 0, False), (ol.F32, 0, True)])
