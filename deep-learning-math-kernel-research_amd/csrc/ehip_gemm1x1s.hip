@@ -22,7 +22,7 @@ namespace ehip {
       int ihw, unsigned ny_rows, unsigned geom, unsigned iow, unsigned ow_magic, void *out
 
 template <int NW, int KPW>
-__global__ __launch_bounds__(64 * NW) void k_gemm1x1_res_split(EHIP_SPLIT_HEAD)
+__global__ __launch_bounds__(64 * NW) void k_gemm1x1_split(EHIP_SPLIT_HEAD)
 {
   __shared__ v4i part[(NW > 1 ? NW - 1 : 1) * 256];   // [wave - 1][quarter of the 16 results][lane]
   const int lane = threadIdx.x & 63;
@@ -127,13 +127,13 @@ typedef void (*split_kernel_t)(EHIP_SPLIT_HEAD);
 split_kernel_t split_kernel(int nks, int &nw)
 {
   nw = nks <= 1 ? 1 : (nks <= 2 ? 2 : (nks <= 16 ? 4 : 8));
-  if (nks <= 1) return k_gemm1x1_res_split<1, 1>;
-  if (nks <= 2) return k_gemm1x1_res_split<2, 1>;
-  if (nks <= 4) return k_gemm1x1_res_split<4, 1>;
-  if (nks <= 8) return k_gemm1x1_res_split<4, 2>;
-  if (nks <= 12) return k_gemm1x1_res_split<4, 3>;
-  if (nks <= 16) return k_gemm1x1_res_split<4, 4>;
-  return nks <= 32 ? k_gemm1x1_res_split<8, 4> : k_gemm1x1_res_split<8, 8>;
+  if (nks <= 1) return k_gemm1x1_split<1, 1>;
+  if (nks <= 2) return k_gemm1x1_split<2, 1>;
+  if (nks <= 4) return k_gemm1x1_split<4, 1>;
+  if (nks <= 8) return k_gemm1x1_split<4, 2>;
+  if (nks <= 12) return k_gemm1x1_split<4, 3>;
+  if (nks <= 16) return k_gemm1x1_split<4, 4>;
+  return nks <= 32 ? k_gemm1x1_split<8, 4> : k_gemm1x1_split<8, 8>;
 }
 }  // namespace
 
@@ -171,7 +171,7 @@ hipError_t plan_gemm1x1_split(LaunchPlan &plan, const GemmArgs &a0)
   const bool dense = a.stride_h == 1 && a.stride_w == 1 && a.iw == a.ow;
   const unsigned geom = (unsigned)a.stride_h | (unsigned)a.stride_w << 8 | (dense ? 1u << 16 : 0u) | (a.in_nhwc ? 1u << 17 : 0u) |
       (a.out_nhwc ? 1u << 18 : 0u) | (unsigned)a.ic2 << 24;
-  plan.name = a.ic2 > 8 ? "k_gemm1x1_res_split" : (a.lean ? "k_gemm_smallk_lean_split" : "k_gemm_smallk_split");
+  plan.name = "k_gemm1x1_split";
   return plan_set(plan, kernel, dim3((unsigned)(a.nx * a.ny)), dim3(64 * nw), 0, a, ArgIn{a.in}, a.w, a.ep.scale, ArgBlock{}, a.p_total,
                   a.ohw, a.ohw_magic, a.ihw, (unsigned)a.ny | (unsigned)(a.ocpp / kOcTile) << 16, geom,
                   (unsigned)a.iw | (unsigned)a.ow << 16, a.ow_magic, ArgOut{a.out});

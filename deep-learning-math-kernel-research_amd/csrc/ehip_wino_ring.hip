@@ -15,7 +15,7 @@ int wino_ring_pick(const WinoFusedArgs &a)
   for (const char *other : {"EHIP_WINO_LANES", "EHIP_WINO_LANES_WRES"})   // (the other forms asked for)
     if (const char *env = getenv(other)) if (env[0] == '0') return -1;
   auto items = [&](int oct, int tt) { return (long long)((a.t + tt - 1) / tt) * ((a.oc2 * 16 + oct - 1) / oct); };
-  if (const char *env = getenv("EHIP_WINO_RING")) {
+  if (const char *env = getenv("EHIP_WINO_RING")) {   // (0, 1, 2: that form where it exists; anything else: none)
     const int form = env[0] - '0';
     return form == 2 ? (nks64 == 4 ? 2 : -1) : (form >= 0 && form < 2 && nks64 > 4 ? form : -1);
   }
@@ -46,7 +46,9 @@ hipError_t plan_wino_gemm_output_ring(LaunchPlan &plan, const WinoFusedArgs &a0,
   slots = slots < 1 ? 1 : slots;
   const int need = (a.nx + 7) / 8;
   a.slots = slots < need ? slots : need;
-  plan.name = "k_wino_gemm_output_lanes_wres";   // (the family of the lanes kernels that read their weights from LDS)
+  static const char *const names[] = {"k_wino_gemm_output_lanes_ring<64,64>", "k_wino_gemm_output_lanes_ring<32,32>",
+                                      "k_wino_gemm_output_lanes_ring<32,64>"};   // channels, tiles of a workgroup
+  plan.name = names[form];
   return plan_set(plan, f.kernel, dim3(8 * a.ny * a.slots), dim3(64 * f.waves), lds, a, ArgBlock{}, ArgOut{a.out}, ArgBias{});
 }
 

@@ -210,11 +210,10 @@ def test_wino_fused_lanes_weights_resident(slots, wres, tile, out_type, with_sum
 @pytest.mark.parametrize("n,ic,oc,hw", [(2, 256, 48, 30), (1, 192, 32, 36), (3, 512, 32, 18)])
 def test_wino_fused_lanes_weights_resident_many_channels(waves, slots, tile, out_type, with_sum, n, ic, oc, hw, monkeypatch):
     """192 / 256 input channels (three / four k-steps of 64 per position): the weights of 16 channels fill most of the
-    LDS, one workgroup per CU, of four or of eight waves (64 / 128 tiles a block); 512 channels: with tile size 4 the
-    same, with tile sizes 6 and 5 two passes over half of the columns each, the first pass's results parked in memory"""
+    LDS, one workgroup per CU, of four or of eight waves (64 / 128 tiles a block); 512 channels, whose weights do not fit:
+    both operands through the ring, whatever these switches say"""
     import torch
     monkeypatch.setenv("EHIP_WINO_LANES_WAVES", waves)
-    monkeypatch.setenv("EHIP_WINO_LANES_TWO_PASS", "1")   # (by itself the library keeps so small a layer on the general kernel)
     if slots:
         monkeypatch.setenv("EHIP_WINO_LANES_SLOTS", slots)
     E, p, d, xq, wb, bias = make_wino_u8(n, ic, oc, hw, seed=63 + tile + ic + out_type, out_type=out_type, tile=tile,
@@ -236,7 +235,7 @@ def test_wino_fused_lanes_weights_resident_many_channels(waves, slots, tile, out
     conv.prepare(dev(wb), d_b)
     conv.execute(d_out, dev(xq), None, d_b)
     torch.cuda.synchronize()
-    assert conv.kernel_name.endswith("k_wino_gemm_output_lanes_wres")
+    assert conv.kernel_name.endswith("k_wino_gemm_output_lanes_wres" if ic <= 256 else "k_wino_gemm_output_lanes_ring<32,32>")
     got = host(d_out)
     assert np.array_equal(bits(got), bits(exp)), "output differs at %d of %d" % (int((got != exp).sum()), got.size)
 
@@ -244,10 +243,10 @@ def test_wino_fused_lanes_weights_resident_many_channels(waves, slots, tile, out
 @pytest.mark.parametrize("out_type", [ol.S8, ol.F32])
 @pytest.mark.parametrize("n,ic,oc,hw", [(8, 64, 64, 224), (16, 128, 128, 112), (16, 256, 256, 56), (64, 512, 512, 28)])
 def test_wino_fused_forms_agree_at_full_size(out_type, n, ic, oc, hw, monkeypatch):
-    """the VGG layers at their real planes (a share of the batch), where the weights-resident workgroups take many blocks
-    of tiles each: the three forms of the fused stage -- lanes with resident weights, lanes with both operands streamed,
-    the general kernel -- written independently of each other, leave the same bytes (each is pinned against the oracle
-    at sizes the oracle finishes in seconds by the tests above)"""
+    """the VGG layers at their real planes (a share of the batch), where the workgroups that walk over blocks of tiles take
+    many of them each: the forms of the fused stage -- lanes with resident weights, lanes with both operands streamed, both
+    operands through a ring in LDS, the general kernel -- written independently of each other, leave the same bytes (each is
+    pinned against the oracle at sizes the oracle finishes in seconds by the tests of this file)"""
     import torch
     E = pkg()
     g = torch.Generator(device="cuda").manual_seed(1234 + ic + hw)
@@ -259,11 +258,17 @@ def test_wino_fused_forms_agree_at_full_size(out_type, n, ic, oc, hw, monkeypatc
                     with_bias=True, with_relu=True, input_quant=(1.0 / 255.0, 0.0), tile_size=6, execution_mode=0xa161,
                     wino_tinput_quant=(22.0 / 255.0, 104.0), output_quant=(out_scale, 0.0))
     outs = {}
-    forms = [("resident", {}), ("streamed", {"EHIP_WINO_LANES_WRES": "0"}), ("general", {"EHIP_WINO_LANES": "0"})]
+    # (switches that ask for it, kernel); own: the library's choice
+    resident, streamed = "k_wino_gemm_output_lanes_wres", "k_wino_gemm_output_lanes"
+    ring = "k_wino_gemm_output_lanes_ring<%d,%d>"
+    forms = {"general": ({"EHIP_WINO_LANES": "0"}, "k_wino_gemm_output")}
     if ic > 256:
-        forms.pop(1)   # (the streamed form stops at 256 input channels; 512: two passes with resident weights)
-    for name, env in forms:
-        for k in ("EHIP_WINO_LANES_WRES", "EHIP_WINO_LANES"):
+        forms.update(own=({}, ring % (64, 64)), small=({"EHIP_WINO_RING": "1"}, ring % (32, 32)))
+    else:
+        forms.update(resident=({"EHIP_WINO_RING": "-"}, resident), streamed=({"EHIP_WINO_LANES_WRES": "0"}, streamed),
+                     own=({}, ring % (32, 64) if ic == 256 else resident))
+    for name, (env, kernel) in forms.items():
+        for k in ("EHIP_WINO_LANES_WRES", "EHIP_WINO_LANES", "EHIP_WINO_RING"):
             monkeypatch.delenv(k, raising=False)
         for k, v in env.items():
             monkeypatch.setenv(k, v)
@@ -272,18 +277,12 @@ def test_wino_fused_forms_agree_at_full_size(out_type, n, ic, oc, hw, monkeypatc
         conv.prepare(w, bias)
         conv.execute(out, x, None, bias)
         torch.cuda.synchronize()
-        outs[name] = (out, conv.kernel_name)
+        assert conv.kernel_name.endswith(kernel), name
+        outs[name] = out
         del conv
-    assert outs["resident"][1].endswith("k_wino_gemm_output_lanes_wres")
-    if "streamed" in outs:
-        assert outs["streamed"][1].endswith("k_wino_gemm_output_lanes")
-    assert outs["general"][1].endswith("k_wino_gemm_output")
-    ref = outs["general"][0]
+    ref = outs["general"]
     assert int((ref.view(torch.uint8) != 0).sum()) > ref.numel() // 8   # (not a layer of zeros)
-    for name in ("resident", "streamed"):
-        if name not in outs:
-            continue
-        got = outs[name][0]
+    for name, got in outs.items():
         assert torch.equal(got.view(torch.uint8), ref.view(torch.uint8)), "%s differs from the general kernel at %d values" % (
             name, int((got != ref).sum()))
 
@@ -664,6 +663,6 @@ def test_wino_fused_ring(form, tile, out_type, with_sum, with_relu, n, ic, oc, h
     conv.prepare(dev(wb), d_b)
     conv.execute(d_out, dev(xq), None, d_b)
     torch.cuda.synchronize()
-    assert conv.kernel_name.endswith("k_wino_gemm_output_lanes_wres")
+    assert conv.kernel_name.endswith("k_wino_gemm_output_lanes_ring<%s>" % {"0": "64,64", "1": "32,32", "2": "32,64"}[form])
     got = host(d_out)
     assert np.array_equal(bits(got), bits(exp)), "output differs at %d of %d" % (int((got != exp).sum()), got.size)
