@@ -34,19 +34,30 @@ def run_and_compare(layer, lazy=False):
 
 
 # ---- 1x1 (CONV_DIRECT_1X1 a160; f32 output goes through CONV_DIRECT a160) ----------------------
+@pytest.fixture(params=["", "0"], ids=["own", "nosplit"])
+def with_and_without_k_split(request, monkeypatch):
+    """layers of a few hundred output tiles take the kernel with the K loop split by themselves; the same layers through the
+    kernels that larger ones take"""
+    if request.param:
+        monkeypatch.setenv("EHIP_GEMM1X1_SPLIT", request.param)
+
+
 @pytest.mark.parametrize("out_type", [ol.S32, ol.U8, ol.S8, ol.F32])
 @pytest.mark.parametrize("n,ic,oc,hw", [(2, 64, 64, 9), (1, 80, 48, 7), (3, 128, 272, 5)])
+@pytest.mark.usefixtures("with_and_without_k_split")
 def test_conv1x1_s1(out_type, n, ic, oc, hw):
     run_and_compare(Layer(n, ic, oc, hw, out_type=out_type, seed=11 + ic + out_type))
 
 
 @pytest.mark.parametrize("out_type", [ol.U8, ol.S8])
+@pytest.mark.usefixtures("with_and_without_k_split")
 def test_conv1x1_sum_relu(out_type):
     run_and_compare(Layer(2, 96, 64, 14, out_type=out_type, with_sum=True, seed=5))
 
 
 @pytest.mark.parametrize("out_type", [ol.U8, ol.S8])
 @pytest.mark.parametrize("with_sum", [False, True])
+@pytest.mark.usefixtures("with_and_without_k_split")
 def test_conv1x1_every_zero_point(out_type, with_sum):
     """input, output and sum zero points all non-zero: the folded shift (compared bit for bit with the
     oracle's, whose contraction pattern is that of the reference's compiled fold) and the result"""
@@ -61,6 +72,7 @@ def test_conv3x3_and_depthwise_output_zero_point():
 
 
 @pytest.mark.parametrize("out_type", [ol.S32, ol.S8])
+@pytest.mark.usefixtures("with_and_without_k_split")
 def test_conv1x1_stride2(out_type):
     run_and_compare(Layer(2, 64, 96, 14, stride=2, out_type=out_type, with_sum=(out_type == ol.S8), seed=6))
 
@@ -84,6 +96,7 @@ def test_conv1x1_resident_pixel_tile_kernel(variant, n, ic, oc, hw, stride, monk
 def test_conv1x1_resident_pixel_tile_kernel_nhwc_output(variant, n, ic, oc, hw, stride, monkeypatch):
     """blocked input, nhwc output, u8 / s8 with ReLU (the lean epilogue's cases): a lane's 16 channels are 16
     contiguous bytes of its pixel's vector; with the sum the old output is read from the same place"""
+    monkeypatch.setenv("EHIP_GEMM1X1_SPLIT", "0")   # (by itself the library splits the K loop of layers this small)
     if variant:
         monkeypatch.setenv("EHIP_GEMM1X1_RES", variant)
     for out_type, with_sum, kw in ((ol.U8, False, {}), (ol.S8, True, {}), (ol.U8, True, {"relu_hi": 200.0})):
@@ -107,6 +120,7 @@ def test_conv1x1_resident_pixel_tile_kernel_nhwc_output(variant, n, ic, oc, hw, 
 def test_conv1x1_resident_pixel_tile_kernel_nhwc_input(variant, n, ic, oc, hw, stride, monkeypatch):
     """nhwc input: the tile pixel-major in LDS (one pad cell per pixel); blocked output with every output
     type, nhwc output with the lean epilogue's cases; generic and unrolled K loops, stride 2, ragged tiles"""
+    monkeypatch.setenv("EHIP_GEMM1X1_SPLIT", "0")   # (by itself the library splits the K loop of layers this small)
     if variant:
         monkeypatch.setenv("EHIP_GEMM1X1_RES", variant)
     for out_type, with_sum in ((ol.U8, False), (ol.S8, True), (ol.F32, False), (ol.S32, False)):
@@ -169,6 +183,7 @@ def test_conv1x1_resident_pixel_tile_kernel_can_be_switched_off(monkeypatch):
     run_and_compare(Layer(2, 256, 256, 14, out_type=ol.S8, with_sum=True, seed=302))
 
 
+@pytest.mark.usefixtures("with_and_without_k_split")
 def test_conv1x1_lazy_first_run_and_no_bias():
     run_and_compare(Layer(1, 64, 32, 6, out_type=ol.U8, with_bias=False, seed=8), lazy=True)
 
@@ -218,12 +233,14 @@ def test_conv1x1_few_input_channels_can_be_switched_off(monkeypatch):
 # values are the oracle's, moved through the closed-form index map [n][c/16][h][w][16] -> [n][h][w][c]
 @pytest.mark.parametrize("in_nhwc,out_nhwc", [(True, True), (True, False), (False, True)])
 @pytest.mark.parametrize("out_type", [ol.S32, ol.U8, ol.S8, ol.F32])
+@pytest.mark.usefixtures("with_and_without_k_split")
 def test_conv1x1_nhwc(in_nhwc, out_nhwc, out_type):
     run_and_compare(Layer(3, 128, 272 if not out_nhwc else 176, 5, out_type=out_type, seed=70 + out_type,
                           in_nhwc=in_nhwc, out_nhwc=out_nhwc))
 
 
 @pytest.mark.parametrize("stride", [1, 2])
+@pytest.mark.usefixtures("with_and_without_k_split")
 def test_conv1x1_nhwc_sum_relu(stride):
     run_and_compare(Layer(2, 96, 64, 14, stride=stride, out_type=ol.S8, with_sum=True, seed=75, in_nhwc=True, out_nhwc=True))
 
@@ -532,13 +549,19 @@ def test_depthwise_on_the_matrix_cores(g, hw, pad, T, relu_hi, in_z, monkeypatch
 def test_depthwise_matrix_core_kernel_is_the_default_where_it_fits(monkeypatch):
     monkeypatch.delenv("EHIP_DW_MFMA", raising=False)
     E = pkg()
-    names = {}
-    for hw in (7, 14, 28, 56, 112):
-        d = E.make_desc(1, 32, 32, hw, hw, 3, 3, pad=1, g=32, output_type=E.U8, relu_bound=(0.0, 255.0), flatting_t=7,
+    w, b = dev(np.zeros((32, 3, 3), np.float32)), dev(np.zeros(32, np.float32))
+
+    def name(n, hw):   # (final once the handle is prepared)
+        d = E.make_desc(n, 32, 32, hw, hw, 3, 3, pad=1, g=32, output_type=E.U8, relu_bound=(0.0, 255.0), flatting_t=7,
                         output_quant=(0.02, 0.0))
-        names[hw] = E.Conv(d).kernel_name
+        conv = E.Conv(d)
+        conv.prepare(w, b)
+        return conv.kernel_name
+
+    names = {hw: name(2048, hw) for hw in (7, 14, 28, 56, 112)}
     assert names[112] == names[56] == names[28] == "k_depthwise3x3_mfma"
     assert names[7] == names[14] == "k_depthwise3x3_u8s8"   # half-empty chunks and strips: the dot4 kernel
+    assert {name(1, hw) for hw in (7, 14, 28, 56, 112)} == {"k_depthwise3x3_u8s8"}   # small layers: one or two rows per lane
 
 
 # stride 2 (MobileNet's down-sampling layers, scripts/best_configs/mobilenetv1-n64-clx-1s-int8.sh:48:
@@ -722,17 +745,26 @@ def test_setup_refuses_what_no_kernel_can_address():
     assert ei.value.code == E.EHIP_UNIMPLEMENTED and "tensor too large" in str(ei.value)
 
 
-@pytest.mark.parametrize("kind", ["1x1 many channels", "1x1 many channels, sum, nhwc", "1x1 few channels", "1x1 few channels f32", "3x3",
-                                  "3x3 stride 2", "depthwise 56", "depthwise 7", "depthwise stride 2", "first layer", "first layer f32"])
-def test_prepared_handle_on_other_buffers(kind):
-    # a handle keeps its launch (kernel, grid, derived and leading scalar arguments) from the first execute; the
+@pytest.mark.parametrize("kind,kernel", [("1x1 many channels", "k_gemm_u8s8"), ("1x1 many channels, sum, nhwc", "k_gemm1x1_res"),
+                                         ("1x1 few channels", "k_gemm_smallk_lean"), ("1x1 few channels f32", "k_gemm_smallk_u8s8"),
+                                         ("1x1 K split", "k_gemm1x1_split"), ("3x3", "k_conv3x3v"), ("3x3 stride 2", "k_conv3x3v"),
+                                         ("depthwise 56", "k_depthwise3x3_mfma"), ("depthwise 7", "k_depthwise3x3_u8s8"),
+                                         ("depthwise stride 2", "k_depthwise3x3_u8s8"), ("first layer", "k_conv_fewch_lean"),
+                                         ("first layer f32", "k_conv_fewch_u8s8")])
+def test_prepared_handle_on_other_buffers(kind, kernel, monkeypatch):
+    # a handle keeps its launch (kernel, grid, derived and leading scalar arguments) from its creation; the
     # next execute must run on the tensors it is given: same bytes into a fresh output at another address
+    if kind.startswith("1x1"):   # (the kernels that larger layers take)
+        monkeypatch.setenv("EHIP_GEMM1X1_SPLIT", "1" if kind == "1x1 K split" else "0")
+    if kind == "depthwise 56":
+        monkeypatch.setenv("EHIP_DW_MFMA", "1")
     layer = {
         "1x1 many channels": lambda: Layer(2, 256, 144, 14, out_type=ol.U8, seed=501),
         "1x1 many channels, sum, nhwc": lambda: Layer(2, 512, 256, 14, stride=2, out_type=ol.S8, with_sum=True, in_nhwc=True,
                                                       out_nhwc=True, seed=502),
         "1x1 few channels": lambda: Layer(2, 64, 128, 14, out_type=ol.U8, seed=503),
         "1x1 few channels f32": lambda: Layer(1, 32, 48, 9, out_type=ol.F32, seed=504),
+        "1x1 K split": lambda: Layer(2, 256, 144, 14, out_type=ol.U8, with_sum=True, seed=512),
         "3x3": lambda: Layer(2, 64, 64, 14, k=3, pad=1, out_type=ol.U8, seed=505),
         "3x3 stride 2": lambda: Layer(2, 32, 32, 15, k=3, pad=1, stride=2, out_type=ol.S8, seed=506),
         "depthwise 56": lambda: Layer(2, 32, 32, 56, k=3, pad=1, depthwise=True, out_type=ol.U8, seed=507, T=14, relu_hi=255.0),
@@ -742,6 +774,7 @@ def test_prepared_handle_on_other_buffers(kind):
         "first layer f32": lambda: Layer(2, 3, 32, 23, k=3, pad=1, stride=2, out_type=ol.F32, seed=511, in_nhwc=True, with_relu=False),
     }[kind]()
     res = run_and_compare(layer)
+    assert res["conv"].kernel_name.startswith(kernel)
     again = layer.rerun_gpu(res["conv"])
     assert again.shape == res["out"].shape and (again == res["out"]).all(), kind
 

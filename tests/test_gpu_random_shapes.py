@@ -15,8 +15,11 @@ def _rng(seed):
     return np.random.default_rng(1000 + seed)
 
 
+@pytest.mark.parametrize("split", ["", "0"])   # (the library splits the K loop of most of these small layers)
 @pytest.mark.parametrize("seed", range(24))
-def test_random_1x1(seed):
+def test_random_1x1(seed, split, monkeypatch):
+    if split:
+        monkeypatch.setenv("EHIP_GEMM1X1_SPLIT", split)
     r = _rng(seed)
     stride = int(r.choice([1, 1, 2]))
     nhwc_in, nhwc_out = bool(r.integers(0, 2)), bool(r.integers(0, 2))

@@ -97,15 +97,16 @@ def test_wino_tinput_under_range_and_both_gathers(tile, buf_gather, monkeypatch)
                                         (2, 256, 64, 9), (1, 272, 32, 6)])
 def test_wino_fused_gemm_and_output_transform(n, ic, oc, hw):
     """Default schedule: GEMM + output transform in one kernel; final output bit for bit."""
-    _fused(n, ic, oc, hw)
+    assert "k_wino_gemm_output_lanes" in _fused(n, ic, oc, hw).kernel_name
 
 
 @pytest.mark.parametrize("ring", ["2", "4", "8"])
 def test_wino_fused_every_operand_ring_depth(ring, monkeypatch):
     """256 input channels = 8 k-steps per position: the fused kernel with its operands requested 2, 4 and 8
     k-steps ahead (three instantiations; 4 is the default where it divides the k-steps)"""
+    monkeypatch.setenv("EHIP_WINO_LANES", "0")   # (the general kernel)
     monkeypatch.setenv("EHIP_WINO_KS", ring)
-    _fused(2, 256, 80, 9)
+    assert _fused(2, 256, 80, 9).kernel_name.endswith("k_wino_gemm_output")
 
 
 @pytest.mark.parametrize("halves", ["1", "2"])
@@ -113,8 +114,9 @@ def test_wino_fused_every_operand_ring_depth(ring, monkeypatch):
 def test_wino_fused_channels_per_workgroup(halves, n, ic, oc, hw, monkeypatch):
     """the fused kernel with workgroups of 32 channels (what layers of few tiles get, so that every CU has a
     workgroup) and of 64; ragged channel counts leave the last workgroup partly past the real channels"""
+    monkeypatch.setenv("EHIP_WINO_LANES", "0")   # (the general kernel)
     monkeypatch.setenv("EHIP_WINO_HALVES", halves)
-    _fused(n, ic, oc, hw)
+    assert _fused(n, ic, oc, hw).kernel_name.endswith("k_wino_gemm_output")
 
 
 @pytest.mark.parametrize("flat", ["0", "1"])
@@ -123,6 +125,7 @@ def test_wino_fused_channels_per_workgroup(halves, n, ic, oc, hw, monkeypatch):
 def test_wino_fused_few_input_channels(flat, tile, ic, monkeypatch):
     """64 / 128 input channels (2 / 4 k-steps per position): the operand ring running ahead over the positions as one
     flat sequence of steps, and filled position by position; 48 channels (padded to 64) as well"""
+    monkeypatch.setenv("EHIP_WINO_LANES", "0")   # (the general kernel)
     monkeypatch.setenv("EHIP_WINO_FLAT", flat)
     import torch
     E, p, d, xq, wb, bias = make_wino_u8(2, ic, 80, 13, seed=31 + tile + ic, out_type=ol.S8, tile=tile)
@@ -136,6 +139,7 @@ def test_wino_fused_few_input_channels(flat, tile, ic, monkeypatch):
     conv.prepare(dev(wb), d_b)
     conv.execute(d_out, dev(xq), None, d_b)
     torch.cuda.synchronize()
+    assert conv.kernel_name.endswith("k_wino_gemm_output")
     got = host(d_out)
     assert np.array_equal(bits(got), bits(exp)), "output differs at %d of %d" % (int((got != exp).sum()), got.size)
 
@@ -307,6 +311,7 @@ def _fused(n, ic, oc, hw):
     assert np.array_equal(conv.query(E.Q_TINPUT_U8).reshape(tin.shape), tin)
     got = host(d_out)
     assert np.array_equal(bits(got), bits(exp)), "output differs at %d of %d" % (int((got != exp).sum()), got.size)
+    return conv
 
 
 def make_wino_u8(n, ic, oc, hw, seed, out_type, with_bias=True, with_relu=True, out_scale=None, out_z=0.0, tile=6):
