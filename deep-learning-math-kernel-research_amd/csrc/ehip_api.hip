@@ -614,7 +614,7 @@ static int plan_execute(ehip_conv *c)
     if (c->fused) {
       WinoFusedArgs f;
       memset(&f, 0, sizeof(f));
-      f.tin = c->tin; f.tin_blocked = c->tin_blocked; f.w = c->wpacked;
+      f.tin = c->tin; f.w = c->wpacked;
       f.scale = c->scale; f.shift = c->shift; f.comp = c->comp;
       f.n = w.n; f.ic2 = c->ic2; f.units_pad = c->units_pad; f.oc2 = c->oc2; f.ocpp = c->ocpp;
       f.oh = d.oh; f.ow = d.ow; f.ht = w.ht; f.wt = w.wt; f.nt = w.nt; f.t = w.t;

@@ -123,8 +123,7 @@ struct WinoArgs {
 };
 
 struct WinoFusedArgs {
-  const uint8_t *tin;   // (tin_blocked) [t / 32][36][ic2][32][16]: code - 128 (the general kernel also reads [36][ic2][t][16])
-  int tin_blocked;
+  const uint8_t *tin;   // [t / 32][36][ic2][32][16]: code - 128
   const int8_t *w;      // [36][units_pad][OCpp][16] s8
   void *out;            // [n][oc2][oh][ow][16] f32 / u8 / s8 (out_type)
   const float *bias;

@@ -615,14 +615,12 @@ __global__ __launch_bounds__(kBlock, 1) void k_wino_gemm_output(const WinoFusedA
   // operand addresses = wave-uniform pointer (scalar arithmetic) + a per-lane 32-bit offset that
   // never changes: lane = packed row / tile l32 of unit 2 * ks + lh
   const unsigned a_lane = (unsigned)(lh * a.ocpp + l32) * 16u;
-  // plain layout: tile `tile` of unit lh; blocked: cell l32 of unit lh inside the block's own run (cells of
-  // tiles past the end hold nothing and are never stored; a block past the last one reads the last one)
-  unsigned b_lane[NT];
+  // cell l32 of unit lh inside the block's own run (cells of tiles past the end hold nothing and are never stored; a
+  // block past the last one reads the last one)
+  const unsigned b_lane = (unsigned)(lh * 32 + l32) * 16u;
   long long b_block[NT];
 #pragma unroll
   for (int j = 0; j < NT; ++j) {
-    const int tile = t0 + 32 * j + l32 < a.t ? t0 + 32 * j + l32 : a.t - 1;
-    b_lane[j] = a.tin_blocked ? (unsigned)(lh * 32 + l32) * 16u : (unsigned)(lh * a.t + tile) * 16u;
     const int nb32 = (a.t + 31) >> 5;
     b_block[j] = bx * NT + j < nb32 ? bx * NT + j : nb32 - 1;
   }
@@ -639,9 +637,8 @@ __global__ __launch_bounds__(kBlock, 1) void k_wino_gemm_output(const WinoFusedA
     const int ksc = ks < ks_last ? ks : ks_last;
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
-      const uint8_t *pb = a.tin_blocked ? a.tin + ((b_block[j] * AA + p) * a.ic2 + 2 * ksc) * 512
-                                        : a.tin + ((long long)p * a.ic2 + 2 * ksc) * a.t * 16;
-      rb[slot][j] = *reinterpret_cast<const v4i *>(pb + b_lane[j]);
+      const uint8_t *pb = a.tin + ((b_block[j] * AA + p) * a.ic2 + 2 * ksc) * 512;
+      rb[slot][j] = *reinterpret_cast<const v4i *>(pb + b_lane);
     }
   };
 

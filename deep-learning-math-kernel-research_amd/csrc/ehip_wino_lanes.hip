@@ -455,7 +455,7 @@ bool wino_lanes_applies(const WinoFusedArgs &a)
   // Measured at N = 64, u8 in / s8 out, against the general kernel (fused stage, us): 64 -> 64 at 56 x 56 28.5 vs 34.1, at
   // 224 x 224 370 vs 459; 128 -> 128 at 112 x 112 238 vs 300; 128 -> 256 at 56 x 56 107 vs 133; 256 -> 256 at 56 x 56 164 vs 171;
   // the weights of 16 channels at every position must fit the LDS (the streamed form: 1, 2 or 4 k-steps): up to 256 channels.
-  return a.tin_blocked && nks64 <= 4 && a.units_pad % 4 == 0 && a.units_pad >= 4 * nks64 && !(a.out_type == EHIP_F32 && a.with_sum) &&
+  return nks64 <= 4 && a.units_pad % 4 == 0 && a.units_pad >= 4 * nks64 && !(a.out_type == EHIP_F32 && a.with_sum) &&
       !(env && env[0] == '0');
 }
 

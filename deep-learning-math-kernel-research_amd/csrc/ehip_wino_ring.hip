@@ -10,7 +10,7 @@ int wino_ring_pick(const WinoFusedArgs &a)
   const int nks64 = (a.ic2 + 3) / 4;
   // whole stages of k-steps; 32-bit offsets into the weights
   const int kc = nks64 <= 4 ? 4 : (nks64 <= 6 ? 6 : (nks64 + 1) / 2 * 2);
-  if (!a.tin_blocked || a.units_pad < 4 * kc || (a.out_type == EHIP_F32 && a.with_sum)) return -1;
+  if (a.units_pad < 4 * kc || (a.out_type == EHIP_F32 && a.with_sum)) return -1;
   if ((long long)A * A * a.units_pad * a.ocpp * 16 > 0xffffffffll) return -1;
   for (const char *other : {"EHIP_WINO_LANES", "EHIP_WINO_LANES_WRES"})   // (the other forms asked for)
     if (const char *env = getenv(other)) if (env[0] == '0') return -1;
