@@ -154,7 +154,8 @@ struct WinoFusedArgs {
 constexpr size_t kMaxKernarg = 104;   // (the step is between 104 and 128)
 constexpr size_t kArgBlock = 512;     // device memory of one argument structure
 struct LaunchPlan {
-  void *args_dev = nullptr;     // kArgBlock bytes of device memory, set when the handle is created
+  void *args = nullptr;         // the argument structure: kArgBlock bytes of the handle, copied to args_dev once planned
+  void *args_dev = nullptr;     // kArgBlock bytes of device memory
   hipFunction_t fn = nullptr;   // of the device the handle was created on
   dim3 grid, block;
   unsigned lds = 0;
@@ -186,8 +187,7 @@ struct KernargWriter {
   template <typename P> void put(const ArgBias &) { raw(nullptr, 8, &p.bias_at); }
   template <typename P> void put(const ArgBlock &) { raw(&p.args_dev, 8); }
 };
-// `a` in the order of the kernel's parameters, each converted to its parameter's type.  (The copy is complete once the null
-// stream has been waited for, as ehip_conv_create does.)
+// `a` in the order of the kernel's parameters, each converted to its parameter's type
 template <typename Args, typename... P, typename... A>
 inline hipError_t plan_set(LaunchPlan &p, void (*kernel)(P...), dim3 grid, dim3 block, size_t lds, const Args &args, A... a)
 {
@@ -205,7 +205,7 @@ inline hipError_t plan_set(LaunchPlan &p, void (*kernel)(P...), dim3 grid, dim3 
   if (lds > 48 * 1024)
     e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e == hipSuccess) e = hipGetFuncBySymbol(&p.fn, reinterpret_cast<const void *>(kernel));
-  if (e == hipSuccess) e = hipMemcpy(p.args_dev, &args, sizeof(Args), hipMemcpyHostToDevice);
+  memcpy(p.args, &args, sizeof(Args));
   return e;
 }
 // The kept plan is only read: the tensors of this call go into a copy of the kernel arguments, so executes of one
