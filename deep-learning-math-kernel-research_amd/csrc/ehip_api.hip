@@ -4,6 +4,7 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <mutex>
 #include <utility>
 #include <vector>
 
@@ -90,11 +91,34 @@ void free_all(ehip_conv *c)
     if (p) (void)hipFree(p);
 }
 
+// What creating a handle puts on the device (cleared workspaces, argument structures) runs on a stream that the library
+// keeps per device, and creation waits for that stream: whatever stream the handle is used on next finds it done, and
+// nobody waits for what the caller has queued on the null stream.
+constexpr int kMaxDevices = 64;
+std::mutex g_setup_mutex;
+hipStream_t g_setup_stream[kMaxDevices];   // by device ordinal; null until the device's first handle
+
+int setup_stream(hipStream_t *s)
+{
+  int dev = -1;
+  HIP_TRY(hipGetDevice(&dev));
+  if (dev < 0 || dev >= kMaxDevices) return fail(EHIP_GENERAL_ERROR, "device ordinal out of range");
+  std::lock_guard<std::mutex> lock(g_setup_mutex);
+  if (!g_setup_stream[dev]) HIP_TRY(hipStreamCreateWithFlags(&g_setup_stream[dev], hipStreamNonBlocking));
+  *s = g_setup_stream[dev];
+  return EHIP_OK;
+}
+
 template <typename T>
 int dev_alloc(T **p, size_t count, bool zero)
 {
   HIP_TRY(hipMalloc(reinterpret_cast<void **>(p), count * sizeof(T)));
-  if (zero) HIP_TRY(hipMemset(*p, 0, count * sizeof(T)));
+  if (zero) {
+    hipStream_t s;
+    const int rc = setup_stream(&s);
+    if (rc != EHIP_OK) return rc;
+    HIP_TRY(hipMemsetAsync(*p, 0, count * sizeof(T), s));
+  }
   return EHIP_OK;
 }
 
@@ -658,12 +682,14 @@ static int plan_execute(ehip_conv *c)
   return EHIP_OK;
 }
 
-// The argument structures to the device, and a wait for everything that creating the handle has put on the null stream
-// (cleared workspaces, this copy): other streams need not wait for that one.
+// The argument structures to the device, and the wait for all that creating the handle has put there.
 static int finish_create(ehip_conv *c)
 {
-  HIP_TRY(hipMemcpyAsync(c->args_dev, c->args, (size_t)c->nplans * kArgBlock, hipMemcpyHostToDevice, nullptr));
-  HIP_TRY(hipStreamSynchronize(nullptr));
+  hipStream_t s;
+  const int rc = setup_stream(&s);
+  if (rc != EHIP_OK) return rc;
+  HIP_TRY(hipMemcpyAsync(c->args_dev, c->args, (size_t)c->nplans * kArgBlock, hipMemcpyHostToDevice, s));
+  HIP_TRY(hipStreamSynchronize(s));
   return EHIP_OK;
 }
 

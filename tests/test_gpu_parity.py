@@ -779,6 +779,27 @@ def test_prepared_handle_on_other_buffers(kind, kernel, monkeypatch):
     assert again.shape == res["out"].shape and (again == res["out"]).all(), kind
 
 
+@pytest.mark.parametrize("kw", [dict(ic=64, oc=96), dict(ic=48, oc=48, k=3, pad=1, T=7), dict(ic=32, oc=32, k=3, pad=1, depthwise=True, T=7)])
+def test_handle_created_and_used_while_the_default_stream_is_busy(kw):
+    """a handle created, prepared and executed on a side stream does not wait for the default stream, so nothing that its
+    creation does (cleared workspaces, argument structures) may be queued there behind the caller's work"""
+    import torch
+    E = pkg()
+    layer = Layer(2, hw=14, out_type=ol.U8, seed=530, **kw)
+    exp = layer.oracle()["out"]
+    d_x, d_w, d_b = dev(layer.xb), dev(layer.wb), dev(layer.bias)
+    d_out = torch.full(exp.shape, 99, dtype=torch.uint8, device="cuda")
+    busy, side = torch.zeros(1 << 24, device="cuda"), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    for _ in range(50):
+        busy.add_(1.0)
+    conv = E.Conv(layer.desc)
+    conv.prepare(d_w, d_b, stream=side.cuda_stream)
+    conv.execute(d_out, d_x, stream=side.cuda_stream)
+    torch.cuda.synchronize()
+    assert np.array_equal(host(d_out), exp)
+
+
 # ---- depthwise: rows per lane by the size of the layer ----------------------------------------------------
 @pytest.mark.parametrize("n,g,hw,stride", [(1, 32, 14, 1), (1, 16, 57, 1), (4, 64, 28, 1), (6, 32, 56, 1), (1, 48, 28, 2), (2, 32, 57, 2),
                                            (64, 32, 7, 1)])
