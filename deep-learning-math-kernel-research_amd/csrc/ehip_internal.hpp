@@ -124,6 +124,7 @@ struct WinoArgs {
 
 struct WinoFusedArgs {
   const uint8_t *tin;   // [t / 32][36][ic2][32][16]: code - 128
+  long long *trace;     // development aid, normally null (see EHIP_TRACE)
   const int8_t *w;      // [36][units_pad][OCpp][16] s8
   void *out;            // [n][oc2][oh][ow][16] f32 / u8 / s8 (out_type)
   const float *bias;
@@ -139,7 +140,6 @@ struct WinoFusedArgs {
   int nx, ny;           // set by the launcher: blocks of 32 tiles, of 64 channels
   int slots;            // set by the lanes launcher: workgroups per XCD and channel block
   int nkc;              // set by the ring launcher: stages per position
-  long long *trace;     // development aid, normally null (see EHIP_TRACE)
 };
 
 // ---- launch plans -------------------------------------------------------------------------------
