@@ -256,6 +256,8 @@ bool depthwise_mfma_applies(int stride, int oh, int ow, int pad_t, int pad_l, in
 hipError_t plan_wino_trans_input(LaunchPlan &plan, const WinoArgs &a);
 hipError_t plan_wino_trans_output(LaunchPlan &plan, const WinoArgs &a);
 hipError_t plan_wino_gemm_output(LaunchPlan &plan, const WinoFusedArgs &a);
+// workgroups of the general fused kernel; halves (may be null): 32-channel halves of a workgroup
+long long wino_general_workgroups(const WinoFusedArgs &a, int *halves);
 // at most 256 input channels: the form without an exchange between GEMMs and transform (ehip_wino_lanes.hip)
 bool wino_lanes_applies(const WinoFusedArgs &a);
 hipError_t plan_wino_gemm_output_lanes(LaunchPlan &plan, const WinoFusedArgs &a);

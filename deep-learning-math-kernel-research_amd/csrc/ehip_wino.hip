@@ -835,6 +835,18 @@ hipError_t plan_wino_trans_output(LaunchPlan &plan, const WinoArgs &a)
   return plan_set(plan, kern, grid, dim3(kBlock), 0, a, ArgBlock{}, ArgOut{a.out}, ArgBias{});
 }
 
+long long wino_general_workgroups(const WinoFusedArgs &a, int *halves)
+{
+  const int A = a.tile ? a.tile : 6, ntb = A == 4 ? 2 : 1, oc = a.oc2 * 16;
+  const long long nx = (a.t + 32 * ntb - 1) / (32 * ntb);
+  // 64 channels per workgroup; 32 where that would leave a quarter of the CUs or more without a workgroup
+  int nh = 2;
+  if (ntb == 1 && nx * ((oc + 63) / 64) <= 192 && oc > 32) nh = 1;
+  if (const char *env = getenv("EHIP_WINO_HALVES")) if (ntb == 1 && (env[0] == '1' || env[0] == '2')) nh = env[0] - '0';
+  if (halves) *halves = nh;
+  return nx * ((oc + 32 * nh - 1) / (32 * nh));
+}
+
 // k-steps per ring block: the largest of 8, 4, 2 that divides the k-steps of a position
 hipError_t plan_wino_gemm_output(LaunchPlan &plan, const WinoFusedArgs &a0)
 {
@@ -845,10 +857,8 @@ hipError_t plan_wino_gemm_output(LaunchPlan &plan, const WinoFusedArgs &a0)
   if (wino_lanes_applies(a)) return plan_wino_gemm_output_lanes(plan, a);
   const int ntb = A == 4 ? 2 : 1;   // blocks of 32 tiles per workgroup
   a.nx = (a.t + 32 * ntb - 1) / (32 * ntb);
-  // 64 channels per workgroup; 32 where that would leave a quarter of the CUs or more without a workgroup
   int nh = 2;
-  if (ntb == 1 && (long long)a.nx * ((a.oc2 * 16 + 63) / 64) <= 192 && a.oc2 * 16 > 32) nh = 1;
-  if (const char *env = getenv("EHIP_WINO_HALVES")) if (ntb == 1 && (env[0] == '1' || env[0] == '2')) nh = env[0] - '0';
+  wino_general_workgroups(a, &nh);
   a.ny = (a.oc2 * 16 + 32 * nh - 1) / (32 * nh);
   const int nks = a.units_pad / 2;
   const size_t lds = (size_t)AA * 32 * 32 * sizeof(float) + 4 * (size_t)((AA + 3) / 4 * 24) * sizeof(float4);   // exchange + constants
