@@ -479,9 +479,6 @@ dw_kernel_t kernel_rb(int stride, int mode)
 }
 }  // namespace
 
-// The matrix-core kernel: stride 1, u8 output with a ReLU inside the code range, pads 0 / 1, and a plane
-// of up to four 32-column chunks whose chunks and 8-row strips are mostly real pixels (EHIP_DW_MFMA=0 / 1
-// overrides the last condition).
 // Lanes of a dot4 launch with one output row per lane.  Small layers are bound by the latency of a lane's chain of loads and
 // rows and by CUs without work, not by the halo rows read again: they take one row per lane, and none runs on the matrix
 // cores, whose workgroups start from eight staged rows.  Measured (us; one row / two / the choice of the large layers):
@@ -492,6 +489,9 @@ dw_kernel_t kernel_rb(int stride, int mode)
 constexpr long long kOneRow = 110000, kTwoRows = 260000, kOneRowStride2 = 450000;
 static long long one_row_lanes(long long planes, int oh, int ow) { return planes * oh * ((ow + 1) / 2) * 4; }
 
+// The matrix-core kernel, for layers that are not small (plan_depthwise asks that first): stride 1, u8 output with a ReLU
+// inside the code range, pads 0 / 1, and a plane of up to four 32-column chunks whose chunks and 8-row strips are mostly
+// real pixels.  EHIP_DW_MFMA=0 / 1 overrides the last condition and the size of the layer.
 bool depthwise_mfma_applies(int stride, int oh, int ow, int pad_t, int pad_l, int out_type, int with_relu, float lo, float hi,
                             long long planes, int ih, int iw)
 {

@@ -8,7 +8,8 @@
 // 100 KB through one CU and multiplies sixteen k-steps in a row.  In this kernel a workgroup owns ONE tile of 32 channels x
 // 32 pixels and its NW waves take KPW k-steps (of 32 channels) each: all of a wave's operands are requested at once,
 // straight into registers, so the chain is one trip to memory, KPW multiplies, one exchange of partial sums through LDS and
-// the epilogue of 16 values per lane.
+// the epilogue of 16 values per lane.  The last two are the first wave's alone: it adds up to eight partial sums and
+// finishes the 32 x 32 values while the others have ended.
 #include "ehip_internal.hpp"
 
 namespace ehip {

@@ -150,7 +150,9 @@ struct WinoFusedArgs {
 // launch finds it there on whatever stream it runs and whether or not that stream waits for the one that packs the weights.
 // What that buys: HIP writes kernel arguments into device memory across PCIe, and a launch with 300 bytes of them
 // costs the host 3.4 us where 16-96 bytes cost 2.6 (128: 3.25, 256: 3.45; empty kernel, back to back) -- as long as a
-// small layer's kernel takes on the GPU.
+// small layer's kernel takes on the GPU.  It is host time: a loop of small layers gains it (1x1 64 -> 256 at 56 x 56, N = 1,
+// 4.0 -> 3.6 us a call), a single call between other work hardly does, because a kernel that needs the structure for its
+// first load waits for a line of memory of its own.
 constexpr size_t kMaxKernarg = 104;   // (the step is between 104 and 128)
 constexpr size_t kArgBlock = 512;     // device memory of one argument structure
 struct LaunchPlan {

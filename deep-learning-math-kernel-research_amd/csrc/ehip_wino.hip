@@ -234,9 +234,10 @@ __device__ __forceinline__ void gather_tile_wide(const WinoArgs &, const TileCoo
 // block: 64 consecutive tiles x 4 channel quads of one 16-channel unit.  Work items are numbered tile
 // block first, then unit, and XCD x (workgroup b runs on XCD b % 8) takes the x-th eighth of them:
 // neighbouring tile blocks read the same two input rows where they meet, and find them in their XCD's L2.
-// Tiles that touch the zero frame take the reference's "border" arithmetic, the others the plain one; a
-// wave that holds both kinds (nearly every wave: two rim tiles per row of tiles) runs the per-lane,
-// branch-free form of the transform instead of both forms under complementary masks.
+// Tiles that touch the zero frame take the reference's "border" arithmetic, the others the plain one; with f32 input a
+// wave that holds both kinds (nearly every wave: two rim tiles per row of tiles) runs the per-lane, branch-free form of
+// the transform instead of both forms under complementary masks.  u8 codes take one form in every wave, with the choice in
+// one product of the last row (tile_input_lanes).
 // Cell = float4 (f32 user input) or unsigned (u8 user input: four codes per lane and pixel).
 template <typename Cell, int A = 6>
 __global__ __launch_bounds__(kBlock) void k_wino_trans_input_u8(const WinoArgs *rest, const void *in)

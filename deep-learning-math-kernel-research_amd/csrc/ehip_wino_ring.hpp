@@ -8,13 +8,19 @@
 // What bounds it: a CU takes 58 bytes a clock through its L1, so the product of a weight and a tile byte is only as cheap
 // as the block of channels x tiles they are shared in.  With the weights of 16 channels resident (ehip_wino_lanes.hip) a
 // byte of the transformed input feeds 16 products; a workgroup of 64 channels x 64 tiles makes it 32 for both operands, and
-// needs no more than a third of the registers for results because the positions are finished one after the other: a
-// position's 64 x 64 sums are requantized and folded into the output transform while the next position is multiplied, so
-// a lane keeps 16 + 4 running values per output channel and tile (Fold) instead of all 36 positions.
+// keeps no more than 16 + 4 running values per output channel and tile in a lane (Fold) instead of all 36 positions,
+// because the positions are finished one after the other: a position's 64 x 64 sums are requantized and folded into the
+// output transform while the next position is multiplied.
+// That still takes all of the 256 registers that a wave has with two on a SIMD: at tile size 6 the forms of 64 tiles (0 and
+// 2) keep 11 to 15 values in scratch memory, stored ahead of the loop over the positions and reloaded in the output phase
+// (2 MB of writes beside 51 MB of output, 256 -> 256 at 56 x 56, N = 64).  A reload waits by the counter that the requests for
+// the next block of tiles are in as well, so it waits for those, too.
 // The operands travel global memory -> LDS without registers, five stages ahead, and LDS -> registers one stage ahead; one
-// barrier per stage.  512 -> 512 at 28 x 28, N = 64 (u8 in, s8 out): 129-136 us with the weights resident in two passes, 74
-// us here, of which the L1 stream is 40 us and the vector work of the transforms, which only partly hides behind it, 25;
-// 256 -> 256 at 56 x 56, f32 in and out: 132 -> 114 us.
+// barrier per stage.  512 -> 512 at 28 x 28, N = 64 (u8 in, s8 out): 114-117 us with the weights resident in two passes over
+// half of the columns each (a form that is gone), 69-74 us here, of which the L1 stream is 40 us and the vector work of the
+// transforms, which only partly hides behind it, 25; 256 -> 256 at 56 x 56 90 -> 78 us, f32 in and out 122 -> 100 us.
+// A workgroup walks whole blocks of 64 tiles: where their number does not divide over the workgroups of a channel block, the
+// last round is short (256 -> 256 at 56 x 56, N = 64: 196 blocks over 64 columns of workgroups, four rounds for 3.06).
 // Tried: splitting the channels over the waves 2 x 4 instead of 4 x 2 (twice the reads of per-channel constants: 4 %
 // slower); all positions unrolled (60 to 120 KB of instructions: 0.28 us per KB and block of tiles); the two waves of a SIMD
 // folding in different stages (the running values are copied where the branches meet: 10 % slower); four k-steps per

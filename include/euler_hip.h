@@ -110,7 +110,8 @@ EHIP_API int ehip_conv_destroy(ehip_conv_t *conv);
  * zero points into one scale/shift pair per output channel
  * (src/elx_int8_conv_direct_1x1.cpp:234-355, src/elx_int8_conv_direct.cpp:311-500,
  *  src/elx_int8_conv_direct_depthwise.cpp:200-292, src/elx_conv_wino_trans_weights.cpp:437-553).
- * weights_dev: f32 OIhw16i16o (depthwise: goihw); bias_dev: f32 [OCp] or NULL. */
+ * weights_dev: f32 OIhw16i16o (depthwise: goihw); bias_dev: f32 [OCp] or NULL.
+ * Asynchronous on `hip_stream`; for Winograd layers it returns when the weights are ready. */
 EHIP_API int ehip_conv_prepare(ehip_conv_t *conv, const void *weights_dev, const void *bias_dev,
                                void *hip_stream);
 
