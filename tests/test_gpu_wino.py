@@ -680,25 +680,34 @@ def test_wino_fused_ring(form, tile, out_type, with_sum, with_relu, n, ic, oc, h
     (5, 1, 640, 48, 9, ""), (5, 1, 640, 256, 9, "_lanes_ring<32,32>"), (5, 64, 640, 256, 14, ""), (4, 1, 640, 48, 9, "_lanes_ring<32,32>")])
 def test_wino_fused_choice_of_form(tile, n, ic, oc, hw, kernel, monkeypatch):
     """which form of the fused stage layers of more than 256 input channels take, around the lines of the rule; the chosen one
-    and each ring form leave the same bytes"""
+    and each ring form leave the same bytes, for every output type, with and without the sum, in both layouts"""
     import torch
     E = pkg()
     g = torch.Generator(device="cuda").manual_seed(5 + ic + oc)
     x = torch.randint(0, 256, (n, ic // 16, hw, hw, 16), dtype=torch.uint8, device="cuda", generator=g)
     w = (torch.randn((oc // 16, ic // 16, 3, 3, 16, 16), device="cuda", generator=g) * 0.02).float()
     bias = (torch.randn(oc, device="cuda", generator=g) * 0.01).float()
-    d = E.make_desc(n, ic, oc, hw, hw, 3, 3, 1, algorithm=E.CONV_WINOGRAD, input_type=E.U8, output_type=E.S8,
-                    input_quant=(1.0 / 255.0, 0.0), tile_size=tile, execution_mode=0xa161,
-                    wino_tinput_quant=(22.0 / 255.0, 104.0), output_quant=(4.0 * 0.02 * np.sqrt(9 * ic / 3.0) / 127.0, 0.0))
-    outs = []
-    for form in ("", "0", "1"):
-        if form:
-            monkeypatch.setenv("EHIP_WINO_RING", form)
-        conv = E.Conv(d)
-        conv.prepare(w, bias)
-        assert form or conv.kernel_name.endswith("k_wino_gemm_output" + kernel)
-        outs.append(torch.zeros((n, oc // 16, hw, hw, 16), dtype=torch.int8, device="cuda"))
-        conv.execute(outs[-1], x, None, bias)
-    torch.cuda.synchronize()
-    assert int((outs[0] != 0).sum()) > outs[0].numel() // 8
-    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+    for out_type, with_sum, with_relu, nhwc in ((ol.S8, 0, True, False), (ol.U8, 1, True, True), (ol.S8, 1, False, False), (ol.F32, 0, True, True)):
+        d = E.make_desc(n, ic, oc, hw, hw, 3, 3, 1, algorithm=E.CONV_WINOGRAD, input_type=E.U8, output_type=out_type, with_relu=with_relu,
+                        with_ip_sum=with_sum, input_quant=(1.0 / 255.0, 0.0), tile_size=tile, execution_mode=0xa161,
+                        wino_tinput_quant=(22.0 / 255.0, 104.0), output_quant=(4.0 * 0.02 * np.sqrt(9 * ic / 3.0) / 127.0, 0.0))
+        xi, shape = x, (n, oc // 16, hw, hw, 16)
+        if nhwc:
+            d.input_fmt = d.output_fmt = E.NHWC
+            xi, shape = x.permute(0, 2, 3, 1, 4).contiguous(), (n, hw, hw, oc)
+        old = torch.randint(0, 60, shape, device="cuda", generator=g, dtype=torch.uint8)
+        old = old.float() if out_type == ol.F32 else old.view(torch.int8 if out_type == ol.S8 else torch.uint8)
+        outs = []
+        for form in ("", "0", "1"):
+            if form:
+                monkeypatch.setenv("EHIP_WINO_RING", form)
+            else:
+                monkeypatch.delenv("EHIP_WINO_RING", raising=False)
+            conv = E.Conv(d)
+            conv.prepare(w, bias)
+            assert form or conv.kernel_name.endswith("k_wino_gemm_output" + kernel)
+            outs.append(old.clone())
+            conv.execute(outs[-1], xi, None, bias)
+        torch.cuda.synchronize()
+        assert int((outs[0] != old).sum()) > old.numel() // 8
+        assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2]), (out_type, with_sum, nhwc)
