@@ -32,7 +32,8 @@ __device__ __forceinline__ void pack_channel(const float *o, float b, int k, boo
       r = r + (OUT == EHIP_U8 ? (float)ob : (float)(int)(signed char)ob);
     }
     if (with_relu) {
-      r = __builtin_amdgcn_fmed3f(r, 0.0f, OUT == EHIP_S8 ? 127.0f : 255.0f);
+      // (v_cvt_pk_u8_f32 itself clamps to 0..255 and makes a NaN 0, all that the ReLU asks for of a u8 code; s8 has its own bound)
+      if (OUT == EHIP_S8) r = __builtin_amdgcn_fmed3f(r, 0.0f, 127.0f);
       if (A == 4) r = __builtin_floorf(r);
       pk[e] = __builtin_amdgcn_cvt_pk_u8_f32(r, k, pk[e]);
     } else if (A == 4) {
