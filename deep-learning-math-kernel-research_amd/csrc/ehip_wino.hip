@@ -26,7 +26,7 @@
 #include <mutex>
 
 #include "ehip_internal.hpp"
-#include "ehip_wino_tiles.hpp"
+#include "ehip_wino_input.hpp"
 
 #ifdef EHIP_TRACE
 #define TRACE_POINT(i)                                                                             \
@@ -41,193 +41,12 @@ namespace ehip {
 
 namespace {
 
-// Buffer addressing (a load whose offset lies outside the buffer returns zero and touches no memory).  The
-// builtins exist in the device pass only.
-#if defined(__HIP_DEVICE_COMPILE__)
-typedef __amdgpu_buffer_rsrc_t BufferRsrc;
-__device__ __forceinline__ BufferRsrc make_rsrc(const void *base, unsigned bytes)
-{
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), (short)0, (int)bytes, 0x00020000);
-}
-__device__ __forceinline__ void buffer_load_cell(BufferRsrc r, unsigned off, float4 &v)
-{
-  typedef float v4f __attribute__((ext_vector_type(4)));
-  const v4f x = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 0));
-  v = make_float4(x.x, x.y, x.z, x.w);
-}
-__device__ __forceinline__ void buffer_load_cell(BufferRsrc r, unsigned off, unsigned &v)
-{
-  v = __builtin_amdgcn_raw_buffer_load_b32(r, (int)off, 0, 0);
-}
-__device__ __forceinline__ void buffer_load_cell(BufferRsrc r, unsigned off, uint4 &v)
-{
-  typedef unsigned v4u __attribute__((ext_vector_type(4)));
-  const v4u x = __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 0));
-  v = make_uint4(x.x, x.y, x.z, x.w);
-}
-// 4 x 4 transpose of dwords between four registers and the four lanes of a quad (lanes 4 n .. 4 n + 3): register j of
-// lane q becomes register q of lane j.  Two exchanges, with the neighbour (lane ^ 1) and across (lane ^ 2); in each a lane
-// sends the register its partner lacks and takes the partner's in its place.
-__device__ __forceinline__ void quad_transpose(unsigned &x0, unsigned &x1, unsigned &x2, unsigned &x3, int lane)
-{
-  const bool odd = (lane & 1) != 0, hi = (lane & 2) != 0;
-  {
-    const unsigned r01 = __builtin_amdgcn_mov_dpp(odd ? x0 : x1, 0xB1, 0xf, 0xf, true);   // quad_perm [1, 0, 3, 2]
-    const unsigned r23 = __builtin_amdgcn_mov_dpp(odd ? x2 : x3, 0xB1, 0xf, 0xf, true);
-    if (odd) { x0 = r01; x2 = r23; } else { x1 = r01; x3 = r23; }
-  }
-  {
-    const unsigned r02 = __builtin_amdgcn_mov_dpp(hi ? x0 : x2, 0x4E, 0xf, 0xf, true);    // quad_perm [2, 3, 0, 1]
-    const unsigned r13 = __builtin_amdgcn_mov_dpp(hi ? x1 : x3, 0x4E, 0xf, 0xf, true);
-    if (hi) { x0 = r02; x1 = r13; } else { x2 = r02; x3 = r13; }
-  }
-}
-#else
-typedef int BufferRsrc;
-__device__ inline BufferRsrc make_rsrc(const void *, unsigned) { return 0; }
-__device__ inline void buffer_load_cell(BufferRsrc, unsigned, float4 &v) { v = float4(); }
-__device__ inline void buffer_load_cell(BufferRsrc, unsigned, unsigned &v) { v = 0u; }
-__device__ inline void buffer_load_cell(BufferRsrc, unsigned, uint4 &v) { v = uint4(); }
-__device__ inline void quad_transpose(unsigned &, unsigned &, unsigned &, unsigned &, int) {}
-#endif
-
-__device__ __forceinline__ float comp_of(const float4 &v, int k)
-{
-  return k == 0 ? v.x : (k == 1 ? v.y : (k == 2 ? v.z : v.w));
-}
-
-// four u8 codes in a dword: the reference turns the codes into floats as they are
-// (src/kernel/elk_conv_wino_4x4_3x3_input.hxx:40-47)
-__device__ __forceinline__ float comp_of(const unsigned &v, int k)
-{
-  return (float)((v >> (8 * k)) & 0xffu);
-}
-
 // order-preserving map float -> unsigned, for atomicMin/atomicMax
 __device__ __forceinline__ unsigned f2ord(float f)
 {
   unsigned u = __float_as_uint(f);
   return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
-
-struct TileCoord {
-  int n, th, tw, h0, w0;
-  bool border;
-};
-template <int A>
-__device__ __forceinline__ TileCoord tile_coord(const WinoArgs &a, int t)
-{
-  TileCoord c;
-  c.n = t / a.nt;
-  const int rem = t - c.n * a.nt;
-  c.th = rem / a.wt;
-  c.tw = rem - c.th * a.wt;
-  c.h0 = (A - 2) * c.th - a.pad_t;
-  c.w0 = (A - 2) * c.tw - a.pad_l;
-  c.border = c.h0 < 0 || c.w0 < 0 || c.h0 + A - 1 >= a.ih || c.w0 + A - 1 >= a.iw;
-  return c;
-}
-
-// the lane's four channels of the A x A pixels of a tile: float4 (f32 input) or 4 packed codes (u8)
-template <int A>
-__device__ __forceinline__ void gather_tile(const WinoArgs &a, const TileCoord &c, int c2, int q, float4 *d)
-{
-  // blocked: the 16-channel plane of (n, c2), 4 quads per pixel; nhwc: quad c2 * 4 + q of every pixel's vector
-  const size_t pq = a.in_nhwc ? (size_t)a.ic2 * 4 : 4;   // quads between neighbouring pixels
-  const float4 *plane = reinterpret_cast<const float4 *>(a.in) +
-      (a.in_nhwc ? (size_t)c.n * a.ih * a.iw * pq + c2 * 4 : ((size_t)c.n * a.ic2 + c2) * a.ih * a.iw * 4) + q;
-#pragma unroll
-  for (int i = 0; i < A; ++i)
-#pragma unroll
-    for (int j = 0; j < A; ++j) {
-      const int h = c.h0 + i, w = c.w0 + j;
-      d[A * i + j] = (h >= 0 && h < a.ih && w >= 0 && w < a.iw) ? plane[((size_t)h * a.iw + w) * pq]
-                                                                   : make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-}
-template <int A>
-__device__ __forceinline__ void gather_tile(const WinoArgs &a, const TileCoord &c, int c2, int q, unsigned *d)
-{
-  const size_t pq = a.in_nhwc ? (size_t)a.ic2 * 4 : 4;
-  const unsigned *plane = reinterpret_cast<const unsigned *>(a.in) +
-      (a.in_nhwc ? (size_t)c.n * a.ih * a.iw * pq + c2 * 4 : ((size_t)c.n * a.ic2 + c2) * a.ih * a.iw * 4) + q;
-#pragma unroll
-  for (int i = 0; i < A; ++i)
-#pragma unroll
-    for (int j = 0; j < A; ++j) {
-      const int h = c.h0 + i, w = c.w0 + j;
-      d[A * i + j] = (h >= 0 && h < a.ih && w >= 0 && w < a.iw) ? plane[((size_t)h * a.iw + w) * pq] : 0u;   // the frame is 0.0f
-    }
-}
-
-// The same gather through buffer addressing, for tensors below 4 GB (WinoArgs::buf_gather).  A cell's byte
-// offset is the lane's first cell's (32 bits, possibly "negative" for a tile that starts in the frame) plus
-// a scalar; rows and columns are tested once each, a cell's test is the AND of two lane masks (scalar
-// instructions), and a cell of the frame is sent to an offset outside the buffer, where the load returns
-// the frame's zero.  Two vector instructions per cell instead of a bounds test, a 64-bit multiply-add and
-// a branch.
-template <int A, typename Cell>
-__device__ __forceinline__ void gather_tile_buf(const WinoArgs &a, const TileCoord &c, int c2, int q, Cell *d)
-{
-  const unsigned pq = a.in_nhwc ? (unsigned)a.ic2 * 4u : 4u;   // cells between neighbouring pixels
-  const unsigned cells = (unsigned)a.n * a.ic2 * a.ih * a.iw * 4u;
-  const BufferRsrc rin = make_rsrc(a.in, cells * (unsigned)sizeof(Cell));
-  const unsigned plane = a.in_nhwc ? (unsigned)c.n * a.ih * a.iw * pq + c2 * 4u
-                                   : ((unsigned)c.n * a.ic2 + c2) * a.ih * a.iw * 4u;
-  const unsigned voff = (plane + (unsigned)(c.h0 * a.iw + c.w0) * pq + q) * (unsigned)sizeof(Cell);
-  bool rv[A], cv[A];
-#pragma unroll
-  for (int i = 0; i < A; ++i) {
-    rv[i] = (unsigned)(c.h0 + i) < (unsigned)a.ih;
-    cv[i] = (unsigned)(c.w0 + i) < (unsigned)a.iw;
-  }
-#pragma unroll
-  for (int i = 0; i < A; ++i)
-#pragma unroll
-    for (int j = 0; j < A; ++j) {
-      const unsigned so = (unsigned)(i * a.iw + j) * pq * (unsigned)sizeof(Cell);   // scalar
-      buffer_load_cell(rin, (rv[i] && cv[j]) ? voff + so : 0xffffff00u, d[A * i + j]);
-    }
-}
-
-// u8 input below 4 GB, by whole cells: the four lanes of a tile (one channel quad each) share the tile's pixels out
-// between them -- lane q loads the 16 bytes (all four quads) of pixels q, 4 + q, 8 + q, ... -- and a transpose inside
-// the quad hands every lane its own quad of four pixels at a time.  A wave's load then covers 16 tiles x four
-// neighbouring pixels = up to 1 KB in lane order, a quarter of the load instructions and of the cache lines looked up
-// per byte (one dword per lane and pixel looks up a 64-byte line for 16 bytes).  Cells of the zero frame are sent
-// to an offset outside the buffer, as in gather_tile_buf.
-template <int A>
-__device__ __forceinline__ void gather_tile_wide(const WinoArgs &a, const TileCoord &c, int c2, int q, unsigned *d)
-{
-  constexpr int AA = A * A;
-  const unsigned pc = a.in_nhwc ? (unsigned)a.ic2 : 1u;   // cells between neighbouring pixels
-  const unsigned cells = (unsigned)a.n * a.ic2 * a.ih * a.iw;
-  const BufferRsrc rin = make_rsrc(a.in, cells * 16u);
-  const unsigned plane = a.in_nhwc ? (unsigned)c.n * a.ih * a.iw * pc + c2 : ((unsigned)c.n * a.ic2 + c2) * a.ih * a.iw;
-  constexpr int NK = (AA + 3) / 4;
-  uint4 v[NK];
-  // every load first (offsets without a branch), then the exchanges
-#pragma unroll
-  for (int k = 0; k < NK; ++k) {
-    const int e = 4 * k + q;       // the lane's pixel of this group
-    const int i = e / A, j = e - A * i;
-    const int h = c.h0 + i, w = c.w0 + j;
-    const bool ok = e < AA && (unsigned)h < (unsigned)a.ih && (unsigned)w < (unsigned)a.iw;
-    const unsigned off = (plane + (unsigned)(h * a.iw + w) * pc) * 16u;
-    buffer_load_cell(rin, ok ? off : 0xffffff00u, v[k]);
-  }
-  __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int k = 0; k < NK; ++k) {
-    quad_transpose(v[k].x, v[k].y, v[k].z, v[k].w, q);
-    d[4 * k] = v[k].x;
-    if (4 * k + 1 < AA) d[4 * k + 1 < AA ? 4 * k + 1 : 0] = v[k].y;
-    if (4 * k + 2 < AA) d[4 * k + 2 < AA ? 4 * k + 2 : 0] = v[k].z;
-    if (4 * k + 3 < AA) d[4 * k + 3 < AA ? 4 * k + 3 : 0] = v[k].w;
-  }
-}
-template <int A>
-__device__ __forceinline__ void gather_tile_wide(const WinoArgs &, const TileCoord &, int, int, float4 *) {}   // (u8 input only)
 
 }  // namespace
 
@@ -245,7 +64,6 @@ __global__ __launch_bounds__(kBlock) void k_wino_trans_input_u8(const WinoArgs *
   WinoArgs a = load_args(rest);
   a.in = in;
   constexpr int AA = A * A;
-  constexpr bool kCodes = sizeof(Cell) == sizeof(unsigned);
   const int q = threadIdx.x & 3;
   const int item = (blockIdx.x & 7) * a.items_per_xcd + (blockIdx.x >> 3);
   if (item >= a.nblocks * a.ic2) return;   // whole workgroup
@@ -256,78 +74,10 @@ __global__ __launch_bounds__(kBlock) void k_wino_trans_input_u8(const WinoArgs *
   if (t >= a.t) return;
   const TileCoord c = tile_coord<A>(a, t);
   Cell d[AA];
-  if (kCodes && a.buf_gather == 2) gather_tile_wide<A>(a, c, c2, q, d);
-  else if (a.buf_gather) gather_tile_buf<A>(a, c, c2, q, d);
+  if (a.buf_gather) gather_tile_buf<A>(a, c, c2, q, d);
   else gather_tile<A>(a, c, c2, q, d);
   unsigned packed[AA];
-  // mixed: the wave holds interior and rim tiles -- the per-lane, branch-free form of the transform.
-  // Quantization: sat_u8(rne_to_u32(V * (in_S / tin_S) + tin_z)), one rounding in the multiply-add.  The
-  // reference's float -> u32 conversion turns everything below -0.5 (and NaN) into 0xffffffff, which then
-  // saturates to 255; v_cvt_pk_u8_f32 rounds to nearest even and saturates the rest.  watch: the plain
-  // conversion, with the quirk's cases only looked for -- two running integer maxima over the values' bit
-  // patterns, one instruction per value instead of a compare and a select -- and the result says whether
-  // one was seen (never, with a calibrated tinput_quant); the caller then runs the exact form again.
-  // u8 user input: the codes are finite, so with finite quantization constants no NaN can arise and ONE running
-  // float minimum (an instruction per two values) says whether anything fell below -0.5; constants that are not
-  // finite send every wave to the exact form.
-  const bool odd_consts = !(__builtin_fabsf(a.mrepS) <= 3.402823466e38f) || !(__builtin_fabsf(a.mz) <= 3.402823466e38f);
-  auto channels = [&](bool mixed, bool watch) {
-    unsigned seen_u = 0u;
-    int seen_s = 0;
-    float seen_min = 0.0f;
-#pragma unroll
-    for (int k = 0; k < AA; ++k) packed[k] = 0u;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      float f[AA], v[AA];
-#pragma unroll
-      for (int e = 0; e < AA; ++e) f[e] = comp_of(d[e], k);
-      if (kCodes || mixed) wino::tile_input_lanes<A, kCodes>(f, v, c.border);
-      else wino::tile_input<A>(f, v, false);
-      if (watch) {
-        float y[AA];
-#pragma unroll
-        for (int e = 0; e < AA; ++e) {
-          y[e] = __builtin_fmaf(v[e], a.mrepS, a.mz);
-          packed[e] = __builtin_amdgcn_cvt_pk_u8_f32(y[e], k, packed[e]);
-        }
-        // bit patterns above 0xbf000000 unsigned: below -0.5, or a negative NaN; above 0x7f800000 signed: a
-        // positive NaN
-        if (kCodes) {
-#pragma unroll
-          for (int e = 0; e + 1 < AA; e += 2) seen_min = __builtin_fminf(seen_min, __builtin_fminf(y[e], y[e + 1]));
-          if (AA & 1) seen_min = __builtin_fminf(seen_min, y[AA - 1]);
-        } else {
-#pragma unroll
-          for (int e = 0; e + 1 < AA; e += 2) {
-            const unsigned b0 = __float_as_uint(y[e]), b1 = __float_as_uint(y[e + 1]);
-            seen_u = max(seen_u, max(b0, b1));
-            seen_s = max(seen_s, max((int)b0, (int)b1));
-          }
-          if (AA & 1) {
-            const unsigned b = __float_as_uint(y[AA - 1]);
-            seen_u = max(seen_u, b);
-            seen_s = max(seen_s, (int)b);
-          }
-        }
-      } else {
-#pragma unroll
-        for (int e = 0; e < AA; ++e) {
-          const float y = __builtin_fmaf(v[e], a.mrepS, a.mz);
-          packed[e] = __builtin_amdgcn_cvt_pk_u8_f32(y >= -0.5f ? y : 300.0f, k, packed[e]);
-        }
-      }
-    }
-    return kCodes ? (seen_min < -0.5f || odd_consts) : (seen_u > 0xbf000000u || seen_s > 0x7f800000);
-  };
-  const bool mixed = !kCodes && __ballot(c.border) != 0;   // wave-uniform
-  bool again;
-  if (mixed) again = channels(true, true);
-  else again = channels(false, true);
-  if (__ballot(again) != 0) {
-    if (mixed) channels(true, false);
-    else channels(false, false);
-  }
+  quantize_tile<Cell, A>(d, c.border, a.mrepS, a.mz, packed);
   // A position's store = a wave-uniform base + position x stride + one 32-bit offset per lane that never changes
   // (47.3 against 48.7 us on 256 channels at 56 x 56 with the index worked out per lane in 64 bits; forcing the scalar
   // base into every store with assembly: no further gain).  Blocked layout: a wave's sixteen tiles lie in one block of 32.
@@ -341,6 +91,86 @@ __global__ __launch_bounds__(kBlock) void k_wino_trans_input_u8(const WinoArgs *
 #pragma unroll
   for (int e = 0; e < AA; ++e)
     *reinterpret_cast<unsigned *>(const_cast<uint8_t *>(base) + e * pos_stride + voff) = packed[e] ^ flip;
+}
+
+// The same for u8 codes below 4 GB into the blocked layout, through LDS: the pixels of a tile change hands there (gather_tile_lds),
+// and the finished codes take the place of the pixels, position by position, so that they leave by 16 bytes a lane.
+// What bounds it is the issue of vector instructions: 1250 per wave and 16 tiles x 16 channels, of which conversions, minima
+// and byte packs issue at 4.35 clocks and multiply-adds, with two or more waves on a SIMD, at 2.6.  So the instructions that
+// are not the transform's own went (exchanges, address arithmetic, two of three stores), and the registers (91, from 163)
+// let five waves share a SIMD instead of three.
+// By execute_stages, N = 64, before -> now: 256 channels at 56 x 56 36.0 -> 30.5 us, 512 at 28 x 28 21.6 -> 19.3, 64 at 56 x 56
+// 15.7 -> 13.4, 128 at 28 x 28 8.8 -> 8.1.
+template <int A>
+__global__ __launch_bounds__(kBlock, 4) void k_wino_trans_input_codes(const WinoArgs *rest, const void *in)
+{
+  WinoArgs a = load_args(rest);
+  a.in = in;
+  constexpr int AA = A * A;
+  __shared__ uint4 lds[4][AA * 16];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int q = lane & 3, tl = lane >> 2;
+  const int item = (blockIdx.x & 7) * a.items_per_xcd + (blockIdx.x >> 3);
+  if (item >= a.nblocks * a.ic2) return;   // whole workgroup
+  const int c2 = item % a.ic2;
+  const int t0 = item / a.ic2 * 64 + wave * 16;
+  if (t0 >= a.t) return;                   // whole wave
+  // (a lane without a tile takes part with the last one: what it leaves lies in the last block's padding)
+  const TileCoord c = tile_coord<A>(a, t0 + tl < a.t ? t0 + tl : a.t - 1);
+  uint4 *cells = lds[wave];
+  unsigned packed[AA];
+  gather_tile_lds<A>(a, c, c2, q, tl, cells);
+  unsigned *quads = reinterpret_cast<unsigned *>(cells + tl) + q;
+  quantize_tile_lds<A>(quads, c.border, a.mrepS, a.mz, packed);
+#pragma unroll
+  for (int e = 0; e < AA; ++e) quads[64 * e] = packed[e] ^ 0x80808080u;   // (signed bytes, see k_wino_trans_input_u8)
+  __builtin_amdgcn_wave_barrier();
+  uint8_t *base = a.tin + ((size_t)(t0 >> 5) * AA * a.ic2 + c2) * 512 + (t0 & 16) * 16;
+  const unsigned pos = (unsigned)a.ic2 * 512u;
+  const unsigned voff = (unsigned)(lane >> 4) * pos + (unsigned)(lane & 15) * 16u;
+#pragma unroll
+  for (int k = 0; k < (AA + 3) / 4; ++k)
+    if (4 * k + 3 < AA || 4 * k + (lane >> 4) < AA)
+      *reinterpret_cast<uint4 *>(base + (size_t)(4 * k) * pos + voff) = cells[64 * k + lane];
+}
+
+// The same for layers that give a SIMD less than two waves of it: a workgroup takes 16 tiles of one unit, and each of its four waves
+// one channel of every quad, so that four times as many waves run a quarter of the instructions each, and the chain from the first load to the last store
+// is as much shorter.  With other tensors on every call, this against the form above: 512 channels at 7 x 7, N = 64 4.8 against 7.3 us, 256 at
+// 14 x 14 6.9 against 8.2 (N = 16 4.0 against 6.3), 128 at 28 x 28 9.0 against 9.8; N = 1 4.0 against 5.1 to 5.9.
+template <int A>
+__global__ __launch_bounds__(kBlock) void k_wino_trans_input_codes_short(const WinoArgs *rest, const void *in)
+{
+  WinoArgs a = load_args(rest);
+  a.in = in;
+  constexpr int AA = A * A;
+  __shared__ uint4 cells[AA * 16];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int q = lane & 3, tl = lane >> 2;
+  const int item = (blockIdx.x & 7) * a.items_per_xcd + (blockIdx.x >> 3);
+  if (item >= a.nblocks * a.ic2) return;   // whole workgroup
+  const int c2 = item % a.ic2;
+  const int t0 = item / a.ic2 * 16;
+  const TileCoord c = tile_coord<A>(a, t0 + tl < a.t ? t0 + tl : a.t - 1);
+  gather_tile_lds<A, 16, 4>(a, c, c2, q, tl, cells, wave);
+  __syncthreads();                         // the pixels are in LDS
+  unsigned *quads = reinterpret_cast<unsigned *>(cells + tl) + q;
+  unsigned codes[AA];
+  quantize_tile_lds<A, 16, 1>(quads, c.border, a.mrepS, a.mz, codes, wave);
+  __syncthreads();                         // and read
+  uint8_t *bytes = reinterpret_cast<uint8_t *>(quads) + wave;
+#pragma unroll
+  for (int e = 0; e < AA; ++e) bytes[256 * e] = (uint8_t)(codes[e] ^ 0x80u);
+  __syncthreads();
+  uint8_t *base = a.tin + ((size_t)(t0 >> 5) * AA * a.ic2 + c2) * 512 + (t0 & 16) * 16;
+  const unsigned pos = (unsigned)a.ic2 * 512u;
+  const unsigned voff = (unsigned)(4 * wave + (lane >> 4)) * pos + (unsigned)(lane & 15) * 16u;
+#pragma unroll
+  for (int k = 0; k < (AA + 15) / 16; ++k)
+    if (16 * (k + 1) <= AA || 16 * k + 4 * wave + (lane >> 4) < AA)
+      *reinterpret_cast<uint4 *>(base + (size_t)(16 * k) * pos + voff) = cells[256 * k + threadIdx.x];
 }
 
 // partials[2 * c2] = ordered-min, [2 * c2 + 1] = ordered-max (see f2ord) of 16-channel unit c2; real
@@ -810,15 +640,26 @@ hipError_t plan_wino_trans_input(LaunchPlan &plan, const WinoArgs &a0)
     const char *env = getenv("EHIP_WINO_BUF_GATHER");
     a.buf_gather = bytes <= 0xffffff00ull && !(env && env[0] == '0');
     const char *wide = getenv("EHIP_WINO_WIDE_GATHER");
-    if (a.buf_gather && a.in_u8 && !(wide && wide[0] == '0')) a.buf_gather = 2;   // whole cells and a transpose inside the quad
+    if (a.buf_gather && a.in_u8 && a.tin_blocked && !(wide && wide[0] == '0')) a.buf_gather = 2;   // k_wino_trans_input_codes
   }
-  a.nblocks = (a.t + 63) / 64;
+  const bool codes = a.buf_gather == 2;
+  const char *short_env = getenv("EHIP_WINO_SHORT");
+  // the short form up to three waves of the other on a SIMD (64 channels at 56 x 56, N = 64: 13.3 against 14.0 us; 256 at 28 x 28 with tile
+  // size 5, 6400 waves: 20.7 against 19.0); at tile size 4, whose waves are short anyway, up to one and a half (784 waves 3.9 against
+  // 4.0, and 11.4 against 12.1 with the stage behind it; 2048 waves 5.7 against 5.4)
+  const bool shorter = codes && (short_env ? short_env[0] != '0' : (long long)((a.t + 15) / 16) * a.ic2 < (a.tile == 4 ? 1536 : 3328));
+  const int tiles = shorter ? 16 : 64;   // of a workgroup
+  a.nblocks = (a.t + tiles - 1) / tiles;
   a.items_per_xcd = (int)(((long long)a.nblocks * a.ic2 + 7) / 8);
   dim3 grid(8 * a.items_per_xcd, 1);
   void (*kern)(const WinoArgs *, const void *) = nullptr;
-  if (a.tile == 4) kern = a.in_u8 ? k_wino_trans_input_u8<unsigned, 4> : k_wino_trans_input_u8<float4, 4>;
-  else if (a.tile == 5) kern = a.in_u8 ? k_wino_trans_input_u8<unsigned, 5> : k_wino_trans_input_u8<float4, 5>;
-  else kern = a.in_u8 ? k_wino_trans_input_u8<unsigned, 6> : k_wino_trans_input_u8<float4, 6>;
+#define EHIP_WI(A)                                                                                          \
+  kern = shorter ? k_wino_trans_input_codes_short<A>                                                        \
+      : codes ? k_wino_trans_input_codes<A> : a.in_u8 ? k_wino_trans_input_u8<unsigned, A> : k_wino_trans_input_u8<float4, A>
+  if (a.tile == 4) EHIP_WI(4);
+  else if (a.tile == 5) EHIP_WI(5);
+  else EHIP_WI(6);
+#undef EHIP_WI
   return plan_set(plan, kern, grid, dim3(kBlock), 0, a, ArgBlock{}, ArgIn{a.in});
 }
 

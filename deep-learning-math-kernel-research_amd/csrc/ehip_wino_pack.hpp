@@ -4,14 +4,13 @@
 #ifndef EHIP_WINO_PACK_HPP
 #define EHIP_WINO_PACK_HPP
 #include "ehip_internal.hpp"
+#include "ehip_wino_input.hpp"
 #include "ehip_wino_tiles.hpp"
 #include <type_traits>
 
 namespace ehip {
 
 namespace {
-
-__device__ __forceinline__ float comp_of(const float4 &v, int k) { return k == 0 ? v.x : (k == 1 ? v.y : (k == 2 ? v.z : v.w)); }
 
 // The pieces of output_tile (ehip_wino.hip) for u8 / s8 output with few registers: one channel at a time, its bytes
 // packed into the pixels' dwords as they come (16 dwords live instead of 4 x 16 floats; the old output of the in-place

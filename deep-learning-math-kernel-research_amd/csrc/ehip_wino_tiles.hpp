@@ -249,6 +249,22 @@ __device__ __forceinline__ void tile_input_lanes(const float *d, float *v, bool 
   }
 }
 
+// One column and one row of tile_input_lanes<A, true> (A = 6, 5)
+template <int A>
+__device__ __forceinline__ void codes_column(const float *f, float *o)
+{
+  if constexpr (A == 6) in6_1d(f, o, false, false);
+  else in5_1d(f, o, true);
+}
+template <int A>
+__device__ __forceinline__ void codes_row(int i, const float *m, float *v, bool border)
+{
+  if constexpr (A == 6) {
+    if (i == 5) in6_1d_lanes(m, v, false, border);
+    else in6_1d(m, v, false, false);
+  } else in5_1d(m, v, true);
+}
+
 // g: [3][3] (kh, kw)
 template <int A>
 __device__ __forceinline__ void tile_weights(const float g[9], float *u);

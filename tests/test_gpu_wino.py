@@ -711,3 +711,50 @@ def test_wino_fused_choice_of_form(tile, n, ic, oc, hw, kernel, monkeypatch):
         torch.cuda.synchronize()
         assert int((outs[0] != old).sum()) > old.numel() // 8
         assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2]), (out_type, with_sum, nhwc)
+
+
+# ---- the input transform of u8 codes ----------------------------------
+def _u8_layer(n, ic, oc, h, w, tile, out_type, with_sum=0, with_relu=True, in_nhwc=False, out_nhwc=False, tin=(22.0 / 255.0, 104.0), seed=0):
+    """(handle's descriptor, device operands, the oracle's transformed input and output, the output's buffer)"""
+    E = pkg()
+    rng = np.random.default_rng(seed)
+    xq = ol.to_blocked(rng.integers(0, 256, (n, ic, h, w)).astype(np.uint8))
+    wb = ol.weights_to_blocked(rng.normal(0, 0.02, (oc, ic, 3, 3)).astype(f32))
+    bias = np.zeros(ol.up16(oc), f32)
+    bias[:oc] = rng.normal(0, 0.01, oc)
+    quant = (4.0 * 0.02 * np.sqrt(9 * ic / 3.0) / (127.0 if out_type == ol.S8 else 255.0), 1.6 if out_type == ol.U8 else 0.0)
+    p = ol.make_params(n, ic, oc, h, w, 3, 3, 1, out_type=out_type, in_scale=1.0 / 255.0, with_bias=True, with_relu=with_relu,
+                       out_scale=quant[0], out_z=quant[1], wino_tile=tile)
+    d = E.make_desc(n, ic, oc, h, w, 3, 3, 1, algorithm=E.CONV_WINOGRAD, input_type=E.U8, output_type=out_type, with_relu=with_relu,
+                    input_quant=(1.0 / 255.0, 0.0), tile_size=tile, execution_mode=0xa161, output_quant=quant)
+    p.with_sum = d.with_ip_sum = with_sum
+    p.tin_scale, p.tin_z = d.tinput_scale, d.tinput_z = tin
+    old = rng.integers(-30 if out_type == ol.S8 else 0, 60, (n, ol.up16(oc) // 16, h, w, 16)).astype(ol.NP_OF[out_type])
+    twq, tscale, tshift = ol.wino_prepare(p, wb)
+    tinput = ol.wino_trans_input(p, xq.astype(f32))
+    tout, _ = ol.wino_gemm(p, tinput, twq, tscale, tshift)
+    exp = ol.wino_trans_output(p, tout, bias, out_init=old if with_sum else None)
+    if in_nhwc:
+        d.input_fmt, xq = E.NHWC, ol.blocked_to_nhwc(xq, ic)
+    if out_nhwc:
+        d.output_fmt, exp, old = E.NHWC, ol.blocked_to_nhwc(exp, oc), ol.blocked_to_nhwc(old, oc)
+    return E, d, (dev(xq), dev(wb), dev(bias)), tinput, exp, dev(old)
+
+
+@pytest.mark.parametrize("short", ["0", "1"])
+@pytest.mark.parametrize("tile", [6, 5, 4])
+@pytest.mark.parametrize("tin", [(22.0 / 255.0, 104.0), (22.0 / 255.0, 4.0), (float("inf"), 104.0), (1e-39, 104.0)])
+@pytest.mark.parametrize("n,ic,hw,nhwc", [(1, 20, 5, False), (3, 32, 11, True), (2, 144, 14, False)])
+def test_wino_transformed_codes(n, ic, hw, nhwc, tin, tile, short, monkeypatch):
+    """The transformed input of u8 codes through LDS: calibrated constants; a zero point too small for the data, where the wave
+    converts once more in the form that sends values below -0.5 to 255; and scales that make the constants zero and infinite; in every kernel that transforms codes"""
+    import torch
+    monkeypatch.setenv("EHIP_WINO_SHORT", short)
+    E, d, (x, wb, b), tinput, exp, old = _u8_layer(n, ic, 24, hw, hw, tile, ol.S8, in_nhwc=nhwc, tin=tin, seed=3 + ic + hw)
+    if tin[1] == 4.0:
+        assert (tinput == 255).sum() > tinput.size // 50
+    conv = E.Conv(d)
+    conv.prepare(wb, b)
+    conv.execute(old, x, None, b)
+    torch.cuda.synchronize()
+    assert np.array_equal(conv.query(E.Q_TINPUT_U8).reshape(tinput.shape), tinput)
