@@ -30,6 +30,7 @@ void set_error(const std::string &msg) { g_last_error = msg; }
   } while (0)
 
 constexpr int kMaxPlans = 3;
+constexpr int kStageWhole = 8;   // not one of the stages that a caller can ask for
 
 struct ehip_conv {
   ehip_conv_desc_t d;
@@ -65,9 +66,11 @@ struct ehip_conv {
   float *tout = nullptr;
   size_t tin_bytes = 0, tout_bytes = 0;
 
-  // what an execute launches, in order, and the stage bit (ehip_conv_execute_stages) each launch belongs to
+  // what an execute launches, in order, and the stage bits (ehip_conv_execute_stages) each launch belongs to.  A Winograd
+  // layer that runs whole in one kernel has that launch behind those of its stages, under a bit of its own
   LaunchPlan plan[kMaxPlans];
   int plan_stage[kMaxPlans] = {7, 7, 7};
+  int execute_stages = 7;
   int nplans = 0;
   alignas(8) unsigned char args[kMaxPlans][kArgBlock] = {};
   void *args_dev = nullptr;   // [kMaxPlans][kArgBlock], behind wsum
@@ -654,6 +657,11 @@ static int plan_execute(ehip_conv *c)
       f.trace = trace_buffer();
       HIP_TRY(plan_wino_gemm_output(c->plan[1], f));
       c->nplans = 2;
+      if (wino_whole_applies(w, f)) {
+        HIP_TRY(plan_wino_whole(c->plan[2], w, f));
+        c->plan_stage[2] = c->execute_stages = kStageWhole;
+        c->nplans = 3;
+      }
       return EHIP_OK;
     }
     GemmArgs a;
@@ -770,6 +778,7 @@ EHIP_API int ehip_conv_prepare(ehip_conv_t *c, const void *weights_dev, const vo
   // from here on the name is that of the kernel the planner chose
   if (c->family == FAM_WINOGRAD) {
     if (c->fused && c->plan[1].name) c->kernel_name = std::string("k_wino_trans_input_u8 + ") + c->plan[1].name;
+    if (c->execute_stages == kStageWhole) c->kernel_name = std::string(c->plan[2].name) + " | " + c->kernel_name;
   } else if (c->plan[0].name) {
     c->kernel_name = c->plan[0].name;
   }
@@ -785,7 +794,7 @@ EHIP_API int ehip_conv_execute(ehip_conv_t *c, void *output_dev, const void *inp
     int rc = ehip_conv_prepare(c, weights_dev, bias_dev, hip_stream);
     if (rc != EHIP_OK) return rc;
   }
-  return run_plans(c, output_dev, input_dev, bias_dev, 7, static_cast<hipStream_t>(hip_stream));
+  return run_plans(c, output_dev, input_dev, bias_dev, c->execute_stages, static_cast<hipStream_t>(hip_stream));
 }
 
 EHIP_API int ehip_conv_execute_stages(ehip_conv_t *c, void *output_dev, const void *input_dev, const void *bias_dev,

@@ -142,6 +142,15 @@ struct WinoFusedArgs {
   int nkc;              // set by the ring launcher: stages per position
 };
 
+// a Winograd layer whole in one kernel (ehip_wino_whole.hpp)
+struct WinoWholeArgs {
+  WinoArgs w;
+  WinoFusedArgs f;
+  int nx;                  // blocks of 16 tiles
+  int splits, per_split;   // workgroups of a block of tiles, groups of 16 output channels of each
+  unsigned nt_magic, wt_magic;   // div_magic of the tiles per image and per row
+};
+
 // ---- launch plans -------------------------------------------------------------------------------
 // Everything about a launch but the tensors is worked out once, when the handle is created (planned): kernel, grid,
 // LDS size, the derived arguments, the EHIP_* knobs read from the environment.  The argument structure goes to device
@@ -274,6 +283,16 @@ RingForm wino_ring_form6(int form, int nks);   // tile sizes 6, 5, 4; nks = k-st
 RingForm wino_ring_form5(int form, int nks);
 RingForm wino_ring_form4(int form, int nks);
 hipError_t plan_wino_gemm_output_ring(LaunchPlan &plan, const WinoFusedArgs &a, int form);
+// the whole layer in one kernel, up to 256 input channels (ehip_wino_whole.hip)
+struct WholeForm {
+  void (*kernel)(const WinoWholeArgs *, const void *, void *, const float *);
+  int waves, lds;                  // of a workgroup
+};
+WholeForm wino_whole_form6(int nks, int nw, int out_type, bool sum);   // tile sizes 6, 5, 4; nks = k-steps of 64 input channels
+WholeForm wino_whole_form5(int nks, int nw, int out_type, bool sum);
+WholeForm wino_whole_form4(int nks, int nw, int out_type, bool sum);
+bool wino_whole_applies(const WinoArgs &w, const WinoFusedArgs &f);
+hipError_t plan_wino_whole(LaunchPlan &plan, const WinoArgs &w, const WinoFusedArgs &f);
 // min / max of the transformed input: partials = 2 * a.ic2 dwords of device scratch, result = two floats
 // of device memory (min, max); three launches on `s`, nothing else
 hipError_t launch_wino_range(const WinoArgs &a, int ic_real, unsigned *partials, float *minmax_out_dev, hipStream_t s);

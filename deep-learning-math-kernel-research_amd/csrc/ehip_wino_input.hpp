@@ -1,5 +1,6 @@
 // The input side of a Winograd layer: a tile's pixels from the user's tensor, V = Bt d B, and the u8 codes of the
-// transformed tile; a lane holds one tile x four channels.
+// transformed tile.  Shared by the stand-alone input transform (ehip_wino.hip) and by the kernel that runs a layer whole
+// (ehip_wino_whole.hpp); a lane holds one tile x four channels.
 #ifndef EHIP_WINO_INPUT_HPP
 #define EHIP_WINO_INPUT_HPP
 #include "ehip_internal.hpp"

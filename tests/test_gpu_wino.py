@@ -713,7 +713,7 @@ def test_wino_fused_choice_of_form(tile, n, ic, oc, hw, kernel, monkeypatch):
         assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2]), (out_type, with_sum, nhwc)
 
 
-# ---- the input transform of u8 codes ----------------------------------
+# ---- the layer whole in one kernel, and the input transform of u8 codes ----------------------------------
 def _u8_layer(n, ic, oc, h, w, tile, out_type, with_sum=0, with_relu=True, in_nhwc=False, out_nhwc=False, tin=(22.0 / 255.0, 104.0), seed=0):
     """(handle's descriptor, device operands, the oracle's transformed input and output, the output's buffer)"""
     E = pkg()
@@ -741,15 +741,49 @@ def _u8_layer(n, ic, oc, h, w, tile, out_type, with_sum=0, with_relu=True, in_nh
     return E, d, (dev(xq), dev(wb), dev(bias)), tinput, exp, dev(old)
 
 
-@pytest.mark.parametrize("short", ["0", "1"])
+@pytest.mark.parametrize("tile", [6, 5, 4])
+@pytest.mark.parametrize("out_type,with_sum,with_relu,in_nhwc,out_nhwc", [
+    (ol.S8, 0, True, False, False), (ol.U8, 0, True, False, True), (ol.U8, 1, False, False, False), (ol.S8, 1, True, True, True),
+    (ol.F32, 0, True, True, False), (ol.S8, 0, False, True, False)])
+@pytest.mark.parametrize("waves,splits,n,ic,oc,h,w", [
+    ("8", "", 1, 16, 16, 4, 4), ("8", "", 2, 64, 80, 13, 11), ("4", "2", 3, 48, 144, 9, 10), ("8", "3", 1, 128, 112, 12, 17),
+    ("4", "1", 3, 80, 208, 7, 9), ("8", "1", 2, 176, 144, 9, 8), ("8", "", 5, 256, 48, 6, 7)])
+def test_wino_whole_layer(waves, splits, n, ic, oc, h, w, out_type, with_sum, with_relu, in_nhwc, out_nhwc, tile, monkeypatch):
+    """Every count of k-steps, with four and eight waves, workgroups that share a block's output channels unevenly, waves with no
+    group, one and several; blocks of tiles that end inside a unit of 32 and across images; every output type, layout and the sum.
+    The handle holds the transformed input afterwards, and its stages still run on their own."""
+    import torch
+    monkeypatch.setenv("EHIP_WINO_WHOLE", "1")
+    monkeypatch.setenv("EHIP_WINO_WHOLE_WAVES", waves)
+    if splits:
+        monkeypatch.setenv("EHIP_WINO_WHOLE_SPLITS", splits)
+    E, d, (x, wb, b), tinput, exp, old = _u8_layer(n, ic, oc, h, w, tile, out_type, with_sum, with_relu, in_nhwc, out_nhwc,
+                                                   seed=17 * n + ic + h + tile)
+    conv = E.Conv(d)
+    conv.prepare(wb, b)
+    assert conv.kernel_name.startswith("k_wino_whole | ")
+    out = old.clone()
+    conv.execute(out, x, None, b)
+    torch.cuda.synchronize()
+    assert np.array_equal(conv.query(E.Q_TINPUT_U8).reshape(tinput.shape), tinput)
+    assert np.array_equal(bits(host(out)), bits(exp)), "output differs at %d of %d" % (int((host(out) != exp).sum()), exp.size)
+    out.copy_(old)
+    conv.execute_stages(out, x, 3, 1, b)
+    torch.cuda.synchronize()
+    assert np.array_equal(bits(host(out)), bits(exp))
+
+
+@pytest.mark.parametrize("whole,short", [("1", ""), ("0", "0"), ("0", "1")])
 @pytest.mark.parametrize("tile", [6, 5, 4])
 @pytest.mark.parametrize("tin", [(22.0 / 255.0, 104.0), (22.0 / 255.0, 4.0), (float("inf"), 104.0), (1e-39, 104.0)])
 @pytest.mark.parametrize("n,ic,hw,nhwc", [(1, 20, 5, False), (3, 32, 11, True), (2, 144, 14, False)])
-def test_wino_transformed_codes(n, ic, hw, nhwc, tin, tile, short, monkeypatch):
+def test_wino_transformed_codes(n, ic, hw, nhwc, tin, tile, whole, short, monkeypatch):
     """The transformed input of u8 codes through LDS: calibrated constants; a zero point too small for the data, where the wave
     converts once more in the form that sends values below -0.5 to 255; and scales that make the constants zero and infinite; in every kernel that transforms codes"""
     import torch
-    monkeypatch.setenv("EHIP_WINO_SHORT", short)
+    monkeypatch.setenv("EHIP_WINO_WHOLE", whole)
+    if short:
+        monkeypatch.setenv("EHIP_WINO_SHORT", short)
     E, d, (x, wb, b), tinput, exp, old = _u8_layer(n, ic, 24, hw, hw, tile, ol.S8, in_nhwc=nhwc, tin=tin, seed=3 + ic + hw)
     if tin[1] == 4.0:
         assert (tinput == 255).sum() > tinput.size // 50
@@ -757,4 +791,33 @@ def test_wino_transformed_codes(n, ic, hw, nhwc, tin, tile, short, monkeypatch):
     conv.prepare(wb, b)
     conv.execute(old, x, None, b)
     torch.cuda.synchronize()
+    assert conv.kernel_name.startswith("k_wino_whole | ") == (whole == "1")
     assert np.array_equal(conv.query(E.Q_TINPUT_U8).reshape(tinput.shape), tinput)
+
+
+@pytest.mark.parametrize("tile,ic,oc,n,hw,whole", [
+    (6, 64, 64, 32, 56, True), (6, 64, 64, 64, 56, False), (6, 64, 64, 2, 28, False), (6, 128, 128, 64, 28, True), (6, 128, 128, 160, 28, False),
+    (6, 192, 192, 20, 28, False), (6, 192, 192, 64, 28, True), (6, 256, 64, 64, 28, True), (6, 256, 256, 64, 14, False), (5, 128, 256, 40, 28, True),
+    (4, 256, 128, 20, 28, True), (4, 64, 48, 1, 7, True)])
+def test_wino_whole_choice(tile, ic, oc, n, hw, whole, monkeypatch):
+    """which layers run whole, around the lines of the rule, and the same bytes from the stages"""
+    import torch
+    E = pkg()
+    g = torch.Generator(device="cuda").manual_seed(5 + ic + oc)
+    x = torch.randint(0, 256, (n, ic // 16, hw, hw, 16), dtype=torch.uint8, device="cuda", generator=g)
+    w = (torch.randn((oc // 16, ic // 16, 3, 3, 16, 16), device="cuda", generator=g) * 0.02).float()
+    bias = (torch.randn(oc, device="cuda", generator=g) * 0.01).float()
+    d = E.make_desc(n, ic, oc, hw, hw, 3, 3, 1, algorithm=E.CONV_WINOGRAD, input_type=E.U8, output_type=E.S8, input_quant=(1.0 / 255.0, 0.0),
+                    tile_size=tile, execution_mode=0xa161, wino_tinput_quant=(22.0 / 255.0, 104.0),
+                    output_quant=(4.0 * 0.02 * np.sqrt(9 * ic / 3.0) / 127.0, 0.0))
+    outs = []
+    for env in ("", "0"):
+        if env:
+            monkeypatch.setenv("EHIP_WINO_WHOLE", env)
+        conv = E.Conv(d)
+        conv.prepare(w, bias)
+        assert conv.kernel_name.startswith("k_wino_whole | ") == (whole and not env)
+        outs.append(torch.zeros((n, oc // 16, hw, hw, 16), dtype=torch.int8, device="cuda"))
+        conv.execute(outs[-1], x, None, bias)
+    torch.cuda.synchronize()
+    assert int((outs[0] != 0).sum()) > outs[0].numel() // 8 and torch.equal(outs[0], outs[1])
