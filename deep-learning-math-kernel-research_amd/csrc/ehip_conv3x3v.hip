@@ -60,6 +60,10 @@ namespace ehip {
 // The staged cells of a unit are stored by residue: cell c at (c % TN) * R + c / TN, which makes the
 // strided read a read of consecutive 16-byte slots; R is chosen so that neighbouring cells written by
 // neighbouring threads land in different banks.
+//
+// KS = 2 ("shared"): eight waves on one CU instead of four.  Both halves own the same channels and pixels; the lower half takes
+// fills 0, 2, ... of the input channels and the upper one 1, 3, ..., each in its own part of the LDS, and the upper half's sums
+// reach the lower one's accumulators through LDS at the end (integers: exact).  See plan_conv3x3v.
 constexpr int conv3x3v_unit_stride(int cells, int tn, bool sp)
 {
   if (!sp || tn == 1) return cells;
@@ -69,9 +73,10 @@ constexpr int conv3x3v_unit_stride(int cells, int tn, bool sp)
   return r * tn;
 }
 
-template <int WM, int WN, int TM, int TN, int CT, int NPASS, int PAIRS, bool SP, bool SL, int S>
+template <int WM, int WN, int TM, int TN, int CT, int NPASS, int PAIRS, bool SP, bool SL, int S, int KS>
 __device__ __forceinline__ void conv3x3v_body(const Conv3x3Args &a)
 {
+  static_assert(KS == 1 || (KS == 2 && PAIRS == 0 && !SP), "channels shared out: loop form");
   static_assert(!SL || (PAIRS > 0 && !SP && TM == 1 && TN == 4), "split last pair: straight-line form, 32 channels x 4 tiles");
   static_assert(S == 1 || (S == 2 && !SP && (CT * NPASS) % 4 == 0), "stride 2: four phase planes per staged unit");
   constexpr int PS = CT * NPASS / 4;   // stride 2: staged cells per phase plane
@@ -85,12 +90,15 @@ __device__ __forceinline__ void conv3x3v_body(const Conv3x3Args &a)
   constexpr int G = kBlock / CT;       // thread groups that split the units of a fill
   static_assert(WM * WN == 4, "four waves per workgroup");
   static_assert(kBlock % CT == 0, "cells per pass");
-  extern __shared__ v4i lds[];         // [chunk_units][STRIDE]
+  extern __shared__ v4i lds_all[];     // [KS][chunk_units][STRIDE]
 #ifdef EHIP_TRACE
   const long long t_entry = wall_clock64();
 #endif
 
-  const int tid = threadIdx.x;
+  // KS = 2: eight waves, of which the upper four do what the lower four do with every other fill
+  const int half = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / kBlock);
+  const int tid = threadIdx.x % kBlock;
+  v4i *lds = lds_all + (KS == 1 ? 0 : half * a.chunk_units * STRIDE);
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform: what depends on it stays scalar
   const int l32 = lane & 31;
@@ -203,13 +211,13 @@ __device__ __forceinline__ void conv3x3v_body(const Conv3x3Args &a)
 #pragma unroll
         for (int j = 0; j < KB; ++j) {
           const int k = k0 + j < nk ? k0 + j : nk - 1;
-          int u = ug + G * k;
+          int u = half * a.chunk_units + ug + G * k;
           u = u < a.ic2 ? u : a.ic2 - 1;   // padded units multiply zero weights
           t[p][j] = *reinterpret_cast<const v4i *>(inb + (long long)u * plane + goff[p]);
         }
       if (k0 == 0) {
 #pragma unroll
-        for (int tap = 0; tap < 9; ++tap) load_a(tap, 0);
+        for (int tap = 0; tap < 9; ++tap) load_a(tap, half * (a.chunk_units / 2));
       }
 #pragma unroll
       for (int p = 0; p < NPASS; ++p)
@@ -252,7 +260,7 @@ __device__ __forceinline__ void conv3x3v_body(const Conv3x3Args &a)
         __builtin_amdgcn_sched_barrier(0);
       }
   };
-  // loop form: the operands of a pair's first tap are read at its start
+  // loop form: the operands of a pair's first tap are read at its start (pair: whose successor's weights are requested)
   auto pair_taps = [&](int pl, int pair, bool last) {
 #pragma unroll
     for (int nt = 0; nt < TN; ++nt) read_b(0, pl, 0, nt);
@@ -322,7 +330,7 @@ __device__ __forceinline__ void conv3x3v_body(const Conv3x3Args &a)
 #pragma unroll
     for (int nt = 0; nt < TN; ++nt)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc[mt][nt][v] = c4[v >> 2][v & 3];
+      for (int v = 0; v < 16; ++v) acc[mt][nt][v] = KS == 1 || half == 0 ? c4[v >> 2][v & 3] : 0;
   }
   // Lean epilogue (a.lean, decided by the launcher): u8 / s8 output, ReLU with bounds 0 <= lo <= hi, no
   // sum -- the case of every direct 3x3 layer of the tuned networks.  Scale and shift of the lane's
@@ -444,6 +452,49 @@ __device__ __forceinline__ void conv3x3v_body(const Conv3x3Args &a)
       for (int st = LAST0; st < 9 * PAIRS; ++st)
         tap_mfmas(st & 1, st % 9, PAIRS - 1, true, st + 1 < 9 * PAIRS ? PAIRS - 1 : -1, (st + 1) % 9);
     }
+  } else if (KS == 2) {
+    // fill 2 i + half in step i; (an odd count of fills: the upper half skips the last step's work, not its barriers)
+    const int steps = (nchunks + 1) / 2;
+    for (int i = 0; i < steps; ++i) {
+      const int chunk = 2 * i + half;
+      const bool mine = chunk < nchunks;
+      if (i) {
+        __syncthreads();
+        if (mine) stage(chunk, false);
+        __syncthreads();
+      }
+      if (mine) {
+        for (int pl = 0; pl < ppc - 1; ++pl) pair_taps(pl, chunk * ppc + pl, false);
+        const bool last = chunk + 2 >= nchunks;
+        if (last && half == 0) load_epilogue_consts();
+        pair_taps(ppc - 1, (chunk + 2) * ppc - 1, last);
+      }
+    }
+    // the upper half's sums through LDS
+    __syncthreads();
+    v4i *sums = lds_all;
+    if (half) {
+#pragma unroll
+      for (int mt = 0; mt < TM; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < TN; ++nt)
+#pragma unroll
+          for (int v = 0; v < 4; ++v)
+            sums[((mt * TN + nt) * 4 + v) * kBlock + tid] =
+                v4i{acc[mt][nt][4 * v], acc[mt][nt][4 * v + 1], acc[mt][nt][4 * v + 2], acc[mt][nt][4 * v + 3]};
+    }
+    __syncthreads();
+    if (half) return;
+#pragma unroll
+    for (int mt = 0; mt < TM; ++mt)
+#pragma unroll
+      for (int nt = 0; nt < TN; ++nt)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const v4i x = sums[((mt * TN + nt) * 4 + v) * kBlock + tid];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) acc[mt][nt][4 * v + j] += x[j];
+        }
   } else
   for (int chunk = 0; chunk < nchunks; ++chunk) {
     if (chunk) {
@@ -511,14 +562,14 @@ __device__ __forceinline__ void conv3x3v_body(const Conv3x3Args &a)
 #define EHIP_CONV3X3V_HEAD                                                                                            \
   const uint8_t *in, const Conv3x3Args *rest, int ih, int iw, int oh, int ow, unsigned pads_cu, int ic2, int vw,        \
       unsigned vw_magic, int gx, int gy, int tiles, int tiles_per_xcd
-template <int WM, int WN, int TM, int TN, int CT, int NPASS, int PAIRS = 0, bool SP = false, bool SL = false, int S = 1>
-__global__ __launch_bounds__(kBlock, 2) void k_conv3x3v_u8s8(EHIP_CONV3X3V_HEAD, void *out)
+template <int WM, int WN, int TM, int TN, int CT, int NPASS, int PAIRS = 0, bool SP = false, bool SL = false, int S = 1, int KS = 1>
+__global__ __launch_bounds__(kBlock * KS, 2) void k_conv3x3v_u8s8(EHIP_CONV3X3V_HEAD, void *out)
 {
   Conv3x3Args a = load_args(rest);
   a.in = in; a.out = out; a.ih = ih; a.iw = iw; a.oh = oh; a.ow = ow; a.pad_t = (int)(pads_cu & 0xffu); a.pad_l = (int)((pads_cu >> 8) & 0xffu);
   a.ic2 = ic2; a.chunk_units = (int)(pads_cu >> 16); a.vw = vw; a.vw_magic = vw_magic; a.gx = gx; a.gy = gy; a.tiles = tiles;
   a.tiles_per_xcd = tiles_per_xcd;
-  conv3x3v_body<WM, WN, TM, TN, CT, NPASS, PAIRS, SP, SL, S>(a);
+  conv3x3v_body<WM, WN, TM, TN, CT, NPASS, PAIRS, SP, SL, S, KS>(a);
 }
 
 namespace {
@@ -531,36 +582,42 @@ struct Variant {
   conv3x3v_kernel_t unrolled[3];   // straight-line K loop for layers of exactly 2, 4, 8 unit pairs, or null
   conv3x3v_kernel_t split[3];      // the same with the last pair split (lean epilogue without the sum), or null
   int stride;                      // 1, or 2: the staged unit is four phase planes of cells / 4 cells each
+  conv3x3v_kernel_t shared;        // eight waves that share the input channels out, or null
 };
 #define V(WM, WN, TM, TN, CT, NPASS)                                                              \
   { "k_conv3x3v_u8s8<" #WM "," #WN "," #TM "," #TN "," #CT "," #NPASS ">", WM * TM * 32, WN * TN * 32, \
-    CT * NPASS, CT * NPASS, k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS>, {nullptr, nullptr, nullptr}, {nullptr, nullptr, nullptr}, 1 }
+    CT * NPASS, CT * NPASS, k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS>, {nullptr, nullptr, nullptr}, {nullptr, nullptr, nullptr}, 1, nullptr }
 #define VU(WM, WN, TM, TN, CT, NPASS)                                                             \
   { "k_conv3x3v_u8s8<" #WM "," #WN "," #TM "," #TN "," #CT "," #NPASS ">", WM * TM * 32, WN * TN * 32, \
     CT * NPASS, CT * NPASS, k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS>,                            \
     {k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 2>, k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 4>,  \
-     k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 8>}, {nullptr, nullptr, nullptr}, 1 }
+     k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 8>}, {nullptr, nullptr, nullptr}, 1, nullptr }
 #define VU2(WM, WN, TM, TN, CT, NPASS) /* straight-line form for two unit pairs only (64 input channels) */ \
   { "k_conv3x3v_u8s8<" #WM "," #WN "," #TM "," #TN "," #CT "," #NPASS ">", WM * TM * 32, WN * TN * 32, \
     CT * NPASS, CT * NPASS, k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS>,                            \
-    {k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 2>, nullptr, nullptr}, {nullptr, nullptr, nullptr}, 1 }
+    {k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 2>, nullptr, nullptr}, {nullptr, nullptr, nullptr}, 1, nullptr }
 #define VK(WM, WN, TM, TN, CT, NPASS)                                                             \
   { "k_conv3x3v_u8s8<" #WM "," #WN "," #TM "," #TN "," #CT "," #NPASS ">", WM * TM * 32, WN * TN * 32, \
     CT * NPASS, CT * NPASS, k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS>,                            \
     {k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 2>, k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 4>,  \
      k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 8>},                                               \
     {k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 2, false, true>, k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 4, false, true>, \
-     k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 8, false, true>}, 1 }
+     k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 8, false, true>}, 1, nullptr }
 #define V2(WM, WN, TM, TN, CT, NPASS) /* stride 2; straight-line forms for two and four unit pairs */ \
   { "k_conv3x3v_u8s8<" #WM "," #WN "," #TM "," #TN "," #CT "," #NPASS ",s2>", WM * TM * 32, WN * TN * 32, \
     CT * NPASS, CT * NPASS, k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 0, false, false, 2>,       \
     {k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 2, false, false, 2>, k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 4, false, false, 2>, \
-     nullptr}, {nullptr, nullptr, nullptr}, 2 }
+     nullptr}, {nullptr, nullptr, nullptr}, 2, nullptr }
+#define V2K(WM, WN, TM, TN, CT, NPASS) /* and the form that shares the input channels out */ \
+  { "k_conv3x3v_u8s8<" #WM "," #WN "," #TM "," #TN "," #CT "," #NPASS ",s2>", WM * TM * 32, WN * TN * 32, \
+    CT * NPASS, CT * NPASS, k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 0, false, false, 2>,       \
+    {k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 2, false, false, 2>, k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 4, false, false, 2>, \
+     nullptr}, {nullptr, nullptr, nullptr}, 2, k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 0, false, false, 2, 2> }
 #define VS(WM, WN, TM, TN, CT, NPASS)                                                             \
   { "k_conv3x3v_u8s8<" #WM "," #WN "," #TM "," #TN "," #CT "," #NPASS ",sp>", WM * TM * 32, WN * TN * 32, \
     CT * NPASS, conv3x3v_unit_stride(CT * NPASS, TN, true), k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 0, true>, \
     {k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 2, true>, k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 4, true>, \
-     k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 8, true>}, {nullptr, nullptr, nullptr}, 1 }
+     k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 8, true>}, {nullptr, nullptr, nullptr}, 1, nullptr }
 const Variant kVariants[] = {
     V(2, 2, 2, 1, 128, 1),  // 0: 128 oc x  64 px, rows up to  31 cells
     V(2, 2, 2, 1, 256, 1),  // 1: 128 oc x  64 px, rows up to  95 cells
@@ -582,9 +639,9 @@ const Variant kVariants[] = {
     VS(2, 2, 2, 2, 256, 1), // 17: as 2, strided pixels
     VS(4, 1, 1, 4, 256, 2), // 18: as 13, strided pixels
     VS(2, 2, 2, 4, 256, 2), // 19: 128 oc x 256 px, rows up to 127 cells, a wave = 64 oc x 128 px, strided pixels
-    V2(4, 1, 1, 2, 128, 3), // 20: stride 2, 128 oc x  64 px, output rows up to 29 pixels, every wave all pixels
+    V2K(4, 1, 1, 2, 128, 3), // 20: stride 2, 128 oc x  64 px, output rows up to 29 pixels, every wave all pixels
     V2(4, 1, 1, 4, 128, 5), // 21: stride 2, 128 oc x 128 px, output rows up to 29 pixels, every wave all pixels
-    V2(4, 1, 1, 2, 256, 2), // 22: stride 2, 128 oc x  64 px, output rows up to 61 pixels
+    V2K(4, 1, 1, 2, 256, 2), // 22: stride 2, 128 oc x  64 px, output rows up to 61 pixels
     V2(1, 4, 2, 1, 128, 5), // 23: stride 2,  64 oc x 128 px, output rows up to 29 pixels
 };
 #undef V
@@ -593,6 +650,7 @@ const Variant kVariants[] = {
 #undef VU2
 #undef VS
 #undef V2
+#undef V2K
 constexpr int kNumVariants = sizeof(kVariants) / sizeof(kVariants[0]);
 constexpr int kLdsBudget = 64 * 1024;
 }  // namespace
@@ -710,8 +768,29 @@ hipError_t plan_conv3x3v(LaunchPlan &plan, const Conv3x3Args &a0, int n, int var
       if (k.split[slot] && (a.lean & 1) && !(a.lean & 4) && want) kernel = k.split[slot];
     }
   }
+  // Stride 2 with more than one fill (over 128 input channels) and a CU for every workgroup: two fills at a time by eight
+  // waves.  A fill is a trip to memory that nothing covers, and the 36 taps behind it run at one wave per SIMD.  With other tensors
+  // on every call, one at a time / two: 512 -> 512 at 14 x 14, N = 1 18.0 / 14.7 us, N = 64 (256 workgroups) 19.0 / 16.9; 256 -> 256 at 28 x 28, N = 1
+  // 10.5 / 9.1, N = 16 (128) 10.3 / 9.0, N = 64 (512 workgroups, two on a CU either way) 18.3 / 20.0.  Stride 1 stages everything in
+  // one fill: 512 -> 512 at 14 x 14, N = 1 10.1 / 9.8, 256 -> 256 6.2 / 7.0, not taken.
+  int threads = kBlock;
+  size_t lds = lds_bytes;
+  const char *shared_env = getenv("EHIP_CONV3X3V_SHARED");   // (0 / 1: never / wherever it can run)
+  if (k.shared && a.units_pad > a.chunk_units && (shared_env ? shared_env[0] != '0' : tiles <= 256)) {
+    int cu = 0;   // units of a fill: as many as two fills have room for
+    for (int c = 2; c <= a.units_pad / 2; c += 2)
+      if (a.units_pad % c == 0 && (size_t)2 * c * k.ustride * 16 <= 150 * 1024) cu = c;
+    if (cu) {
+      a.chunk_units = cu;
+      const size_t sums = (size_t)k.oc_t * k.p_t * sizeof(int);
+      lds = (size_t)2 * cu * k.ustride * 16;
+      lds = lds < sums ? sums : lds;
+      kernel = k.shared;
+      threads = 2 * kBlock;
+    }
+  }
   if (a.pad_t > 255 || a.pad_l > 255 || a.chunk_units >= 65536) return hipErrorInvalidValue;   // pads_cu's fields
-  return plan_set(plan, kernel, grid, dim3(kBlock), lds_bytes, a, ArgIn{a.in}, ArgBlock{}, a.ih, a.iw, a.oh, a.ow,
+  return plan_set(plan, kernel, grid, dim3(threads), lds, a, ArgIn{a.in}, ArgBlock{}, a.ih, a.iw, a.oh, a.ow,
                   (unsigned)a.pad_t | (unsigned)a.pad_l << 8 | (unsigned)a.chunk_units << 16, a.ic2, a.vw, a.vw_magic, a.gx, a.gy,
                   a.tiles, a.tiles_per_xcd, ArgOut{a.out});
 }

@@ -390,6 +390,18 @@ def test_direct_3x3_stride2_phase_planes(variant, n, ic, oc, hw, pad, out_hw, mo
         assert "s2" in res["conv"].kernel_name
 
 
+@pytest.mark.parametrize("variant,n,ic,oc,hw,out_type", [
+    ("", 2, 256, 64, 14, ol.S8), ("20", 1, 144, 144, 9, ol.U8), ("22", 1, 272, 48, 21, ol.F32), ("20", 1, 880, 32, 8, ol.S32), ("22", 3, 512, 136, 14, ol.U8)])
+def test_direct_3x3_stride2_channels_shared_out(variant, n, ic, oc, hw, out_type, monkeypatch):
+    """eight waves that take two fills of input channels at a time: two, four and an odd count of fills, and padded units"""
+    if variant:
+        monkeypatch.setenv("EHIP_CONV3X3V_VARIANT", variant)
+    for shared in ("1", "0"):
+        monkeypatch.setenv("EHIP_CONV3X3V_SHARED", shared)
+        res = run_and_compare(Layer(n, ic, oc, hw, k=3, pad=1, stride=2, out_type=out_type, seed=195 + ic + hw))
+        assert "s2" in res["conv"].kernel_name
+
+
 def test_direct_3x3_stride2_phase_planes_can_be_switched_off(monkeypatch):
     monkeypatch.setenv("EHIP_CONV3X3V_S2", "0")
     res = run_and_compare(Layer(2, 64, 48, 14, k=3, pad=1, stride=2, out_type=ol.S8, seed=97))
