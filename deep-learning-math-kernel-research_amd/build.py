@@ -25,7 +25,7 @@ SOURCES = [
     "ehip_wino.hip",
     "ehip_wino_lanes.hip",
     "ehip_wino_ring.hip", "ehip_wino_ring6.hip", "ehip_wino_ring5.hip", "ehip_wino_ring4.hip",
-    "ehip_wino_split.hip",
+    "ehip_wino_cols.hip",
     "ehip_wino_whole.hip", "ehip_wino_whole6.hip", "ehip_wino_whole5.hip", "ehip_wino_whole4.hip",
     "ehip_prepare.hip",
     "ehip_harness.hip",
@@ -61,7 +61,7 @@ EXTRA_FLAGS = {
                                     "-amdgpu-kernarg-preload-count=16"] for a in (6, 5, 4)},
     **{"ehip_wino_whole%d.hip" % a: ["-mllvm", "-amdgpu-mfma-vgpr-form=1", "-mllvm", "-pragma-unroll-threshold=1000000", "-mllvm",
                                      "-amdgpu-kernarg-preload-count=16"] for a in (6, 5, 4)},
-    "ehip_wino_split.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1", "-mllvm", "-amdgpu-kernarg-preload-count=16"],
+    "ehip_wino_cols.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1", "-mllvm", "-amdgpu-kernarg-preload-count=16"],
     "ehip_wino.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=16"],
     "ehip_fewch.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=16"],
     "ehip_gemm1x1s.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=16"],

@@ -283,9 +283,10 @@ RingForm wino_ring_form6(int form, int nks);   // tile sizes 6, 5, 4; nks = k-st
 RingForm wino_ring_form5(int form, int nks);
 RingForm wino_ring_form4(int form, int nks);
 hipError_t plan_wino_gemm_output_ring(LaunchPlan &plan, const WinoFusedArgs &a, int form);
-// few output values: the input channels shared out among the waves of a workgroup (ehip_wino_split.hip)
-bool wino_split_applies(const WinoFusedArgs &a);
-hipError_t plan_wino_gemm_output_split(LaunchPlan &plan, const WinoFusedArgs &a);
+// about one round of workgroups: the columns of the positions shared out among the waves of a workgroup (ehip_wino_cols.hip); the
+// form for the layer, or -1
+int wino_cols_pick(const WinoFusedArgs &a);
+hipError_t plan_wino_gemm_output_cols(LaunchPlan &plan, const WinoFusedArgs &a, int form);
 // the whole layer in one kernel, up to 256 input channels (ehip_wino_whole.hip)
 struct WholeForm {
   void (*kernel)(const WinoWholeArgs *, const void *, void *, const float *);

@@ -694,7 +694,8 @@ hipError_t plan_wino_gemm_output(LaunchPlan &plan, const WinoFusedArgs &a0)
 {
   WinoFusedArgs a = a0;
   const int A = a.tile ? a.tile : 6, AA = A * A;
-  if (wino_split_applies(a)) return plan_wino_gemm_output_split(plan, a);
+  const int cols = wino_cols_pick(a);
+  if (cols >= 0) return plan_wino_gemm_output_cols(plan, a, cols);
   const int ring = wino_ring_pick(a);
   if (ring >= 0) return plan_wino_gemm_output_ring(plan, a, ring);
   if (wino_lanes_applies(a)) return plan_wino_gemm_output_lanes(plan, a);

@@ -16,14 +16,14 @@ namespace {
 // packed into the pixels' dwords as they come (16 dwords live instead of 4 x 16 floats; the old output of the in-place
 // sum stays packed as well).  Same operations in the same order per value as output_tile.
 // pack_channel: channel k of the lane's four -- bias, output scale, old output, ReLU, rounding, byte k of the dwords.
-template <int OUT, int A>
+// (E: pixels, the tile's or one row of it)
+template <int OUT, int A, int E = (A - 2) * (A - 2)>
 __device__ __forceinline__ void pack_channel(const float *o, float b, int k, bool with_relu, float repS, float z, bool with_sum,
                                              const unsigned *old, unsigned *pk)
 {
   static_assert(OUT == EHIP_U8 || OUT == EHIP_S8, "quantized output");
-  constexpr int M = A - 2;
 #pragma unroll
-  for (int e = 0; e < M * M; ++e) {
+  for (int e = 0; e < E; ++e) {
     float r = o[e] + b;
     r = __builtin_fmaf(r, repS, z);
     if (with_sum) {
@@ -66,43 +66,53 @@ __device__ __forceinline__ void rows_transpose(unsigned &x0, unsigned &x1, unsig
 // column g of the tile's row i and writes it with one 16-byte store (a wave then covers 16 tiles x 4 pixels of an
 // image row = up to 1 KB in one piece, where dword stores leave 16 pieces of 16 bytes per instruction).
 // block: the tile's image and channel block; ok: the tile exists.  Called by all lanes.
+// (store_row: row i of the tile, pk its M pixels)
+template <int A>
+__device__ __forceinline__ void store_row(const unsigned *pk, uint8_t *block, int i, int g, bool ok, int th, int tw, int oh_n, int ow_n,
+                                          int px)
+{
+  constexpr int M = A - 2;
+  unsigned c0 = pk[0], c1 = pk[1], c2 = M > 2 ? pk[M > 2 ? 2 : 0] : 0u, c3 = M > 3 ? pk[M > 3 ? 3 : 0] : 0u;
+  rows_transpose(c0, c1, c2, c3);
+  const int oh = M * th + i, ow = M * tw + g;
+  if (ok && g < M && oh < oh_n && ow < ow_n) {
+    // (non-temporal: the output would only push the transformed input, which the other channel blocks' workgroups
+    // still read, out of the L2 -- 128 -> 128 at 112 x 112: 130 -> 100 us)
+    typedef unsigned v4u __attribute__((ext_vector_type(4)));
+    const v4u vv = {c0, c1, c2, c3};
+    __builtin_nontemporal_store(vv, reinterpret_cast<v4u *>(block + ((size_t)oh * ow_n + ow) * px));
+  }
+}
 template <int A>
 __device__ __forceinline__ void store_cells(const unsigned *pk, uint8_t *block, int g, bool ok, int th, int tw, int oh_n, int ow_n,
                                             int px)
 {
   constexpr int M = A - 2;
 #pragma unroll
-  for (int i = 0; i < M; ++i) {
-    unsigned c0 = pk[M * i], c1 = pk[M * i + 1], c2 = M > 2 ? pk[M * i + (M > 2 ? 2 : 0)] : 0u, c3 = M > 3 ? pk[M * i + (M > 3 ? 3 : 0)] : 0u;
-    rows_transpose(c0, c1, c2, c3);
-    const int oh = M * th + i, ow = M * tw + g;
-    if (ok && g < M && oh < oh_n && ow < ow_n) {
-      // (non-temporal: the output would only push the transformed input, which the other channel blocks' workgroups
-      // still read, out of the L2 -- 128 -> 128 at 112 x 112: 130 -> 100 us)
-      typedef unsigned v4u __attribute__((ext_vector_type(4)));
-      const v4u vv = {c0, c1, c2, c3};
-      __builtin_nontemporal_store(vv, reinterpret_cast<v4u *>(block + ((size_t)oh * ow_n + ow) * px));
-    }
-  }
+  for (int i = 0; i < M; ++i) store_row<A>(pk + M * i, block, i, g, ok, th, tw, oh_n, ow_n, px);
 }
 
 // the old output of the in-place sum the same way round: cells in, the lane's four channels of every pixel out
+template <int A>
+__device__ __forceinline__ void load_old_row(unsigned *old, const uint8_t *block, int i, int g, int th, int tw, int oh_n, int ow_n, int px)
+{
+  constexpr int M = A - 2;
+  const int oh = M * th + i, ow = M * tw + g;
+  const bool in = g < M && oh < oh_n && ow < ow_n;
+  const uint4 c = *reinterpret_cast<const uint4 *>(block + (in ? ((size_t)oh * ow_n + ow) * px : 0));
+  unsigned c0 = c.x, c1 = c.y, c2 = c.z, c3 = c.w;
+  rows_transpose(c0, c1, c2, c3);
+  old[0] = c0;
+  old[1] = c1;
+  if (M > 2) old[M > 2 ? 2 : 0] = c2;
+  if (M > 3) old[M > 3 ? 3 : 0] = c3;
+}
 template <int A>
 __device__ __forceinline__ void load_old_cells(unsigned *old, const uint8_t *block, int g, int th, int tw, int oh_n, int ow_n, int px)
 {
   constexpr int M = A - 2;
 #pragma unroll
-  for (int i = 0; i < M; ++i) {
-    const int oh = M * th + i, ow = M * tw + g;
-    const bool in = g < M && oh < oh_n && ow < ow_n;
-    const uint4 c = *reinterpret_cast<const uint4 *>(block + (in ? ((size_t)oh * ow_n + ow) * px : 0));
-    unsigned c0 = c.x, c1 = c.y, c2 = c.z, c3 = c.w;
-    rows_transpose(c0, c1, c2, c3);
-    old[M * i] = c0;
-    old[M * i + 1] = c1;
-    if (M > 2) old[M * i + (M > 2 ? 2 : 0)] = c2;
-    if (M > 3) old[M * i + (M > 3 ? 3 : 0)] = c3;
-  }
+  for (int i = 0; i < M; ++i) load_old_row<A>(old + M * i, block, i, g, th, tw, oh_n, ow_n, px);
 }
 
 // All positions of the lane's tile x four channels -> the output: Y = At M A channel by channel, packed, and written by

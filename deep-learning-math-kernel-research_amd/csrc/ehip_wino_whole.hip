@@ -21,15 +21,23 @@ namespace ehip {
 //     0.97 / 0.94; 256 -> 64, 65 0.83; 256 -> 128, 100 / 125 1.07 / 0.88; 256 -> 256, 163 1.02
 //   tile size 4: 64 -> 128, 4 / 784 0.84 / 0.93; 64 -> 256, 392 / 784 0.86 / 1.02; 128 -> 128, 40 / 65 / 466 0.97 / 0.95 / 0.82; 128 -> 256, 392 0.94; 128 -> 512, 160 1.12;
 //     192 -> 64, 65 0.91; 192 -> 128, 98 / 123 1.03 / 0.92; 192 -> 256, 160 / 245 0.98 / 0.91; 256 -> 128, 98 / 123 1.03 / 0.91; 256 -> 256, 196 / 245 0.95 / 0.98
+// and where the stages have the kernel that shares the columns of the positions out (ehip_wino_cols.hip), planes of 14 x 14 / 12 x 12 / 8 x 8:
+//   tile size 6: 64 -> 64, 64 / 98 / 196 blocks 1.09 / 0.92 / 0.82; 64 -> 128, 32 / 48 / 98 1.16 / 1.02 / 0.96; 128 -> 64, 64 / 98 / 128 1.31 / 1.03 / 0.90; 128 -> 128, 64 / 98 / 128
+//     1.33 / 1.03 / 0.95; 192 -> 64, 64 / 98 1.40 / 0.98; 256 -> 64, 64 / 98 / 128 1.30 / 1.04 / 0.98
+//   tile size 5: 64 -> 64, 16 / 64 / 98 1.03 / 1.00 / 0.90; 64 -> 128, 32 / 48 1.11 / 0.96; 128 -> 64, 64 / 98 1.16 / 0.96; 128 -> 128, 64 / 98 1.21 / 0.99; 192 -> 64, 98 / 128
+//     1.08 / 0.94; 256 -> 64, 98 / 128 1.00 / 0.94
+//   tile size 4: 128 -> 128, 64 / 98 1.12 / 0.95; 256 -> 64, 64 / 98 1.09 / 0.99
 static bool wino_whole_pays(int A, int nks, int blocks, int groups)
 {
   // blocks from (at most 64 output channels; more) and to, groups of 16 output channels, blocks x groups; by k-steps of 64 input
   // channels
   struct Limit { int least_few, least, most, groups, work; };
   static const Limit limits[3][4] = {
-      {{1, 1, 1200, 64, 6300}, {1, 48, 480, 16, 6300}, {56, 110, 256, 16, 4000}, {56, 115, 256, 16, 3200}},     // tile size 4
-      {{1, 32, 1200, 64, 4700}, {32, 90, 480, 16, 4000}, {48, 110, 256, 16, 4000}, {48, 110, 256, 8, 4000}},
-      {{24, 48, 400, 64, 3300}, {56, 112, 480, 8, 4000}, {90, 120, 256, 12, 4000}, {110, 125, 256, 8, 4000}}};
+      {{1, 1, 1200, 64, 6300}, {1, 90, 480, 16, 6300}, {56, 110, 256, 16, 4000}, {90, 115, 256, 16, 3200}},     // tile size 4
+      {{1, 40, 1200, 64, 4700}, {80, 90, 480, 16, 4000}, {110, 110, 256, 16, 4000}, {110, 110, 256, 8, 4000}},
+      {{24, 56, 400, 64, 3300}, {110, 112, 480, 8, 4000}, {95, 120, 256, 12, 4000}, {110, 125, 256, 8, 4000}}};
+  // (the fused stage with a workgroup of its own on a CU for every 16 channels x 16 tiles: the stages)
+  if (A >= 5 && (long long)blocks * groups <= 256) return false;
   const Limit &l = limits[A - 4][nks - 1];
   return blocks >= (groups <= 4 ? l.least_few : l.least) && blocks <= l.most && groups <= l.groups && (long long)blocks * groups <= l.work;
 }

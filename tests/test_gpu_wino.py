@@ -823,34 +823,38 @@ def test_wino_whole_choice(tile, ic, oc, n, hw, whole, monkeypatch):
     assert int((outs[0] != 0).sum()) > outs[0].numel() // 8 and torch.equal(outs[0], outs[1])
 
 
-# ---- few output values: the input channels shared out among the waves of a workgroup ----------------------
+# ---- about one round of workgroups: the columns of the positions shared out among the waves ----------------
+@pytest.mark.parametrize("form", ["0", "1", "2"])
 @pytest.mark.parametrize("tile", [6, 5, 4])
 @pytest.mark.parametrize("out_type,with_sum,with_relu,out_nhwc", [(ol.S8, 0, True, False), (ol.U8, 1, True, True), (ol.S8, 1, False, False),
                                                                   (ol.U8, 0, False, True), (ol.F32, 0, True, True), (ol.F32, 0, False, False)])
-@pytest.mark.parametrize("n,ic,oc,h,w", [(1, 16, 16, 4, 5), (3, 100, 24, 7, 9), (2, 256, 48, 9, 13), (1, 272, 80, 11, 6), (5, 400, 16, 5, 7), (1, 512, 32, 14, 13)])
-def test_wino_fused_split(n, ic, oc, h, w, out_type, with_sum, with_relu, out_nhwc, tile, monkeypatch):
-    """Waves without a k-step and with a part of one, channel tails, blocks of tiles that end early, across images and inside a unit of
-    32; every output type, layout and the sum"""
+@pytest.mark.parametrize("n,ic,oc,h,w", [(1, 16, 16, 4, 5), (3, 100, 24, 7, 9), (2, 256, 48, 9, 13), (1, 272, 80, 11, 6), (5, 400, 16, 5, 7), (1, 640, 32, 14, 13),
+                                         (7, 64, 144, 9, 11)])
+def test_wino_fused_columns(n, ic, oc, h, w, out_type, with_sum, with_relu, out_nhwc, tile, form, monkeypatch):
+    """k-steps that do not fill the ring and last ones in part, channel tails and an odd last half, blocks of tiles that end early, across
+    images and inside a unit of 32, a last pair of them with one; every output type, layout and the sum"""
     import torch
     if out_nhwc and oc % 16:
         oc = ol.up16(oc)
     monkeypatch.setenv("EHIP_WINO_WHOLE", "0")
-    monkeypatch.setenv("EHIP_WINO_SPLIT", "1")
+    monkeypatch.setenv("EHIP_WINO_COLS", form)
     E, d, (x, wb, b), tinput, exp, out = _u8_layer(n, ic, oc, h, w, tile, out_type, with_sum, with_relu, False, out_nhwc, seed=n + ic + h + tile)
     conv = E.Conv(d)
     conv.prepare(wb, b)
-    assert conv.kernel_name.endswith("_split")
+    assert conv.kernel_name.endswith(("_cols<16,16>", "_cols<32,16>", "_cols<32,32>")[int(form)])
     conv.execute(out, x, None, b)
     torch.cuda.synchronize()
     assert np.array_equal(bits(host(out)), bits(exp)), "output differs at %d of %d" % (int((host(out) != exp).sum()), exp.size)
 
 
-@pytest.mark.parametrize("tile,n,ic,oc,hw,split", [(6, 2, 512, 512, 28, True), (6, 3, 512, 512, 28, False), (6, 1, 192, 256, 28, True), (6, 1, 128, 256, 28, False),
-                                                   (5, 2, 256, 256, 28, True), (4, 1, 256, 256, 14, True), (6, 1, 512, 512, 14, False)])
-def test_wino_fused_split_choice(tile, n, ic, oc, hw, split):
+@pytest.mark.parametrize("tile,n,ic,oc,hw,form", [
+    (6, 2, 512, 512, 28, "<16,16>"), (6, 3, 512, 512, 28, "<32,16>"), (6, 64, 256, 256, 14, "<32,32>"), (6, 65, 256, 256, 14, ""), (6, 1, 256, 256, 14, "<16,16>"),
+    (6, 1, 512, 512, 14, "<16,16>"), (6, 1, 512, 256, 14, ""), (5, 3, 1024, 256, 28, "<32,16>"), (5, 64, 128, 256, 14, ""), (4, 1, 256, 256, 14, "<16,16>"), (4, 1, 128, 512, 14, ""), (4, 12, 128, 512, 8, "<32,16>")])
+def test_wino_fused_columns_choice(tile, n, ic, oc, hw, form, monkeypatch):
+    monkeypatch.setenv("EHIP_WINO_WHOLE", "0")
     E = pkg()
     d = E.make_desc(n, ic, oc, hw, hw, 3, 3, 1, algorithm=E.CONV_WINOGRAD, input_type=E.U8, output_type=E.S8, input_quant=(1.0 / 255.0, 0.0),
                     tile_size=tile, execution_mode=0xa161, wino_tinput_quant=(22.0 / 255.0, 104.0))
     conv = E.Conv(d)
     conv.prepare(dev(np.zeros((oc // 16, ic // 16, 3, 3, 16, 16), f32)), dev(np.zeros(oc, f32)))
-    assert conv.kernel_name.endswith("_split") == split
+    assert (conv.kernel_name.endswith("_cols" + form) if form else "_cols" not in conv.kernel_name)
