@@ -93,6 +93,49 @@ __global__ __launch_bounds__(kBlock) void k_wino_trans_input_u8(const WinoArgs *
     *reinterpret_cast<unsigned *>(const_cast<uint8_t *>(base) + e * pos_stride + voff) = packed[e] ^ flip;
 }
 
+// f32 input, tile size 6: a lane = a tile x TWO channels (a wave = eight tiles x one unit).  With four channels the tile alone is 144
+// registers and two waves fill a SIMD, whose vector units then wait a third of the time; with two channels (166 registers) three
+// waves fit, and each is half as long a chain.  The lane's bytes meet in LDS and leave by whole cells, 128 bytes of a position in one
+// piece.  Against the form above, other tensors on every call: 256 channels at 56 x 56, N = 64 71.4 -> 67.1 us (320 MB: a
+// conversion of floats to halves moves the same bytes in 55), 64 channels 24.6 -> 21.2, 512 channels at 7 x 7 7.3 -> 5.6, one image of
+// 56 x 56 6.5 -> 4.7.  (Where input, codes and output together are far beyond what the memory-side cache holds, 256 channels at 56 x 56
+// with three sets of tensors in turn, the fused stage behind it loses what this one gains: 196.7 -> 196.5 us a layer.)  At tile sizes 5 and 4 the tile is 100 and 64 registers and the halves cost more than they give: 256 channels at
+// 56 x 56 81.7 against 83.8 and 86.4 against 102.
+template <int A>
+__global__ __launch_bounds__(kBlock, 3) void k_wino_trans_input_floats(const WinoArgs *rest, const void *in)
+{
+  WinoArgs a = load_args(rest);
+  a.in = in;
+  constexpr int AA = A * A;
+  __shared__ uint4 lds[4][AA * 8];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int o2 = lane & 7, tl = lane >> 3;
+  const int item = (blockIdx.x & 7) * a.items_per_xcd + (blockIdx.x >> 3);
+  if (item >= a.nblocks * a.ic2) return;   // whole workgroup
+  const int c2 = item % a.ic2;
+  const int t32 = item / a.ic2, t0 = t32 * 32 + wave * 8;
+  if (t0 >= a.t) return;                   // whole wave
+  // (a lane without a tile takes part with the last one: what it leaves lies in the last block's padding)
+  const TileCoord c = tile_coord<A>(a, t0 + tl < a.t ? t0 + tl : a.t - 1);
+  float2 d[AA];
+  unsigned packed[AA];
+  gather_tile_pairs<A>(a, c, c2, o2, d);
+  quantize_tile<float2, A>(d, c.border, a.mrepS, a.mz, packed);
+  uint4 *cells = lds[wave];
+  unsigned short *mine = reinterpret_cast<unsigned short *>(cells + tl) + o2;
+#pragma unroll
+  for (int e = 0; e < AA; ++e) mine[64 * e] = (unsigned short)(packed[e] ^ 0x8080u);   // (signed bytes, see k_wino_trans_input_u8)
+  __builtin_amdgcn_wave_barrier();
+  uint8_t *base = a.tin + ((size_t)t32 * AA * a.ic2 + c2) * 512 + wave * 128;
+  const unsigned pos = (unsigned)a.ic2 * 512u;
+  const unsigned voff = (unsigned)(lane >> 3) * pos + (unsigned)(lane & 7) * 16u;
+#pragma unroll
+  for (int k = 0; k < (AA + 7) / 8; ++k)
+    if (8 * k + 7 < AA || 8 * k + (lane >> 3) < AA)
+      *reinterpret_cast<uint4 *>(base + (size_t)(8 * k) * pos + voff) = cells[64 * k + lane];
+}
+
 // The same for u8 codes below 4 GB into the blocked layout, through LDS: the pixels of a tile change hands there (gather_tile_lds),
 // and the finished codes take the place of the pixels, position by position, so that they leave by 16 bytes a lane.
 // What bounds it is the issue of vector instructions: 1250 per wave and 16 tiles x 16 channels, of which conversions, minima
@@ -643,12 +686,13 @@ hipError_t plan_wino_trans_input(LaunchPlan &plan, const WinoArgs &a0)
     if (a.buf_gather && a.in_u8 && a.tin_blocked && !(wide && wide[0] == '0')) a.buf_gather = 2;   // k_wino_trans_input_codes
   }
   const bool codes = a.buf_gather == 2;
+  const bool floats = a.tile != 4 && a.tile != 5 && a.buf_gather && !a.in_u8 && a.tin_blocked && (unsigned long long)a.n * a.ic2 * a.ih * a.iw * 64 <= 0x3f000000ull;
   const char *short_env = getenv("EHIP_WINO_SHORT");
   // the short form up to three waves of the other on a SIMD (64 channels at 56 x 56, N = 64: 13.3 against 14.0 us; 256 at 28 x 28 with tile
   // size 5, 6400 waves: 20.7 against 19.0); at tile size 4, whose waves are short anyway, up to one and a half (784 waves 3.9 against
   // 4.0, and 11.4 against 12.1 with the stage behind it; 2048 waves 5.7 against 5.4)
   const bool shorter = codes && (short_env ? short_env[0] != '0' : (long long)((a.t + 15) / 16) * a.ic2 < (a.tile == 4 ? 1536 : 3328));
-  const int tiles = shorter ? 16 : 64;   // of a workgroup
+  const int tiles = shorter ? 16 : floats ? 32 : 64;   // of a workgroup
   a.nblocks = (a.t + tiles - 1) / tiles;
   a.items_per_xcd = (int)(((long long)a.nblocks * a.ic2 + 7) / 8);
   dim3 grid(8 * a.items_per_xcd, 1);
@@ -658,6 +702,7 @@ hipError_t plan_wino_trans_input(LaunchPlan &plan, const WinoArgs &a0)
       : codes ? k_wino_trans_input_codes<A> : a.in_u8 ? k_wino_trans_input_u8<unsigned, A> : k_wino_trans_input_u8<float4, A>
   if (a.tile == 4) EHIP_WI(4);
   else if (a.tile == 5) EHIP_WI(5);
+  else if (floats) kern = k_wino_trans_input_floats<6>;
   else EHIP_WI(6);
 #undef EHIP_WI
   return plan_set(plan, kern, grid, dim3(kBlock), 0, a, ArgBlock{}, ArgIn{a.in});

@@ -35,6 +35,12 @@ __device__ __forceinline__ void buffer_load_cell(BufferRsrc r, unsigned off, uin
   const v4u x = __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 0));
   v = make_uint4(x.x, x.y, x.z, x.w);
 }
+__device__ __forceinline__ void buffer_load_cell(BufferRsrc r, unsigned off, float2 &v)
+{
+  typedef float v2f __attribute__((ext_vector_type(2)));
+  const v2f x = __builtin_bit_cast(v2f, __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, 0, 0));
+  v = make_float2(x.x, x.y);
+}
 // (off: the lane's bytes, checked against the buffer; at: a wave-uniform offset on top)
 __device__ __forceinline__ void buffer_load_cell(BufferRsrc r, unsigned off, unsigned at, v4i &v)
 {
@@ -44,6 +50,7 @@ __device__ __forceinline__ void buffer_load_cell(BufferRsrc r, unsigned off, uns
 typedef int BufferRsrc;
 __device__ inline BufferRsrc make_rsrc(const void *, unsigned) { return 0; }
 __device__ inline void buffer_load_cell(BufferRsrc, unsigned, float4 &v) { v = float4(); }
+__device__ inline void buffer_load_cell(BufferRsrc, unsigned, float2 &v) { v = float2(); }
 __device__ inline void buffer_load_cell(BufferRsrc, unsigned, unsigned &v) { v = 0u; }
 __device__ inline void buffer_load_cell(BufferRsrc, unsigned, uint4 &v) { v = uint4(); }
 __device__ inline void buffer_load_cell(BufferRsrc, unsigned, unsigned, v4i &v) { v = v4i(); }
@@ -53,6 +60,8 @@ __device__ __forceinline__ float comp_of(const float4 &v, int k)
 {
   return k == 0 ? v.x : (k == 1 ? v.y : (k == 2 ? v.z : v.w));
 }
+
+__device__ __forceinline__ float comp_of(const float2 &v, int k) { return k == 0 ? v.x : v.y; }
 
 // four u8 codes in a dword: the reference turns the codes into floats as they are
 // (src/kernel/elk_conv_wino_4x4_3x3_input.hxx:40-47)
@@ -140,6 +149,27 @@ __device__ __forceinline__ void gather_tile_buf(const WinoArgs &a, const TileCoo
       buffer_load_cell(rin, (rv[i] && cv[j]) ? voff + so : 0xffffff00u, d[A * i + j]);
     }
 }
+// The lane's two channels (o2: their place among a unit's eight pairs) of an f32 tensor of at most 2^30 - 2^24 bytes.  A row and a column
+// outside the image each add enough to leave the buffer, and their sum does not come round, so that an address is one addition.
+template <int A>
+__device__ __forceinline__ void gather_tile_pairs(const WinoArgs &a, const TileCoord &c, int c2, int o2, float2 *d)
+{
+  const unsigned px = a.in_nhwc ? (unsigned)a.ic2 * 64u : 64u;   // bytes between neighbouring pixels
+  const BufferRsrc rin = make_rsrc(a.in, (unsigned)a.n * a.ic2 * a.ih * a.iw * 64u);
+  const unsigned plane = a.in_nhwc ? (unsigned)c.n * a.ih * a.iw * px + c2 * 64u : ((unsigned)c.n * a.ic2 + c2) * a.ih * a.iw * 64u;
+  const unsigned at = plane + (unsigned)(c.h0 * a.iw + c.w0) * px + (unsigned)o2 * 8u, row = (unsigned)a.iw * px;
+  unsigned ro[A], co[A];
+#pragma unroll
+  for (int i = 0; i < A; ++i) {
+    ro[i] = (unsigned)(c.h0 + i) < (unsigned)a.ih ? at + i * row : 0x80000000u;
+    co[i] = (unsigned)(c.w0 + i) < (unsigned)a.iw ? i * px : 0x40000000u;
+  }
+#pragma unroll
+  for (int i = 0; i < A; ++i)
+#pragma unroll
+    for (int j = 0; j < A; ++j) buffer_load_cell(rin, ro[i] + co[j], d[A * i + j]);
+}
+
 
 // u8 input below 4 GB, by whole cells and through LDS: `cells` = the wave's own [A x A pixels][16 tiles] cells of 16 bytes, S
 // cells from pixel to pixel.  Lane (tile, q) fetches the cells (all four channel quads) of pixels q, 4 + q, ... of its tile --
@@ -174,31 +204,44 @@ __device__ __forceinline__ void gather_tile_lds(const WinoArgs &a, const TileCoo
   __builtin_amdgcn_wave_barrier();
 }
 
-// packed[position]: the lane's four channels of the transformed tile as u8 codes.
+// min(s, a, b) in one instruction (left to itself the compiler pairs the values up first: three for four values, not two)
+__device__ __forceinline__ float min3(float s, float a, float b)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm("v_min3_f32 %0, %0, %1, %2" : "+v"(s) : "v"(a), "v"(b));
+#endif
+  return s;
+}
+// the same with a NaN for a NaN
+__device__ __forceinline__ float minimum3(float s, float a, float b)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm("v_minimum3_f32 %0, %0, %1, %2" : "+v"(s) : "v"(a), "v"(b));
+#endif
+  return s;
+}
+// packed[position]: the lane's four (float2 cells: two) channels of the transformed tile as u8 codes.
 template <typename Cell, int A>
 __device__ __forceinline__ void quantize_tile(const Cell *d, bool border, float mrepS, float mz, unsigned *packed)
 {
   constexpr int AA = A * A;
   constexpr bool kCodes = sizeof(Cell) == sizeof(unsigned);
+  constexpr int kChannels = sizeof(Cell) == sizeof(float2) ? 2 : 4;
   // mixed: the wave holds interior and rim tiles -- the per-lane, branch-free form of the transform.
   // Quantization: sat_u8(rne_to_u32(V * (in_S / tin_S) + tin_z)), one rounding in the multiply-add.  The
   // reference's float -> u32 conversion turns everything below -0.5 (and NaN) into 0xffffffff, which then
   // saturates to 255; v_cvt_pk_u8_f32 rounds to nearest even and saturates the rest.  watch: the plain
-  // conversion, with the quirk's cases only looked for -- two running integer maxima over the values' bit
-  // patterns, one instruction per value instead of a compare and a select -- and the result says whether
-  // one was seen (never, with a calibrated tinput_quant); the caller then runs the exact form again.
-  // u8 user input: the codes are finite, so with finite quantization constants no NaN can arise and ONE running
-  // float minimum (an instruction per two values) says whether anything fell below -0.5; constants that are not
+  // conversion, with the quirk's cases only looked for: a running minimum that a NaN sticks to, an instruction per two values,
+  // says whether one was seen (never, with a calibrated tinput_quant); the caller then runs the exact form again.
+  // u8 user input: the codes are finite, so with finite quantization constants no NaN can arise; constants that are not
   // finite send every wave to the exact form.
   const bool odd_consts = !(__builtin_fabsf(mrepS) <= 3.402823466e38f) || !(__builtin_fabsf(mz) <= 3.402823466e38f);
   auto channels = [&](bool mixed, bool watch) {
-    unsigned seen_u = 0u;
-    int seen_s = 0;
-    float seen_min = 0.0f;
+    float seen = 0.0f;
 #pragma unroll
     for (int k = 0; k < AA; ++k) packed[k] = 0u;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
+    for (int k = 0; k < kChannels; ++k) {
       float f[AA], v[AA];
 #pragma unroll
       for (int e = 0; e < AA; ++e) f[e] = comp_of(d[e], k);
@@ -211,25 +254,9 @@ __device__ __forceinline__ void quantize_tile(const Cell *d, bool border, float 
           y[e] = __builtin_fmaf(v[e], mrepS, mz);
           packed[e] = __builtin_amdgcn_cvt_pk_u8_f32(y[e], k, packed[e]);
         }
-        // bit patterns above 0xbf000000 unsigned: below -0.5, or a negative NaN; above 0x7f800000 signed: a
-        // positive NaN
-        if (kCodes) {
 #pragma unroll
-          for (int e = 0; e + 1 < AA; e += 2) seen_min = __builtin_fminf(seen_min, __builtin_fminf(y[e], y[e + 1]));
-          if (AA & 1) seen_min = __builtin_fminf(seen_min, y[AA - 1]);
-        } else {
-#pragma unroll
-          for (int e = 0; e + 1 < AA; e += 2) {
-            const unsigned b0 = __float_as_uint(y[e]), b1 = __float_as_uint(y[e + 1]);
-            seen_u = max(seen_u, max(b0, b1));
-            seen_s = max(seen_s, max((int)b0, (int)b1));
-          }
-          if (AA & 1) {
-            const unsigned b = __float_as_uint(y[AA - 1]);
-            seen_u = max(seen_u, b);
-            seen_s = max(seen_s, (int)b);
-          }
-        }
+        for (int e = 0; e + 1 < AA; e += 2) seen = kCodes ? __builtin_fminf(seen, __builtin_fminf(y[e], y[e + 1])) : minimum3(seen, y[e], y[e + 1]);
+        if (AA & 1) seen = kCodes ? __builtin_fminf(seen, y[AA - 1]) : minimum3(seen, y[AA - 1], y[AA - 1]);
       } else {
 #pragma unroll
         for (int e = 0; e < AA; ++e) {
@@ -238,7 +265,7 @@ __device__ __forceinline__ void quantize_tile(const Cell *d, bool border, float 
         }
       }
     }
-    return kCodes ? (seen_min < -0.5f || odd_consts) : (seen_u > 0xbf000000u || seen_s > 0x7f800000);
+    return kCodes ? (seen < -0.5f || odd_consts) : !(seen >= -0.5f);
   };
   const bool mixed = !kCodes && __ballot(border) != 0;   // wave-uniform
   bool again;
@@ -250,14 +277,6 @@ __device__ __forceinline__ void quantize_tile(const Cell *d, bool border, float 
   }
 }
 
-// min(s, a, b) in one instruction (left to itself the compiler pairs the values up first: three for four values, not two)
-__device__ __forceinline__ float min3(float s, float a, float b)
-{
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm("v_min3_f32 %0, %0, %1, %2" : "+v"(s) : "v"(a), "v"(b));
-#endif
-  return s;
-}
 // The same for the pixels that gather_tile_lds left in LDS (quads: the lane's, 4 S dwords from pixel to pixel), with few
 // registers: every channel reads its bytes, column by column, and a row of the result is packed as it is finished.  At 128
 // registers four waves fit on a SIMD.  (CH < 4: that many channels of the quad, from the k0-th on, in the low bytes.)  The channels are a loop: a quarter of the instructions to fetch, which a layer between

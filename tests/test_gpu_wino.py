@@ -795,6 +795,49 @@ def test_wino_transformed_codes(n, ic, hw, nhwc, tin, tile, whole, short, monkey
     assert np.array_equal(conv.query(E.Q_TINPUT_U8).reshape(tinput.shape), tinput)
 
 
+@pytest.mark.parametrize("nhwc", [False, True])
+@pytest.mark.parametrize("n,ic,h,w", [(1, 16, 4, 4), (3, 32, 5, 9), (2, 144, 13, 11), (5, 48, 7, 6), (1, 20, 33, 35)])
+@pytest.mark.parametrize("data", ["calibrated", "under range", "not finite"])
+def test_wino_transformed_floats(n, ic, h, w, nhwc, data, monkeypatch):
+    """The transformed input of f32 tensors, two channels a lane: tiles in every place of a wave's eight and a block's 32, rims; values
+    below -0.5, which end as 255 in the wave's second pass; and infinities and NaN, which the kernel with the plain gather turns into the same codes"""
+    import torch
+    if nhwc and ic % 16:
+        ic = ol.up16(ic)
+    E, p, d, xb, wb, bias = make_wino(n, ic, 32, max(h, w), seed=13 + ic + h)
+    d.ih = d.oh = p.ih = p.oh = h
+    d.iw = d.ow = p.iw = p.ow = w
+    xb = np.ascontiguousarray(xb[:, :, :h, :w])
+    mn, mx = ol.wino_tinput_range(p, xb)
+    s_t = float((f32(mx) - f32(mn)) / f32(255.0))
+    p.tin_scale, p.tin_z = d.tinput_scale, d.tinput_z = s_t, float(-f32(mn) / f32(s_t)) * (0.5 if data == "under range" else 1.0)
+    tin = ol.wino_trans_input(p, xb)
+    x = xb
+    if data == "not finite":
+        x = x.copy()
+        rng = np.random.default_rng(n + h)
+        flat = x.reshape(-1)
+        flat[rng.integers(0, flat.size, 6)] = [np.nan, -np.nan, np.inf, -np.inf, 3e38, -3e38]
+    if nhwc:
+        d.input_fmt, x = E.NHWC, ol.blocked_to_nhwc(x, ic)
+    got = []
+    for gather in ("1", "0"):
+        monkeypatch.setenv("EHIP_WINO_BUF_GATHER", gather)
+        conv = E.Conv(d)
+        d_b = dev(bias)
+        conv.prepare(dev(wb), d_b)
+        d_out = torch.zeros((n, 2, h, w, 16), dtype=torch.float32, device="cuda")
+        conv.execute(d_out, dev(x), None, d_b)
+        torch.cuda.synchronize()
+        got.append(conv.query(E.Q_TINPUT_U8).reshape(tin.shape))
+    assert np.array_equal(got[0], got[1])
+    if data == "not finite":
+        assert (got[0] == 255).sum() > (tin == 255).sum()
+    else:
+        assert np.array_equal(got[0], tin), "u8 transformed input differs at %d cells" % int((got[0] != tin).sum())
+        assert data != "under range" or (tin == 255).sum() > 4   # (else no wave converts twice)
+
+
 @pytest.mark.parametrize("tile,ic,oc,n,hw,whole", [
     (6, 64, 64, 32, 56, True), (6, 64, 64, 64, 56, False), (6, 64, 64, 2, 28, False), (6, 128, 128, 64, 28, True), (6, 128, 128, 160, 28, False),
     (6, 192, 192, 20, 28, False), (6, 192, 192, 64, 28, True), (6, 256, 64, 64, 28, True), (6, 256, 256, 64, 14, False), (5, 128, 256, 40, 28, True),
