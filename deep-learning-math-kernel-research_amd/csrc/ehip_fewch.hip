@@ -15,6 +15,8 @@
 //      a byte address of any alignment, read as five dwords and shifted into place;
 //   3. kh * nu / 2 MFMAs per tile against the weights in registers, then the shared epilogue.
 // The four waves split into a.wo channel tiles x 4 / a.wo pixel tiles.
+#include <type_traits>
+
 #include "ehip_internal.hpp"
 
 namespace ehip {
@@ -177,30 +179,37 @@ __device__ __forceinline__ FewChTables fewch_stage(const FewChArgs &a, unsigned 
     __syncthreads();
     uint8_t *lb = reinterpret_cast<uint8_t *>(rows_lds);
     const int total = a.nrows_in * a.iw;
-    for (int base = 0; base < total; base += kBlock * kStageDepth) {
-      unsigned v[kStageDepth];
-      int at[kStageDepth];   // LDS byte of the pixel, -1: nothing to store
+    auto stage_cells = [&](auto depth_c) {
+      constexpr int DEPTH = decltype(depth_c)::value;
+      for (int base = 0; base < total; base += kBlock * DEPTH) {
+        unsigned v[DEPTH];
+        int at[DEPTH];   // LDS byte of the pixel, -1: nothing to store
 #pragma unroll
-      for (int u = 0; u < kStageDepth; ++u) {
-        int idx = base + u * kBlock + tid;
-        const bool in_range = idx < total;
-        idx = in_range ? idx : total - 1;
-        const int r = fastdiv(idx, a.iw, a.iw_magic);
-        const int x = idx - r * a.iw;
-        const int h = ihb + r;
-        const bool inside = in_range && h >= 0 && h < a.ih;
-        at[u] = inside ? r * a.lrow + (x + a.pad_l) * a.icl : -1;
-        v[u] = *reinterpret_cast<const unsigned *>(a.in + (inside ? ((long long)(img * a.ih + h) * a.iw + x) * 16 : 0));
-      }
-#pragma unroll
-      for (int u = 0; u < kStageDepth; ++u)
-        if (at[u] >= 0) {
-          const unsigned q = v[u] ^ 0x80808080u;
-#pragma unroll
-          for (int c = 0; c < 4; ++c)
-            if (c < a.ic) lb[at[u] + c] = (uint8_t)(q >> (8 * c));
+        for (int u = 0; u < DEPTH; ++u) {
+          int idx = base + u * kBlock + tid;
+          const bool in_range = idx < total;
+          idx = in_range ? idx : total - 1;
+          const int r = fastdiv(idx, a.iw, a.iw_magic);
+          const int x = idx - r * a.iw;
+          const int h = ihb + r;
+          const bool inside = in_range && h >= 0 && h < a.ih;
+          at[u] = inside ? r * a.lrow + (x + a.pad_l) * a.icl : -1;
+          v[u] = *reinterpret_cast<const unsigned *>(a.in + (inside ? ((long long)(img * a.ih + h) * a.iw + x) * 16 : 0));
         }
-    }
+#pragma unroll
+        for (int u = 0; u < DEPTH; ++u)
+          if (at[u] >= 0) {
+            const unsigned q = v[u] ^ 0x80808080u;
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+              if (c < a.ic) lb[at[u] + c] = (uint8_t)(q >> (8 * c));
+          }
+      }
+    };
+    // (tall strips of many pixels: two trips to memory instead of four, 7x7 s2 3 -> 64 at 224 x 224, N = 64 33.4 -> 30.8 us; a short strip's
+    // batch is mostly repeats, 3x3 s2 1 -> 64 at 112 x 112 7.3 -> 8.6)
+    if (total > 16 * kBlock) stage_cells(std::integral_constant<int, 2 * kStageDepth>{});
+    else stage_cells(std::integral_constant<int, kStageDepth>{});
   }
   store_tables();
   return FewChTables{lds_shift, lds_cls_h, lds_cls_w};
@@ -348,10 +357,17 @@ __global__ __launch_bounds__(kBlock, 3) void k_conv_fewch_u8s8(const FewChArgs *
 }
 
 // The same tiles for u8 / s8 output with ReLU (FewChArgs::lean; TAB: the shift row of the pixel's border class
-// comes from LDS): nothing but that epilogue, so the tile loop is straight-line code with 32-bit output offsets,
-// and the cells of a wave's next tile are read while the present one is scaled and stored.
+// comes from LDS): nothing but that epilogue, so the tile loop is straight-line code with 32-bit output offsets.
+// What bounds it (7x7 s2 3 -> 64 at 224 x 224, N = 64: 51 MB out, 9 us at the rate of a large fill; matrix instructions 4.6 us, vector
+// instructions 6): the strips are all staged at the same time, and then the stores, the matrix cores and the vector units
+// share what is left.  Without the stores 14.5 of 21.6 us are left, without the staging 20, without the scaling 17.4.
+// The chain of a tile's matrix instructions and the scaling of the tile before it are one stream of instructions: one after the
+// other, the waves of a SIMD fell into step and its units took turns (22.4 -> 21.5 us; N = 16 10.8 -> 9.3; 3x3 at stride 1 51.3 -> 49.4).
+// Tried: both channel tiles in one wave (half of the reads of cells; 21.4, but 3x3 16 -> 18.5), the weights ahead of the
+// staging (+0.7), six groups of pixels in flight (+0.2), nhwc cells paired in LDS so that neighbouring lanes write neighbouring
+// bytes (+0.9).
 template <int KS, bool CLAMP, bool TAB>
-__global__ __launch_bounds__(kBlock, 3) void k_conv_fewch_lean(const FewChArgs *rest, const uint8_t *in, void *out)
+__global__ __launch_bounds__(kBlock, KS == 7 ? 2 : 3) void k_conv_fewch_lean(const FewChArgs *rest, const uint8_t *in, void *out)
 {
   FewChArgs a = load_args(rest);
   a.in = in; a.out = out;
@@ -406,63 +422,126 @@ __global__ __launch_bounds__(kBlock, 3) void k_conv_fewch_lean(const FewChArgs *
   const int row_step = a.stride_h * a.lrow, px_step = a.stride_w * a.icl;
   const int ntiles = (npix + 31) >> 5;
 
-  int ro, ox;   // output row (in the strip) and column of the lane's pixel of the tile whose cells were read last
-  v4i b[KS];
-  auto read_cells = [&](int tile) {
+  // The matrix instructions of a tile are a chain of KS, with the cells of the tile after next read and a slice of the epilogue of the
+  // tile before it between any two of them: left in phases, the waves of a SIMD fall into step, and its matrix cores and vector
+  // units take turns.
+  // (what the lambdas below take of `a`, by value: a captured structure stays in memory)
+  const int ow = a.ow, out_nhwc = a.out_nhwc;
+  const unsigned ow_magic = a.ow_magic;
+  const float lo = a.ep.lo;
+  int ro, ox;   // output row (in the strip) and column of the lane's pixel of the tile that `place` saw last
+  int at0;      // LDS byte of its first cell
+  auto place = [&](int tile) {
     int p = tile * 32 + l32;
     p = p < npix ? p : npix - 1;   // also beyond the wave's last tile: some cell of the strip
-    ro = fastdiv(p, a.ow, a.ow_magic);
-    ox = p - ro * a.ow;
-    const int at0 = ro * row_step + ox * px_step;
-    if (a.icl == 4 && (a.stride_w & 1) == 0) {
+    ro = fastdiv(p, ow, ow_magic);
+    ox = p - ro * ow;
+    at0 = ro * row_step + ox * px_step;
+  };
+  v4i b[KS];
+  auto read_cell = [&](auto form, int ks) {
+    if (decltype(form)::value == 0) {
       // every cell starts on eight bytes: one read of twice eight bytes per cell, and neighbouring lanes' pieces follow each
       // other (as four dwords, eight bytes apart from lane to lane, half of the banks idle)
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const uint2 *src = reinterpret_cast<const uint2 *>(reinterpret_cast<const char *>(rows_lds) + at0 + cell_at[ks]);
-        const uint2 lo = src[0], hi = src[1];
-        b[ks] = v4i{(int)lo.x, (int)lo.y, (int)hi.x, (int)hi.y};
-      }
-    } else if (a.icl == 4) {
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const unsigned *src = rows_lds + ((at0 + cell_at[ks]) >> 2);
-        b[ks] = v4i{(int)src[0], (int)src[1], (int)src[2], (int)src[3]};
-      }
+      const uint2 *src = reinterpret_cast<const uint2 *>(reinterpret_cast<const char *>(rows_lds) + at0 + cell_at[ks]);
+      const uint2 lo = src[0], hi = src[1];
+      b[ks] = v4i{(int)lo.x, (int)lo.y, (int)hi.x, (int)hi.y};
+    } else if (decltype(form)::value == 1) {
+      const unsigned *src = rows_lds + ((at0 + cell_at[ks]) >> 2);
+      b[ks] = v4i{(int)src[0], (int)src[1], (int)src[2], (int)src[3]};
     } else {
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const int A = at0 + cell_at[ks];
-        const unsigned *src = rows_lds + (A >> 2);
-        const unsigned sh = A & 3;
-        const unsigned d0 = src[0], d1 = src[1], d2 = src[2], d3 = src[3], d4 = src[4];
-        b[ks] = v4i{(int)__builtin_amdgcn_alignbyte(d1, d0, sh), (int)__builtin_amdgcn_alignbyte(d2, d1, sh),
-                    (int)__builtin_amdgcn_alignbyte(d3, d2, sh), (int)__builtin_amdgcn_alignbyte(d4, d3, sh)};
-      }
+      const int A = at0 + cell_at[ks];
+      const unsigned *src = rows_lds + (A >> 2);
+      const unsigned sh = A & 3;
+      const unsigned d0 = src[0], d1 = src[1], d2 = src[2], d3 = src[3], d4 = src[4];
+      b[ks] = v4i{(int)__builtin_amdgcn_alignbyte(d1, d0, sh), (int)__builtin_amdgcn_alignbyte(d2, d1, sh),
+                  (int)__builtin_amdgcn_alignbyte(d3, d2, sh), (int)__builtin_amdgcn_alignbyte(d4, d3, sh)};
     }
   };
-  read_cells(wp);
-  for (int tile = wp; tile < ntiles; tile += wpn) {
-    v16i acc[1][1];
-    acc[0][0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wreg[0], b[0], comp0, 0, 0, 0);
+  const float hi = a.ep.out_type == EHIP_S8 ? __builtin_fminf(a.ep.hi, 127.0f) : a.ep.hi;
+  // (TAB: where the shift row of the lane's pixel starts, floats from the first)
+  auto shift_row = [&]() { return TAB ? (tabs.cls_h[ro] + tabs.cls_w[ox]) * tab_width : 0; };
+  auto load_row = [&](int row) {
+    if (TAB)
 #pragma unroll
-    for (int ks = 1; ks < KS; ++ks) acc[0][0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wreg[ks], b[ks], acc[0][0], 0, 0, 0);
-    if (TAB) {
-      const float *row = shift_rows + (tabs.cls_h[ro] + tabs.cls_w[ox]) * tab_width;
+      for (int q = 0; q < 4; ++q) lk[0].sh[q] = *reinterpret_cast<const float4 *>(shift_rows + row + 4 * q);
+  };
+  // four values of a finished tile
+  auto finish = [&](const v16i &acc, int q) -> int {
+    const float sc[4] = {lk[0].sc[q].x, lk[0].sc[q].y, lk[0].sc[q].z, lk[0].sc[q].w};
+    const float sh[4] = {lk[0].sh[q].x, lk[0].sh[q].y, lk[0].sh[q].z, lk[0].sh[q].w};
+    unsigned pk = 0;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) lk[0].sh[q] = *reinterpret_cast<const float4 *>(row + 4 * q);
+    for (int j = 0; j < 4; ++j) {
+      float f = __builtin_fmaf((float)acc[4 * q + j], sc[j], sh[j]);
+      if (CLAMP) f = __builtin_amdgcn_fmed3f(f, lo, hi);
+      pk = __builtin_amdgcn_cvt_pk_u8_f32(f, j, pk);
     }
-    __builtin_amdgcn_sched_barrier(0);
-    read_cells(tile + wpn);   // the MFMAs above have taken their operands
-    __builtin_amdgcn_sched_barrier(0);
+    return (int)pk;
+  };
+  const bool oc_ok = oc0 + 16 * lh < oc_real;
+  auto store = [&](int tile, const v4i &out) {
     const int p0 = tile * 32;
-    const bool pvalid[1] = {p0 + l32 < npix};
-    uint8_t *const cell[1] = {out_base + ((unsigned)p0 * px_stride + lane_off)};
-    // blocked output: non-temporal stores (3x3 s2 3 -> 32 at 224 x 224, N = 64: 15.9 -> 14.3 us); in nhwc a line's
-    // 16-byte pieces come from several waves and should meet in L2 (7x7 s2 3 -> 64: 32.9 -> 37.6 us with them)
-    if (a.out_nhwc) lean_store_typed<1, 1, false, CLAMP, false>(a.ep, acc, lk, cell, pvalid, oc0 + 16 * lh, oc_real, 0, nullptr);
-    else lean_store_typed<1, 1, false, CLAMP, true>(a.ep, acc, lk, cell, pvalid, oc0 + 16 * lh, oc_real, 0, nullptr);
-  }
+    if (p0 + l32 < npix && oc_ok) {
+      uint8_t *cell = out_base + ((unsigned)p0 * px_stride + lane_off);
+      // blocked output: non-temporal stores (3x3 s2 3 -> 32 at 224 x 224, N = 64: 15.9 -> 14.3 us); in nhwc a line's
+      // 16-byte pieces come from several waves and should meet in L2 (7x7 s2 3 -> 64: 32.9 -> 37.6 us with them)
+      if (out_nhwc) store_out16<false>(cell, out);
+      else store_out16<true>(cell, out);
+    }
+  };
+  auto walk = [&](auto form) {
+    v16i acc[2];
+    int row, row_next;   // shift rows: of the tile that is finished next, of the one behind it
+    // the matrix instructions of tile t (its cells are in b) into acc[I]; between them the cells of tile t + wpn are read and, with
+    // LAST, tile t - wpn leaves
+    auto step = [&](auto ic, auto last, int t) {
+      constexpr int I = decltype(ic)::value;
+      constexpr bool LAST = decltype(last)::value;
+      if (LAST) load_row(row);
+      row = row_next;
+      place(t + wpn);
+      v4i out;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        acc[I] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wreg[ks], b[ks], ks == 0 ? comp0 : acc[I], 0, 0, 0);
+        read_cell(form, ks);
+        if (LAST)
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            if (q * KS / 4 == ks) out[q] = finish(acc[1 - I], q);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      row_next = shift_row();
+      if (LAST) store(t - wpn, out);
+    };
+    auto leave = [&](const v16i &acc, int t) {
+      load_row(row);
+      v4i out;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) out[q] = finish(acc, q);
+      store(t, out);
+    };
+    using C0 = std::integral_constant<int, 0>;
+    using C1 = std::integral_constant<int, 1>;
+    int t = wp;
+    place(t);
+    row_next = shift_row();
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) read_cell(form, ks);
+    step(C0{}, std::false_type{}, t);
+    for (;;) {
+      if (t + wpn >= ntiles) { leave(acc[0], t); break; }
+      step(C1{}, std::true_type{}, t + wpn);
+      if (t + 2 * wpn >= ntiles) { leave(acc[1], t + wpn); break; }
+      step(C0{}, std::true_type{}, t + 2 * wpn);
+      t += 2 * wpn;
+    }
+  };
+  if (wp >= ntiles) return;
+  if (a.icl == 4 && (a.stride_w & 1) == 0) walk(std::integral_constant<int, 0>{});
+  else if (a.icl == 4) walk(std::integral_constant<int, 1>{});
+  else walk(std::integral_constant<int, 2>{});
 }
 
 int conv_fewch_icl(int ic, int kw)
@@ -535,18 +614,22 @@ hipError_t plan_conv_fewch(LaunchPlan &plan, FewChArgs &a)
       const int nrows_in = (r - 1) * a.stride_h + a.kh;
       const size_t dyn = (size_t)nrows_in * a.lrow + 32;
       if (dyn > 40 * 1024) break;
-      // workgroups of 4 waves resident per CU: registers (3 waves per SIMD; 4 for the lean kernel with at most
-      // five operands, which stays below 128 registers), LDS (the general kernel's 16 KB static exchange patch +
-      // the rows).  3x3 s2 3 -> 32 at 224 x 224, N = 64: strips of 7 rows (4 workgroups per CU) 12.0 us, of 10 rows
+      // workgroups of 4 waves resident per CU: registers (3 waves per SIMD; the lean kernel 4 with two operands,
+      // 2 with seven), LDS (the general kernel's 16 KB static exchange patch + the rows).  3x3 s2 3 -> 32 at 224 x 224, N = 64: strips of 7 rows (4 workgroups per CU) 12.0 us, of 10 rows
       // (3 per CU) 12.6 us.
-      int resident = (a.lean && (a.cells + 1) / 2 <= 5) ? 4 : 3;
+      const int ks = (a.cells + 1) / 2;
+      int resident = !a.lean ? 3 : ks <= 2 ? 4 : ks <= 5 ? 3 : 2;
       const int by_lds = (int)((160 * 1024) / ((a.lean ? 0 : 16 * 1024) + dyn));
       if (by_lds < resident) resident = by_lds < 1 ? 1 : by_lds;
       const double slots = (double)n_cu * resident;
       const double wgs = (double)a.n * ((a.oh + r - 1) / r) * gy;
       const double rounds = (double)(long long)((wgs + slots - 1) / slots);
       const int tiles = (r * a.ow + 31) / 32;
-      const double cost = rounds * slots / wgs                                   // idle slots of the last round
+      // idle slots of the last round; with one round, idle CUs (the lean kernel keeps a CU almost as busy with two workgroups as with
+      // three: 5x5 s2 3 -> 96 at 224 x 224, N = 24: two of 16 rows 16.5 us, three of 12 18.6)
+      double idle = rounds * slots / wgs;
+      if (a.lean && rounds == 1.0 && wgs > n_cu && wgs <= 2.0 * n_cu && resident == 3) idle = 1.08 * 2.0 * n_cu / wgs;
+      const double cost = idle
           * ((tiles + wpn - 1) / wpn * wpn * 32.0 / (r * a.ow))                  // idle waves and lanes of the last tiles
           * ((double)((a.oh + r - 1) / r) * r / a.oh)                             // rows of the last strip below the image
           * (1.0 + 0.2 * nrows_in / (r * a.stride_h));                            // staging, relative to the tile work

@@ -492,6 +492,21 @@ def test_direct_few_input_channels_lean_kernel(lean_kernel, out_type, out_nhwc, 
         assert res["conv"].kernel_name == want
 
 
+@pytest.mark.parametrize("oc,rows", [(32, 1), (32, 9), (128, 1), (128, 4), (128, 5), (64, 8)])
+@pytest.mark.parametrize("ic,k,stride,in_z", [(3, 7, 2, 128.0), (3, 3, 1, 0.0), (4, 5, 1, 0.0), (1, 3, 2, 5.0)])
+def test_direct_few_input_channels_lean_walk(oc, rows, ic, k, stride, in_z, monkeypatch):
+    """waves that take no tile, one, an even and an odd number of them, where the next tile's matrix instructions run between the scaling of the last"""
+    monkeypatch.setenv("EHIP_FEWCH_ROWS", str(rows))
+    res = run_and_compare(Layer(1, ic, oc, 27 * stride, k=k, pad=k // 2, stride=stride, out_type=ol.S8, seed=290 + rows + k, in_z=in_z, in_nhwc=True))
+    assert res["conv"].kernel_name == "k_conv_fewch_lean"
+
+
+def test_direct_few_input_channels_tall_strip_of_cells(monkeypatch):
+    """blocked input whose strip is staged sixteen cells a thread at a time, the last batch in part"""
+    monkeypatch.setenv("EHIP_FEWCH_ROWS", "40")
+    run_and_compare(Layer(1, 3, 32, 100, k=3, pad=1, stride=1, out_type=ol.U8, seed=301))
+
+
 @pytest.mark.parametrize("rows", [1, 2, 3, 5, 16])
 def test_direct_few_input_channels_strip_heights(rows, monkeypatch):
     # output rows per workgroup, including strips that end below the image
