@@ -20,6 +20,7 @@ SOURCES = [
     "ehip_gemm1x1w.hip",
     "ehip_gemm1x1s.hip",
     "ehip_conv3x3v.hip",
+    "ehip_convs.hip",
     "ehip_fewch.hip",
     "ehip_depthwise.hip",
     "ehip_wino.hip",

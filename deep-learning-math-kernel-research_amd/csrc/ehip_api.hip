@@ -613,6 +613,24 @@ static int plan_execute(ehip_conv *c)
     a.vw = d.stride_h == 2 ? d.ow + 1 : d.ow + 2;
     a.vw_magic = div_magic(a.vw);
     a.trace = trace_buffer();
+    {
+      GemmArgs g;
+      memset(&g, 0, sizeof(g));
+      g.w = a.w;
+      g.ep = a.ep;
+      g.p_total = d.n * d.oh * d.ow;
+      g.ohw = d.oh * d.ow; g.ow = d.ow;
+      g.ohw_magic = div_magic(g.ohw); g.ow_magic = div_magic(g.ow);
+      g.ihw = d.ih * d.iw; g.ih = d.ih; g.iw = d.iw;
+      g.kh = d.kh; g.kw = d.kw; g.pad_t = d.pad_t; g.pad_l = d.pad_l;
+      g.stride_h = d.stride_h; g.stride_w = d.stride_w;
+      g.ic2 = c->ic2; g.units_pad = c->units_pad; g.oc2 = c->oc2; g.ocpp = c->ocpp;
+      const int form = conv_split_pick(g, 1, true);
+      if (form >= 0) {
+        HIP_TRY(plan_conv_split(*p, g, form, true));
+        break;
+      }
+    }
     HIP_TRY(plan_conv3x3v(*p, a, d.n, c->variant));
     break;
   }

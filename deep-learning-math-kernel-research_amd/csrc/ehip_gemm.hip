@@ -781,6 +781,10 @@ hipError_t plan_gemm(LaunchPlan &plan, const GemmArgs &a0, int nbatch, int varia
     const int rv = gemm1x1_res_pick(a0, nbatch);
     if (rv >= 0) return plan_gemm1x1_res(plan, a0, rv);
   }
+  {
+    const int form = conv_split_pick(a0, nbatch, false);
+    if (form >= 0) return plan_conv_split(plan, a0, form, false);
+  }
   const Variant &k = kVariants[variant];
   GemmArgs a = a0;
   a.lean = lean_mode(a.ep, false);   // blocked and nhwc output alike

@@ -254,6 +254,11 @@ hipError_t plan_gemm1x1_wres(LaunchPlan &plan, const GemmArgs &a);
 bool gemm1x1_split_applies(const GemmArgs &a, int nbatch);
 hipError_t plan_gemm1x1_split(LaunchPlan &plan, const GemmArgs &a);
 
+// k x k layers with few output values: K shared out among the waves of a workgroup (ehip_convs.hip); the form, or -1
+// (planes: a layer that the 3x3 kernel would run, with its weights)
+int conv_split_pick(const GemmArgs &a, int nbatch, bool planes);
+hipError_t plan_conv_split(LaunchPlan &plan, const GemmArgs &a, int form, bool planes);
+
 hipError_t plan_conv3x3v(LaunchPlan &plan, const Conv3x3Args &a, int n, int variant);
 int conv3x3v_pick_variant(int n, int oh, int ow, int oc2, int stride);   // stride 1 or 2 (both directions); -1: rows too wide for every variant
 int conv3x3v_chunk_units(int variant, int ic2);

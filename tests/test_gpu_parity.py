@@ -425,6 +425,33 @@ def test_direct_zero_point_with_padding(out_type, n, ic, oc, hw, k, pad, stride,
         assert res["conv"].kernel_name.startswith("k_conv_fewch" if ic <= 4 else "k_gemm_u8s8")
 
 
+# few output values: K shared out among the waves of a workgroup
+@pytest.mark.parametrize("form", ["0", "1", "2"])
+@pytest.mark.parametrize("out_type,nhwc,in_z", [(ol.U8, False, 0.0), (ol.S8, True, 0.0), (ol.F32, False, 128.0), (ol.S32, False, 0.0), (ol.F32, True, 0.0)])
+@pytest.mark.parametrize("n,ic,oc,hw,k,pad,stride,out_hw", [
+    (1, 16, 16, 8, 3, 1, 1, None),      # a unit a tap: fewer steps than waves and slots
+    (2, 48, 48, 11, 5, 2, 2, None),     # an odd count of units: the last half of a tap multiplies nothing
+    (3, 80, 80, 9, 7, 3, 1, None),      # channels and pixels that fill no tile
+    (1, 112, 144, 13, 3, 0, 2, 6),      # 3x3, stride 2, pads only right / bottom
+    (1, 512, 32, 7, 3, 1, 1, None),     # more steps than the ring, several rounds
+])
+def test_direct_k_shared_out(form, out_type, nhwc, in_z, n, ic, oc, hw, k, pad, stride, out_hw, monkeypatch):
+    monkeypatch.setenv("EHIP_CONV_SPLIT", form)
+    res = run_and_compare(Layer(n, ic, oc, hw, k=k, pad=pad, stride=stride, out_type=out_type, seed=240 + k + ic, out_hw=out_hw, in_z=in_z,
+                                in_nhwc=nhwc, out_nhwc=nhwc, with_relu=(out_type != ol.F32)))
+    assert "_split<%s" % ("32,32", "32,64", "64,64")[int(form)] in res["conv"].kernel_name
+
+
+@pytest.mark.parametrize("n,ic,oc,hw,k,stride,nhwc,split", [
+    (2, 64, 32, 14, 5, 1, False, "k_gemm_u8s8_split<32,32>"), (1, 32, 32, 14, 3, 1, True, ""), (8, 64, 64, 28, 5, 1, False, "k_gemm_u8s8_split<32,64>"),
+    (16, 64, 64, 28, 5, 1, False, "k_gemm_u8s8_split<64,64>"), (32, 64, 64, 28, 5, 1, False, ""),
+    (2, 256, 64, 14, 3, 1, False, "k_conv3x3v_u8s8_split<32,32>"), (2, 128, 64, 14, 3, 1, False, ""), (2, 256, 64, 14, 3, 2, False, "k_conv3x3v_u8s8_split<32,32,s2>"),
+    (10, 512, 256, 14, 3, 1, False, "k_conv3x3v_u8s8_split<32,64>"), (10, 256, 256, 14, 3, 1, False, "")])
+def test_direct_k_shared_out_choice(n, ic, oc, hw, k, stride, nhwc, split):
+    res = run_and_compare(Layer(n, ic, oc, hw, k=k, pad=k // 2, stride=stride, out_type=ol.S8, seed=250 + k + ic, in_nhwc=nhwc))
+    assert res["conv"].kernel_name == split if split else "_split" not in res["conv"].kernel_name
+
+
 # at most four input channels (first layers; the reference feeds them 3-channel nhwc,
 # scripts/best_configs/resnetv1_5-n64-clx-1s-int8.sh:12): 16 / ic pixels per operand cell, a kernel row
 # is ceil(kw / (16 / ic)) cells, input rows staged compactly in LDS
