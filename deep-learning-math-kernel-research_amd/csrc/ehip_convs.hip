@@ -22,7 +22,8 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void k_gemm_u8s8_split(const GemmA
 {
   GemmArgs a = load_args(rest);
   a.in = in; a.out = out;
-  constexpr int T = TM * TN, D = T == 1 ? 10 : (T == 2 ? 8 : 6);   // tiles; k-steps in flight
+  constexpr int T = TM * TN, D = T == 1 ? 10 : (T == 2 ? 8 : (T == 4 ? 6 : 3));   // tiles; k-steps in flight
+  constexpr int PW = T <= 4 ? NW : NW / 2;   // waves whose sums fit the LDS at once
   extern __shared__ v4i part[];        // [wave][tile][quarter of the 16 results][lane]
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -110,14 +111,33 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void k_gemm_u8s8_split(const GemmA
     }
   }
   // ---- the parts meet in LDS; a wave finishes a tile ------------------------------------------------------------------
+  auto leave = [&](int at) {
 #pragma unroll
-  for (int mt = 0; mt < TM; ++mt)
+    for (int mt = 0; mt < TM; ++mt)
 #pragma unroll
-    for (int nt = 0; nt < TN; ++nt)
+      for (int nt = 0; nt < TN; ++nt)
 #pragma unroll
-      for (int q = 0; q < 4; ++q)
-        part[((wave * T + mt * TN + nt) * 4 + q) * 64 + lane] =
-            v4i{acc[mt][nt][4 * q], acc[mt][nt][4 * q + 1], acc[mt][nt][4 * q + 2], acc[mt][nt][4 * q + 3]};
+        for (int q = 0; q < 4; ++q)
+          part[((at * T + mt * TN + nt) * 4 + q) * 64 + lane] =
+              v4i{acc[mt][nt][4 * q], acc[mt][nt][4 * q + 1], acc[mt][nt][4 * q + 2], acc[mt][nt][4 * q + 3]};
+  };
+  if constexpr (PW < NW) {             // the upper half's sums first, into the lower half's
+    if (wave >= PW) leave(wave - PW);
+    __syncthreads();
+    if (wave < PW)
+#pragma unroll
+      for (int mt = 0; mt < TM; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < TN; ++nt)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const v4i x = part[((wave * T + mt * TN + nt) * 4 + q) * 64 + lane];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc[mt][nt][4 * q + j] += x[j];
+          }
+    __syncthreads();
+    if (wave < PW) leave(wave);
+  } else leave(wave);
   __syncthreads();
   if (wave >= T) return;
   const int oc_real = a.oc2 * 16, oc = oc0 + 32 * (wave / TN) + 16 * lh, p0 = pix0 + 32 * (wave % TN);
@@ -128,7 +148,7 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void k_gemm_u8s8_split(const GemmA
   for (int q = 0; q < 4; ++q) {
     v4i s = k0.comp[q];
 #pragma unroll
-    for (int w = 0; w < NW; ++w) s += part[((w * T + wave) * 4 + q) * 64 + lane];
+    for (int w = 0; w < PW; ++w) s += part[((w * T + wave) * 4 + q) * 64 + lane];
 #pragma unroll
     for (int j = 0; j < 4; ++j) sum[0][0][4 * q + j] = s[j];
   }
@@ -159,7 +179,7 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void k_gemm_u8s8_split(const GemmA
                                   pixT, validT, cls);
 }
 
-// The form for a layer: 0, 1, 2 = 32 x 32, 32 x 64, 64 x 64 channels x pixels a workgroup, -1 = none.  The smallest whose workgroups have
+// The form for a layer: 0, 1, 2, 3, 4 = 32 x 32, 32 x 64, 64 x 64, 32 x 128, 64 x 128 channels x pixels a workgroup, -1 = none.  The smallest whose workgroups have
 // a CU of their own; a second round costs what the first did.  The kernel that ran before / the three forms, us, by units of 16
 // channels of all taps:
 //   instead of the general kernel (nhwc input, 5x5 or 7x7, zero points): 36 units 5.3 / 5.6 6.1 6.6 (98 workgroups of 32 x 32); 50 7.5 / 6.8 7.3 7.4 (98); 72 7.6 / 10.3 7.5 7.6
@@ -167,6 +187,9 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void k_gemm_u8s8_split(const GemmA
 //     20.0 10.7 (980), 14.4 / 37.5 35.6 19.7 (1568)
 //   instead of the 3x3 kernel: 72 units 4.7 / 5.3 6.0 6.4 (98); 144 6.7 / 5.3 7.3 7.7 (98), 5.8 / 9.3 7.4 7.7 (490), 8.2 / 17.2 13.5 8.1 (980); 288 15.8 / 7.2 8.7 9.0 (196), 10.0 / 11.5 8.9
 //     9.3 (490), 13.6 / 23.1 18.0 11.1 (980); stride 2, 288 13.1 / 6.5 9.0 9.4 (32), 15.1 / 29.1 25.5 15.6 (980)
+// and 32 x 128 and 64 x 128 with 31360 pixels, 32 and 64 channels: the general kernel 72 units 9.1 / 10.0, 9.2 / 11.7; 100 12.4 / 10.2, 12.5 / 11.2; 3x3, 144 14.5 / 15.1,
+// 15.3 / 16.3; 7x7, 196 21.6 / 12.9, 21.9 / 15.0; 5x5, 200 20.1 / 18.0, 20.5 / 19.9; the 3x3 kernel 144 8.8 / 9.9, 14.0 / 11.4 (7840 and 256 channels 11.1 / 11.3); 288
+// 16.2 / 13.3, 26.7 / 16.6.
 int conv_split_pick(const GemmArgs &a, int nbatch, bool planes)
 {
   const int taps = a.kh * a.kw;
@@ -174,7 +197,7 @@ int conv_split_pick(const GemmArgs &a, int nbatch, bool planes)
   if (planes && (a.pad_t > 255 || a.pad_l > 255)) return -1;   // (what the 3x3 kernel refuses)
   const long long in_bytes = (long long)(a.p_total / a.ohw) * a.ic2 * a.ihw * 16, w_bytes = (long long)taps * a.units_pad * a.ocpp * 16;
   if (in_bytes > 0x7fffffffll || w_bytes > 0x7fffffffll) return -1;
-  if (const char *env = getenv("EHIP_CONV_SPLIT")) return env[0] >= '0' && env[0] <= '2' ? env[0] - '0' : -1;
+  if (const char *env = getenv("EHIP_CONV_SPLIT")) return env[0] >= '0' && env[0] <= '4' ? env[0] - '0' : -1;
   // (another kernel asked for)
   for (const char *other : {"EHIP_GEMM_VARIANT", "EHIP_GEMM_SMALLK", "EHIP_CONV3X3V_VARIANT", "EHIP_CONV3X3V_UNROLL", "EHIP_CONV3X3V_SPLIT_LAST",
                             "EHIP_CONV3X3V_SHARED"})
@@ -183,25 +206,30 @@ int conv_split_pick(const GemmArgs &a, int nbatch, bool planes)
   const long long px32 = (a.p_total + 31) / 32, px64 = (a.p_total + 63) / 64, oc32 = (a.oc2 + 1) / 2, oc64 = (a.oc2 + 3) / 4;
   if (px32 * oc32 <= 256) return units >= (planes ? 128 : 40) ? 0 : -1;
   if (px64 * oc32 <= 256) return units >= (planes ? 216 : 64) ? 1 : -1;
-  if (px64 * oc64 <= 256) return units >= (planes ? 216 : 96) && !(planes && a.stride_h > 1) ? 2 : -1;
-  return -1;
+  if (planes && a.stride_h > 1) return -1;
+  const long long px128 = (a.p_total + 127) / 128;
+  if (units < (planes ? 216 : 96)) return -1;
+  if (px64 * oc64 <= 256) return 2;
+  if (px128 * oc32 <= 256) return 3;
+  return px128 * oc64 <= 256 && (planes || taps > 9) ? 4 : -1;
 }
 
 hipError_t plan_conv_split(LaunchPlan &plan, const GemmArgs &a0, int form, bool planes)
 {
   GemmArgs a = a0;
   a.k_real = a.kh * a.kw * a.units_pad;
-  const int tm = form == 2 ? 2 : 1, tn = form >= 1 ? 2 : 1;
+  const int tm = form == 2 || form == 4 ? 2 : 1, tn = form >= 3 ? 4 : (form >= 1 ? 2 : 1);
   a.nx = (a.p_total + 32 * tn - 1) / (32 * tn);
   a.ny = (a.oc2 * 16 + 32 * tm - 1) / (32 * tm);
   void (*kernel)(const GemmArgs *, const uint8_t *, void *) =
-      form == 0 ? k_gemm_u8s8_split<1, 1, 8> : form == 1 ? k_gemm_u8s8_split<1, 2, 8> : k_gemm_u8s8_split<2, 2, 8>;
+      form == 0 ? k_gemm_u8s8_split<1, 1, 8> : form == 1 ? k_gemm_u8s8_split<1, 2, 8> : form == 2 ? k_gemm_u8s8_split<2, 2, 8> :
+      form == 3 ? k_gemm_u8s8_split<1, 4, 8> : k_gemm_u8s8_split<2, 4, 8>;
   // (channels, pixels of a workgroup)
-  static const char *const names[][3] = {{"k_gemm_u8s8_split<32,32>", "k_gemm_u8s8_split<32,64>", "k_gemm_u8s8_split<64,64>"},
-                                         {"k_conv3x3v_u8s8_split<32,32>", "k_conv3x3v_u8s8_split<32,64>", "k_conv3x3v_u8s8_split<64,64>"},
-                                         {"k_conv3x3v_u8s8_split<32,32,s2>", "k_conv3x3v_u8s8_split<32,64,s2>", "k_conv3x3v_u8s8_split<64,64,s2>"}};
+  static const char *const names[][5] = {{"k_gemm_u8s8_split<32,32>", "k_gemm_u8s8_split<32,64>", "k_gemm_u8s8_split<64,64>", "k_gemm_u8s8_split<32,128>", "k_gemm_u8s8_split<64,128>"},
+                                         {"k_conv3x3v_u8s8_split<32,32>", "k_conv3x3v_u8s8_split<32,64>", "k_conv3x3v_u8s8_split<64,64>", "k_conv3x3v_u8s8_split<32,128>", "k_conv3x3v_u8s8_split<64,128>"},
+                                         {"k_conv3x3v_u8s8_split<32,32,s2>", "k_conv3x3v_u8s8_split<32,64,s2>", "k_conv3x3v_u8s8_split<64,64,s2>", "k_conv3x3v_u8s8_split<32,128,s2>", "k_conv3x3v_u8s8_split<64,128,s2>"}};
   plan.name = names[planes ? a.stride_h : 0][form];
-  return plan_set(plan, kernel, dim3((unsigned)(a.nx * a.ny)), dim3(512), (size_t)8 * tm * tn * 4096, a, ArgBlock{}, ArgIn{a.in}, ArgOut{a.out});
+  return plan_set(plan, kernel, dim3((unsigned)(a.nx * a.ny)), dim3(512), (size_t)(tm * tn > 4 ? 4 : 8) * tm * tn * 4096, a, ArgBlock{}, ArgIn{a.in}, ArgOut{a.out});
 }
 
 }  // namespace ehip

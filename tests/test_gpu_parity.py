@@ -426,7 +426,7 @@ def test_direct_zero_point_with_padding(out_type, n, ic, oc, hw, k, pad, stride,
 
 
 # few output values: K shared out among the waves of a workgroup
-@pytest.mark.parametrize("form", ["0", "1", "2"])
+@pytest.mark.parametrize("form", ["0", "1", "2", "3", "4"])
 @pytest.mark.parametrize("out_type,nhwc,in_z", [(ol.U8, False, 0.0), (ol.S8, True, 0.0), (ol.F32, False, 128.0), (ol.S32, False, 0.0), (ol.F32, True, 0.0)])
 @pytest.mark.parametrize("n,ic,oc,hw,k,pad,stride,out_hw", [
     (1, 16, 16, 8, 3, 1, 1, None),      # a unit a tap: fewer steps than waves and slots
@@ -439,12 +439,13 @@ def test_direct_k_shared_out(form, out_type, nhwc, in_z, n, ic, oc, hw, k, pad, 
     monkeypatch.setenv("EHIP_CONV_SPLIT", form)
     res = run_and_compare(Layer(n, ic, oc, hw, k=k, pad=pad, stride=stride, out_type=out_type, seed=240 + k + ic, out_hw=out_hw, in_z=in_z,
                                 in_nhwc=nhwc, out_nhwc=nhwc, with_relu=(out_type != ol.F32)))
-    assert "_split<%s" % ("32,32", "32,64", "64,64")[int(form)] in res["conv"].kernel_name
+    assert "_split<%s" % ("32,32", "32,64", "64,64", "32,128", "64,128")[int(form)] in res["conv"].kernel_name
 
 
 @pytest.mark.parametrize("n,ic,oc,hw,k,stride,nhwc,split", [
     (2, 64, 32, 14, 5, 1, False, "k_gemm_u8s8_split<32,32>"), (1, 32, 32, 14, 3, 1, True, ""), (8, 64, 64, 28, 5, 1, False, "k_gemm_u8s8_split<32,64>"),
-    (16, 64, 64, 28, 5, 1, False, "k_gemm_u8s8_split<64,64>"), (32, 64, 64, 28, 5, 1, False, ""),
+    (16, 64, 64, 28, 5, 1, False, "k_gemm_u8s8_split<64,64>"), (32, 64, 64, 28, 5, 1, False, "k_gemm_u8s8_split<64,128>"), (64, 64, 64, 28, 5, 1, False, ""),
+    (32, 64, 32, 28, 5, 1, False, "k_gemm_u8s8_split<32,128>"),
     (2, 256, 64, 14, 3, 1, False, "k_conv3x3v_u8s8_split<32,32>"), (2, 128, 64, 14, 3, 1, False, ""), (2, 256, 64, 14, 3, 2, False, "k_conv3x3v_u8s8_split<32,32,s2>"),
     (10, 512, 256, 14, 3, 1, False, "k_conv3x3v_u8s8_split<32,64>"), (10, 256, 256, 14, 3, 1, False, "")])
 def test_direct_k_shared_out_choice(n, ic, oc, hw, k, stride, nhwc, split):
