@@ -145,7 +145,8 @@ EHIP_API int ehip_conv_execute_stages(ehip_conv_t *conv, void *output_dev, const
 EHIP_API int ehip_conv_query(ehip_conv_t *conv, int what, void *host_dst, size_t *bytes);
 
 /* Name of the kernel variant execute() launches (for profiles), and its launch geometry.  Where the launcher chooses
- * between forms of a kernel (epilogue forms, the fused Winograd stage), the name is final once the handle is prepared. */
+ * between forms of a kernel (epilogue forms, the fused Winograd stage), the name is final once the handle is prepared.
+ * A Winograd layer that execute() runs in one launch reads "k_wino_whole | " and then the stages of ehip_conv_execute_stages. */
 EHIP_API const char *ehip_conv_kernel_name(ehip_conv_t *conv);
 
 /* Replaces the harness-side fp32 -> u8 activation quantization
