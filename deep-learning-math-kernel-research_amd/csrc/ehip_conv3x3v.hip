@@ -97,7 +97,7 @@ __device__ __forceinline__ void conv3x3v_body(const Conv3x3Args &a)
 
   // KS = 2: eight waves, of which the upper four do what the lower four do with every other fill
   const int half = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / kBlock);
-  const int tid = threadIdx.x % kBlock;
+  const int tid = KS == 1 ? threadIdx.x : threadIdx.x % kBlock;
   v4i *lds = lds_all + (KS == 1 ? 0 : half * a.chunk_units * STRIDE);
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform: what depends on it stays scalar
@@ -452,7 +452,7 @@ __device__ __forceinline__ void conv3x3v_body(const Conv3x3Args &a)
       for (int st = LAST0; st < 9 * PAIRS; ++st)
         tap_mfmas(st & 1, st % 9, PAIRS - 1, true, st + 1 < 9 * PAIRS ? PAIRS - 1 : -1, (st + 1) % 9);
     }
-  } else if (KS == 2) {
+  } else if constexpr (KS == 2) {
     // fill 2 i + half in step i; (an odd count of fills: the upper half skips the last step's work, not its barriers)
     const int steps = (nchunks + 1) / 2;
     for (int i = 0; i < steps; ++i) {
