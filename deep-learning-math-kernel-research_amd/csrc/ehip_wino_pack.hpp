@@ -16,8 +16,8 @@ namespace {
 // packed into the pixels' dwords as they come (16 dwords live instead of 4 x 16 floats; the old output of the in-place
 // sum stays packed as well).  Same operations in the same order per value as output_tile.
 // pack_channel: channel k of the lane's four -- bias, output scale, old output, ReLU, rounding, byte k of the dwords.
-// (E: pixels, the tile's or one row of it)
-template <int OUT, int A, int E = (A - 2) * (A - 2)>
+// (E: pixels, the tile's or one row of it; CLAMP: both bounds of the ReLU explicitly, see below)
+template <int OUT, int A, int E = (A - 2) * (A - 2), bool CLAMP = false>
 __device__ __forceinline__ void pack_channel(const float *o, float b, int k, bool with_relu, float repS, float z, bool with_sum,
                                              const unsigned *old, unsigned *pk)
 {
@@ -31,8 +31,10 @@ __device__ __forceinline__ void pack_channel(const float *o, float b, int k, boo
       r = r + (OUT == EHIP_U8 ? (float)ob : (float)(int)(signed char)ob);
     }
     if (with_relu) {
-      // (v_cvt_pk_u8_f32 itself clamps to 0..255 and makes a NaN 0, all that the ReLU asks for of a u8 code; s8 has its own bound)
-      if (OUT == EHIP_S8) r = __builtin_amdgcn_fmed3f(r, 0.0f, 127.0f);
+      // (v_cvt_pk_u8_f32 itself clamps to 0..255 and makes a NaN 0, all that the ReLU asks for of a u8 code; s8 has its own
+      // bound.  The ring kernel keeps both: it has no registers to spare, and without this instruction in the u8 branch the compiler
+      // places the values of all branches otherwise, 25 instead of 15 of them in scratch memory with 64 channels x 64 tiles)
+      if (OUT == EHIP_S8 || CLAMP) r = __builtin_amdgcn_fmed3f(r, 0.0f, OUT == EHIP_S8 ? 127.0f : 255.0f);
       if (A == 4) r = __builtin_floorf(r);
       pk[e] = __builtin_amdgcn_cvt_pk_u8_f32(r, k, pk[e]);
     } else if (A == 4) {

@@ -393,7 +393,7 @@ __global__ __launch_bounds__(64 * WO * WT, 2) void k_wino_gemm_output_lanes_ring
             for (int k = 0; k < 4; ++k) {
               float y[M * M];
               value(k, y);
-              pack_channel<OUT, A>(y, comp_of(bias, k), k, RELU, a.out_repS, a.out_z, SUM, old, pk);
+              pack_channel<OUT, A, (A - 2) * (A - 2), true>(y, comp_of(bias, k), k, RELU, a.out_repS, a.out_z, SUM, old, pk);
 #pragma unroll
               for (int q = 0; q < M * M; ++q) asm volatile("" : "+v"(pk[q]));
               __builtin_amdgcn_sched_barrier(0);
