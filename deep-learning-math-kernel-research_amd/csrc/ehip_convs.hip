@@ -4,6 +4,7 @@
 // Replaces, for those layers, elx_int8_conv_direct_t::conv_a160 + gemm_a160 and the u8s8 GEMM micro-kernel
 // (src/elx_int8_conv_direct.cpp:227-423, src/kernel/elk_u8s8_gemm.hxx:66-406).
 #include "ehip_internal.hpp"
+#include "ehip_convs_at.hpp"
 #include "ehip_wino_input.hpp"
 
 namespace ehip {
@@ -31,7 +32,7 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void k_gemm_u8s8_split(const GemmA
   const int bx = blockIdx.x / a.ny, oc0 = (blockIdx.x - bx * a.ny) * 32 * TM;
   const int pix0 = bx * 32 * TN;
   // ---- the lane's pixels: input row and column of the first tap, byte of the image and unit -----------------------
-  const unsigned pxs = a.in_nhwc ? (unsigned)a.ic2 * 16u : 16u, us = a.in_nhwc ? 16u : (unsigned)a.ihw * 16u;
+  const SplitStrides strides = split_strides(a.in_nhwc != 0, a.ic2, a.ihw);
   int ihb[TN], iwb[TN];
   unsigned base[TN];
 #pragma unroll
@@ -42,18 +43,14 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void k_gemm_u8s8_split(const GemmA
     const int r = gp - n * a.ohw, oh = fastdiv(r, a.ow, a.ow_magic);
     ihb[nt] = oh * a.stride_h - a.pad_t;
     iwb[nt] = (r - oh * a.ow) * a.stride_w - a.pad_l;
-    base[nt] = (unsigned)n * a.ic2 * a.ihw * 16u + lh * us;
+    base[nt] = split_image(strides, n, lh, a.ic2, a.ihw);
   }
   const int images = (a.p_total + a.ohw - 1) / a.ohw;
   const BufferRsrc rin = make_rsrc(a.in, (unsigned)images * a.ic2 * a.ihw * 16u);
   const BufferRsrc rw = make_rsrc(a.w, (unsigned)a.k_real * a.ocpp * 16u);
-  unsigned aoff[TM], aoff_tail[TM];    // (of an odd count's last unit: the second half multiplies nothing)
-  const bool odd = (a.ic2 & 1) != 0;
+  unsigned aoff[TM];
 #pragma unroll
-  for (int mt = 0; mt < TM; ++mt) {
-    aoff[mt] = (unsigned)(lh * a.ocpp + oc0 + 32 * mt + l32) * 16u;
-    aoff_tail[mt] = odd && lh ? 0x80000000u : aoff[mt];
-  }
+  for (int mt = 0; mt < TM; ++mt) aoff[mt] = (unsigned)(lh * a.ocpp + oc0 + 32 * mt + l32) * 16u;
   // ---- the wave's k-steps: pairs of units, tap by tap ---------------------------------------------------------------
   const int P = (a.ic2 + 1) >> 1, S = a.kh * a.kw * P;
   const int s0 = S * wave / NW, s1 = S * (wave + 1) / NW;
@@ -62,21 +59,18 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void k_gemm_u8s8_split(const GemmA
   auto at_tap = [&]() {
     const int kr = tap / a.kw, kc = tap - kr * a.kw;
 #pragma unroll
-    for (int nt = 0; nt < TN; ++nt) {
-      const int ih = ihb[nt] + kr, iw = iwb[nt] + kc;
-      const bool inside = (unsigned)ih < (unsigned)a.ih && (unsigned)iw < (unsigned)a.iw;
-      voff[nt] = inside ? base[nt] + (unsigned)(ih * a.iw + iw) * pxs : 0x80000000u;   // (outside: past the buffer, code 0)
-    }
+    for (int nt = 0; nt < TN; ++nt) voff[nt] = split_tap(strides, base[nt], ihb[nt] + kr, iwb[nt] + kc, a.ih, a.iw);
   };
   at_tap();
   v4i ra[D][TM], rb[D][TN];
   auto issue = [&](int slot) {
-    const bool live = si < s1, tail = pr == P - 1;
-    const unsigned wat = (unsigned)(tap * a.units_pad + 2 * pr) * (unsigned)a.ocpp * 16u, iat = (unsigned)(2 * pr) * us;   // scalar
+    const bool live = si < s1;
+    const int units = live ? a.ic2 : 0;   // (past the last step every lane is past the buffers)
+    const unsigned wat = (unsigned)(tap * a.units_pad + 2 * pr) * (unsigned)a.ocpp * 16u, iat = split_step(strides, pr);   // scalar
 #pragma unroll
-    for (int mt = 0; mt < TM; ++mt) buffer_load_cell(rw, live ? (tail ? aoff_tail[mt] : aoff[mt]) : 0x80000000u, live ? wat : 0u, ra[slot][mt]);
+    for (int mt = 0; mt < TM; ++mt) buffer_load_cell(rw, split_lane(aoff[mt], pr, lh, units), live ? wat : 0u, ra[slot][mt]);
 #pragma unroll
-    for (int nt = 0; nt < TN; ++nt) buffer_load_cell(rin, live ? voff[nt] : 0x80000000u, live ? iat : 0u, rb[slot][nt]);
+    for (int nt = 0; nt < TN; ++nt) buffer_load_cell(rin, split_lane(voff[nt], pr, lh, units), live ? iat : 0u, rb[slot][nt]);
     ++si;
     if (++pr == P) {
       pr = 0;
