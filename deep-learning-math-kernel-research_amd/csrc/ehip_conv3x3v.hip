@@ -90,7 +90,7 @@ __device__ __forceinline__ void conv3x3v_body(const Conv3x3Args &a)
   constexpr int G = kBlock / CT;       // thread groups that split the units of a fill
   static_assert(WM * WN == 4, "four waves per workgroup");
   static_assert(kBlock % CT == 0, "cells per pass");
-  extern __shared__ v4i lds_all[];     // [KS][chunk_units][STRIDE]
+  extern __shared__ v4i lds[];         // [KS][chunk_units][STRIDE]
 #ifdef EHIP_TRACE
   const long long t_entry = wall_clock64();
 #endif
@@ -98,7 +98,9 @@ __device__ __forceinline__ void conv3x3v_body(const Conv3x3Args &a)
   // KS = 2: eight waves, of which the upper four do what the lower four do with every other fill
   const int half = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / kBlock);
   const int tid = KS == 1 ? threadIdx.x : threadIdx.x % kBlock;
-  v4i *lds = lds_all + (KS == 1 ? 0 : half * a.chunk_units * STRIDE);
+  // (an offset and not a pointer: KS = 1 has to index `lds` itself, whose address the compiler folds into its reads and writes; behind
+  // a pointer all of that form's kernels came out otherwise, 64 -> 64 at 14 x 14, stride 2, 3.9 -> 4.05 us)
+  const int half_at = KS == 1 ? 0 : half * a.chunk_units * STRIDE;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform: what depends on it stays scalar
   const int l32 = lane & 31;
@@ -192,7 +194,7 @@ __device__ __forceinline__ void conv3x3v_body(const Conv3x3Args &a)
           if (k0 + j < nk) {
             const v4i x = t[j] ^ (int)0x80808080;
             const v4i z = {(int)0x80808080, (int)0x80808080, (int)0x80808080, (int)0x80808080};
-            lds[(ug + G * (k0 + j)) * STRIDE + slot(tid % CT + p * CT)] = gin[p] ? x : z;
+            lds[half_at + (ug + G * (k0 + j)) * STRIDE + slot(tid % CT + p * CT)] = gin[p] ? x : z;
           }
         }
       }
@@ -226,7 +228,7 @@ __device__ __forceinline__ void conv3x3v_body(const Conv3x3Args &a)
           if (k0 + j < nk) {
             const v4i x = t[p][j] ^ (int)0x80808080;
             const v4i z = {(int)0x80808080, (int)0x80808080, (int)0x80808080, (int)0x80808080};
-            lds[(ug + G * (k0 + j)) * STRIDE + slot(tid % CT + p * CT)] = gin[p] ? x : z;
+            lds[half_at + (ug + G * (k0 + j)) * STRIDE + slot(tid % CT + p * CT)] = gin[p] ? x : z;
           }
         }
     }
@@ -242,7 +244,7 @@ __device__ __forceinline__ void conv3x3v_body(const Conv3x3Args &a)
   // tap's last MFMA by the weight request for the next channel pair; sched_barrier pins that order.
   v4i bq[2][TN];
   auto read_b = [&](int par, int pl, int tap, int nt) {
-    const v4i *tile = lds + (2 * pl + lh) * STRIDE + pw0 + l32;
+    const v4i *tile = lds + half_at + (2 * pl + lh) * STRIDE + pw0 + l32;
     const int kh = tap / 3, kw = tap % 3;
     bq[par][nt] = tile[nt * 32 + (S == 2 ? ((kh & 1) * 2 + (kw & 1)) * PS + (kh >> 1) * VW + (kw >> 1) : kh * VW + kw)];
   };
@@ -282,7 +284,7 @@ __device__ __forceinline__ void conv3x3v_body(const Conv3x3Args &a)
   v4i q[2][TN + 2];
   // operands of kernel row kh of the pair staged at pl, into buffer par
   auto load_q = [&](int par, int pl, int kh) {
-    const v4i *ub = lds + (2 * pl + lh) * STRIDE + l32;
+    const v4i *ub = lds + half_at + (2 * pl + lh) * STRIDE + l32;
 #pragma unroll
     for (int o = 0; o < TN + 2; ++o) q[par][o] = ub[soff[kh][o]];
   };
@@ -300,7 +302,7 @@ __device__ __forceinline__ void conv3x3v_body(const Conv3x3Args &a)
           acc[mt][nt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a_reg[tap][mt], q[par][nt + kw], acc[mt][nt], 0, 0, 0);
           __builtin_amdgcn_sched_barrier(0);
           if (next_pl >= 0 && issued < TN + 2) {
-            const v4i *ub = lds + (2 * next_pl + lh) * STRIDE + l32;
+            const v4i *ub = lds + half_at + (2 * next_pl + lh) * STRIDE + l32;
             q[par ^ 1][issued] = ub[soff[next_kh][issued]];
             ++issued;
           }
@@ -472,7 +474,7 @@ __device__ __forceinline__ void conv3x3v_body(const Conv3x3Args &a)
     }
     // the upper half's sums through LDS
     __syncthreads();
-    v4i *sums = lds_all;
+    v4i *sums = lds;
     if (half) {
 #pragma unroll
       for (int mt = 0; mt < TM; ++mt)
