@@ -625,7 +625,8 @@ static int plan_execute(ehip_conv *c)
       g.kh = d.kh; g.kw = d.kw; g.pad_t = d.pad_t; g.pad_l = d.pad_l;
       g.stride_h = d.stride_h; g.stride_w = d.stride_w;
       g.ic2 = c->ic2; g.units_pad = c->units_pad; g.oc2 = c->oc2; g.ocpp = c->ocpp;
-      const int form = conv_split_pick(g, 1, true);
+      const Conv3x3Tiles tiles = conv3x3v_tiles(c->variant, d.n, d.oh, d.ow, c->oc2, d.stride_h);
+      const int form = conv_split_pick(g, 1, &tiles);
       if (form >= 0) {
         HIP_TRY(plan_conv_split(*p, g, form, true));
         break;

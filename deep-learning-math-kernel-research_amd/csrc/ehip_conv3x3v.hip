@@ -585,41 +585,42 @@ struct Variant {
   conv3x3v_kernel_t split[3];      // the same with the last pair split (lean epilogue without the sum), or null
   int stride;                      // 1, or 2: the staged unit is four phase planes of cells / 4 cells each
   conv3x3v_kernel_t shared;        // eight waves that share the input channels out, or null
+  int wm;                          // waves beside each other along the channels
 };
 #define V(WM, WN, TM, TN, CT, NPASS)                                                              \
   { "k_conv3x3v_u8s8<" #WM "," #WN "," #TM "," #TN "," #CT "," #NPASS ">", WM * TM * 32, WN * TN * 32, \
-    CT * NPASS, CT * NPASS, k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS>, {nullptr, nullptr, nullptr}, {nullptr, nullptr, nullptr}, 1, nullptr }
+    CT * NPASS, CT * NPASS, k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS>, {nullptr, nullptr, nullptr}, {nullptr, nullptr, nullptr}, 1, nullptr, WM }
 #define VU(WM, WN, TM, TN, CT, NPASS)                                                             \
   { "k_conv3x3v_u8s8<" #WM "," #WN "," #TM "," #TN "," #CT "," #NPASS ">", WM * TM * 32, WN * TN * 32, \
     CT * NPASS, CT * NPASS, k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS>,                            \
     {k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 2>, k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 4>,  \
-     k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 8>}, {nullptr, nullptr, nullptr}, 1, nullptr }
+     k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 8>}, {nullptr, nullptr, nullptr}, 1, nullptr, WM }
 #define VU2(WM, WN, TM, TN, CT, NPASS) /* straight-line form for two unit pairs only (64 input channels) */ \
   { "k_conv3x3v_u8s8<" #WM "," #WN "," #TM "," #TN "," #CT "," #NPASS ">", WM * TM * 32, WN * TN * 32, \
     CT * NPASS, CT * NPASS, k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS>,                            \
-    {k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 2>, nullptr, nullptr}, {nullptr, nullptr, nullptr}, 1, nullptr }
+    {k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 2>, nullptr, nullptr}, {nullptr, nullptr, nullptr}, 1, nullptr, WM }
 #define VK(WM, WN, TM, TN, CT, NPASS)                                                             \
   { "k_conv3x3v_u8s8<" #WM "," #WN "," #TM "," #TN "," #CT "," #NPASS ">", WM * TM * 32, WN * TN * 32, \
     CT * NPASS, CT * NPASS, k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS>,                            \
     {k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 2>, k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 4>,  \
      k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 8>},                                               \
     {k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 2, false, true>, k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 4, false, true>, \
-     k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 8, false, true>}, 1, nullptr }
+     k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 8, false, true>}, 1, nullptr, WM }
 #define V2(WM, WN, TM, TN, CT, NPASS) /* stride 2; straight-line forms for two and four unit pairs */ \
   { "k_conv3x3v_u8s8<" #WM "," #WN "," #TM "," #TN "," #CT "," #NPASS ",s2>", WM * TM * 32, WN * TN * 32, \
     CT * NPASS, CT * NPASS, k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 0, false, false, 2>,       \
     {k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 2, false, false, 2>, k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 4, false, false, 2>, \
-     nullptr}, {nullptr, nullptr, nullptr}, 2, nullptr }
+     nullptr}, {nullptr, nullptr, nullptr}, 2, nullptr, WM }
 #define V2K(WM, WN, TM, TN, CT, NPASS) /* and the form that shares the input channels out */ \
   { "k_conv3x3v_u8s8<" #WM "," #WN "," #TM "," #TN "," #CT "," #NPASS ",s2>", WM * TM * 32, WN * TN * 32, \
     CT * NPASS, CT * NPASS, k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 0, false, false, 2>,       \
     {k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 2, false, false, 2>, k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 4, false, false, 2>, \
-     nullptr}, {nullptr, nullptr, nullptr}, 2, k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 0, false, false, 2, 2> }
+     nullptr}, {nullptr, nullptr, nullptr}, 2, k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 0, false, false, 2, 2>, WM }
 #define VS(WM, WN, TM, TN, CT, NPASS)                                                             \
   { "k_conv3x3v_u8s8<" #WM "," #WN "," #TM "," #TN "," #CT "," #NPASS ",sp>", WM * TM * 32, WN * TN * 32, \
     CT * NPASS, conv3x3v_unit_stride(CT * NPASS, TN, true), k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 0, true>, \
     {k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 2, true>, k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 4, true>, \
-     k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 8, true>}, {nullptr, nullptr, nullptr}, 1, nullptr }
+     k_conv3x3v_u8s8<WM, WN, TM, TN, CT, NPASS, 8, true>}, {nullptr, nullptr, nullptr}, 1, nullptr, WM }
 const Variant kVariants[] = {
     V(2, 2, 2, 1, 128, 1),  // 0: 128 oc x  64 px, rows up to  31 cells
     V(2, 2, 2, 1, 256, 1),  // 1: 128 oc x  64 px, rows up to  95 cells
@@ -664,6 +665,13 @@ bool conv3x3v_fits(int v, int ow, int stride)
   if (kVariants[v].stride != stride) return false;
   if (stride == 2) return kVariants[v].p_t + (ow + 1) + 2 <= kVariants[v].cells / 4;   // a phase plane: tile + a row + a cell
   return kVariants[v].p_t + 2 * (ow + 2) + 2 <= kVariants[v].cells;
+}
+
+Conv3x3Tiles conv3x3v_tiles(int v, int n, int oh, int ow, int oc2, int stride)
+{
+  const Variant &k = kVariants[v];
+  const int vw = stride == 2 ? ow + 1 : ow + 2;
+  return Conv3x3Tiles{(long long)((oh * vw + k.p_t - 1) / k.p_t) * ((oc2 * 16 + k.oc_t - 1) / k.oc_t) * n, k.oc_t, k.wm == 4 || k.wm == 1};
 }
 
 // units of 16 input channels staged per LDS fill: all of them if they fit the budget

@@ -184,7 +184,20 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void k_gemm_u8s8_split(const GemmA
 // and 32 x 128 and 64 x 128 with 31360 pixels, 32 and 64 channels: the general kernel 72 units 9.1 / 10.0, 9.2 / 11.7; 100 12.4 / 10.2, 12.5 / 11.2; 3x3, 144 14.5 / 15.1,
 // 15.3 / 16.3; 7x7, 196 21.6 / 12.9, 21.9 / 15.0; 5x5, 200 20.1 / 18.0, 20.5 / 19.9; the 3x3 kernel 144 8.8 / 9.9, 14.0 / 11.4 (7840 and 256 channels 11.1 / 11.3); 288
 // 16.2 / 13.3, 26.7 / 16.6.
-int conv_split_pick(const GemmArgs &a, int nbatch, bool planes)
+// (50 units, blocked input: 7.0 / 7.1 and 7.2 with 98 to 245 workgroups, hence 64 there.)
+// The 3x3 kernel, stride 1, is at its best where its workgroups come to one round, no wave is without channels or shares its own
+// with another, and one fill of the LDS holds all input channels (up to 512: 288 units).  There it takes less for more pixels, because it
+// reads them once for 128 channels, where a workgroup here has 32 or 64.  427 layers of 128 to 1024 input channels, 3x3 kernel / the form:
+//   32 x 64, 288 units, more than 2048 pixels: 9.8 / 9.7 to 10.4 (up to 2048: 9.7 to 10.7 / 8.7 to 9.1; 216 units 8.1 to 8.3 / 7.5 to 8.0);
+//   64 x 64: 216 units 8.1 to 8.8 / 9.1 to 10.1; 288 units, more than 2048 pixels 10.0 to 10.8 / 10.4 to 10.8 (up to 2048: 9.9 to 10.7 / 9.2 to 9.5);
+//   32 x 128, 32 channels: 216 units 11.3 to 12.0 / 11.5 to 11.9; 288 units 12.9 / 12.9 to 13.5;
+//   64 x 128: 512 -> 512 at 7 x 7, N = 64 11.6 to 14.1 / 15.4 (it moves with the box and its clock, this kernel does not); 384 -> 512 there
+//     9.3 to 10.9 / 13.3; 768 21.1 to 24.6 / 19.3 to 19.6, 1024 21.8 to 25.3 / 23.5.
+// Two rounds of it still beat 32 x 128 and 64 x 128 (216 units 10.9 to 13.4 / 12.3 to 13.3, 288 14.2 to 17.1 / 14.9 to 15.7), not 64 x 64 (13.8 /
+// 11.0); nor do three (384 -> 192 at 14 x 14, N = 48, 18.8 / 14.8; 512 -> 512 at 14 x 14, N = 20 22.5 to 23.7 / 15.7 to 17.6).  With more
+// channels it fills twice (432 units, one round: 18.0 / 11.8 to 15.0), with half of the waves idle (64 channels) it takes 15 to 19 us for 10
+// to 16, with wide rows 14 to 17 for 8 to 16.
+int conv_split_pick(const GemmArgs &a, int nbatch, const Conv3x3Tiles *planes)
 {
   const int taps = a.kh * a.kw;
   if (nbatch != 1 || taps <= 1 || taps > 64 || a.ep.with_sum) return -1;
@@ -198,14 +211,20 @@ int conv_split_pick(const GemmArgs &a, int nbatch, bool planes)
     if (const char *env = getenv(other)) if (env[0]) return -1;
   const int units = taps * a.ic2;
   const long long px32 = (a.p_total + 31) / 32, px64 = (a.p_total + 63) / 64, oc32 = (a.oc2 + 1) / 2, oc64 = (a.oc2 + 3) / 4;
-  if (px32 * oc32 <= 256) return units >= (planes ? 128 : 40) ? 0 : -1;
-  if (px64 * oc32 <= 256) return units >= (planes ? 216 : 64) ? 1 : -1;
+  const bool apart = planes && a.stride_h == 1 && planes->apart && 32 * a.oc2 > planes->channels, best = apart && units <= 288;   // (see above)
+  const bool one = best && planes->count <= 256;
+  if (px32 * oc32 <= 256) return units >= (planes ? 128 : a.in_nhwc ? 40 : 64) ? 0 : -1;
+  if (px64 * oc32 <= 256) {
+    if (one && units >= 256 && a.p_total > 2048 && planes->channels == 128) return -1;
+    return units >= (planes ? 216 : 64) ? 1 : -1;
+  }
   if (planes && a.stride_h > 1) return -1;
   const long long px128 = (a.p_total + 127) / 128;
   if (units < (planes ? 216 : 96)) return -1;
-  if (px64 * oc64 <= 256) return 2;
+  if (px64 * oc64 <= 256) return one && (units < 256 || a.p_total > 2048) ? -1 : 2;
+  if (best && planes->count <= 512) return -1;
   if (px128 * oc32 <= 256) return 3;
-  return px128 * oc64 <= 256 && (planes || taps > 9) ? 4 : -1;
+  return px128 * oc64 <= 256 && (planes ? !(apart && planes->count <= 256) : taps > 9) ? 4 : -1;
 }
 
 hipError_t plan_conv_split(LaunchPlan &plan, const GemmArgs &a0, int form, bool planes)

@@ -782,7 +782,7 @@ hipError_t plan_gemm(LaunchPlan &plan, const GemmArgs &a0, int nbatch, int varia
     if (rv >= 0) return plan_gemm1x1_res(plan, a0, rv);
   }
   {
-    const int form = conv_split_pick(a0, nbatch, false);
+    const int form = conv_split_pick(a0, nbatch, nullptr);
     if (form >= 0) return plan_conv_split(plan, a0, form, false);
   }
   const Variant &k = kVariants[variant];

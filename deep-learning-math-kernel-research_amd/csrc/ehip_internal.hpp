@@ -255,13 +255,19 @@ bool gemm1x1_split_applies(const GemmArgs &a, int nbatch);
 hipError_t plan_gemm1x1_split(LaunchPlan &plan, const GemmArgs &a);
 
 // k x k layers with few output values: K shared out among the waves of a workgroup (ehip_convs.hip); the form, or -1
-// (planes: a layer that the 3x3 kernel would run, with its weights)
-int conv_split_pick(const GemmArgs &a, int nbatch, bool planes);
+// (planes: how the 3x3 kernel would run a layer that is its own, and has its weights; null for the others)
+struct Conv3x3Tiles {
+  long long count;     // workgroups
+  int channels;        // of a workgroup
+  bool apart;          // no two waves of a workgroup work on the same channels and others do not (four beside each other, or one)
+};
+int conv_split_pick(const GemmArgs &a, int nbatch, const Conv3x3Tiles *planes);
 hipError_t plan_conv_split(LaunchPlan &plan, const GemmArgs &a, int form, bool planes);
 
 hipError_t plan_conv3x3v(LaunchPlan &plan, const Conv3x3Args &a, int n, int variant);
 int conv3x3v_pick_variant(int n, int oh, int ow, int oc2, int stride);   // stride 1 or 2 (both directions); -1: rows too wide for every variant
 int conv3x3v_chunk_units(int variant, int ic2);
+Conv3x3Tiles conv3x3v_tiles(int variant, int n, int oh, int ow, int oc2, int stride);
 int conv3x3v_num_variants();
 const char *conv3x3v_variant_name(int variant);
 

@@ -453,6 +453,21 @@ def test_direct_k_shared_out_choice(n, ic, oc, hw, k, stride, nhwc, split):
     assert res["conv"].kernel_name == split if split else "_split" not in res["conv"].kernel_name
 
 
+@pytest.mark.parametrize("n,ic,oc,hw,k,split", [
+    # one round of the 3x3 kernel with one fill and all of its waves at work: on both sides of the lines
+    (64, 512, 512, 7, 3, ""), (16, 512, 512, 14, 3, ""), (20, 512, 512, 14, 3, "<64,128>"), (64, 384, 512, 7, 3, ""), (48, 384, 192, 14, 3, "<64,128>"), (24, 384, 256, 14, 3, ""),
+    (16, 384, 192, 14, 3, ""), (8, 512, 512, 14, 3, "<64,64>"), (4, 512, 256, 28, 3, ""), (20, 512, 256, 14, 3, "<64,64>"), (16, 768, 256, 14, 3, "<64,64>"),
+    (4, 512, 128, 28, 3, ""), (8, 512, 64, 28, 3, "<32,64>"), (2, 512, 128, 56, 3, "<64,64>"), (24, 384, 32, 28, 3, ""),
+    (8, 32, 64, 14, 5, ""), (8, 64, 64, 14, 5, "<32,32>")])
+def test_direct_k_shared_out_lines(n, ic, oc, hw, k, split):
+    E = pkg()
+    d = E.make_desc(n, ic, oc, hw, hw, k, k, k // 2, 1, algorithm=E.CONV_DIRECT, input_type=E.U8, output_type=E.S8, with_relu=True,
+                    relu_bound=(0.0, 127.0), input_quant=(1.0 / 255.0, 0.0), output_quant=(0.1, 0.0))
+    conv = E.Conv(d)
+    conv.prepare(dev(np.zeros((oc // 16, ic // 16, k, k, 16, 16), np.float32)), dev(np.zeros(oc, np.float32)))
+    assert conv.kernel_name.endswith("_split" + split) if split else "_split" not in conv.kernel_name
+
+
 # at most four input channels (first layers; the reference feeds them 3-channel nhwc,
 # scripts/best_configs/resnetv1_5-n64-clx-1s-int8.sh:12): 16 / ic pixels per operand cell, a kernel row
 # is ceil(kw / (16 / ic)) cells, input rows staged compactly in LDS
