@@ -225,6 +225,41 @@ __global__ __launch_bounds__(64 * A, A == 4 ? 1 : 2) void k_wino_gemm_output_lan
   }
 }
 
+// The workgroups of form 0, 1, 2 = 16 channels x 16 tiles, 32 x 16, 32 x 32 for so many blocks of 16 tiles and of 16 channels, and which of them an
+// XCD takes: a rectangle of nxx x nyy, the one of least reading (its share of the weights and its share of the tiles) among those that give each
+// of its 32 CUs one workgroup at most, if there are any.
+struct ColsGrid {
+  int nx, ny;     // groups of tiles, of channels
+  int slots;      // log2 of the XCDs beside each other along the tiles
+  int nxx, nyy;
+};
+static ColsGrid cols_grid(int blocks, int oc2, int form)
+{
+  const int ro = form >= 1 ? 2 : 1, rt = form == 2 ? 2 : 1;
+  ColsGrid g;
+  g.nx = (blocks + rt - 1) / rt;
+  g.ny = (oc2 + ro - 1) / ro;
+  long long best = -1;
+  bool best_fits = false;
+  for (int xa = 0; xa <= 3; ++xa) {
+    const int nxx = (g.nx + (1 << xa) - 1) >> xa, nyy = (g.ny + (8 >> xa) - 1) / (8 >> xa);
+    const long long read = (long long)nxx * rt + (long long)nyy * ro;   // (times A * A * ic2 * 256 bytes)
+    const bool fits = (long long)nxx * nyy <= 32;
+    if (best >= 0 && (fits == best_fits ? read >= best : best_fits)) continue;
+    best = read;
+    best_fits = fits;
+    g.slots = xa;
+    g.nxx = nxx;
+    g.nyy = nyy;
+  }
+  return g;
+}
+static bool cols_one_round(int blocks, int oc2, int form)
+{
+  const ColsGrid g = cols_grid(blocks, oc2, form);
+  return (long long)g.nxx * g.nyy <= 32;
+}
+
 // The form for a layer: 0, 1, 2 = 16 channels x 16 tiles, 32 x 16, 32 x 32 a workgroup, -1 = none.  Each is the fastest while every
 // workgroup has a CU of its own, the smaller one first; a second round costs as much as the first, and the other kernels share what
 // they read among more products.  Fused stage, other tensors on every call, us: the kernel that ran before / the three forms, at
@@ -238,6 +273,9 @@ __global__ __launch_bounds__(64 * A, A == 4 ? 1 : 2) void k_wino_gemm_output_lan
 //     256 channels 8.6 / 7.2 8.4 10.4 (256), 11.9 / 10.6 8.6 10.6 (512), 12.4 / - 15.4 11.3 (1024); 512 channels 17.1 / - 21.3 16.0 (1024)
 //   tile size 4: 128 channels 5.0 / 5.6 4.8 6.0 (256), 6.3 / 7.4 5.4 6.2 (512); 256 channels 6.9 / 5.9 6.2 7.4 (256), 7.7 / 8.4 6.3 7.4 (512), 7.9 / - 8.2 7.5 (640);
 //     512 channels 9.0 / 7.9 8.0 9.7 (256), 11.5 / - 12.9 10.7 (1024)
+// An XCD has 32 of the CUs, and takes a rectangle of the workgroups: 49 x 5 of them do not come to one round on any XCD (at best 35
+// on one), and cost two.  Then the next form is the faster one, or none: 160 -> 160, 49 blocks of tiles, tile size 6, with the input transform
+// 16.6 / 21.1 with 32 x 16; 453 -> 275, 54 blocks, tile size 5 28.9 / 36.5 with 32 x 32; 184 -> 80, 49 blocks 16.7 with 16 x 16, 15.2 with 32 x 16.
 // 32 x 32 with up to 256 input channels only from 192 output channels on: with fewer, the layer has so many tiles that they are what
 // it reads, and resident weights read them once (with the input transform, 256 -> 64, 160 blocks of tiles 28.7 / 29.7; 192 -> 32, 390
 // blocks 34.3 / 36.5).
@@ -253,10 +291,9 @@ int wino_cols_pick(const WinoFusedArgs &a)
   // (more than 256 channels, up to 16 workgroups: the forms that the tests of the choice pin for such layers; 512 -> 256, one block of
   // tiles, tile size 6 20 / 12 us)
   if (nks > 4 && (long long)blocks * a.oc2 <= 16) return -1;
-  const int halves = (a.oc2 + 1) / 2;
-  if ((long long)blocks * a.oc2 <= 256) return A == 4 && nks < 3 ? -1 : 0;
-  if ((long long)blocks * halves <= 256) return A == 6 || nks >= 2 ? 1 : -1;
-  if ((long long)((blocks + 1) / 2) * halves <= 256) return nks > 4 || (nks >= (A == 4 ? 4 : 3) && a.oc2 >= 12) ? 2 : -1;
+  if (cols_one_round(blocks, a.oc2, 0)) return A == 4 && nks < 3 ? -1 : 0;
+  if (cols_one_round(blocks, a.oc2, 1)) return A == 6 || nks >= 2 ? 1 : -1;
+  if (cols_one_round(blocks, a.oc2, 2)) return nks > 4 || (nks >= (A == 4 ? 4 : 3) && a.oc2 >= 12) ? 2 : -1;
   return -1;
 }
 
@@ -271,19 +308,9 @@ hipError_t plan_wino_gemm_output_cols(LaunchPlan &plan, const WinoFusedArgs &a0,
   else if (A == 5) EHIP_WC(5);
   else EHIP_WC(6);
 #undef EHIP_WC
-  a.nx = ((a.t + 15) / 16 + blocks - 1) / blocks;
-  a.ny = (a.oc2 + ro - 1) / ro;
-  // what an XCD reads: its share of the weights and its share of the tiles
-  dim3 grid;
-  long long best = -1;
-  for (int xa = 0; xa <= 3; ++xa) {
-    const int nxx = (a.nx + (1 << xa) - 1) >> xa, nyy = (a.ny + (8 >> xa) - 1) / (8 >> xa);
-    const long long read = (long long)nxx * blocks + (long long)nyy * ro;   // (times A * A * ic2 * 256 bytes)
-    if (best >= 0 && read >= best) continue;
-    best = read;
-    a.slots = xa;
-    grid = dim3(8 * nxx, nyy);
-  }
+  const ColsGrid g = cols_grid((a.t + 15) / 16, a.oc2, form);
+  a.nx = g.nx; a.ny = g.ny; a.slots = g.slots;
+  const dim3 grid(8 * g.nxx, g.nyy);
   const size_t lds = (size_t)ro * blocks * (A == 4 ? A : A - 2) * A * 1024 + (size_t)A * 3 * A * 64 * ro;
   static const char *const names[] = {"k_wino_gemm_output_lanes_cols<16,16>", "k_wino_gemm_output_lanes_cols<32,16>",
                                       "k_wino_gemm_output_lanes_cols<32,32>"};   // channels, tiles of a workgroup

@@ -892,7 +892,9 @@ def test_wino_fused_columns(n, ic, oc, h, w, out_type, with_sum, with_relu, out_
 
 @pytest.mark.parametrize("tile,n,ic,oc,hw,form", [
     (6, 2, 512, 512, 28, "<16,16>"), (6, 3, 512, 512, 28, "<32,16>"), (6, 64, 256, 256, 14, "<32,32>"), (6, 65, 256, 256, 14, ""), (6, 1, 256, 256, 14, "<16,16>"),
-    (6, 1, 512, 512, 14, "<16,16>"), (6, 1, 512, 256, 14, ""), (5, 3, 1024, 256, 28, "<32,16>"), (5, 64, 128, 256, 14, ""), (4, 1, 256, 256, 14, "<16,16>"), (4, 1, 128, 512, 14, ""), (4, 12, 128, 512, 8, "<32,16>")])
+    (6, 1, 512, 512, 14, "<16,16>"), (6, 1, 512, 256, 14, ""), (5, 3, 1024, 256, 28, "<32,16>"), (5, 64, 128, 256, 14, ""), (4, 1, 256, 256, 14, "<16,16>"), (4, 1, 128, 512, 14, ""), (4, 12, 128, 512, 8, "<32,16>"),
+    # 245 workgroups that no rectangle per XCD takes in one round: the next form, or none
+    (6, 16, 192, 80, 28, "<32,16>"), (6, 16, 160, 160, 28, "")])
 def test_wino_fused_columns_choice(tile, n, ic, oc, hw, form, monkeypatch):
     monkeypatch.setenv("EHIP_WINO_WHOLE", "0")
     E = pkg()
