@@ -3,6 +3,28 @@
 
 namespace ehip {
 
+struct WholeSplit {
+  int waves;               // of a workgroup
+  int splits, per_split;   // workgroups of a block of tiles, groups of 16 output channels of each
+};
+static WholeSplit whole_split(int nks, int blocks, int groups)
+{
+  // eight waves where no CU gets a second block (128 -> 128, 196 blocks: 17.8 against 22.1 us), else four, so that the phases of two
+  // or three blocks overlap on a CU (402 blocks: 29.6 against 31.9; 64 -> 64, 784 blocks: 28.0 against 41.6)
+  WholeSplit s;
+  s.waves = blocks <= 256 || nks > 2 ? 8 : 4;
+  if (const char *env = getenv("EHIP_WINO_WHOLE_WAVES")) s.waves = env[0] == '8' || nks > 2 ? 8 : 4;
+  // fewer blocks than CUs: the output channels of a block are shared out, as long as that leaves every wave some
+  s.splits = 256 / blocks;
+  const int most = (groups + s.waves - 1) / s.waves;
+  s.splits = s.splits > most ? most : s.splits;
+  if (const char *env = getenv("EHIP_WINO_WHOLE_SPLITS")) s.splits = atoi(env);
+  s.splits = s.splits < 1 ? 1 : s.splits > groups ? groups : s.splits;
+  s.per_split = (groups + s.splits - 1) / s.splits;
+  s.splits = (groups + s.per_split - 1) / s.per_split;
+  return s;
+}
+
 // Where one kernel is the faster one.  It saves a launch, the trip of the transformed input through memory and the start of a second
 // kernel with cold caches; it pays with input transforms that the workgroups sharing a block of tiles repeat, with weights
 // that every block streams for itself, and with phases that overlap only where a CU holds several workgroups.  So it wins
@@ -27,19 +49,32 @@ namespace ehip {
 //   tile size 5: 64 -> 64, 16 / 64 / 98 1.03 / 1.00 / 0.90; 64 -> 128, 32 / 48 1.11 / 0.96; 128 -> 64, 64 / 98 1.16 / 0.96; 128 -> 128, 64 / 98 1.21 / 0.99; 192 -> 64, 98 / 128
 //     1.08 / 0.94; 256 -> 64, 98 / 128 1.00 / 0.94
 //   tile size 4: 128 -> 128, 64 / 98 1.12 / 0.95; 256 -> 64, 64 / 98 1.09 / 0.99
+// A wave takes whole groups of 16 output channels, so 9 groups cost four waves as much as 12 and eight as much as 16.  Where the waves go
+// through more than one round of them (`full`: blocks from which on that pays with eight waves; 1000 random layers):
+//   eight waves, tile size 6: 64 -> 160, 133 / 144 / 157 / 196 / 256 blocks 1.19 / 1.15 / 1.09 / 0.94 / 0.86; 192 -> 160, 172 / 222 1.11 / 0.93; tile size
+//     5: 64 -> 160 .. 256, 135 to 256 1.01 to 0.89; 128 -> 144 .. 192, 144 to 188 1.13 to 1.06, 252 0.90; 192 -> 144 .. 224, 163 to 179 1.01 to 1.18;
+//     tile size 4: up to 128 channels 0.77 to 0.98; 192, 154 / 158 1.04, 196 0.90; 256 -> 208, 153 / 245 1.08
+//   four waves, up to 400 blocks: two rounds, tile size 6 260 / 300 / 341 / 378 blocks 1.35 / 1.24 / 1.11 / 1.11 (336 and seven groups 0.94), tile size 5 0.87 to
+//     1.09, tile size 4 0.75 to 0.84; three, tile size 6 324 / 338 1.20 / 1.16, 5 258 to 384
+//     1.16 to 1.06, 4 0.82 to 0.92 with 64 channels and 1.05 to 1.11 with 128; four, tile size 4 1.03 to 1.11
 static bool wino_whole_pays(int A, int nks, int blocks, int groups)
 {
   // blocks from (at most 64 output channels; more) and to, groups of 16 output channels, blocks x groups; by k-steps of 64 input
   // channels
-  struct Limit { int least_few, least, most, groups, work; };
+  struct Limit { int least_few, least, most, groups, work, full; };
   static const Limit limits[3][4] = {
-      {{1, 1, 1200, 64, 6300}, {1, 90, 480, 16, 6300}, {56, 110, 256, 16, 4000}, {90, 115, 256, 16, 3200}},     // tile size 4
-      {{1, 40, 1200, 64, 4700}, {80, 90, 480, 16, 4000}, {110, 110, 256, 16, 4000}, {110, 110, 256, 8, 4000}},
-      {{24, 56, 400, 64, 3300}, {110, 112, 480, 8, 4000}, {95, 120, 256, 12, 4000}, {110, 125, 256, 8, 4000}}};
+      {{1, 1, 1200, 64, 6300, 1}, {1, 90, 480, 16, 6300, 1}, {56, 110, 256, 16, 4000, 160}, {90, 115, 256, 12, 3200, 160}},     // tile size 4
+      {{1, 40, 1200, 64, 4700, 128}, {80, 90, 480, 16, 4000, 193}, {110, 110, 256, 16, 4000, 193}, {110, 120, 256, 8, 4000, 193}},
+      {{24, 56, 400, 64, 3300, 193}, {110, 112, 480, 8, 4000, 193}, {95, 120, 256, 12, 4000, 193}, {110, 125, 256, 8, 4000, 193}}};
   // (the fused stage with a workgroup of its own on a CU for every 16 channels x 16 tiles: the stages)
   if (A >= 5 && (long long)blocks * groups <= 256) return false;
   const Limit &l = limits[A - 4][nks - 1];
-  return blocks >= (groups <= 4 ? l.least_few : l.least) && blocks <= l.most && groups <= l.groups && (long long)blocks * groups <= l.work;
+  if (blocks < (groups <= 4 ? l.least_few : l.least) || blocks > l.most || groups > l.groups || (long long)blocks * groups > l.work) return false;
+  const WholeSplit s = whole_split(nks, blocks, groups);
+  const int rounds = (s.per_split + s.waves - 1) / s.waves;   // of a wave's groups of output channels
+  if (rounds == 1) return true;
+  if (s.waves == 8) return blocks * s.splits >= l.full;
+  return (long long)blocks * 4 * rounds <= l.work && blocks >= (rounds > (A == 4 && nks == 1 ? 3 : 2) ? 400 : A == 6 ? 384 : 257);
 }
 
 bool wino_whole_applies(const WinoArgs &w, const WinoFusedArgs &f)
@@ -70,20 +105,11 @@ hipError_t plan_wino_whole(LaunchPlan &plan, const WinoArgs &w, const WinoFusedA
   a.f = f;
   const int nks = (f.ic2 + 3) / 4;
   a.nx = (f.t + 15) / 16;
-  // eight waves where no CU gets a second block (128 -> 128, 196 blocks: 17.8 against 22.1 us), else four, so that the phases of two
-  // or three blocks overlap on a CU (402 blocks: 29.6 against 31.9; 64 -> 64, 784 blocks: 28.0 against 41.6)
-  int nw = a.nx <= 256 ? 8 : 4;
-  if (const char *env = getenv("EHIP_WINO_WHOLE_WAVES")) nw = env[0] == '8' ? 8 : 4;
-  const WholeForm form = f.tile == 4 ? wino_whole_form4(nks, nw, f.out_type, f.with_sum != 0)
-      : f.tile == 5 ? wino_whole_form5(nks, nw, f.out_type, f.with_sum != 0) : wino_whole_form6(nks, nw, f.out_type, f.with_sum != 0);
-  // fewer blocks than CUs: the output channels of a block are shared out, as long as that leaves every wave some
-  int splits = 256 / a.nx;
-  const int most = (f.oc2 + form.waves - 1) / form.waves;
-  splits = splits > most ? most : splits;
-  if (const char *env = getenv("EHIP_WINO_WHOLE_SPLITS")) splits = atoi(env);
-  splits = splits < 1 ? 1 : splits > f.oc2 ? f.oc2 : splits;
-  a.per_split = (f.oc2 + splits - 1) / splits;
-  a.splits = (f.oc2 + a.per_split - 1) / a.per_split;
+  const WholeSplit split = whole_split(nks, a.nx, f.oc2);
+  const WholeForm form = f.tile == 4 ? wino_whole_form4(nks, split.waves, f.out_type, f.with_sum != 0)
+      : f.tile == 5 ? wino_whole_form5(nks, split.waves, f.out_type, f.with_sum != 0) : wino_whole_form6(nks, split.waves, f.out_type, f.with_sum != 0);
+  a.splits = split.splits;
+  a.per_split = split.per_split;
   a.nt_magic = div_magic(f.nt);
   a.wt_magic = div_magic(f.wt);
   plan.name = "k_wino_whole";

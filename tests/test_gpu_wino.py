@@ -841,7 +841,10 @@ def test_wino_transformed_floats(n, ic, h, w, nhwc, data, monkeypatch):
 @pytest.mark.parametrize("tile,ic,oc,n,hw,whole", [
     (6, 64, 64, 32, 56, True), (6, 64, 64, 64, 56, False), (6, 64, 64, 2, 28, False), (6, 128, 128, 64, 28, True), (6, 128, 128, 160, 28, False),
     (6, 192, 192, 20, 28, False), (6, 192, 192, 64, 28, True), (6, 256, 64, 64, 28, True), (6, 256, 256, 64, 14, False), (5, 128, 256, 40, 28, True),
-    (4, 256, 128, 20, 28, True), (4, 64, 48, 1, 7, True)])
+    (4, 256, 128, 20, 28, True), (4, 64, 48, 1, 7, True),
+    # groups of output channels that the waves do not share evenly
+    (6, 32, 144, 32, 52, False), (6, 64, 80, 24, 56, False), (6, 64, 144, 16, 56, True), (6, 64, 160, 11, 56, False), (5, 128, 144, 23, 28, False),
+    (4, 128, 160, 22, 28, False), (4, 64, 144, 26, 28, True)])
 def test_wino_whole_choice(tile, ic, oc, n, hw, whole, monkeypatch):
     """which layers run whole, around the lines of the rule, and the same bytes from the stages"""
     import torch
