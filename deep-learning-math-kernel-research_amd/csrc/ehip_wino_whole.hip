@@ -50,22 +50,25 @@ static WholeSplit whole_split(int nks, int blocks, int groups)
 //     1.08 / 0.94; 256 -> 64, 98 / 128 1.00 / 0.94
 //   tile size 4: 128 -> 128, 64 / 98 1.12 / 0.95; 256 -> 64, 64 / 98 1.09 / 0.99
 // A wave takes whole groups of 16 output channels, so 9 groups cost four waves as much as 12 and eight as much as 16.  Where the waves go
-// through more than one round of them (`full`: blocks from which on that pays with eight waves; 1000 random layers):
-//   eight waves, tile size 6: 64 -> 160, 133 / 144 / 157 / 196 / 256 blocks 1.19 / 1.15 / 1.09 / 0.94 / 0.86; 192 -> 160, 172 / 222 1.11 / 0.93; tile size
-//     5: 64 -> 160 .. 256, 135 to 256 1.01 to 0.89; 128 -> 144 .. 192, 144 to 188 1.13 to 1.06, 252 0.90; 192 -> 144 .. 224, 163 to 179 1.01 to 1.18;
-//     tile size 4: up to 128 channels 0.77 to 0.98; 192, 154 / 158 1.04, 196 0.90; 256 -> 208, 153 / 245 1.08
-//   four waves, up to 400 blocks: two rounds, tile size 6 260 / 300 / 341 / 378 blocks 1.35 / 1.24 / 1.11 / 1.11 (336 and seven groups 0.94), tile size 5 0.87 to
-//     1.09, tile size 4 0.75 to 0.84; three, tile size 6 324 / 338 1.20 / 1.16, 5 258 to 384
-//     1.16 to 1.06, 4 0.82 to 0.92 with 64 channels and 1.05 to 1.11 with 128; four, tile size 4 1.03 to 1.11
+// through more than one round of them it pays (`full`) with eight waves from so many CUs on whose waves would all be at work, 2000 random
+// layers:
+//   tile size 6: 64 -> 160, 133 / 144 / 157 blocks (82 / 89 / 108 CUs) 1.19 / 1.15 / 1.09; 64 -> 144, 192 / 196 / 224 / 256 (108 / 110 / 126 / 144) 1.08 / 0.94 / 0.93 / 0.94; 64 ->
+//     176, 179 (123) 0.90; 192 -> 160, 172 (107) 1.11; 192 -> 144, 204 / 222 (115 / 125) 0.92 / 0.93
+//   tile size 5: 64 -> 160 .. 256, 135 to 256 (110 to 224) 1.01 to 0.89; 128 -> 144 .. 192, 144 to 188 (81 to 118) 1.13 to 1.06, 252 (205) 0.90; 192 -> 144 /
+//     160, 179 / 167 (101 / 104) 1.18 / 1.16
+//   tile size 4, by blocks: up to 128 channels 0.77 to 0.98; 192, 154 to 160 1.04, 180 / 196 0.90; 256 -> 160 .. 208, 153 / 160 1.08 / 0.97
+// with four waves, tile size 6 only next to the next round of blocks (two rounds of groups, 260 / 300 / 341 / 378 blocks 1.35 / 1.24 / 1.11 / 1.11); tile
+//   size 5, two rounds, 257 to 319 blocks 1.19 to 1.04, 324 to 522 0.97 to 0.87, three, 258 to 384 1.16 to 1.06, 387 to 398 0.95; tile size 4, three or
+//   four, 128 channels, 259 to 338 blocks 1.11 to 1.05, 359 to 392 0.96 to 0.93, 64 channels 0.82 to 0.92.
 static bool wino_whole_pays(int A, int nks, int blocks, int groups)
 {
   // blocks from (at most 64 output channels; more) and to, groups of 16 output channels, blocks x groups; by k-steps of 64 input
   // channels
   struct Limit { int least_few, least, most, groups, work, full; };
   static const Limit limits[3][4] = {
-      {{1, 1, 1200, 64, 6300, 1}, {1, 90, 480, 16, 6300, 1}, {56, 110, 256, 16, 4000, 160}, {90, 115, 256, 12, 3200, 160}},     // tile size 4
-      {{1, 40, 1200, 64, 4700, 128}, {80, 90, 480, 16, 4000, 193}, {110, 110, 256, 16, 4000, 193}, {110, 120, 256, 8, 4000, 193}},
-      {{24, 56, 400, 64, 3300, 193}, {110, 112, 480, 8, 4000, 193}, {95, 120, 256, 12, 4000, 193}, {110, 125, 256, 8, 4000, 193}}};
+      {{1, 1, 1200, 64, 6300, 0}, {1, 90, 480, 16, 6300, 0}, {56, 110, 256, 16, 4000, 165}, {90, 115, 256, 12, 3200, 160}},     // tile size 4
+      {{1, 40, 1200, 64, 4700, 112}, {80, 90, 480, 16, 4000, 120}, {110, 110, 256, 16, 4000, 120}, {110, 120, 256, 8, 4000, 120}},
+      {{24, 56, 400, 64, 3300, 109}, {110, 112, 480, 8, 4000, 109}, {95, 128, 256, 12, 4000, 109}, {110, 128, 256, 8, 4000, 109}}};
   // (the fused stage with a workgroup of its own on a CU for every 16 channels x 16 tiles: the stages)
   if (A >= 5 && (long long)blocks * groups <= 256) return false;
   const Limit &l = limits[A - 4][nks - 1];
@@ -73,8 +76,9 @@ static bool wino_whole_pays(int A, int nks, int blocks, int groups)
   const WholeSplit s = whole_split(nks, blocks, groups);
   const int rounds = (s.per_split + s.waves - 1) / s.waves;   // of a wave's groups of output channels
   if (rounds == 1) return true;
-  if (s.waves == 8) return blocks * s.splits >= l.full;
-  return (long long)blocks * 4 * rounds <= l.work && blocks >= (rounds > (A == 4 && nks == 1 ? 3 : 2) ? 400 : A == 6 ? 384 : 257);
+  if (s.waves == 8) return A == 4 ? blocks >= l.full : blocks * groups >= l.full * 8 * rounds;
+  if (A == 6) return blocks >= 384 && blocks * 4 * rounds <= l.work;
+  return A == 5 ? blocks >= (rounds == 2 ? 320 : 385) : rounds == 2 || nks == 1 || blocks >= 350;
 }
 
 bool wino_whole_applies(const WinoArgs &w, const WinoFusedArgs &f)
