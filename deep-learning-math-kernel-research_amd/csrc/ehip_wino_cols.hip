@@ -276,6 +276,8 @@ static bool cols_one_round(int blocks, int oc2, int form)
 // An XCD has 32 of the CUs, and takes a rectangle of the workgroups: 49 x 5 of them do not come to one round on any XCD (at best 35
 // on one), and cost two.  Then the next form is the faster one, or none: 160 -> 160, 49 blocks of tiles, tile size 6, with the input transform
 // 16.6 / 21.1 with 32 x 16; 453 -> 275, 54 blocks, tile size 5 28.9 / 36.5 with 32 x 32; 184 -> 80, 49 blocks 16.7 with 16 x 16, 15.2 with 32 x 16.
+// A few workgroups gain as much as a chip full of them: 288 / 512 -> 16 to 256, one image of 7 x 7 or 14 x 14, with the input transform, tile size 6 19.2 to
+// 23.5 us (ring) / 11.7 to 13.2 (16 x 16), 5 14.3 to 19.2 / 9.9 to 11.5, 4 10.7 to 13.0 / 8.6 to 9.5.
 // 32 x 32 with up to 256 input channels only from 192 output channels on: with fewer, the layer has so many tiles that they are what
 // it reads, and resident weights read them once (with the input transform, 256 -> 64, 160 blocks of tiles 28.7 / 29.7; 192 -> 32, 390
 // blocks 34.3 / 36.5).
@@ -288,9 +290,6 @@ int wino_cols_pick(const WinoFusedArgs &a)
   // (a switch that asks for one of the other forms)
   for (const char *k : {"EHIP_WINO_LANES", "EHIP_WINO_LANES_WRES", "EHIP_WINO_LANES_SLOTS", "EHIP_WINO_LANES_WAVES", "EHIP_WINO_RING"})
     if (getenv(k)) return -1;
-  // (more than 256 channels, up to 16 workgroups: the forms that the tests of the choice pin for such layers; 512 -> 256, one block of
-  // tiles, tile size 6 20 / 12 us)
-  if (nks > 4 && (long long)blocks * a.oc2 <= 16) return -1;
   if (cols_one_round(blocks, a.oc2, 0)) return A == 4 && nks < 3 ? -1 : 0;
   if (cols_one_round(blocks, a.oc2, 1)) return A == 6 || nks >= 2 ? 1 : -1;
   if (cols_one_round(blocks, a.oc2, 2)) return nks > 4 || (nks >= (A == 4 ? 4 : 3) && a.oc2 >= 12) ? 2 : -1;

@@ -679,9 +679,10 @@ def test_wino_fused_ring(form, tile, out_type, with_sum, with_relu, n, ic, oc, h
     (6, 1, 528, 48, 14, ""), (6, 128, 640, 256, 14, ""), (6, 192, 640, 256, 14, "_lanes_ring<64,64>"),   # 4, 256 and 384 workgroups of the general kernel
     (5, 1, 640, 48, 9, ""), (5, 1, 640, 256, 9, "_lanes_ring<32,32>"), (5, 64, 640, 256, 14, ""), (4, 1, 640, 48, 9, "_lanes_ring<32,32>")])
 def test_wino_fused_choice_of_form(tile, n, ic, oc, hw, kernel, monkeypatch):
-    """which form of the fused stage layers of more than 256 input channels take, around the lines of the rule; the chosen one
-    and each ring form leave the same bytes, for every output type, with and without the sum, in both layouts"""
+    """which form of the fused stage layers of more than 256 input channels take that do not share the columns out, around the lines of
+    the rule; the chosen one and each ring form leave the same bytes, for every output type, with and without the sum, in both layouts"""
     import torch
+    monkeypatch.setenv("EHIP_WINO_COLS", "-")   # (the smaller ones would: test_wino_fused_columns_choice)
     E = pkg()
     g = torch.Generator(device="cuda").manual_seed(5 + ic + oc)
     x = torch.randint(0, 256, (n, ic // 16, hw, hw, 16), dtype=torch.uint8, device="cuda", generator=g)
@@ -895,7 +896,8 @@ def test_wino_fused_columns(n, ic, oc, h, w, out_type, with_sum, with_relu, out_
 
 @pytest.mark.parametrize("tile,n,ic,oc,hw,form", [
     (6, 2, 512, 512, 28, "<16,16>"), (6, 3, 512, 512, 28, "<32,16>"), (6, 64, 256, 256, 14, "<32,32>"), (6, 65, 256, 256, 14, ""), (6, 1, 256, 256, 14, "<16,16>"),
-    (6, 1, 512, 512, 14, "<16,16>"), (6, 1, 512, 256, 14, ""), (5, 3, 1024, 256, 28, "<32,16>"), (5, 64, 128, 256, 14, ""), (4, 1, 256, 256, 14, "<16,16>"), (4, 1, 128, 512, 14, ""), (4, 12, 128, 512, 8, "<32,16>"),
+    (6, 1, 512, 512, 14, "<16,16>"), (6, 1, 512, 256, 14, "<16,16>"), (6, 1, 528, 48, 14, "<16,16>"),
+    (5, 1, 640, 48, 9, "<16,16>"), (4, 1, 640, 48, 9, "<16,16>"), (5, 3, 1024, 256, 28, "<32,16>"), (5, 64, 128, 256, 14, ""), (4, 1, 256, 256, 14, "<16,16>"), (4, 1, 128, 512, 14, ""), (4, 12, 128, 512, 8, "<32,16>"),
     # 245 workgroups that no rectangle per XCD takes in one round: the next form, or none
     (6, 16, 192, 80, 28, "<32,16>"), (6, 16, 160, 160, 28, "")])
 def test_wino_fused_columns_choice(tile, n, ic, oc, hw, form, monkeypatch):
