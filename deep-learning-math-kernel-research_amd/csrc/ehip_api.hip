@@ -628,7 +628,7 @@ static int plan_execute(ehip_conv *c)
       const Conv3x3Tiles tiles = conv3x3v_tiles(c->variant, d.n, d.oh, d.ow, c->oc2, d.stride_h);
       const int form = conv_split_pick(g, 1, &tiles);
       if (form >= 0) {
-        HIP_TRY(plan_conv_split(*p, g, form, true));
+        HIP_TRY(plan_conv_split(*p, g, form));
         break;
       }
     }
@@ -796,7 +796,7 @@ EHIP_API int ehip_conv_prepare(ehip_conv_t *c, const void *weights_dev, const vo
   }
   // from here on the name is that of the kernel the planner chose
   if (c->family == FAM_WINOGRAD) {
-    if (c->fused && c->plan[1].name) c->kernel_name = std::string("k_wino_trans_input_u8 + ") + c->plan[1].name;
+    if (c->fused) c->kernel_name = std::string(c->plan[0].name) + " + " + c->plan[1].name;
     if (c->execute_stages == kStageWhole) c->kernel_name = std::string(c->plan[2].name) + " | " + c->kernel_name;
   } else if (c->plan[0].name) {
     c->kernel_name = c->plan[0].name;

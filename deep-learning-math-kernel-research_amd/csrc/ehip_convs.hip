@@ -227,7 +227,7 @@ int conv_split_pick(const GemmArgs &a, int nbatch, const Conv3x3Tiles *planes)
   return px128 * oc64 <= 256 && (planes ? !(apart && planes->count <= 256) : taps > 9) ? 4 : -1;
 }
 
-hipError_t plan_conv_split(LaunchPlan &plan, const GemmArgs &a0, int form, bool planes)
+hipError_t plan_conv_split(LaunchPlan &plan, const GemmArgs &a0, int form)
 {
   GemmArgs a = a0;
   a.k_real = a.kh * a.kw * a.units_pad;
@@ -238,10 +238,9 @@ hipError_t plan_conv_split(LaunchPlan &plan, const GemmArgs &a0, int form, bool 
       form == 0 ? k_gemm_u8s8_split<1, 1, 8> : form == 1 ? k_gemm_u8s8_split<1, 2, 8> : form == 2 ? k_gemm_u8s8_split<2, 2, 8> :
       form == 3 ? k_gemm_u8s8_split<1, 4, 8> : k_gemm_u8s8_split<2, 4, 8>;
   // (channels, pixels of a workgroup)
-  static const char *const names[][5] = {{"k_gemm_u8s8_split<32,32>", "k_gemm_u8s8_split<32,64>", "k_gemm_u8s8_split<64,64>", "k_gemm_u8s8_split<32,128>", "k_gemm_u8s8_split<64,128>"},
-                                         {"k_conv3x3v_u8s8_split<32,32>", "k_conv3x3v_u8s8_split<32,64>", "k_conv3x3v_u8s8_split<64,64>", "k_conv3x3v_u8s8_split<32,128>", "k_conv3x3v_u8s8_split<64,128>"},
-                                         {"k_conv3x3v_u8s8_split<32,32,s2>", "k_conv3x3v_u8s8_split<32,64,s2>", "k_conv3x3v_u8s8_split<64,64,s2>", "k_conv3x3v_u8s8_split<32,128,s2>", "k_conv3x3v_u8s8_split<64,128,s2>"}};
-  plan.name = names[planes ? a.stride_h : 0][form];
+  static const char *const names[] = {"k_gemm_u8s8_split<32,32>", "k_gemm_u8s8_split<32,64>", "k_gemm_u8s8_split<64,64>", "k_gemm_u8s8_split<32,128>",
+                                      "k_gemm_u8s8_split<64,128>"};
+  plan.name = names[form];
   return plan_set(plan, kernel, dim3((unsigned)(a.nx * a.ny)), dim3(512), (size_t)(tm * tn > 4 ? 4 : 8) * tm * tn * 4096, a, ArgBlock{}, ArgIn{a.in}, ArgOut{a.out});
 }
 

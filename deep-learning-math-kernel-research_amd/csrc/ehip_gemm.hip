@@ -783,7 +783,7 @@ hipError_t plan_gemm(LaunchPlan &plan, const GemmArgs &a0, int nbatch, int varia
   }
   {
     const int form = conv_split_pick(a0, nbatch, nullptr);
-    if (form >= 0) return plan_conv_split(plan, a0, form, false);
+    if (form >= 0) return plan_conv_split(plan, a0, form);
   }
   const Variant &k = kVariants[variant];
   GemmArgs a = a0;

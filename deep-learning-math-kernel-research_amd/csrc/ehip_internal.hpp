@@ -262,7 +262,7 @@ struct Conv3x3Tiles {
   bool apart;          // no two waves of a workgroup work on the same channels and others do not (four beside each other, or one)
 };
 int conv_split_pick(const GemmArgs &a, int nbatch, const Conv3x3Tiles *planes);
-hipError_t plan_conv_split(LaunchPlan &plan, const GemmArgs &a, int form, bool planes);
+hipError_t plan_conv_split(LaunchPlan &plan, const GemmArgs &a, int form);
 
 hipError_t plan_conv3x3v(LaunchPlan &plan, const Conv3x3Args &a, int n, int variant);
 int conv3x3v_pick_variant(int n, int oh, int ow, int oc2, int stride);   // stride 1 or 2 (both directions); -1: rows too wide for every variant

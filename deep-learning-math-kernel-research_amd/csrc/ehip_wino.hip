@@ -696,6 +696,7 @@ hipError_t plan_wino_trans_input(LaunchPlan &plan, const WinoArgs &a0)
   a.nblocks = (a.t + tiles - 1) / tiles;
   a.items_per_xcd = (int)(((long long)a.nblocks * a.ic2 + 7) / 8);
   dim3 grid(8 * a.items_per_xcd, 1);
+  plan.name = shorter ? "k_wino_trans_input_codes_short" : codes ? "k_wino_trans_input_codes" : floats ? "k_wino_trans_input_floats" : "k_wino_trans_input_u8";
   void (*kern)(const WinoArgs *, const void *) = nullptr;
 #define EHIP_WI(A)                                                                                          \
   kern = shorter ? k_wino_trans_input_codes_short<A>                                                        \
@@ -750,6 +751,7 @@ hipError_t plan_wino_gemm_output(LaunchPlan &plan, const WinoFusedArgs &a0)
   wino_general_workgroups(a, &nh);
   a.ny = (a.oc2 * 16 + 32 * nh - 1) / (32 * nh);
   const int nks = a.units_pad / 2;
+  plan.name = "k_wino_gemm_output";
   const size_t lds = (size_t)AA * 32 * 32 * sizeof(float) + 4 * (size_t)((AA + 3) / 4 * 24) * sizeof(float4);   // exchange + constants
   dim3 grid(8 * a.ny * ((a.nx + 7) / 8));
   // operand ring depth in k-steps.  Measured (C4a / C4b / C4a_i8 / C4b_i8, us): 8 deep 261.7 / 177.3 / 247.6 /

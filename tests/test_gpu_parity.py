@@ -331,8 +331,9 @@ def test_conv3x3_strided_pixels_output_types(variant, out_type, monkeypatch):
     run_and_compare(Layer(1, 128, 80, 9, k=3, pad=0, out_type=out_type, seed=61 + variant + out_type))
 
 
-def test_conv3x3_virtual_rows_many_channels_restage():
+def test_conv3x3_virtual_rows_many_channels_restage(monkeypatch):
     # 1040 input channels = 65 units: more than one LDS fill of the virtual-row kernel, odd unit count
+    monkeypatch.setenv("EHIP_CONV_SPLIT", "-")   # (a layer of so few values would share K out)
     res = run_and_compare(Layer(1, 1040, 48, 9, k=3, pad=1, out_type=ol.S8, seed=91, w_sigma=0.02))
     assert res["conv"].kernel_name.startswith("k_conv3x3v_u8s8")
 
@@ -382,6 +383,7 @@ def test_direct_kxk_strided(out_type, n, ic, oc, hw, k, pad, stride, out_hw):
 ])
 def test_direct_3x3_stride2_phase_planes(variant, n, ic, oc, hw, pad, out_hw, monkeypatch):
     """3x3 stride 2 through the 3x3 kernel: the staged input as four phase planes, every tile variant, every output type"""
+    monkeypatch.setenv("EHIP_CONV_SPLIT", "-")
     if variant:
         monkeypatch.setenv("EHIP_CONV3X3V_VARIANT", variant)
     for out_type in (ol.U8, ol.S8, ol.F32, ol.S32):
@@ -399,7 +401,7 @@ def test_direct_3x3_stride2_channels_shared_out(variant, n, ic, oc, hw, out_type
     for shared in ("1", "0"):
         monkeypatch.setenv("EHIP_CONV3X3V_SHARED", shared)
         res = run_and_compare(Layer(n, ic, oc, hw, k=3, pad=1, stride=2, out_type=out_type, seed=195 + ic + hw))
-        assert "s2" in res["conv"].kernel_name
+        assert res["conv"].kernel_name.startswith("k_conv3x3v_u8s8") and res["conv"].kernel_name.endswith(",s2,shared>" if shared == "1" else ",s2>")
 
 
 def test_direct_3x3_stride2_phase_planes_can_be_switched_off(monkeypatch):
@@ -418,11 +420,15 @@ def test_direct_3x3_stride2_phase_planes_can_be_switched_off(monkeypatch):
     (1, 24, 16, 11, 5, 2, 2, None),
     (2, 16, 16, 8, 3, 0, 1, None),      # no padding: one class, plain shift
 ])
-def test_direct_zero_point_with_padding(out_type, n, ic, oc, hw, k, pad, stride, out_hw):
-    res = run_and_compare(Layer(n, ic, oc, hw, k=k, pad=pad, stride=stride, out_type=out_type, seed=140 + k + stride,
-                                out_hw=out_hw, in_z=128.0, with_relu=(out_type != ol.F32)))
-    if pad or out_hw:
-        assert res["conv"].kernel_name.startswith("k_conv_fewch" if ic <= 4 else "k_gemm_u8s8")
+def test_direct_zero_point_with_padding(out_type, n, ic, oc, hw, k, pad, stride, out_hw, monkeypatch):
+    # (the general kernel, and the one that shares K out)
+    for split in ("-", "0") if ic > 4 else ("",):
+        monkeypatch.setenv("EHIP_CONV_SPLIT", split)
+        res = run_and_compare(Layer(n, ic, oc, hw, k=k, pad=pad, stride=stride, out_type=out_type, seed=140 + k + stride,
+                                    out_hw=out_hw, in_z=128.0, with_relu=(out_type != ol.F32)))
+        if pad or out_hw:
+            assert res["conv"].kernel_name.startswith("k_conv_fewch" if ic <= 4 else "k_gemm_u8s8")
+            assert ("_split" in res["conv"].kernel_name) == (split == "0")
 
 
 # few output values: K shared out among the waves of a workgroup
@@ -446,8 +452,8 @@ def test_direct_k_shared_out(form, out_type, nhwc, in_z, n, ic, oc, hw, k, pad, 
     (2, 64, 32, 14, 5, 1, False, "k_gemm_u8s8_split<32,32>"), (1, 32, 32, 14, 3, 1, True, ""), (8, 64, 64, 28, 5, 1, False, "k_gemm_u8s8_split<32,64>"),
     (16, 64, 64, 28, 5, 1, False, "k_gemm_u8s8_split<64,64>"), (32, 64, 64, 28, 5, 1, False, "k_gemm_u8s8_split<64,128>"), (64, 64, 64, 28, 5, 1, False, ""),
     (32, 64, 32, 28, 5, 1, False, "k_gemm_u8s8_split<32,128>"),
-    (2, 256, 64, 14, 3, 1, False, "k_conv3x3v_u8s8_split<32,32>"), (2, 128, 64, 14, 3, 1, False, ""), (2, 256, 64, 14, 3, 2, False, "k_conv3x3v_u8s8_split<32,32,s2>"),
-    (10, 512, 256, 14, 3, 1, False, "k_conv3x3v_u8s8_split<32,64>"), (10, 256, 256, 14, 3, 1, False, "")])
+    (2, 256, 64, 14, 3, 1, False, "k_gemm_u8s8_split<32,32>"), (2, 128, 64, 14, 3, 1, False, ""), (2, 256, 64, 14, 3, 2, False, "k_gemm_u8s8_split<32,32>"),
+    (10, 512, 256, 14, 3, 1, False, "k_gemm_u8s8_split<32,64>"), (10, 256, 256, 14, 3, 1, False, "")])
 def test_direct_k_shared_out_choice(n, ic, oc, hw, k, stride, nhwc, split):
     res = run_and_compare(Layer(n, ic, oc, hw, k=k, pad=k // 2, stride=stride, out_type=ol.S8, seed=250 + k + ic, in_nhwc=nhwc))
     assert res["conv"].kernel_name == split if split else "_split" not in res["conv"].kernel_name

@@ -870,6 +870,24 @@ def test_wino_whole_choice(tile, ic, oc, n, hw, whole, monkeypatch):
     assert int((outs[0] != 0).sum()) > outs[0].numel() // 8 and torch.equal(outs[0], outs[1])
 
 
+@pytest.mark.parametrize("tile,in_type,n,ic,hw,env,kernel", [
+    (6, ol.F32, 2, 64, 14, "", "floats"), (6, ol.F32, 2, 64, 14, "EHIP_WINO_BUF_GATHER", "u8"), (5, ol.F32, 2, 64, 14, "", "u8"), (4, ol.F32, 2, 64, 14, "", "u8"),
+    (6, ol.U8, 2, 64, 14, "", "codes_short"), (6, ol.U8, 70, 256, 28, "", "codes"), (6, ol.U8, 2, 64, 14, "EHIP_WINO_SHORT", "codes"),
+    (5, ol.U8, 16, 64, 28, "", "codes_short"), (4, ol.U8, 2, 64, 14, "", "codes_short"), (4, ol.U8, 40, 64, 28, "", "codes"),
+    (6, ol.U8, 2, 64, 14, "EHIP_WINO_WIDE_GATHER", "u8"), (6, ol.U8, 2, 64, 14, "EHIP_WINO_FUSED", "u8")])
+def test_wino_input_transform_is_named(tile, in_type, n, ic, hw, env, kernel, monkeypatch):
+    """the handle's name says which form of the input transform runs"""
+    E = pkg()
+    if env:
+        monkeypatch.setenv(env, "0")
+    d = E.make_desc(n, ic, 64, hw, hw, 3, 3, 1, algorithm=E.CONV_WINOGRAD, input_type=in_type, output_type=E.F32 if in_type == ol.F32 else E.S8,
+                    input_quant=(1.0 if in_type == ol.F32 else 1.0 / 255.0, 0.0), tile_size=tile, execution_mode=0xa161,
+                    wino_tinput_quant=(22.0 / 255.0, 104.0))
+    conv = E.Conv(d)
+    conv.prepare(dev(np.zeros((4, ic // 16, 3, 3, 16, 16), f32)), dev(np.zeros(64, f32)))
+    assert conv.kernel_name.split(" | ")[-1].startswith("k_wino_trans_input_%s + " % kernel)
+
+
 # ---- about one round of workgroups: the columns of the positions shared out among the waves ----------------
 @pytest.mark.parametrize("form", ["0", "1", "2"])
 @pytest.mark.parametrize("tile", [6, 5, 4])
