@@ -131,9 +131,10 @@ def build(verbose=True, jobs=8, incremental=False):
     if verbose:
         print(" ".join(cmd), flush=True)
     subprocess.check_call(cmd)
-    # the address arithmetic of a kernel that reads past no buffer, walked by the CPU tests (host code only)
+    # address arithmetic that keeps kernels from reading past a buffer, walked by the CPU tests (host code only)
     cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-shared", "-fPIC", "-I" + CSRC,
-           os.path.join(ROOT, "tests", "cxx", "conv_split_check.cpp"), "-o", os.path.join(objdir, "libconv_split_check.so")]
+           os.path.join(ROOT, "tests", "cxx", "conv_split_check.cpp"), os.path.join(ROOT, "tests", "cxx", "sum_operand_check.cpp"),
+           "-o", os.path.join(objdir, "libreads_check.so")]
     if verbose:
         print(" ".join(cmd), flush=True)
     subprocess.check_call(cmd)

@@ -258,7 +258,7 @@ __global__ __launch_bounds__(kBlock, 1) void k_gemm1x1_res(EHIP_RES_HEAD, void *
 #pragma unroll
       for (int mt = 0; mt < TM; ++mt) {
         const bool ok = pv[nt] && oc0 + 16 * lh + 32 * mt < oc_real;
-        old[mt][nt] = *reinterpret_cast<const v4i *>(ok ? cell[nt] + (size_t)mt * tile_stride : cell[nt]);
+        old[mt][nt] = *reinterpret_cast<const v4i *>(sum_operand(cell[nt], mt * tile_stride, ok, a.ep.comp));
       }
     }
   }

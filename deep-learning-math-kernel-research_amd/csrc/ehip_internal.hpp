@@ -8,6 +8,7 @@
 #include <string>
 
 #include "euler_hip.h"
+#include "ehip_sum_at.hpp"
 
 namespace ehip {
 
@@ -786,7 +787,7 @@ __device__ __forceinline__ void lean_store_typed(const Epilogue &ep, const v16i 
           old[mt] = old_in[mt][nt];
         } else {
           const bool ok = pvalid[nt] && oc_first + 32 * mt < oc_real;
-          old[mt] = *reinterpret_cast<const v4i *>(ok ? cell[nt] + mt * tile_stride : cell[nt]);
+          old[mt] = *reinterpret_cast<const v4i *>(sum_operand(cell[nt], mt * tile_stride, ok, ep.scale));
         }
       }
     }

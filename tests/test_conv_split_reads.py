@@ -7,14 +7,14 @@ import os
 import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-LIB = os.path.join(ROOT, "deep-learning-math-kernel-research_amd", "build", "libconv_split_check.so")
+LIB = os.path.join(ROOT, "deep-learning-math-kernel-research_amd", "build", "libreads_check.so")
 
 
 @pytest.mark.parametrize("nhwc", [0, 1])
 @pytest.mark.parametrize("n,ic2,ih,iw,k,stride,pad", [
     (1, 1, 8, 8, 3, 1, 1), (2, 3, 11, 9, 5, 2, 2), (3, 5, 9, 7, 7, 1, 3), (1, 7, 13, 13, 3, 2, 0), (2, 2, 6, 7, 3, 1, 1), (1, 4, 5, 5, 5, 1, 2)])
 def test_split_kernel_reads(nhwc, n, ic2, ih, iw, k, stride, pad):
-    assert os.path.exists(LIB), "libconv_split_check.so is not built (python -c 'import __graft_entry__ as g; g.build()')"
+    assert os.path.exists(LIB), "libreads_check.so is not built (python -c 'import __graft_entry__ as g; g.build()')"
     lib = ctypes.CDLL(LIB)
     lib.conv_split_check.restype = ctypes.c_longlong
     oh, ow = ((d + 2 * pad - k) // stride + 1 for d in (ih, iw))

@@ -196,6 +196,21 @@ def test_conv1x1_every_kernel_variant(variant, monkeypatch):
     assert res["conv"].kernel_name.startswith("k_gemm_u8s8")
 
 
+@pytest.mark.parametrize("env,n,ic,oc,hw,out_type,out_nhwc,kernel", [
+    ("", 2, 64, 1040, 37, ol.U8, False, "k_gemm_smallk_lean"), ("", 3, 32, 560, 21, ol.S8, True, "k_gemm_smallk_lean"),
+    ("EHIP_LEAN_EPILOGUE=0", 2, 64, 1040, 21, ol.S8, False, "k_gemm_smallk"), ("EHIP_GEMM_VARIANT=2", 2, 144, 272, 19, ol.U8, False, "k_gemm_u8s8"),
+    ("EHIP_GEMM1X1_RES=4", 2, 256, 272, 19, ol.S8, False, "k_gemm1x1_res"), ("EHIP_GEMM1X1_WRES=1", 1, 256, 272, 19, ol.S8, True, "k_gemm1x1_wres")])
+def test_conv1x1_sum_with_channels_that_fill_up(env, n, ic, oc, hw, out_type, out_nhwc, kernel, monkeypatch):
+    """the in-place sum where many of a workgroup's channels, and pixels, are not there: their operands are not read"""
+    monkeypatch.setenv("EHIP_GEMM1X1_SPLIT", "0")
+    if env:
+        monkeypatch.setenv(*env.split("="))
+        if "VARIANT" in env:
+            monkeypatch.setenv("EHIP_GEMM1X1_RES", "0")
+    res = run_and_compare(Layer(n, ic, oc, hw, out_type=out_type, with_sum=True, out_nhwc=out_nhwc, seed=420 + ic + oc + hw))
+    assert res["conv"].kernel_name.startswith(kernel)
+
+
 # layers with at most 128 input channels take the weights-in-registers kernel
 @pytest.mark.parametrize("out_type", [ol.S32, ol.U8, ol.S8, ol.F32])
 @pytest.mark.parametrize("n,ic,oc,hw,stride,nhwc", [(2, 64, 256, 9, 1, False), (3, 32, 64, 7, 1, False), (1, 128, 512, 6, 1, True),
