@@ -96,7 +96,7 @@ bool wino_whole_applies(const WinoArgs &w, const WinoFusedArgs &f)
   if (env && env[0] == '1') return true;
   // (a switch that asks for a form of the separate stages asks for the stages)
   for (const char *k : {"EHIP_WINO_LANES", "EHIP_WINO_LANES_WRES", "EHIP_WINO_LANES_SLOTS", "EHIP_WINO_LANES_WAVES", "EHIP_WINO_RING",
-                        "EHIP_WINO_BUF_GATHER", "EHIP_WINO_WIDE_GATHER"})
+                        "EHIP_WINO_COLS", "EHIP_WINO_BUF_GATHER", "EHIP_WINO_WIDE_GATHER", "EHIP_WINO_SHORT"})
     if (getenv(k)) return false;
   return wino_whole_pays(f.tile, nks, (f.t + 15) / 16, f.oc2);
 }

@@ -870,6 +870,24 @@ def test_wino_whole_choice(tile, ic, oc, n, hw, whole, monkeypatch):
     assert int((outs[0] != 0).sum()) > outs[0].numel() // 8 and torch.equal(outs[0], outs[1])
 
 
+@pytest.mark.parametrize("env,value", [
+    ("EHIP_WINO_LANES", "1"), ("EHIP_WINO_LANES_WRES", "0"), ("EHIP_WINO_LANES_SLOTS", "8"), ("EHIP_WINO_LANES_WAVES", "8"), ("EHIP_WINO_RING", "1"),
+    ("EHIP_WINO_COLS", "1"), ("EHIP_WINO_BUF_GATHER", "1"), ("EHIP_WINO_WIDE_GATHER", "1"), ("EHIP_WINO_SHORT", "0")])
+def test_wino_whole_gives_way(env, value, monkeypatch):
+    """a layer that would run whole runs by stages where a switch asks for a form of theirs"""
+    E = pkg()
+    d = E.make_desc(64, 128, 128, 28, 28, 3, 3, 1, algorithm=E.CONV_WINOGRAD, input_type=E.U8, output_type=E.S8, input_quant=(1.0 / 255.0, 0.0),
+                    tile_size=6, execution_mode=0xa161, wino_tinput_quant=(22.0 / 255.0, 104.0))
+    names = []
+    for asked in (False, True):
+        if asked:
+            monkeypatch.setenv(env, value)
+        conv = E.Conv(d)
+        conv.prepare(dev(np.zeros((8, 8, 3, 3, 16, 16), f32)), dev(np.zeros(128, f32)))
+        names.append(conv.kernel_name)
+    assert names[0].startswith("k_wino_whole | ") and not names[1].startswith("k_wino_whole")
+
+
 @pytest.mark.parametrize("tile,in_type,n,ic,hw,env,kernel", [
     (6, ol.F32, 2, 64, 14, "", "floats"), (6, ol.F32, 2, 64, 14, "EHIP_WINO_BUF_GATHER", "u8"), (5, ol.F32, 2, 64, 14, "", "u8"), (4, ol.F32, 2, 64, 14, "", "u8"),
     (6, ol.U8, 2, 64, 14, "", "codes_short"), (6, ol.U8, 70, 256, 28, "", "codes"), (6, ol.U8, 2, 64, 14, "EHIP_WINO_SHORT", "codes"),
