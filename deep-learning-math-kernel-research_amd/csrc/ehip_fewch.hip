@@ -14,7 +14,7 @@
 //   2. a wave walks over 32-pixel tiles of the strip: a lane's cell is 16 consecutive LDS bytes at
 //      a byte address of any alignment, read as five dwords and shifted into place;
 //   3. kh * nu / 2 MFMAs per tile against the weights in registers, then the shared epilogue.
-// The four waves split into a.wo channel tiles x 4 / a.wo pixel tiles.
+// The four waves split into a.wo channel tiles x 4 / a.wo pixel tiles (three channel tiles: also as four, the last wave without one).
 #include <type_traits>
 
 #include "ehip_internal.hpp"
@@ -538,7 +538,7 @@ __global__ __launch_bounds__(kBlock, KS == 7 ? 2 : 3) void k_conv_fewch_lean(con
       t += 2 * wpn;
     }
   };
-  if (wp >= ntiles) return;
+  if (wp >= ntiles || oc0 >= oc_real) return;   // (a wave without a tile, of pixels or of channels)
   if (a.icl == 4 && (a.stride_w & 1) == 0) walk(std::integral_constant<int, 0>{});
   else if (a.icl == 4) walk(std::integral_constant<int, 1>{});
   else walk(std::integral_constant<int, 2>{});
@@ -590,46 +590,81 @@ hipError_t plan_conv_fewch(LaunchPlan &plan, FewChArgs &a)
   if (!conv_fewch_applies(a.ic, a.kh, a.kw)) return hipErrorInvalidValue;
   a.lrow = conv_fewch_row_pitch(a.icl, a.kw, a.iw, a.ow, a.stride_w, a.pad_l);
   const int octiles = up(a.oc2 * 16, 32) / 32;   // <= ocpp / 32
+  const int ks = (a.cells + 1) / 2;
+  // LDS of a workgroup's strip and tables of shift rows (0: the tables do not fit; see tab_lds)
+  auto lds_of = [&](int r, int wo) -> size_t {
+    const size_t strip = (size_t)((r - 1) * a.stride_h + a.kh) * a.lrow + 32;
+    if (!a.ep.shift_tab) return strip;
+    const size_t tab = (size_t)(r + a.ow + a.nclass * wo * 32) * 4;
+    return strip + tab <= 48 * 1024 ? (size_t)up((int)strip, 16) + tab : 0;
+  };
+  static int n_cu = 0;
+  if (!n_cu) {
+    int dev = 0, v = 0;
+    if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0)
+      n_cu = v;
+    else
+      n_cu = 256;
+  }
+  // Strip height (output rows per workgroup) and the waves' split.  A taller strip stages fewer overlap rows per output row;
+  // what it must not do is leave waves without tiles, or put a few workgroups more into the grid than the chip runs at once.
   a.wo = octiles % 4 == 0 ? 4 : octiles % 2 == 0 ? 2 : 1;
-  const int gy = octiles / a.wo, wpn = 4 / a.wo;
-  // Strip height (output rows per workgroup).  A taller strip stages fewer overlap rows per output
-  // row; what it must not do is leave waves without tiles, end in a nearly empty strip, or put a
-  // few workgroups more into the grid than the chip runs at once (they would run alone in a second
-  // round).  All of that goes into one relative cost, minimised over the heights whose rows fit in LDS.
+  const char *env_wo = getenv("EHIP_FEWCH_WO");   // (1 / 2 / 4: channel tiles beside each other)
+  const bool forced_wo = env_wo && (env_wo[0] == '1' || env_wo[0] == '2' || env_wo[0] == '4');
+  if (forced_wo) a.wo = env_wo[0] - '0';
   int rows = 1;
   const char *env = getenv("EHIP_FEWCH_ROWS");
+  double best = 0.0;
   if (env && env[0]) {
     rows = atoi(env);
-  } else {
-    static int n_cu = 0;
-    if (!n_cu) {
-      int dev = 0, v = 0;
-      if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0)
-        n_cu = v;
-      else
-        n_cu = 256;
+  } else if (a.lean) {
+    // The lean kernel: its time in us but for what no choice changes, fitted to 2178 random layers (1x1 to 64 images of 32 to 320 rows
+    // and columns, 16 to 128 channels, 3x3 to 7x7) at 17 heights and three splits each.  Per round of workgroups the chain of one:
+    // its start, the staging (KB of pixels; in nhwc it is hidden) and its tiles one after the other; per workgroup of a CU its share of what
+    // they have in common.  Three channel tiles are best beside each other, with a wave that has none, where one by one they stage
+    // the strip three times and write nhwc pixels 32 bytes at a time.  The choice costs 2 % more
+    // than the best of all.  5x5 s2 3 -> 48 at 256 x 256, N = 18 one row 19.2, five 13.2 us; 3x3 s2 3 -> 32, N = 40 one 18.6, eleven 10.8;
+    // 7x7 s2 3 -> 96, N = 4 one 16.2, four 9.6.  7293 other layers: 8 % faster than this kernel's predecessor (three workgroups a CU instead
+    // of two, tiles in phases) with its rule; 201 of them are 5 % or more behind it, most with three channel tiles at stride 1.
+    for (int wo = 1; wo <= 4; wo *= 2) {
+      if (forced_wo ? wo != a.wo : wo >= 2 * octiles) continue;
+      const int groups = (octiles + wo - 1) / wo, waves = 4 / wo;
+      for (int r = 1; r <= a.oh && r <= 32; ++r) {
+        const int nrows_in = (r - 1) * a.stride_h + a.kh;
+        if ((size_t)nrows_in * a.lrow + 32 > 40 * 1024) break;
+        const size_t lds = lds_of(r, wo);
+        if (!lds) break;
+        // resident workgroups of a CU: registers, LDS
+        int resident = ks <= 2 ? 4 : ks <= 5 ? 3 : 2;
+        const int by_lds = (int)((160 * 1024) / lds);
+        if (by_lds < resident) resident = by_lds;
+        const long long wgs = (long long)a.n * ((a.oh + r - 1) / r) * groups;
+        const double per_cu = (double)((wgs + n_cu - 1) / n_cu), rounds = (double)(long long)((per_cu + resident - 1) / resident);
+        const int tiles = ((r * a.ow + 31) / 32 + waves - 1) / waves;   // of a wave
+        const double staged = nrows_in * a.iw / 1024.0;
+        double cost = rounds * (0.94 + (a.in_nhwc ? 0.0 : 0.28 * staged) + tiles * (0.206 + 0.0077 * ks))
+            + per_cu * (0.42 + (a.in_nhwc ? 0.216 : 0.391) * staged + 0.0064 * ks * tiles);
+        if (a.out_nhwc && groups > 1) cost += 0.064e-6 * (double)a.n * a.oh * a.ow * a.oc2 * 16;   // (lines in pieces)
+        if (best == 0.0 || cost < best) { best = cost; rows = r; a.wo = wo; }
+      }
     }
-    double best = 0.0;
+  }
+  const int gy = (octiles + a.wo - 1) / a.wo, wpn = 4 / a.wo;
+  if (best == 0.0 && !(env && env[0])) {
+    // The general kernel: one relative cost
     for (int r = 1; r <= a.oh && r <= 32; ++r) {
       const int nrows_in = (r - 1) * a.stride_h + a.kh;
       const size_t dyn = (size_t)nrows_in * a.lrow + 32;
       if (dyn > 40 * 1024) break;
-      // workgroups of 4 waves resident per CU: registers (3 waves per SIMD; the lean kernel 4 with two operands,
-      // 2 with seven), LDS (the general kernel's 16 KB static exchange patch + the rows).  3x3 s2 3 -> 32 at 224 x 224, N = 64: strips of 7 rows (4 workgroups per CU) 12.0 us, of 10 rows
-      // (3 per CU) 12.6 us.
-      const int ks = (a.cells + 1) / 2;
-      int resident = !a.lean ? 3 : ks <= 2 ? 4 : ks <= 5 ? 3 : 2;
-      const int by_lds = (int)((160 * 1024) / ((a.lean ? 0 : 16 * 1024) + dyn));
+      // workgroups of 4 waves resident per CU: registers (3 waves per SIMD), LDS (the 16 KB static exchange patch + the rows)
+      int resident = 3;
+      const int by_lds = (int)((160 * 1024) / (16 * 1024 + dyn));
       if (by_lds < resident) resident = by_lds < 1 ? 1 : by_lds;
       const double slots = (double)n_cu * resident;
       const double wgs = (double)a.n * ((a.oh + r - 1) / r) * gy;
       const double rounds = (double)(long long)((wgs + slots - 1) / slots);
       const int tiles = (r * a.ow + 31) / 32;
-      // idle slots of the last round; with one round, idle CUs (the lean kernel keeps a CU almost as busy with two workgroups as with
-      // three: 5x5 s2 3 -> 96 at 224 x 224, N = 24: two of 16 rows 16.5 us, three of 12 18.6)
-      double idle = rounds * slots / wgs;
-      if (a.lean && rounds == 1.0 && wgs > n_cu && wgs <= 2.0 * n_cu && resident == 3) idle = 1.08 * 2.0 * n_cu / wgs;
-      const double cost = idle
+      const double cost = rounds * slots / wgs                                    // idle slots of the last round
           * ((tiles + wpn - 1) / wpn * wpn * 32.0 / (r * a.ow))                  // idle waves and lanes of the last tiles
           * ((double)((a.oh + r - 1) / r) * r / a.oh)                             // rows of the last strip below the image
           * (1.0 + 0.2 * nrows_in / (r * a.stride_h));                            // staging, relative to the tile work
@@ -644,10 +679,10 @@ hipError_t plan_conv_fewch(LaunchPlan &plan, FewChArgs &a)
   size_t lds = (size_t)a.nrows_in * a.lrow + 32;
   a.tab_lds = 0;
   if (a.ep.shift_tab) {
-    const size_t tab = (size_t)(rows + a.ow + a.nclass * a.wo * 32) * 4;
-    if (lds + tab <= 48 * 1024) {
+    const size_t with_tables = lds_of(rows, a.wo);
+    if (with_tables) {
       a.tab_lds = (int)(up((int)lds, 16) / 4);   // dword offset of the tables
-      lds = (size_t)a.tab_lds * 4 + tab;
+      lds = with_tables;
     }
   }
   if (lds > 48 * 1024 + 64 || (long long)a.nrows_in * a.lrow >= (1ll << 30) ||
@@ -659,7 +694,6 @@ hipError_t plan_conv_fewch(LaunchPlan &plan, FewChArgs &a)
   a.lrow16_magic = div_magic(a.lrow / 16 > 0 ? a.lrow / 16 : 1);
   if ((long long)a.nrows_in * (a.lrow / 4) * (a.lrow / 4) >= (1ll << 32) || (long long)a.nrows_in * a.iw * a.iw >= (1ll << 32))
     return hipErrorInvalidValue;
-  const int ks = (a.cells + 1) / 2;
   void (*kern)(const FewChArgs *, const uint8_t *, void *) = ks <= 2 ? k_conv_fewch_u8s8<2> : ks == 3 ? k_conv_fewch_u8s8<3> : ks == 4 ? k_conv_fewch_u8s8<4>
       : ks == 5 ? k_conv_fewch_u8s8<5> : k_conv_fewch_u8s8<7>;
   const char *name = "k_conv_fewch_u8s8";

@@ -565,6 +565,23 @@ def test_direct_few_input_channels_lean_walk(oc, rows, ic, k, stride, in_z, monk
     assert res["conv"].kernel_name == "k_conv_fewch_lean"
 
 
+@pytest.mark.parametrize("wo", ["1", "2", "4"])
+@pytest.mark.parametrize("lean_kernel", ["0", "1"])
+@pytest.mark.parametrize("oc,k,stride,in_z,nhwc", [(80, 7, 2, 128.0, True), (96, 3, 2, 0.0, False), (16, 7, 2, 0.0, True), (160, 5, 1, 128.0, False), (272, 3, 1, 7.0, True)])
+def test_direct_few_input_channels_waves_split(wo, lean_kernel, oc, k, stride, in_z, nhwc, monkeypatch):
+    """one, two and four channel tiles beside each other, where the last waves have none: one, three, five and nine tiles"""
+    monkeypatch.setenv("EHIP_FEWCH_WO", wo)
+    monkeypatch.setenv("EHIP_FEWCH_LEAN_KERNEL", lean_kernel)
+    run_and_compare(Layer(2, 3, oc, 19 * stride, k=k, pad=k // 2, stride=stride, out_type=ol.S8, seed=310 + oc + k, in_z=in_z, in_nhwc=nhwc, out_nhwc=nhwc))
+
+
+@pytest.mark.parametrize("n,ic,oc,hw,k,in_z", [(2, 3, 96, 224, 7, 128.0), (1, 1, 48, 320, 7, 200.0), (2, 3, 96, 300, 7, 0.0)])
+def test_direct_few_input_channels_tables_fit(n, ic, oc, hw, k, in_z):
+    """the strip is chosen so that the tables of shift rows find room beside it, and the lean kernel runs"""
+    res = run_and_compare(Layer(n, ic, oc, hw, k=k, pad=k // 2, stride=2, out_type=ol.U8, seed=330 + oc + hw, in_z=in_z, in_nhwc=True, out_nhwc=True))
+    assert res["conv"].kernel_name == "k_conv_fewch_lean"
+
+
 def test_direct_few_input_channels_tall_strip_of_cells(monkeypatch):
     """blocked input whose strip is staged sixteen cells a thread at a time, the last batch in part"""
     monkeypatch.setenv("EHIP_FEWCH_ROWS", "40")
