@@ -489,6 +489,31 @@ def test_direct_k_shared_out_lines(n, ic, oc, hw, k, split):
     assert conv.kernel_name.endswith("_split" + split) if split else "_split" not in conv.kernel_name
 
 
+@pytest.mark.parametrize("ic,split", [(16384, True), (16400, False)])
+def test_direct_k_shared_out_largest(ic, split, monkeypatch):
+    """inputs of 2147.0 and 2149.1 MB, on both sides of 2^31 bytes; the same output as by the general kernel"""
+    import torch
+    E = pkg()
+    g = torch.Generator(device="cuda").manual_seed(ic)
+    x = torch.randint(0, 256, (1, 362, 362, ic), dtype=torch.uint8, device="cuda", generator=g)
+    w = torch.randn((2, ic // 16, 3, 3, 16, 16), device="cuda", generator=g) * 0.04
+    bias = torch.zeros(32, device="cuda")
+    d = E.make_desc(1, ic, 32, 362, 362, 3, 3, 1, 2, algorithm=E.CONV_DIRECT, input_type=E.U8, output_type=E.S8, with_relu=False,
+                    input_quant=(1.0 / 255.0, 0.0), output_quant=(0.2, 0.0))
+    d.input_fmt = E.NHWC
+    outs = []
+    for env in ("", "-"):
+        if env:
+            monkeypatch.setenv("EHIP_CONV_SPLIT", env)
+        conv = E.Conv(d)
+        conv.prepare(w, bias)
+        assert ("_split<32,128>" in conv.kernel_name) == (split and not env)
+        outs.append(torch.zeros((1, 2, 181, 181, 16), dtype=torch.int8, device="cuda"))
+        conv.execute(outs[-1], x, None, bias)
+    torch.cuda.synchronize()
+    assert bool((outs[0][:, :, -1] != 0).any()) and torch.equal(outs[0], outs[1])
+
+
 # at most four input channels (first layers; the reference feeds them 3-channel nhwc,
 # scripts/best_configs/resnetv1_5-n64-clx-1s-int8.sh:12): 16 / ic pixels per operand cell, a kernel row
 # is ceil(kw / (16 / ic)) cells, input rows staged compactly in LDS

@@ -839,6 +839,31 @@ def test_wino_transformed_floats(n, ic, h, w, nhwc, data, monkeypatch):
         assert data != "under range" or (tin == 255).sum() > 4   # (else no wave converts twice)
 
 
+@pytest.mark.parametrize("n,floats", [(4032, True), (4033, False)])
+def test_wino_transformed_floats_largest(n, floats, monkeypatch):
+    """the largest f32 tensor whose addresses the two-channel form makes by additions that may leave the buffer (0x3f000000 bytes: 4032
+    images of 64 x 64 x 16), and the next; the same output by the kernel with the plain gather"""
+    import torch
+    E = pkg()
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x = torch.rand((n, 1, 64, 64, 16), device="cuda", generator=g)
+    w = torch.randn((1, 1, 3, 3, 16, 16), device="cuda", generator=g) * 0.02
+    bias = torch.zeros(16, device="cuda")
+    d = E.make_desc(n, 16, 16, 64, 64, 3, 3, 1, algorithm=E.CONV_WINOGRAD, input_type=E.F32, output_type=E.F32, input_quant=(1.0, 0.0),
+                    tile_size=6, execution_mode=0xa161, wino_tinput_quant=(22.0 / 255.0, 104.0))
+    outs = []
+    for gather in ("", "0"):
+        if gather:
+            monkeypatch.setenv("EHIP_WINO_BUF_GATHER", gather)
+        conv = E.Conv(d)
+        conv.prepare(w, bias)
+        assert conv.kernel_name.startswith("k_wino_trans_input_%s + " % ("floats" if floats and not gather else "u8"))
+        outs.append(torch.zeros(x.shape, device="cuda"))
+        conv.execute(outs[-1], x, None, bias)
+    torch.cuda.synchronize()
+    assert bool((outs[0][-1] != 0).any()) and torch.equal(outs[0].view(torch.int32), outs[1].view(torch.int32))
+
+
 @pytest.mark.parametrize("tile,ic,oc,n,hw,whole", [
     (6, 64, 64, 32, 56, True), (6, 64, 64, 64, 56, False), (6, 64, 64, 2, 28, False), (6, 128, 128, 64, 28, True), (6, 128, 128, 160, 28, False),
     (6, 192, 192, 20, 28, False), (6, 192, 192, 64, 28, True), (6, 256, 64, 64, 28, True), (6, 256, 256, 64, 14, False), (5, 128, 256, 40, 28, True),
@@ -944,3 +969,28 @@ def test_wino_fused_columns_choice(tile, n, ic, oc, hw, form, monkeypatch):
     conv = E.Conv(d)
     conv.prepare(dev(np.zeros((oc // 16, ic // 16, 3, 3, 16, 16), f32)), dev(np.zeros(oc, f32)))
     assert (conv.kernel_name.endswith("_cols" + form) if form else "_cols" not in conv.kernel_name)
+
+
+@pytest.mark.parametrize("hw,cols", [(340, True), (344, False)])
+def test_wino_fused_columns_largest(hw, cols, monkeypatch):
+    """transformed inputs of 2130 and 2158 MB, on both sides of 2^31 bytes: 8192 channels, 226 and 229 units of 32 tiles; the same
+    output as by the kernels before"""
+    import torch
+    E = pkg()
+    g = torch.Generator(device="cuda").manual_seed(hw)
+    x = torch.randint(0, 256, (1, 512, hw, hw, 16), dtype=torch.uint8, device="cuda", generator=g)
+    w = torch.randn((2, 512, 3, 3, 16, 16), device="cuda", generator=g) * 0.02
+    bias = torch.zeros(32, device="cuda")
+    d = E.make_desc(1, 8192, 32, hw, hw, 3, 3, 1, algorithm=E.CONV_WINOGRAD, input_type=E.U8, output_type=E.S8, input_quant=(1.0 / 255.0, 0.0),
+                    tile_size=6, execution_mode=0xa161, wino_tinput_quant=(22.0 / 255.0, 104.0), output_quant=(0.05, 0.0))
+    outs = []
+    for env in ("", "-"):
+        if env:
+            monkeypatch.setenv("EHIP_WINO_COLS", env)
+        conv = E.Conv(d)
+        conv.prepare(w, bias)
+        assert ("_cols<32,32>" in conv.kernel_name) == (cols and not env)
+        outs.append(torch.zeros((1, 2, hw, hw, 16), dtype=torch.int8, device="cuda"))
+        conv.execute(outs[-1], x, None, bias)
+    torch.cuda.synchronize()
+    assert bool((outs[0][:, :, -4:] != 0).any()) and torch.equal(outs[0], outs[1])
