@@ -782,9 +782,9 @@ hipError_t plan_conv3x3v(LaunchPlan &plan, const Conv3x3Args &a0, int n, int var
   }
   // Stride 2 with more than one fill (over 128 input channels) and a CU for every workgroup: two fills at a time by eight
   // waves.  A fill is a trip to memory that nothing covers, and the 36 taps behind it run at one wave per SIMD.  With other tensors
-  // on every call, one at a time / two: 512 -> 512 at 14 x 14, N = 1 18.0 / 14.7 us, N = 64 (256 workgroups) 19.0 / 16.9; 256 -> 256 at 28 x 28, N = 1
-  // 10.5 / 9.1, N = 16 (128) 10.3 / 9.0, N = 64 (512 workgroups, two on a CU either way) 18.3 / 20.0.  Stride 1 stages everything in
-  // one fill: 512 -> 512 at 14 x 14, N = 1 10.1 / 9.8, 256 -> 256 6.2 / 7.0, not taken.
+  // on every call, one at a time / two: 512 -> 512 at 14 x 14, N = 64 (256 workgroups) 19.0 / 16.9 us; 256 -> 256 at 28 x 28,
+  // N = 16 (128) 10.3 / 9.0, N = 64 (512 workgroups, two on a CU either way) 18.3 / 20.0.  (One image of them shares all of K out:
+  // conv_split_pick.)  Stride 1 stages everything in one fill: 512 -> 512 at 14 x 14, N = 1 10.1 / 9.8, 256 -> 256 6.2 / 7.0, not taken.
   int threads = kBlock;
   size_t lds = lds_bytes;
   const char *shared_env = getenv("EHIP_CONV3X3V_SHARED");   // (0 / 1: never / wherever it can run)

@@ -12,7 +12,7 @@ namespace ehip {
 // Such a layer is bound by one workgroup's chain: 64 x 64 results walk K = taps x channels in fills of 64 to 128 that pass the LDS with
 // a barrier each, 0.11 us a step of 32 (7x7, 480 -> 16 at 34 x 34, N = 2: 735 steps, 83 us, on 37 CUs).  Here the eight waves of a
 // workgroup take an eighth of the steps each, with their operands straight from memory six to ten steps ahead, no barrier and
-// no LDS until the sums meet: the chain is an eighth, and what is left is the L1's 98 GB/s (2 KB a step: 735 steps 15 us).  A tap is
+// no LDS until the sums meet: the chain is an eighth, and what is left is the stream into a CU (2 KB a step: 735 steps 15 us, 98 GB/s; loads alone get 115 from the L2).  A tap is
 // the same for a wave's lanes, so the pixels' addresses are worked out once per tap and a step adds a scalar.  Taps outside the
 // image are read past the end of the buffer, which gives code 0 as the padding does.  The sums are integers: exact in any order.
 // us, with other tensors in turn: that layer 83.1 -> 19.1; 7x7 380 -> 256 at 14 x 14, N = 4 84.0 -> 14.5; 5x5 s2 160 -> 32 at 14 x 14, N = 5 21.3 -> 6.4; 5x5 256 ->

@@ -140,10 +140,11 @@ __global__ __launch_bounds__(kBlock, 3) void k_wino_trans_input_floats(const Win
 // and the finished codes take the place of the pixels, position by position, so that they leave by 16 bytes a lane.
 // What bounds it is the issue of vector instructions: 1250 per wave and 16 tiles x 16 channels, of which conversions, minima
 // and byte packs issue at 4.35 clocks and multiply-adds, with two or more waves on a SIMD, at 2.6.  So the instructions that
-// are not the transform's own went (exchanges, address arithmetic, two of three stores), and the registers (91, from 163)
-// let five waves share a SIMD instead of three.
-// By execute_stages, N = 64, before -> now: 256 channels at 56 x 56 36.0 -> 30.5 us, 512 at 28 x 28 21.6 -> 19.3, 64 at 56 x 56
-// 15.7 -> 13.4, 128 at 28 x 28 8.8 -> 8.1.
+// are not the transform's own went (exchanges, address arithmetic, two of three stores), and four waves share a SIMD
+// instead of three (91 registers, from 163, would let five; at tile size 6 the 37 KB of LDS of a workgroup are what counts).
+// The transform alone by execute_stages, N = 64, before -> now: 256 channels at 56 x 56 40.8 -> 31.2 us, 512 at 28 x 28 23.1 -> 20.9 (tile
+// size 5 33.2 -> 25.0, 4 29.1 -> 22.8).  Run over and over it finds its tensors in the caches; with the fused stage in between, which itself takes
+// the same after either form, the two together gain 118.4 -> 114.5, 93.6 -> 93.2, 119.4 -> 113.6 and 124.8 -> 119.6.
 template <int A>
 __global__ __launch_bounds__(kBlock, 4) void k_wino_trans_input_codes(const WinoArgs *rest, const void *in)
 {
@@ -178,7 +179,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_wino_trans_input_codes(const Wino
       *reinterpret_cast<uint4 *>(base + (size_t)(4 * k) * pos + voff) = cells[64 * k + lane];
 }
 
-// The same for layers that give a SIMD less than two waves of it: a workgroup takes 16 tiles of one unit, and each of its four waves
+// The same for layers that give a SIMD less than about three waves of it (see plan_wino_trans_input): a workgroup takes 16 tiles of one unit, and each of its four waves
 // one channel of every quad, so that four times as many waves run a quarter of the instructions each, and the chain from the first load to the last store
 // is as much shorter.  With other tensors on every call, this against the form above: 512 channels at 7 x 7, N = 64 4.8 against 7.3 us, 256 at
 // 14 x 14 6.9 against 8.2 (N = 16 4.0 against 6.3), 128 at 28 x 28 9.0 against 9.8; N = 1 4.0 against 5.1 to 5.9.

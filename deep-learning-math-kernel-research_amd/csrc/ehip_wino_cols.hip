@@ -20,7 +20,7 @@ namespace ehip {
 // it is; what is left of it (A - 2 values) meets the other columns in LDS, and the waves share the rows of the output.  Tile
 // size 4, a two-dimensional formula in the reference, meets as positions.
 // The bytes through the L1 of a CU are what is left: 3 KB for two matrix instructions with 32 channels x 16 tiles a workgroup, 885 KB a CU
-// for 512 -> 512, 256 tiles (15.8 us; the 58 bytes a clock that an L1 delivers would be 6.4).  Both halves of a group of 32 packed rows
+// for 512 -> 512, 256 tiles (15.8 us; the 115 GB/s that a CU gets from its L2 while all of them read would be 7.7).  Both halves of a group of 32 packed rows
 // belong to a workgroup of 32 channels, because a half alone uses half of every cache line: 16.7 against 18.4 us for 16 channels x 32
 // tiles, of the same bytes.  An XCD takes neighbouring groups of channels, not every eighth, for the same reason (13.3 / 12.6).
 // Tried: two k-steps less ahead by the compiler's order of the first loads (17.6 against 15.8: hence the scheduling barriers), twelve

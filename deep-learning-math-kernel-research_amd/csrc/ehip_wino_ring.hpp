@@ -5,7 +5,7 @@
 // runs them per thread (a161, src/elx_int8_conv_wino_xopt.hpp:21-179; src/elx_int8_conv_wino_gemm.cpp:23-205,
 // src/elx_conv_wino_trans_output.cpp:212-423).
 //
-// What bounds it: a CU takes 58 bytes a clock through its L1, so the product of a weight and a tile byte is only as cheap
+// What bounds it: a CU takes 48 bytes a clock from its L2 while all of them do (56 where the L1 has them), so the product of a weight and a tile byte is only as cheap
 // as the block of channels x tiles they are shared in.  With the weights of 16 channels resident (ehip_wino_lanes.hip) a
 // byte of the transformed input feeds 16 products; a workgroup of 64 channels x 64 tiles makes it 32 for both operands, and
 // keeps no more than 16 + 4 running values per output channel and tile in a lane (Fold) instead of all 36 positions,
@@ -420,8 +420,8 @@ __global__ __launch_bounds__(64 * WO * WT, 2) void k_wino_gemm_output_lanes_ring
   wait_all_loads();   // (the requests behind the last stage still write this workgroup's LDS)
 }
 
-// Form 0: 64 channels x 64 tiles, eight waves, one workgroup per CU.  A stage of two k-steps (16 KB) takes the L1 280
-// clocks at its 58 bytes a clock, the matrix cores 134 and the LDS about as long as the L1 (203 clocks of reads beside
+// Form 0: 64 channels x 64 tiles, eight waves, one workgroup per CU.  A stage of two k-steps (16 KB) takes the L1 340
+// clocks at 48 bytes a clock, the matrix cores 134 and the LDS less than the L1 (203 clocks of reads beside
 // the 16 KB coming in).  Form 1: 32 x 32, four waves, two workgroups per CU: twice the operand bytes per product, for
 // layers of few tiles.  Form 2: 32 x 64, four waves, two workgroups per CU that hide each other's transforms and stores,
 // which with 256 input channels weigh more than the operand stream.

@@ -60,6 +60,7 @@ static WholeSplit whole_split(int nks, int blocks, int groups)
 // with four waves, tile size 6 only next to the next round of blocks (two rounds of groups, 260 / 300 / 341 / 378 blocks 1.35 / 1.24 / 1.11 / 1.11); tile
 //   size 5, two rounds, 257 to 319 blocks 1.19 to 1.04, 324 to 522 0.97 to 0.87, three, 258 to 384 1.16 to 1.06, 387 to 398 0.95; tile size 4, three or
 //   four, 128 channels, 259 to 338 blocks 1.11 to 1.05, 359 to 392 0.96 to 0.93, 64 channels 0.82 to 0.92.
+// (Points on either side of a line differ by 2 to 5 %, about what two boxes differ by: nearer than that a line is not known.)
 static bool wino_whole_pays(int A, int nks, int blocks, int groups)
 {
   // blocks from (at most 64 output channels; more) and to, groups of 16 output channels, blocks x groups; by k-steps of 64 input
